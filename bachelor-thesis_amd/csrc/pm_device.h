@@ -140,21 +140,20 @@ __device__ __forceinline__ int32_t pm_key(float x, float inv_h)
 // ulp) corrected to the correctly rounded result by the signs of the residuals
 // x - s' s of its neighbours s' = s -+ 1 ulp -- the expansion the compiler emits
 // for sqrtf at x >= 2^-96, without its scaling of smaller inputs and its
-// special-value fix-up.  Below 2^-96 the hardware result is kept: there
-// q = sqrt(x) / h < 2^-14 for any h > 2^-34, and W(q) = sigma (6 (q^3 - q^2) + 1)
-// rounds to sigma exactly whatever the last bit of the root.
+// special-value fix-up.  Below 2^-96 the residuals may round: the result is
+// then still within an ulp of the hardware's (at 0 the lower neighbour is a NaN
+// and every test fails), there q = sqrt(x) / h < 2^-14 for any h > 2^-34, and
+// W(q) = sigma (6 (q^3 - q^2) + 1) rounds to sigma exactly whatever the last
+// bit of the root.
 __device__ __forceinline__ float pm_sqrt_w(float x)
 {
-    float s = __builtin_amdgcn_sqrtf(x);
-    if (x >= 0x1p-96f) {
-        const float sm = __uint_as_float(__float_as_uint(s) - 1u);
-        const float sp = __uint_as_float(__float_as_uint(s) + 1u);
-        const float rm = __builtin_fmaf(-sm, s, x);
-        const float rp = __builtin_fmaf(-sp, s, x);
-        s = rm <= 0.0f ? sm : s;
-        s = rp > 0.0f ? sp : s;
-    }
-    return s;
+    const float s = __builtin_amdgcn_sqrtf(x);
+    const float sm = __uint_as_float(__float_as_uint(s) - 1u);
+    const float sp = __uint_as_float(__float_as_uint(s) + 1u);
+    const float rm = __builtin_fmaf(-sm, s, x);
+    const float rp = __builtin_fmaf(-sp, s, x);
+    const float t = rm <= 0.0f ? sm : s;
+    return rp > 0.0f ? sp : t;
 }
 
 // Kernel.cpp:16-32 on a squared distance known to be < h^2.
@@ -279,111 +278,168 @@ __device__ __forceinline__ uint32_t pm_cand27(const GridDev &g, float qx, float 
     return cand;
 }
 
-// Same sum as pm_density32, with the in-support candidates compacted through a
-// per-lane LDS buffer before W is evaluated.  A wave walks its rows together;
-// the distance test is cheap and the W evaluation (sqrt, branch, compensated
-// add) then runs over each lane's own short list, so lanes whose candidates are
-// mostly out of support no longer hold the wave in the expensive branch.  The
-// buffer is drained in order, so the summation order -- and the result -- is
-// exactly that of pm_density32.
-//   buf: this lane's slot 0; slot j is buf[j * 64] (lane-interleaved: no bank
-//   conflicts whatever slot each lane is at).
-template <int CAP>
-__device__ __forceinline__ void pm_drain(const GridDev &g, const float *buf, int n, float &s, float &c)
+// ---- the walk through a candidate list ----
+// Same sum as pm_density32, in two steps.  First the lane lists the indices of
+// its stencil's candidates, in order, in its LDS slots: a plane of five rows
+// (one dz) at a time, the next plane's row bounds in flight meanwhile, so the
+// 25 rows cost five load latencies that overlap the listing instead of 50 in a
+// chain.  Then it takes the list four candidates at a time, the next four
+// gathers in flight: rows of different lengths do not idle the other lanes (a
+// wave runs to its longest list, not to each row's longest), and the four W
+// evaluations are independent.  A list that fills up is taken early; the order
+// -- and the result -- is that of pm_density32.
+//   lst: this lane's slot 0; slot j is lst[j * 64] (lane-interleaved: no bank
+//   conflicts); CAP + kListPad slots.
+static constexpr int kListPad = 4;
+
+struct RowPlane {
+    uint32_t b[5], e[5];
+};
+
+// Bounds of the five rows of plane dz; a dropped row gets an empty range (both
+// bounds from one cell).  in = false: no rows (w.base is then a cell whose
+// stencil is inside the grid).
+__device__ __forceinline__ void pm_fine_plane(const GridDev &g, const FineWalk &w, bool in, int dz, RowPlane &P)
 {
-    for (int j = 0; j < n; j++) {
-        float w = pm_W_in(buf[j * 64], g.inv_h, g.sig);
-        pm_neu_add(s, c, w);
+    const float tz = pm_fine_off(dz, w.fz), tz2 = in ? tz * tz : INFINITY;
+    const uint32_t row0 = w.base + (uint32_t)(dz * (int)w.sz);
+#pragma unroll
+    for (int i = 0; i < 5; i++) {
+        const float ty = pm_fine_off(i - 2, w.fy);
+        const float r2 = ty * ty + tz2;
+        const bool kept = r2 < PM_FINE_LIM;
+        int lo = (w.xm2 + r2 < PM_FINE_LIM) ? -2 : ((w.xm1 + r2 < PM_FINE_LIM) ? -1 : 0);
+        int hi = (w.xp2 + r2 < PM_FINE_LIM) ? 3 : ((w.xp1 + r2 < PM_FINE_LIM) ? 2 : 1);
+        lo = kept ? lo : 0;
+        hi = kept ? hi : 0;
+        const uint32_t row = row0 + (uint32_t)((i - 2) * (int)w.sy);
+        P.b[i] = g.fcell_start[row + (uint32_t)lo];
+        P.e[i] = g.fcell_start[row + (uint32_t)hi];
     }
 }
 
-// Distance test of candidate p against q; appends |p - q|^2 to the lane's
-// buffer when it is inside the support.  The store is unconditional (slot n
-// is free and in bounds: the caller keeps n + remaining candidates <= CAP) and
-// only the count depends on the test, so the loop has no branch.
-__device__ __forceinline__ void pm_test_append(const GridDev &g, float4 p, float qx, float qy, float qz, float *buf,
-                                               int &n)
+// Lists the five rows of a plane: n slots are taken; drain(n) takes the listed
+// candidates in order.  Called by any set of lanes; those drain together.
+template <int CAP, class Drain>
+__device__ __forceinline__ void pm_list_plane(const RowPlane &P, uint32_t *lst, int &n, Drain &&drain)
 {
-    float rx = p.x - qx, ry = p.y - qy, rz = p.z - qz;
-    float r2 = (rx * rx + ry * ry) + rz * rz;
-    buf[n * 64] = r2;
-    n += r2 < g.h2 ? 1 : 0;
-}
-
-// UNROLL candidates are loaded before any is tested, so each lane keeps UNROLL
-// independent gathers in flight instead of one dependent load per iteration.
-template <int CAP, int UNROLL>
-__device__ __forceinline__ float pm_density32_lds(const GridDev &g, float qx, float qy, float qz, float *buf,
-                                                  uint32_t &cand, uint32_t &nsup)
-{
-    static_assert(UNROLL >= 1 && UNROLL <= CAP, "unroll");
-    FineWalk fw;
-    float s = 0.0f, c = 0.0f;
-    bool in = pm_fine_begin(g, qx, qy, qz, fw);
-    int n = 0;
-    uint32_t drained = 0;
-    if (in) {
-        _Pragma("unroll 1") for (int dz = -2; dz <= 2; dz++) {
-            const float tz2 = pm_fine_tz2(fw, dz);
-            _Pragma("unroll 1") for (int dy = -2; dy <= 2; dy++) {
-                uint32_t b, e;
-                pm_fine_row(g, fw, dy, dz, tz2, b, e);
-                cand += e - b;
-                if (__ballot(e > b) == 0) continue;         // no lane has candidates in this row
-                if (__ballot(n + (int)(e - b) >= CAP) != 0) {  // some lane might fill the buffer:
-                    pm_drain<CAP>(g, buf, n, s, c);           // all drain together
-                    drained += (uint32_t)n;
-                    n = 0;
-                }
-                if ((int)(e - b) < CAP) {
-                    // groups of UNROLL loads, the last group's unused slots re-reading
-                    // the group's first candidate; slot n stays free for their stores
-                    const int m = (int)(e - b);
-                    const float4 *const p0 = g.fsorted + b;
-                    for (int i = 0; i < m; i += UNROLL) {
-                        float4 v[UNROLL];
+    int mp = 0;
 #pragma unroll
-                        for (int u = 0; u < UNROLL; u++) v[u] = p0[i + u < m ? i + u : i];
+    for (int i = 0; i < 5; i++) mp += (int)(P.e[i] - P.b[i]);
+    if (__ballot(mp != 0) == 0) return;
+    if (__ballot(n + mp > CAP) != 0) {
+        drain(n);
+        n = 0;
+        if (__ballot(mp > CAP) != 0) {        // a plane longer than the list (dense clusters)
+            _Pragma("unroll 1") for (int i = 0; i < 5; i++) {
+                uint32_t b = P.b[0], e = P.e[0];
 #pragma unroll
-                        for (int u = 0; u < UNROLL; u++) {
-                            const float rx = v[u].x - qx, ry = v[u].y - qy, rz = v[u].z - qz;
-                            const float r2 = (rx * rx + ry * ry) + rz * rz;
-                            buf[n * 64] = r2;
-                            n += (i + u < m && r2 < g.h2) ? 1 : 0;
-                        }
-                    }
-                } else {
-                    // a row longer than the buffer (dense clusters hold hundreds of
-                    // particles per row): in chunks that fit, loaded UNROLL at a time
-                    const float4 *p = g.fsorted + b;
-                    const float4 *const pe = g.fsorted + e;
-                    while (p < pe) {
-                        const float4 *const ce = p + (CAP - n) < pe ? p + (CAP - n) : pe;
-                        for (; p + UNROLL <= ce; p += UNROLL) {
-                            float4 v[UNROLL];
-#pragma unroll
-                            for (int u = 0; u < UNROLL; u++) v[u] = p[u];
-#pragma unroll
-                            for (int u = 0; u < UNROLL; u++) pm_test_append(g, v[u], qx, qy, qz, buf, n);
-                        }
-                        for (; p < ce; p++) pm_test_append(g, *p, qx, qy, qz, buf, n);
-                        if (p < pe) { pm_drain<CAP>(g, buf, n, s, c); drained += (uint32_t)n; n = 0; }
-                    }
+                for (int k = 1; k < 5; k++) { b = i == k ? P.b[k] : b; e = i == k ? P.e[k] : e; }
+                while (__ballot(b < e) != 0) {
+                    const int take = min((int)(e - b), CAP - n);
+                    for (int k = 0; k < take; k++) lst[(n + k) * 64] = b + (uint32_t)k;
+                    n += take;
+                    b += (uint32_t)take;
+                    if (__ballot(b < e) != 0) { drain(n); n = 0; }
                 }
             }
+            return;
         }
     }
-    pm_drain<CAP>(g, buf, n, s, c);
-    nsup += drained + (uint32_t)n;
-    return s + c;
+#pragma unroll
+    for (int i = 0; i < 5; i++) {
+        const uint32_t b = P.b[i];
+        const int m = (int)(P.e[i] - b);
+        // four slots at once; those past the row are the next row's
+        uint32_t *const q = lst + n * 64;
+#pragma unroll
+        for (int k = 0; k < 4; k++) q[k * 64] = b + (uint32_t)k;
+        if (__ballot(m > 4) != 0)
+            for (int k = 4; k < m; k++) q[k * 64] = b + (uint32_t)k;
+        n += m;
+    }
 }
 
-template <int CAP, int UNROLL>
-__device__ __forceinline__ float pm_density32_lds(const GridDev &g, float qx, float qy, float qz, float *buf,
-                                                  uint32_t &cand)
+// W on a squared distance (pm_W_in's operations, both branches evaluated).
+__device__ __forceinline__ float pm_W_sel(float r2, float inv_h, float sig)
+{
+    const float q = pm_sqrt_w(r2) * inv_h;
+    const float qq = 1.0f - q, t = q * q;
+    const float a = 2.0f * qq * qq * qq;
+    const float b = 6.0f * (t * q - t) + 1.0f;
+    return sig * (q >= 0.5f ? a : b);
+}
+
+// Takes n listed candidates into the compensated sum (s, c); a slot outside
+// the support adds an exact zero.  s alone is the plain sum.
+__device__ __forceinline__ void pm_list_density(const GridDev &g, const uint32_t *lst, int n, float qx, float qy,
+                                                float qz, float &s, float &c, uint32_t &nsup)
+{
+    if (__ballot(n > 0) == 0) return;
+    float vx[4], vy[4], vz[4];
+    auto load = [&](int i) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const uint32_t l = lst[(i + u) * 64];
+            const float4 *const p = g.fsorted + (i + u < n ? l : 0u);
+            vx[u] = p->x; vy[u] = p->y; vz[u] = p->z;
+        }
+    };
+    load(0);
+    int i = 0;
+    while (true) {
+        float w[4];
+        float r2[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const float rx = vx[u] - qx, ry = vy[u] - qy, rz = vz[u] - qz;
+            r2[u] = (rx * rx + ry * ry) + rz * rz;
+        }
+        const int i0 = i;
+        i += 4;
+        const bool more = __ballot(i < n) != 0;
+        if (more) load(i);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const bool in = i0 + u < n && r2[u] < g.h2;
+            w[u] = in ? pm_W_sel(r2[u], g.inv_h, g.sig) : 0.0f;
+            nsup += in ? 1u : 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) pm_neu_add(s, c, w[u]);
+        if (!more) break;
+    }
+}
+
+template <int CAP>
+__device__ __forceinline__ float pm_density32_list(const GridDev &g, float qx, float qy, float qz, bool comp,
+                                                   uint32_t *lst, uint32_t &cand, uint32_t &nsup)
+{
+    FineWalk fw;
+    float s = 0.0f, c = 0.0f;
+    const bool in = pm_fine_begin(g, qx, qy, qz, fw);
+    if (!in) fw.base = 2u + 2u * fw.sy + 2u * fw.sz;
+    int n = 0;
+    auto drain = [&](int k) { pm_list_density(g, lst, k, qx, qy, qz, s, c, nsup); };
+    RowPlane P, Q;
+    pm_fine_plane(g, fw, in, -2, P);
+    _Pragma("unroll 1") for (int dz = -2; dz <= 2; dz++) {
+        if (dz < 2) pm_fine_plane(g, fw, in, dz + 1, Q);
+#pragma unroll
+        for (int k = 0; k < 5; k++) cand += P.e[k] - P.b[k];
+        pm_list_plane<CAP>(P, lst, n, drain);
+        P = Q;
+    }
+    drain(n);
+    return comp ? s + c : s;
+}
+
+template <int CAP>
+__device__ __forceinline__ float pm_density32_list(const GridDev &g, float qx, float qy, float qz, bool comp,
+                                                   uint32_t *lst, uint32_t &cand)
 {
     uint32_t nsup = 0;
-    return pm_density32_lds<CAP, UNROLL>(g, qx, qy, qz, buf, cand, nsup);
+    return pm_density32_list<CAP>(g, qx, qy, qz, comp, lst, cand, nsup);
 }
 
 // ---- fused central differences ----
@@ -497,61 +553,9 @@ __device__ __forceinline__ void pm_acc6(const GridDev &g, float px, float py, fl
     }
 }
 
-// The six central-difference densities of q = (x[0], x[1], x[2]) in one walk.
-// A kept candidate is added to the six sums at once (about nine in ten pass the
-// union test).
-__device__ __forceinline__ Cdiff6 pm_cdiff6(const GridDev &g, float qx, float qy, float qz, float eps, bool comp)
-{
-    Cdiff6 out;
-    const float x[3] = { qx, qy, qz };
-    const float xp[3] = { qx + eps, qy + eps, qz + eps }, xm[3] = { qx - eps, qy - eps, qz - eps };
-    BoxWalk w;
-    if (!pm_box_begin(g, xm, xp, w)) {
-        out.cand = 0xffffffffu;
-#pragma unroll
-        for (int k = 0; k < 6; k++) out.v[k] = 0.0f;
-        return out;
-    }
-    const float he = (g.h + eps) * 1.0009765625f;
-    const float R2 = he * he;
-    Acc6 a;
-#pragma unroll
-    for (int k = 0; k < 6; k++) { a.s[k] = 0.0f; a.c[k] = 0.0f; }
-    uint32_t cand = 0;
-    int jy = 0, jz = 0;
-    uint32_t nb, ne;
-    pm_box_row(g, w, 0, 0, nb, ne);
-    const int nr = w.ny * w.nz;
-    _Pragma("unroll 1") for (int r = 0; __ballot(r < nr) != 0; r++) {
-        const uint32_t b = nb, e = ne;
-        cand += e - b;
-        const bool any = __ballot(e > b) != 0;
-        if (++jy == w.ny) { jy = 0; jz++; }
-        pm_box_row(g, w, jy, jz, nb, ne);                 // next row in flight
-        if (!any) continue;
-        const int m = (int)(e - b);
-        const float4 *const p0 = g.fsorted + b;
-        for (int i = 0; i < m; i += 4) {
-            float4 v[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) v[u] = p0[i + u < m ? i + u : i];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const float rx = v[u].x - qx, ry = v[u].y - qy, rz = v[u].z - qz;
-                if (i + u < m && (rx * rx + ry * ry) + rz * rz < R2) pm_acc6(g, v[u].x, v[u].y, v[u].z, x, xp, xm, comp, a);
-            }
-        }
-    }
-    out.cand = cand;
-#pragma unroll
-    for (int k = 0; k < 6; k++) out.v[k] = comp ? a.s[k] + a.c[k] : a.s[k];
-    return out;
-}
-
-// The same six densities with the kept candidates compacted first through the
-// lane's LDS slots (buf: lane-interleaved, CAP floats; entries of three floats)
-// and added from there: better where every lane of the wave finishes a hit at
-// once (the finish kernel), worse inside the march kernel's own finishing.
+// The six central-difference densities of q = (x[0], x[1], x[2]) in one walk,
+// the kept candidates compacted through the lane's LDS slots (buf:
+// lane-interleaved, CAP floats; entries of three floats) and added from there.
 template <int CAP>
 __device__ __forceinline__ Cdiff6 pm_cdiff6_lds(const GridDev &g, float qx, float qy, float qz, float eps, float *buf,
                                              bool comp)

@@ -56,8 +56,7 @@ struct MarchLaunch {
     float4 *nrm;
     float *t;             // may be null
     unsigned long long *counters;
-    uint32_t *band_ctr;        // 8 per-XCD tile counters (persistent schedule)
-    uint32_t persist_blocks;   // workgroups of the persistent schedule, 0 = default
+    uint32_t *band_ctr;        // per-XCD tile counters and the hit-list length (anisotropic march, schedule 1)
     // learned step proposal
     CoarseDev cg;
     MlpDev net;

@@ -3,51 +3,41 @@
 // Replaces RayMarcher::PerPixel_Isotropic (RayMarcher.cpp:256-344) and the
 // ThreadPool that drives it (ThreadPool.cpp:38-55).
 //
-// Work mapping: one wave64 per 8x8 pixel tile at a time, one ray per lane, four
-// waves per 256-thread workgroup; persistent workgroups take the tiles from
-// per-XCD bands (blockIdx % 8 names the XCD), so each XCD's L2 holds the
-// particles of its band.
-//
-// Every lane runs a small state machine (march -> FP32 bisection; the learned
-// form adds step proposals) and each loop iteration performs exactly one FP32
-// density evaluation per busy lane, whatever its phase, so the candidate loop
-// stays converged across the wave while rays hit at different steps.  A ray's
-// march ends at its hit record; the FP64 step, the normal and the outputs
-// follow per tile (finish_hit).  Schedule 1 (k_march_simple) marches one ray
-// per lane to its end with a direct walk for every sample: the plain form the
-// persistent one is checked against.
+// Work mapping: one wave64 per 8x8 pixel tile, one ray per lane.  A tile
+// pre-pass lists the tiles a ray of which can hit; the march kernel takes one
+// listed tile per wave up to each ray's hit bracket or miss, the finish kernel
+// then takes the same tiles through bisection, FP64 step, normal and outputs.
+// In each kernel every lane does the same kind of work at the same time: the
+// march ends where its rays' work would diverge.  (One kernel that bisected a
+// ray's hit while other lanes of the wave still marched took 23 density
+// evaluations per wave at the median, 1.11 ms at 1080p on the 1 M dam break;
+// split, 0.33 + 0.46 ms.)  Schedule 1 (k_march_simple) marches one ray per lane
+// to its end with a direct walk for every sample: the plain form the product
+// is checked against.
 #include "pm_features.h"
 #include "pm_internal.h"
 #include "pm_ray.h"
 
 namespace pm {
 
-// The ray's hit is known up to what k_finish does: its record (at the
-// pixel) holds t itself (fp64 = false), or the bracket [lo, hi] of the FP64
-// bisection step.  Record: (1 | fp64 << 1, lo, hi, 0); a miss leaves zeros.
+// The first sample k at or above iso is known and the ray's march ends: its
+// record (at the pixel) holds the bracket [t_{k-1}, t_k] of the bisection, or
+// t itself (the ray starts inside the surface, or no bisection is asked for).
+// Record: (1 | bracket << 1, lo, hi, 0); a miss leaves zeros.
 // lead: this lane writes (the others of a lane group share the ray).
-__device__ __forceinline__ void to_emit(const MarchLaunch &L, RayState &r, bool fp64, float lo, float hi,
-                                       bool lead = true)
-{
-    if (lead) L.hit_rec[r.idx] = make_uint4(fp64 ? 3u : 1u, __float_as_uint(lo), __float_as_uint(hi), 0u);
-    r.phase = PH_DONE;
-}
-
-// The first sample k at or above iso is known: bracket [t_{k-1}, t_k] and
-// start the bisection (or take t_0 when the ray starts inside the surface).
-__device__ __forceinline__ void start_bracket(const MarchLaunch &L, RayState &r, int n32, bool lead = true)
+__device__ __forceinline__ void emit_hit(const MarchLaunch &L, RayState &r, bool lead = true)
 {
     const pm_settings &s = L.s;
-    if (r.k == 0) {
-        to_emit(L, r, false, r.tn, r.tn, lead);
-        return;
+    float lo = r.tn, hi = r.tn;
+    bool bracket = false;
+    if (r.k != 0) {
+        lo = r.tn + (float)(r.k - 1) * s.step;
+        hi = r.tn + (float)r.k * s.step;
+        bracket = s.bisect_iters > 0;
+        if (!bracket) lo = hi = (lo + hi) * 0.5f;
     }
-    r.lo = r.tn + (float)(r.k - 1) * s.step;
-    r.hi = r.tn + (float)r.k * s.step;
-    r.it = 0;
-    if (n32 > 0) r.phase = PH_BISECT;
-    else if (s.final_fp64 && s.bisect_iters > 0) to_emit(L, r, true, r.lo, r.hi, lead);
-    else { const float t = (r.lo + r.hi) * 0.5f; to_emit(L, r, false, t, t, lead); }
+    if (lead) L.hit_rec[r.idx] = make_uint4(bracket ? 3u : 1u, __float_as_uint(lo), __float_as_uint(hi), 0u);
+    r.phase = PH_DONE;
 }
 
 // First half of one step: the sample point of the lane's next FP32 density
@@ -61,32 +51,26 @@ __device__ __forceinline__ bool ray_prepare(const MarchLaunch &L, RayState &r, f
     const GridDev &g = L.g;
     const float o0 = L.cam[0], o1 = L.cam[1], o2 = L.cam[2];
 
-    if (r.phase == PH_MARCH) {
-        // at most HOPS skips per step: a lane crossing much skippable space
-        // then idles for a step instead of holding the whole wave in this loop
-        // (a skip costs a few dozen instructions, a step a density walk)
-        for (int hop = 0;; hop++) {
-            float t = r.tn + (float)r.k * s.step;
-            if (t > r.tf || (s.max_steps > 0 && r.k >= s.max_steps)) {
-                march_miss(L, r.idx);
-                r.phase = PH_DONE;
-                return false;
-            }
-            qx = o0 + t * r.d0; qy = o1 + t * r.d1; qz = o2 + t * r.d2;
-            int kn;
-            if (s.skip_mode == PM_SKIP_BOUND) kn = pm_skip_bound(g, o0, o1, o2, r, qx, qy, qz, L.inv_step);
-            else if (s.skip_mode == PM_SKIP_EMPTY) kn = pm_skip_empty(g, o0, o1, o2, r, qx, qy, qz, s.step);
-            else break;
-            if (kn == r.k) break;
-            r.k = kn;
-            r.lrn = s.learned;
-            if (hop == HOPS - 1) return false;
+    // at most HOPS skips per step: a lane crossing much skippable space
+    // then idles for a step instead of holding the whole wave in this loop
+    // (a skip costs a few dozen instructions, a step a density walk)
+    for (int hop = 0;; hop++) {
+        float t = r.tn + (float)r.k * s.step;
+        if (t > r.tf || (s.max_steps > 0 && r.k >= s.max_steps)) {
+            march_miss(L, r.idx);
+            r.phase = PH_DONE;
+            return false;
         }
-    } else {  // PH_BISECT
-        float tm = (r.lo + r.hi) * 0.5f;
-        qx = o0 + tm * r.d0; qy = o1 + tm * r.d1; qz = o2 + tm * r.d2;
+        qx = o0 + t * r.d0; qy = o1 + t * r.d1; qz = o2 + t * r.d2;
+        int kn;
+        if (s.skip_mode == PM_SKIP_BOUND) kn = pm_skip_bound(g, o0, o1, o2, r, qx, qy, qz, L.inv_step);
+        else if (s.skip_mode == PM_SKIP_EMPTY) kn = pm_skip_empty(g, o0, o1, o2, r, qx, qy, qz, s.step);
+        else return true;
+        if (kn == r.k) return true;
+        r.k = kn;
+        r.lrn = s.learned;
+        if (hop == HOPS - 1) return false;
     }
-    return true;
 }
 
 // The counts of one FP32 density evaluation at q (instrumented launches also
@@ -108,38 +92,23 @@ __device__ __forceinline__ void count_sample(const GridDev &g, float qx, float q
 }
 
 // Second half: the sample's density rho (and its stencil candidate count)
-// drives the lane's state machine.
+// ends the march, asks for a proposal or moves to the next sample.
 template <bool INSTR>
 __device__ __forceinline__ void ray_finish(const MarchLaunch &L, RayState &r, float rho, uint32_t cand, float qx,
                                            float qy, float qz, Counts &cn)
 {
-    const pm_settings &s = L.s;
-    const bool fp64 = s.final_fp64 && s.bisect_iters > 0;
-    const int n32 = fp64 ? s.bisect_iters - 1 : s.bisect_iters;
-    count_sample<INSTR>(L.g, qx, qy, qz, cand, r.phase == PH_MARCH, cn);
-
-    if (r.phase == PH_MARCH) {
-        if (rho >= s.iso) {
-            start_bracket(L, r, n32);
-        } else if (r.lrn && rho < L.mlp_gate_rho) {
-            r.rho = rho;
-            r.phase = PH_PROPOSE;
-        } else {
-            r.k++;
-        }
-    } else {  // PH_BISECT
-        float tm = (r.lo + r.hi) * 0.5f;
-        if (rho >= s.iso) r.hi = tm; else r.lo = tm;
-        r.it++;
-        if (r.it >= n32) {
-            if (fp64) to_emit(L, r, true, r.lo, r.hi);
-            else { const float t = (r.lo + r.hi) * 0.5f; to_emit(L, r, false, t, t); }
-        }
+    count_sample<INSTR>(L.g, qx, qy, qz, cand, true, cn);
+    if (rho >= L.s.iso) {
+        emit_hit(L, r);
+    } else if (r.lrn && rho < L.mlp_gate_rho) {
+        r.rho = rho;
+        r.phase = PH_PROPOSE;
+    } else {
+        r.k++;
     }
 }
 
-// One density evaluation of this ray, whatever its phase, and the transition
-// it implies.  Dens(q, cand) is the FP32 density.  HOPS: skips per step before
+// One march sample of this ray and the transition it implies.  Dens(q, cand) is the FP32 density.  HOPS: skips per step before
 // a lane idles -- 16 in the single-view march, whose end is spent on few long
 // rays with idle lanes beside them; 8 in the batch, whose lanes stay busy.
 template <bool INSTR, int HOPS, class Dens>
@@ -155,33 +124,30 @@ __device__ __forceinline__ void ray_step(const MarchLaunch &L, RayState &r, Dens
 // ---- lane groups: the end of a persistent launch ----
 // Once no tile is left, a wave's remaining rays are spread over its idle lanes:
 // G lanes (a power of two) per ray, every lane of a group holding the same
-// RayState.  A march step then evaluates the G lattice samples k .. k+G-1 at
-// once and takes the first at or above iso; a bisection step evaluates the
-// 2^L - 1 midpoints of the next L levels (L = floor(log2(G + 1))) and descends
-// through them.  Each sample is computed as the one-lane march computes it,
-// and a sample the skip would pass has its density below iso, so the first
-// crossing, the bracket and the image are those of the one-lane march.
-// Counters count what the one-lane march evaluates: the samples the skip
-// keeps, up to the crossing, and the bisection's path.
+// RayState.  A step then evaluates the G lattice samples k .. k+G-1 at once and
+// takes the first at or above iso.  Each sample is computed as the one-lane
+// march computes it, and a sample the skip would pass has its density below
+// iso, so the first crossing, the bracket and the image are those of the
+// one-lane march.  Counters count what the one-lane march evaluates: the
+// samples the skip keeps, up to the crossing.
 
 // The ray's state to LDS and back (region: 64 floats per field).
 __device__ __forceinline__ void state_put(float *region, uint32_t slot, const RayState &r)
 {
     float *p = region + slot;
     p[0 * 64] = r.d0; p[1 * 64] = r.d1; p[2 * 64] = r.d2; p[3 * 64] = r.tn; p[4 * 64] = r.tf;
-    p[5 * 64] = r.lo; p[6 * 64] = r.hi; p[7 * 64] = __int_as_float(r.k); p[8 * 64] = __int_as_float(r.it);
-    p[9 * 64] = __int_as_float(r.phase); p[10 * 64] = __uint_as_float(r.idx); p[11 * 64] = r.id0;
-    p[12 * 64] = r.id1; p[13 * 64] = r.id2;
+    p[5 * 64] = __int_as_float(r.k); p[6 * 64] = __int_as_float(r.phase); p[7 * 64] = __uint_as_float(r.idx);
+    p[8 * 64] = r.id0; p[9 * 64] = r.id1; p[10 * 64] = r.id2;
 }
 
 __device__ __forceinline__ void state_get(const float *region, uint32_t slot, RayState &r)
 {
     const float *p = region + slot;
     r.d0 = p[0 * 64]; r.d1 = p[1 * 64]; r.d2 = p[2 * 64]; r.tn = p[3 * 64]; r.tf = p[4 * 64];
-    r.lo = p[5 * 64]; r.hi = p[6 * 64]; r.k = __float_as_int(p[7 * 64]); r.it = __float_as_int(p[8 * 64]);
-    r.phase = __float_as_int(p[9 * 64]); r.idx = __float_as_uint(p[10 * 64]); r.id0 = p[11 * 64];
-    r.id1 = p[12 * 64]; r.id2 = p[13 * 64];
+    r.k = __float_as_int(p[5 * 64]); r.phase = __float_as_int(p[6 * 64]); r.idx = __float_as_uint(p[7 * 64]);
+    r.id0 = p[8 * 64]; r.id1 = p[9 * 64]; r.id2 = p[10 * 64];
     r.lrn = 0;
+    if (r.phase == PH_PROPOSE) { r.phase = PH_MARCH; r.k++; }   // below iso, and no proposals in groups
 }
 
 // Widens the groups when the busy rays fit in fewer lanes: G becomes the
@@ -211,51 +177,34 @@ __device__ __forceinline__ bool group_prepare(const MarchLaunch &L, RayState &r,
     const GridDev &g = L.g;
     const float o0 = L.cam[0], o1 = L.cam[1], o2 = L.cam[2];
     nonskip = false;
-    if (r.phase == PH_MARCH) {
-        // the group's first sample, as ray_prepare finds it; the wave has few
-        // rays left, so a group may take 8 G skips in one step
-        const int hop_cap = 8 * G - 1;
-        for (int hop = 0;; hop++) {
-            float t = r.tn + (float)r.k * s.step;
-            if (t > r.tf || (s.max_steps > 0 && r.k >= s.max_steps)) {
-                if (j == 0) march_miss(L, r.idx);
-                r.phase = PH_DONE;
-                return false;
-            }
-            qx = o0 + t * r.d0; qy = o1 + t * r.d1; qz = o2 + t * r.d2;
-            int kn = r.k;
-            if (s.skip_mode == PM_SKIP_BOUND) kn = pm_skip_bound(g, o0, o1, o2, r, qx, qy, qz, L.inv_step);
-            if (kn == r.k) break;
-            r.k = kn;
-            if (hop == hop_cap) return false;
+    // the group's first sample, as ray_prepare finds it; the wave has few
+    // rays left, so a group may take 8 G skips in one step
+    const int hop_cap = 8 * G - 1;
+    for (int hop = 0;; hop++) {
+        float t = r.tn + (float)r.k * s.step;
+        if (t > r.tf || (s.max_steps > 0 && r.k >= s.max_steps)) {
+            if (j == 0) march_miss(L, r.idx);
+            r.phase = PH_DONE;
+            return false;
         }
-        if (j == 0) { nonskip = true; return true; }
-        const int kj = r.k + j;
-        const float t = r.tn + (float)kj * s.step;
-        if (t > r.tf || (s.max_steps > 0 && kj >= s.max_steps)) return false;
         qx = o0 + t * r.d0; qy = o1 + t * r.d1; qz = o2 + t * r.d2;
-        nonskip = s.skip_mode != PM_SKIP_BOUND || pm_skip_bound(g, o0, o1, o2, r, qx, qy, qz, L.inv_step) == r.k;
-        return true;
+        int kn = r.k;
+        if (s.skip_mode == PM_SKIP_BOUND) kn = pm_skip_bound(g, o0, o1, o2, r, qx, qy, qz, L.inv_step);
+        else if (s.skip_mode == PM_SKIP_EMPTY) kn = pm_skip_empty(g, o0, o1, o2, r, qx, qy, qz, s.step);
+        if (kn == r.k) break;
+        r.k = kn;
+        if (hop == hop_cap) return false;
     }
-    if (r.phase == PH_BISECT) {
-        const bool fp64 = s.final_fp64 && s.bisect_iters > 0;
-        const int n32 = fp64 ? s.bisect_iters - 1 : s.bisect_iters;
-        int lv = 31 - __clz(G + 1);                 // floor(log2(G + 1))
-        if (lv > n32 - r.it) lv = n32 - r.it;
-        const int node = j + 1;                     // heap order: 1 = the next midpoint
-        if (node >= (1 << lv)) return false;
-        const int depth = 31 - __clz(node);
-        float lo = r.lo, hi = r.hi;
-        for (int b = depth - 1; b >= 0; b--) {      // left child: the crossing lies below the midpoint
-            const float tm = (lo + hi) * 0.5f;
-            if ((node >> b) & 1) lo = tm; else hi = tm;
-        }
-        const float tm = (lo + hi) * 0.5f;
-        qx = o0 + tm * r.d0; qy = o1 + tm * r.d1; qz = o2 + tm * r.d2;
-        nonskip = true;
-        return true;
-    }
-    return false;
+    if (j == 0) { nonskip = true; return true; }
+    const int kj = r.k + j;
+    const float t = r.tn + (float)kj * s.step;
+    if (t > r.tf || (s.max_steps > 0 && kj >= s.max_steps)) return false;
+    qx = o0 + t * r.d0; qy = o1 + t * r.d1; qz = o2 + t * r.d2;
+    // (a skip returns a later sample than r.k exactly where q may be skipped)
+    nonskip = s.skip_mode == PM_SKIP_BOUND   ? pm_skip_bound(g, o0, o1, o2, r, qx, qy, qz, L.inv_step) == r.k
+              : s.skip_mode == PM_SKIP_EMPTY ? pm_skip_empty(g, o0, o1, o2, r, qx, qy, qz, s.step) == r.k
+                                             : true;
+    return true;
 }
 
 // The group's transition from its lanes' densities.  Called by all 64 lanes.
@@ -263,76 +212,46 @@ template <bool INSTR>
 __device__ __forceinline__ void group_finish(const MarchLaunch &L, RayState &r, int G, int j, bool want, bool nonskip,
                                              float rho, uint32_t cand, float qx, float qy, float qz, Counts &cn)
 {
-    const pm_settings &s = L.s;
-    const bool fp64 = s.final_fp64 && s.bisect_iters > 0;
-    const int n32 = fp64 ? s.bisect_iters - 1 : s.bisect_iters;
     const uint32_t lane = threadIdx.x & 63, gbase = lane & ~(uint32_t)(G - 1);
     const unsigned long long gmask = G == 64 ? ~0ull : ((1ull << G) - 1ull);
-    const unsigned long long cross = (__ballot(want && rho >= s.iso) >> gbase) & gmask;
+    const unsigned long long cross = (__ballot(want && rho >= L.s.iso) >> gbase) & gmask;
     const unsigned long long wants = (__ballot(want) >> gbase) & gmask;
-    // bisection: descend through the evaluated midpoints (uniform trip count)
-    const int lvmax = 31 - __clz(G + 1);
-    const bool bis = r.phase == PH_BISECT && (wants & 1ull);
-    int node = 1;
-    for (int l = 0; l < lvmax; l++) {
-        const float rn = __shfl(rho, (int)gbase + node - 1, 64);
-        const uint32_t cn_n = __shfl(cand, (int)gbase + node - 1, 64);
-        if (bis && r.it < n32 && ((wants >> (node - 1)) & 1ull)) {
-            const float tm = (r.lo + r.hi) * 0.5f;
-            if (j == 0)
-                count_sample<INSTR>(L.g, L.cam[0] + tm * r.d0, L.cam[1] + tm * r.d1, L.cam[2] + tm * r.d2, cn_n, false,
-                                    cn);
-            if (rn >= s.iso) { r.hi = tm; node = 2 * node; } else { r.lo = tm; node = 2 * node + 1; }
-            r.it++;
-        }
-    }
-    if (bis && r.it >= n32) {
-        if (fp64) to_emit(L, r, true, r.lo, r.hi, j == 0);
-        else { const float t = (r.lo + r.hi) * 0.5f; to_emit(L, r, false, t, t, j == 0); }
-        return;
-    }
     if (r.phase != PH_MARCH || !(wants & 1ull)) return;
     const int jc = cross ? __ffsll((long long)cross) - 1 : G;
     if (want && nonskip && j <= jc) count_sample<INSTR>(L.g, qx, qy, qz, cand, true, cn);
     if (cross) {
         r.k += jc;
-        start_bracket(L, r, n32, j == 0);
+        emit_hit(L, r, j == 0);
     } else {
         r.k += G;
     }
 }
 
-struct DensPlain {
+// FP32 density through the lane's candidate list (compensated or plain sum).
+// CAP: 36 candidates -- near the surface a stencil holds about 41, so most
+// samples take their list once or twice -- and 10 KB of LDS per wave, which
+// keeps 16 waves on a CU.
+static constexpr int kListCap = 36;
+static constexpr int kListWords = (kListCap + kListPad) * 64;   // per wave
+
+struct DensList {
     const GridDev *g;
+    uint32_t *lst;
     bool comp;
     __device__ float operator()(float x, float y, float z, uint32_t &cand) const
     {
-        return pm_density32(*g, x, y, z, comp, cand);
+        return pm_density32_list<kListCap>(*g, x, y, z, comp, lst, cand);
     }
 };
 
-template <int CAP, int UNROLL>
-struct DensLds {
-    const GridDev *g;
-    float *buf;
-    __device__ float operator()(float x, float y, float z, uint32_t &cand) const
-    {
-        return pm_density32_lds<CAP, UNROLL>(*g, x, y, z, buf, cand);
-    }
-};
+static constexpr int kLdsCap = 32;   // floats per lane of the six-sample walk's compaction
 
-static constexpr int kLdsCap = 32;
-static constexpr uint32_t kOwnTiles = 32;   // tiles a persistent wave finishes itself
-
-// Band b of the T tiles is [T b / 8, T (b+1) / 8).
-__device__ __forceinline__ uint32_t band_lo(uint32_t T, uint32_t b) { return (uint32_t)(((uint64_t)T * b) >> 3); }
-
-// Tile pre-pass of the persistent schedules.  tile_buf = flag[T+1] | pos[T+1] |
+// Tile pre-pass.  tile_buf = flag[T+1] | pos[T+1] |
 // order[T+1] | scan scratch: flag = 1 for a tile one of whose rays enters the
 // padded AABB (the ray set-up and slab test of ray_setup, bit for bit) -- in
 // reference mode, one of whose pixels has a depth other than 1 -- pos
 // its exclusive scan, order the active tiles in row order (order[T] = their
-// count).  The persistent waves take only active tiles; k_miss_tiles writes
+// count).  The march takes only active tiles; k_miss_tiles writes
 // the misses of the others.
 __global__ __launch_bounds__(256) void k_tile_flags(MarchLaunch L, uint32_t T)
 {
@@ -386,7 +305,7 @@ __global__ __launch_bounds__(256) void k_miss_tiles(MarchLaunch L, uint32_t T)
 // Schedule 1: one 8x8 tile per wave, one ray per lane to its end -- march,
 // bisection, FP64 step, normal, outputs -- every sample with its own direct
 // walk (no compaction, no lists, no hit records).  The plain form of the
-// configured march the persistent schedule is checked against.
+// configured march the product is checked against.
 __global__ __launch_bounds__(256) void k_march_simple(MarchLaunch L)
 {
     uint32_t px, py;
@@ -637,24 +556,38 @@ __device__ __forceinline__ void wave_propose_step(const MarchLaunch &L, RayState
 }
 
 // ---- finish ----
-// Per hit record: the FP64 bisection step when the settings ask for it, the
-// normal (the six central differences in one fused walk, or the sum of gradW)
-// and the pixel's outputs.  Every lane of a wave does the same kind of work
+// Per hit record: the bisection of the bracket (the last step in FP64 when the
+// settings ask for it), the normal (the six central differences in one fused
+// walk, or the sum of gradW) and the pixel's outputs.  Every lane of a wave does the same kind of work
 // and none of the march's state is held, so this runs packed and short; the
 // march kernels keep only the phases that decide where the hit is.
-template <bool INSTR, bool LDS_NORMALS>
+template <bool INSTR>
 __device__ __forceinline__ void finish_hit(const MarchLaunch &L, uint32_t px, uint32_t py, uint4 rec, float *buf,
                                            Counts &cn)
 {
     const pm_settings &s = L.s;
     const GridDev &g = L.g;
     const uint32_t idx = py * L.W + px;
-    const float lo = __uint_as_float(rec.y), hi = __uint_as_float(rec.z);
+    float lo = __uint_as_float(rec.y), hi = __uint_as_float(rec.z);
     float d[3];
     pm_ray_dir(L, px, py, d);
     const float o0 = L.cam[0], o1 = L.cam[1], o2 = L.cam[2];
     float xs[3], th;
+    const bool fp64 = s.final_fp64 && s.bisect_iters > 0;
     if (rec.x & 2u) {
+        const int n32 = fp64 ? s.bisect_iters - 1 : s.bisect_iters;
+#pragma unroll 1
+        for (int it = 0; it < n32; it++) {
+            const float tm = (lo + hi) * 0.5f;
+            const float qx = o0 + tm * d[0], qy = o1 + tm * d[1], qz = o2 + tm * d[2];
+            uint32_t cand = 0;
+            const float rho = pm_density32_list<kListCap>(g, qx, qy, qz, s.compensated != 0, (uint32_t *)buf, cand);
+            count_sample<INSTR>(g, qx, qy, qz, cand, false, cn);
+            if (rho >= s.iso) hi = tm; else lo = tm;
+        }
+        if (!fp64) lo = hi = (lo + hi) * 0.5f;
+    }
+    if ((rec.x & 2u) && fp64) {
         // the last bisection step in double (RayMarcher.cpp:316-326 in FP64)
         const double tmd = ((double)lo + (double)hi) * 0.5;
         const double x = (double)o0 + tmd * (double)d[0];
@@ -687,8 +620,7 @@ __device__ __forceinline__ void finish_hit(const MarchLaunch &L, uint32_t px, ui
         const bool comp = s.compensated != 0;
         const float e = s.normal_eps;
         float gv[3];
-        const Cdiff6 o = LDS_NORMALS ? pm_cdiff6_lds<kLdsCap>(g, xs[0], xs[1], xs[2], e, buf, comp)
-                                     : pm_cdiff6(g, xs[0], xs[1], xs[2], e, comp);
+        const Cdiff6 o = pm_cdiff6_lds<kLdsCap>(g, xs[0], xs[1], xs[2], e, buf, comp);
         if (o.cand != 0xffffffffu) {
             cn.samples += 6;
             cn.cand += o.cand;
@@ -700,8 +632,7 @@ __device__ __forceinline__ void finish_hit(const MarchLaunch &L, uint32_t px, ui
                 float q[3] = { xs[0], xs[1], xs[2] };
                 q[k >> 1] = (k & 1) ? xs[k >> 1] - e : xs[k >> 1] + e;
                 uint32_t cand = 0;
-                const float rho = comp ? pm_density32_lds<kLdsCap, 4>(g, q[0], q[1], q[2], buf, cand)
-                                       : pm_density32(g, q[0], q[1], q[2], false, cand);
+                const float rho = pm_density32_list<kListCap>(g, q[0], q[1], q[2], comp, (uint32_t *)buf, cand);
                 cn.samples++;
                 cn.cand += cand;
                 if (k & 1) gv[k >> 1] -= rho; else gv[k >> 1] = rho;
@@ -731,139 +662,95 @@ __device__ __forceinline__ void finish_hit(const MarchLaunch &L, uint32_t px, ui
 }
 
 // One 8x8 tile per wave, one pixel per lane: the lanes whose pixel holds a
-// hit record finish it.  LDS_NORMALS: the six-sample normal walk compacts its
-// candidates through LDS first -- the finish kernel, where every lane of every
-// wave finishes hits; the march kernel's own finishing adds them directly
-// (measured: 1080p 1.11 -> 1.08 ms, 4K pool 10.4 -> 9.4 ms in the march
-// kernel; 54 against 62 ms per batch replay in the finish kernel).
-template <bool INSTR, bool LDS_NORMALS>
+// hit record finish it.
+template <bool INSTR>
 __device__ __forceinline__ void finish_tile(const MarchLaunch &L, uint32_t tile, float *buf, Counts &cn)
 {
     const uint32_t lane = threadIdx.x & 63, tiles_x = (L.W + 7) / 8;
     const uint32_t px = (tile % tiles_x) * 8 + (lane & 7u), py = (tile / tiles_x) * 8 + (lane >> 3);
     if (px >= L.W || py >= L.H) return;
     const uint4 rec = L.hit_rec[py * L.W + px];
-    if (rec.x & 1u) finish_hit<INSTR, LDS_NORMALS>(L, px, py, rec, buf, cn);
+    if (rec.x & 1u) finish_hit<INSTR>(L, px, py, rec, buf, cn);
 }
 
-// Schedule 0: persistent waves.  The image is cut into 8x8 tiles and the tiles
-// into 8 contiguous bands, one per XCD (workgroups are dispatched round-robin
-// over the XCDs, so blockIdx % 8 names the XCD); a wave takes tiles from its
-// band's counter and, once the band is drained, from the other bands.  A lane
-// whose ray is finished takes the next ray of the wave's current tile before
-// the next density evaluation, so all 64 lanes stay busy until the image runs
-// out.  Rays that miss the AABB are retired during refill.  Every wave exits
-// once no tile is left and its lanes are idle.
-// LEARNED adds the step proposals; its LDS region per wave holds either the
-// density compaction buffer or the network's activations (never both at once).
-// INSTR adds the per-sample counts of instrumented launches.  The walk waits
-// on the cache far more than it computes, so the kernel keeps 4 waves per SIMD
-// (<= 128 VGPRs; all 1,024 workgroups resident at once).
-template <bool LEARNED, bool INSTR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_march_persist(
-    MarchLaunch L, uint32_t *__restrict__ band_ctr)
+// Active tile i of a launch's list for wave `w` of the grid (one-wave
+// workgroups, dispatched to the 8 XCDs round-robin): runs of kXcdRun
+// consecutive tiles go to the XCDs in turn, so neighbouring tiles share an L2
+// and every XCD gets its share of a dense region.
+static constexpr uint32_t kXcdRun = 32;
+__device__ __forceinline__ uint32_t xcd_tile(uint32_t w)
 {
-    constexpr int CAP = kLdsCap;
-    // floats per wave: the compaction buffer, or X[64][32] + H[32][64] bf16 + Y[64]
-    constexpr int kRegion = LEARNED ? 2112 : CAP * 64;
-    __shared__ float lds[4 * kRegion];
-    __shared__ uint32_t own[4][kOwnTiles];       // tiles this wave marched (finished by it at the end)
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    float *region = lds + wave * kRegion;
-    float *buf = region + lane;
-    const uint32_t tiles_x = (L.W + 7) / 8, tiles_y = (L.H + 7) / 8, T = tiles_x * tiles_y;
-    uint32_t nown = 0;
-    const uint32_t xcd = blockIdx.x & 7u;
-    const bool use_lds = L.s.compensated != 0;
+    const uint32_t local = w >> 3;
+    return ((local / kXcdRun) * 8 + (w & 7u)) * kXcdRun + local % kXcdRun;
+}
 
+// Workgroups for T tiles (all of them may be active): a multiple of a full
+// round of runs; beyond kMaxWaves each wave takes several tiles.
+static constexpr uint32_t kMaxWaves = 16384;
+__host__ __device__ __forceinline__ uint32_t tile_waves_of(uint32_t T)
+{
+    return (T + 8 * kXcdRun - 1) / (8 * kXcdRun) * (8 * kXcdRun);
+}
+
+// Schedule 0: one wave per active 8x8 tile, one ray per lane up to the ray's
+// hit or miss.  As rays end, the others spread over the idle lanes (lane
+// groups), so the tile's last rays take several samples per step.  The tiles
+// come from the list by position: no queue.  (Persistent waves that drew tiles
+// from counters spent 0.30 of 0.64 ms at 1080p on the counters: 4,096 waves
+// each found all eight bands empty, one serialised atomic per band.)
+// LEARNED adds the step proposals; its LDS region holds either the lanes'
+// candidate lists or the network's activations (never both at once).
+// INSTR adds the per-sample counts of instrumented launches.
+template <bool LEARNED, bool INSTR>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_march_tiles(MarchLaunch L)
+{
+    // the lanes' candidate lists, or X[64][32] + H[32][64] bf16 + Y[64]
+    static_assert(kListWords >= 2112, "network region");
+    __shared__ float region[kListWords];
+    const uint32_t lane = threadIdx.x;
+    uint32_t *lst = (uint32_t *)region + lane;
+    const uint32_t tiles_x = (L.W + 7) / 8, T = tiles_x * ((L.H + 7) / 8);
+    const uint32_t *order = L.tile_buf + 2 * (T + 1);
+    const uint32_t TA = order[T];
+    const bool comp = L.s.compensated != 0;
     Counts cn;
-    RayState r{};
-    r.phase = PH_DONE;
-    uint32_t tile = 0, steal = 0;
-    int qpos = 64;
-    bool exhausted = false;
-    const unsigned long long lt_mask = (1ull << lane) - 1ull;
-    // lane groups at the end of the launch (the one-lane march otherwise)
-    int G = 1;
-    const bool group_ok = L.s.skip_mode == PM_SKIP_BOUND || L.s.skip_mode == PM_SKIP_NONE;
-
-    while (true) {
-        // refill idle lanes from the wave's tile queue
-        while (!exhausted) {
-            unsigned long long needy = __ballot(r.phase == PH_DONE);
-            if (needy == 0) break;
-            if (qpos >= 64) {
-                uint32_t t = 0xffffffffu;
-                if (lane == 0) {
-                    // the bands split the active tiles (the pre-pass lists them)
-                    const uint32_t TA = L.tile_buf[2 * (T + 1) + T];
-                    while (steal < 8) {
-                        uint32_t b = (xcd + steal) & 7u;
-                        uint32_t lo = band_lo(TA, b), hi = band_lo(TA, b + 1);
-                        uint32_t v = atomicAdd(&band_ctr[b], 1u);
-                        if (v < hi - lo) { t = L.tile_buf[2 * (T + 1) + lo + v]; break; }
-                        steal++;
-                    }
-                }
-                t = __shfl(t, 0, 64);
-                steal = __shfl(steal, 0, 64);
-                if (t == 0xffffffffu) { exhausted = true; break; }
-                if (nown < kOwnTiles) {
-                    if (lane == 0) own[wave][nown] = t;
-                    nown++;
-                }
-                tile = t;
-                qpos = 0;
-            }
-            int rank = __popcll(needy & lt_mask);
-            int take = __popcll(needy);
-            if (r.phase == PH_DONE && qpos + rank < 64) {
-                uint32_t j = (uint32_t)(qpos + rank);
-                uint32_t px = (tile % tiles_x) * 8 + (j & 7u), py = (tile / tiles_x) * 8 + (j >> 3);
-                if (px < L.W && py < L.H) ray_setup(L, r, px, py, cn);
-            }
-            qpos = qpos + take < 64 ? qpos + take : 64;
-        }
-        if (__ballot(r.phase != PH_DONE) == 0) break;
-        // The network is batched across the wave (the wave pays for it
-        // whenever any lane needs it): it runs once half of the busy lanes wait
-        // for a proposal, or at the end (before the lane groups, which take no
-        // proposals).  Waiting lanes sit out.
-        if (LEARNED) {
+    bool any = false;
+    for (uint32_t w = blockIdx.x; w < tile_waves_of(TA); w += gridDim.x) {
+        const uint32_t i = xcd_tile(w);
+        if (i >= TA) continue;
+        any = true;
+        const uint32_t tile = order[i];
+        const uint32_t px = (tile % tiles_x) * 8 + (lane & 7u), py = (tile / tiles_x) * 8 + (lane >> 3);
+        RayState r{};
+        r.phase = PH_DONE;
+        if (px < L.W && py < L.H) ray_setup(L, r, px, py, cn);
+        int G = 1;
+        while (__ballot(r.phase != PH_DONE) != 0) {
+            // The network is batched across the wave (the wave pays for it
+            // whenever any lane needs it): it runs once half of the busy
+            // lanes wait for a proposal, or when few rays are left; waiting
+            // lanes sit out.  Lane groups take no proposals: the learned march
+            // groups its last 16 rays only.
             const int nbusy = __popcll(__ballot(r.phase != PH_DONE));
-            const int nwant = __popcll(__ballot(r.phase == PH_PROPOSE));
-            if (nwant > 0 && (2 * nwant >= nbusy || exhausted))
-                wave_propose_step(L, r, cn, region);
-        }
-        if (exhausted && group_ok) regroup(r, G, region);
-        if (G == 1) {
-            if (r.phase == PH_MARCH || r.phase == PH_BISECT) {
-                if (use_lds) ray_step<INSTR, 16>(L, r, DensLds<CAP, 4>{ &L.g, buf }, cn);
-                else ray_step<INSTR, 16>(L, r, DensPlain{ &L.g, false }, cn);
+            if (LEARNED && G == 1) {
+                const int nwant = __popcll(__ballot(r.phase == PH_PROPOSE));
+                if (nwant > 0 && (2 * nwant >= nbusy || nbusy <= 16)) wave_propose_step(L, r, cn, region);
             }
-        } else {
-            const int j = (int)(lane & (uint32_t)(G - 1));
-            float qx = 0.f, qy = 0.f, qz = 0.f, rho = 0.f;
-            bool nonskip = false, want = false;
-            uint32_t cand = 0;
-            if (r.phase != PH_DONE) want = group_prepare(L, r, G, j, qx, qy, qz, nonskip);
-            if (want) rho = use_lds ? pm_density32_lds<CAP, 4>(L.g, qx, qy, qz, buf, cand)
-                                    : pm_density32(L.g, qx, qy, qz, false, cand);
-            group_finish<INSTR>(L, r, G, j, want, nonskip, rho, cand, qx, qy, qz, cn);
+            if (!LEARNED || nbusy <= 16) regroup(r, G, region);
+            if (G == 1) {
+                if (r.phase == PH_MARCH) ray_step<INSTR, 16>(L, r, DensList{ &L.g, lst, comp }, cn);
+            } else {
+                const int j = (int)(lane & (uint32_t)(G - 1));
+                float qx = 0.f, qy = 0.f, qz = 0.f, rho = 0.f;
+                bool nonskip = false, want = false;
+                uint32_t cand = 0;
+                if (r.phase != PH_DONE) want = group_prepare(L, r, G, j, qx, qy, qz, nonskip);
+                if (want) rho = pm_density32_list<kListCap>(L.g, qx, qy, qz, comp, lst, cand);
+                group_finish<INSTR>(L, r, G, j, want, nonskip, rho, cand, qx, qy, qz, cn);
+            }
         }
     }
-    // The tiles this wave marched have all their rays done: their FP64 steps,
-    // normals and outputs are computed here, while other waves still march
-    // (k_finish then skips them).
-    if (nown > 0) {
-        wave_lds_sync();
-        for (uint32_t i = 0; i < nown; i++) {
-            const uint32_t t = own[wave][i];
-            finish_tile<INSTR, false>(L, t, buf, cn);
-            if (lane == 0) L.tile_buf[t] = 2u;
-        }
-    }
-    flush_counts(L.counters, cn);
+    if (any) flush_counts(L.counters, cn);
 }
 
 __global__ void k_zero_u32(uint32_t *p, int n)
@@ -992,12 +879,12 @@ __global__ __launch_bounds__(256) void k_march_reference_active(MarchLaunch L)
 template <bool LEARNED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_march_batch(BatchLaunch B)
 {
-    constexpr int kRegion = LEARNED ? 2112 : kLdsCap * 64;
+    constexpr int kRegion = kListWords;
     __shared__ float lds[4 * kRegion];
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     float *region = lds + wave * kRegion;
-    float *buf = region + lane;
-    const bool use_lds = B.base.s.compensated != 0;
+    uint32_t *lst = (uint32_t *)region + lane;
+    const bool comp = B.base.s.compensated != 0;
 
     const MarchLaunch *Lp = B.jobs;
     Counts cn;
@@ -1058,9 +945,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
         }
         if (group_ok && draining) regroup(r, G, region);
         if (G == 1) {
-            if (r.phase == PH_MARCH || r.phase == PH_BISECT) {
-                if (use_lds) ray_step<false, 8>(*Lp, r, DensLds<kLdsCap, 4>{ &Lp->g, buf }, cn);
-                else ray_step<false, 8>(*Lp, r, DensPlain{ &Lp->g, false }, cn);
+            if (r.phase == PH_MARCH) {
+                ray_step<false, 8>(*Lp, r, DensList{ &Lp->g, lst, comp }, cn);
             }
         } else {
             const int j = (int)(lane & (uint32_t)(G - 1));
@@ -1068,15 +954,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
             bool nonskip = false, want = false;
             uint32_t cand = 0;
             if (r.phase != PH_DONE) want = group_prepare(*Lp, r, G, j, qx, qy, qz, nonskip);
-            if (want) rho = use_lds ? pm_density32_lds<kLdsCap, 4>(Lp->g, qx, qy, qz, buf, cand)
-                                    : pm_density32(Lp->g, qx, qy, qz, false, cand);
+            if (want) rho = pm_density32_list<kListCap>(Lp->g, qx, qy, qz, comp, lst, cand);
             group_finish<false>(*Lp, r, G, j, want, nonskip, rho, cand, qx, qy, qz, cn);
         }
     }
     flush_counts(B.base.counters, cn);
 }
 
-// Single launch: the active tiles no march wave finished; batch: the tiles of
+// Single launch: the active tiles; batch: the tiles of
 // the chunks, one chunk per workgroup at a time.  Four waves per SIMD
 // (registers capped at 128) hide more of the walks' latency than three would
 // at 150 registers.
@@ -1084,23 +969,24 @@ template <bool BATCH, bool INSTR>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_finish(MarchLaunch L0, const MarchLaunch *__restrict__ jobs,
                                                 const BatchChunk *__restrict__ chunks, uint32_t nchunks)
 {
-    __shared__ float lds[4 * kLdsCap * 64];
+    __shared__ float lds[4 * kListWords];
     const uint32_t wave = threadIdx.x >> 6;
-    float *buf = lds + wave * kLdsCap * 64 + (threadIdx.x & 63);
+    float *buf = lds + wave * kListWords + (threadIdx.x & 63);
     Counts cn;
     if (BATCH) {
         for (uint32_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
             const BatchChunk ch = chunks[c];
             const MarchLaunch *Lp = jobs + __builtin_amdgcn_readfirstlane(ch.job);
-            for (uint32_t t = wave; t < ch.ntiles; t += 4) finish_tile<INSTR, true>(*Lp, ch.tile0 + t, buf, cn);
+            for (uint32_t t = wave; t < ch.ntiles; t += 4) finish_tile<INSTR>(*Lp, ch.tile0 + t, buf, cn);
         }
     } else {
         const uint32_t T = ((L0.W + 7) / 8) * ((L0.H + 7) / 8);
         const uint32_t TA = L0.tile_buf[2 * (T + 1) + T];
-        for (uint32_t i = blockIdx.x * 4 + wave; i < TA; i += gridDim.x * 4) {
-            const uint32_t tile = L0.tile_buf[2 * (T + 1) + i];
-            if (L0.tile_buf[tile] == 2u) continue;     // finished by the march
-            finish_tile<INSTR, true>(L0, tile, buf, cn);
+        // four consecutive tiles per workgroup, runs of kXcdRun per XCD
+        for (uint32_t b = blockIdx.x; 4 * b < tile_waves_of(TA); b += gridDim.x) {
+            const uint32_t local = b >> 3, i = ((local / (kXcdRun / 4)) * 8 + (b & 7u)) * kXcdRun +
+                                               (local % (kXcdRun / 4)) * 4 + wave;
+            if (i < TA) finish_tile<INSTR>(L0, L0.tile_buf[2 * (T + 1) + i], buf, cn);
         }
     }
     flush_counts(L0.counters, cn);
@@ -1109,8 +995,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
 static hipError_t launch_finish(const MarchLaunch &L0, hipStream_t st)
 {
     const uint32_t T = ((L0.W + 7) / 8) * ((L0.H + 7) / 8);
-    const uint32_t b = (T + 3) / 4;
-    const dim3 grid(b < 2048 ? b : 2048), blk(256);
+    const uint32_t b = tile_waves_of(T) / 4;
+    const dim3 grid(b < 8192 ? b : 8192), blk(256);
     if (L0.s.instrument) hipLaunchKernelGGL((k_finish<false, true>), grid, blk, 0, st, L0, nullptr, nullptr, 0u);
     else hipLaunchKernelGGL((k_finish<false, false>), grid, blk, 0, st, L0, nullptr, nullptr, 0u);
     return hipGetLastError();
@@ -1168,7 +1054,7 @@ hipError_t launch_miss_tiles(const MarchLaunch &L, uint32_t T, hipStream_t st)
 }
 
 // The configured isotropic march of one view: schedule 1, or the tile
-// pre-pass, the persistent march and the finish of the tiles its waves left
+// pre-pass, the march and the finish of its tiles
 // (L.tile_buf and L.hit_rec set).
 hipError_t launch_tile_prepass(const MarchLaunch &L, hipStream_t st)
 {
@@ -1189,21 +1075,18 @@ static hipError_t launch_march_config(const MarchLaunch &L, hipStream_t st)
         hipLaunchKernelGGL(k_march_simple, dim3((tiles + 3) / 4), dim3(256), 0, st, L);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, st, L.band_ctr, 8);
     hipError_t e = launch_tile_prepass(L, st);
     if (e != hipSuccess) return e;
-    // enough resident waves to fill the chip; extra waves find no tile and exit
-    uint32_t blocks = L.persist_blocks ? L.persist_blocks : 1024;
-    const uint32_t need = (tiles + 3) / 4;
-    if (blocks > need) blocks = (need + 7) & ~7u;
-    const dim3 grid(blocks), blk(256);
+    // a wave per tile that may be active; beyond kMaxWaves each takes several
+    const uint32_t need = tile_waves_of(tiles);
+    const dim3 grid(need < kMaxWaves ? need : kMaxWaves), blk(64);
     const bool instr = L.s.instrument != 0;
     if (L.s.learned) {
-        if (instr) hipLaunchKernelGGL((k_march_persist<true, true>), grid, blk, 0, st, L, L.band_ctr);
-        else hipLaunchKernelGGL((k_march_persist<true, false>), grid, blk, 0, st, L, L.band_ctr);
+        if (instr) hipLaunchKernelGGL((k_march_tiles<true, true>), grid, blk, 0, st, L);
+        else hipLaunchKernelGGL((k_march_tiles<true, false>), grid, blk, 0, st, L);
     } else {
-        if (instr) hipLaunchKernelGGL((k_march_persist<false, true>), grid, blk, 0, st, L, L.band_ctr);
-        else hipLaunchKernelGGL((k_march_persist<false, false>), grid, blk, 0, st, L, L.band_ctr);
+        if (instr) hipLaunchKernelGGL((k_march_tiles<false, true>), grid, blk, 0, st, L);
+        else hipLaunchKernelGGL((k_march_tiles<false, false>), grid, blk, 0, st, L);
     }
     e = hipGetLastError();
     if (e != hipSuccess) return e;

@@ -78,9 +78,8 @@ typedef struct pm_settings {
     int32_t schedule;      /* kernel schedule, same images and counters: 0 = over the
                               8x8 tiles a ray of which enters the AABB (reference
                               mode: with a drawn depth), the others answered as misses
-                              at once -- the isotropic configured march with persistent
-                              waves, ray refill, lane groups and per-wave finishing,
-                              the anisotropic and reference marches one tile per wave
+                              at once -- one tile per wave, the isotropic configured
+                              march with lane groups and a finish kernel for its hits
                               (the product); 1 = every tile, one ray per lane to its
                               end, direct sums (the anisotropic configured march:
                               persistent waves with ray refill) -- the schedules the

@@ -1,0 +1,43 @@
+"""The candidate-list walk at its edges: lists that fit, fill up between planes,
+or are shorter than one plane or one row of the stencil.  Images and counters
+equal the oracle's, bit for bit."""
+import numpy as np
+import pytest
+
+import oracle as O
+from pmarch import scenes
+
+pytestmark = pytest.mark.gpu
+
+KEYS = dict(O.Settings._fields_)
+COUNTERS = ("rays", "rays_in_aabb", "hits", "samples", "march_samples", "march_cand")
+
+
+def _check(marcher, sc, **kw):
+    c = sc.cameras[0]
+    st = sc.settings(**kw)
+    pos, nrm, t, got = marcher.march(60, st, c.inv_pv, c.eye, c.width, c.height)
+    o = O.march(O.Grid(sc.xyz, sc.h), O.make_settings(**{k: v for k, v in st.items() if k in KEYS}), c.inv_pv, c.eye,
+                c.width, c.height)
+    assert np.array_equal(pos, o[0]) and np.array_equal(nrm, o[1]) and np.array_equal(t, o[2])
+    for k in COUNTERS:
+        assert got[k] == o[3][k], (k, got[k], o[3][k])
+    return got
+
+
+@pytest.mark.parametrize("per_cell", [1, 3, 9, 40])
+@pytest.mark.parametrize("compensated", [0, 1])
+def test_list_walk_fill(marcher, per_cell, compensated):
+    """per_cell particles in each h/2 cell: a 25-cell plane holds up to 25, 75,
+    225 and 1,000 candidates, a 5-cell row up to 200, against 36 list slots."""
+    rng = np.random.default_rng(per_cell)
+    h = 0.1
+    base = np.stack(np.meshgrid(*[np.arange(9)] * 3, indexing="ij"), -1).reshape(-1, 1, 3) * (h / 2)
+    xyz = (base + rng.uniform(0, h / 2, (base.shape[0], per_cell, 3))).reshape(-1, 3).astype(np.float32)
+    sc = scenes.tiny_scene(xyz, h, eye=(0.9, 0.8, -0.7), target=(0.22, 0.22, 0.22), width=44, height=37)
+    sc.iso *= per_cell
+    print(f"list walk, {per_cell} per cell, compensated {compensated}", flush=True)
+    marcher.set_frame(60, sc.xyz, sc.h)
+    for skip in (0, 1, 4):
+        got = _check(marcher, sc, skip_mode=skip, compensated=compensated)
+        assert got["hits"] > 100
