@@ -44,7 +44,7 @@ struct Frame {
     pm_frame_info info{};
     GridDev g{};
     DevBuf sorted, cell_start, cell_of, counts, cursor, scan_tmp, xyz, bounds_partial, bounds, scattered;
-    DevBuf empty27, dg_box, dg_cons, dg_count, coarse, bound;
+    DevBuf empty27, clear, clear_tmp, dg_box, dg_cons, dg_count, coarse, bound;
     DevBuf fsorted, fcell_start;    // march grid (cells of h/2)
     bool bound_ok = false;      // bound holds the sub-box bits for bound_iso and bound_boxes
     hipEvent_t bound_ev[2] = { nullptr, nullptr };   // around the last bound build
@@ -58,7 +58,7 @@ struct Frame {
         coarse.release();
         sorted.release(); cell_start.release(); cell_of.release(); counts.release(); cursor.release();
         scan_tmp.release(); xyz.release(); bounds_partial.release(); bounds.release(); scattered.release();
-        empty27.release(); dg_box.release(); dg_cons.release(); dg_count.release(); bound.release();
+        empty27.release(); clear.release(); clear_tmp.release(); dg_box.release(); dg_cons.release(); dg_count.release(); bound.release();
         fsorted.release(); fcell_start.release();
         for (hipEvent_t &e : bound_ev)
             if (e) { hipEventDestroy(e); e = nullptr; }
@@ -375,6 +375,11 @@ static int build_frame(pm_ctx *c, int32_t frame, const float *d_src, uint64_t n,
     HIPCHK(c, f->empty27.ensure(nc));
     HIPCHK(c, launch_empty27((const uint32_t *)f->cell_start.p, I.dims[0], I.dims[1], I.dims[2], (uint8_t *)f->empty27.p, st));
     g.empty27 = (const uint8_t *)f->empty27.p;
+    HIPCHK(c, f->clear.ensure(nc));
+    HIPCHK(c, f->clear_tmp.ensure(nc));
+    HIPCHK(c, launch_clear(g.empty27, I.dims[0], I.dims[1], I.dims[2], (uint8_t *)f->clear_tmp.p,
+                           (uint8_t *)f->clear.p, st));
+    g.clear = (const uint8_t *)f->clear.p;
     uint64_t dgn = 1;
     for (int a2 = 0; a2 < 3; a2++) {
         float cw = 1.0f * h;                            // Dataset.cpp:96

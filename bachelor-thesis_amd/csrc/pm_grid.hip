@@ -248,6 +248,57 @@ hipError_t launch_empty27(const uint32_t *cs, int32_t nx, int32_t ny, int32_t nz
     return hipGetLastError();
 }
 
+// Distance field of empty27: clear[c] is the Chebyshev distance, in cells, from
+// c to the nearest cell whose 27-neighbourhood holds a particle, at most
+// kClearMax (cells outside the grid hold none).  A ray inside a cell with
+// clear = D > 0 may cross the (2 D - 1)^3 cells around it at once.  The
+// Chebyshev distance is separable: along x, then min over d of max(|d|, .)
+// along y and z.  Two passes of at most 2 kClearMax - 1 byte loads per cell.
+static constexpr int kClearMax = 8;
+
+__global__ __launch_bounds__(kThreads) void k_clear_x(const uint8_t *__restrict__ empty27, int32_t nx, uint32_t n,
+                                                      uint8_t *__restrict__ out)
+{
+    const uint32_t c = blockIdx.x * kThreads + threadIdx.x;
+    if (c >= n) return;
+    const int32_t x = (int32_t)(c % (uint32_t)nx);
+    int D = 0;
+    for (; D < kClearMax; D++) {
+        const bool lo = x - D >= 0 && !empty27[c - (uint32_t)D], hi = x + D < nx && !empty27[c + (uint32_t)D];
+        if (lo || hi) break;
+    }
+    out[c] = (uint8_t)D;
+}
+
+__global__ __launch_bounds__(kThreads) void k_clear_yz(const uint8_t *__restrict__ in, int32_t nx, int32_t ny, int32_t nz,
+                                                       uint8_t *__restrict__ out)
+{
+    const uint32_t c = blockIdx.x * kThreads + threadIdx.x;
+    if (c >= (uint32_t)nx * (uint32_t)ny * (uint32_t)nz) return;
+    const int32_t y = (int32_t)((c / (uint32_t)nx) % (uint32_t)ny), z = (int32_t)(c / ((uint32_t)nx * (uint32_t)ny));
+    int D = in[c];
+    // rows in rings of growing max(|dy|, |dz|): none at distance >= D matters
+    for (int r = 1; r < D; r++)
+        for (int a = -r; a <= r; a++)
+            for (int side = 0; side < 4; side++) {
+                const int dy = side < 2 ? a : (side == 2 ? -r : r), dz = side < 2 ? (side == 0 ? -r : r) : a;
+                if (y + dy < 0 || y + dy >= ny || z + dz < 0 || z + dz >= nz) continue;
+                const int v = in[(int64_t)c + (int64_t)nx * (dy + (int64_t)ny * dz)];
+                D = min(D, max(r, v));
+            }
+    out[c] = (uint8_t)D;
+}
+
+hipError_t launch_clear(const uint8_t *empty27, int32_t nx, int32_t ny, int32_t nz, uint8_t *tmp, uint8_t *out,
+                        hipStream_t st)
+{
+    const uint32_t n = (uint32_t)nx * ny * nz;
+    const dim3 grid((n + kThreads - 1) / kThreads), blk(kThreads);
+    hipLaunchKernelGGL(k_clear_x, grid, blk, 0, st, empty27, nx, n, tmp);
+    hipLaunchKernelGGL(k_clear_yz, grid, blk, 0, st, (const uint8_t *)tmp, nx, ny, nz, out);
+    return hipGetLastError();
+}
+
 // Density bound per sub-box.  Every cell of the dense grid is split into
 // 8x8x8 sub-boxes (eighth boxes); sub-box (fx, fy, fz) holds the points whose
 // u = inv_h * x lies in [key + f/8, key + (f+1)/8) on every axis, and quarter

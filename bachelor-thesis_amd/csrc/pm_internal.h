@@ -160,6 +160,9 @@ hipError_t launch_depth_sprites(const SpriteLaunch &S, const float4 *pts, uint32
 hipError_t launch_depth_smooth(const float *in, float *out, uint32_t W, uint32_t H, int N, const float *K,
                                hipStream_t st);
 hipError_t launch_empty27(const uint32_t *cs, int32_t nx, int32_t ny, int32_t nz, uint8_t *out, hipStream_t st);
+// The distance field of empty27 (GridDev::clear); tmp: one byte per cell.
+hipError_t launch_clear(const uint8_t *empty27, int32_t nx, int32_t ny, int32_t nz, uint8_t *tmp, uint8_t *out,
+                        hipStream_t st);
 hipError_t launch_densitygrid(const GridDev &g, int32_t dnx, int32_t dny, int32_t dnz, uint8_t *flag_box, uint8_t *flag_cons,
                               uint32_t *count_box, hipStream_t st);
 

@@ -268,7 +268,9 @@ __device__ __forceinline__ int pm_skip_empty(const GridDev &g, float o0, float o
 // Bound skip: when the sample's eighth box (8x8x8 per cell) has its bit set
 // in g.bound, no point of the box reaches iso, so the march resumes at the
 // first sample past the box exit; when all eight eighth boxes of its quarter
-// box (4x4x4 per cell) are set, past the quarter box's exit.  Every sample it
+// box (4x4x4 per cell) are set, past the quarter box's exit; and when the cells
+// around it are clear of particles' neighbourhoods (g.clear = D > 0: every bit
+// of the (2 D - 1)^3 cells is set), past those cells' exit.  Every sample it
 // passes lies in a set box (within the widening the bound was computed for)
 // and would have been below iso.  Returns the next sample index (r.k when
 // there is nothing to skip).
@@ -293,21 +295,17 @@ __device__ __forceinline__ int pm_skip_bound(const GridDev &g, float o0, float o
     const int f2 = min(7, (int)((u2 - (float)k2) * 8.0f));
     const uint32_t l = (uint32_t)((f0 >> 1) + 4 * (f1 >> 1) + 16 * (f2 >> 1));
     const uint64_t cell = (uint64_t)cx + (uint64_t)g.nx * ((uint64_t)cy + (uint64_t)g.ny * (uint64_t)cz);
-    const uint32_t byte = (uint32_t)(g.bound[8 * cell + (l >> 3)] >> (8 * (l & 7u))) & 0xffu;
-    if (byte == 0u) return r.k;
-    float l0, l1, l2, span;
-    if (byte == 0xffu) {   // the whole quarter box
-        l0 = (float)k0 + 0.25f * (float)(f0 >> 1);
-        l1 = (float)k1 + 0.25f * (float)(f1 >> 1);
-        l2 = (float)k2 + 0.25f * (float)(f2 >> 1);
-        span = 0.25f;
-    } else {
-        if (!((byte >> ((f0 & 1) + 2 * (f1 & 1) + 4 * (f2 & 1))) & 1u)) return r.k;
-        l0 = (float)k0 + 0.125f * (float)f0;
-        l1 = (float)k1 + 0.125f * (float)f1;
-        l2 = (float)k2 + 0.125f * (float)f2;
-        span = 0.125f;
-    }
+    const int clear = (int)g.clear[cell];
+    const uint32_t byte = (uint32_t)((const uint8_t *)g.bound)[64 * cell + l];
+    const bool whole = byte == 0xffu;
+    if (!whole && !((byte >> ((f0 & 1) + 2 * (f1 & 1) + 4 * (f2 & 1))) & 1u)) return r.k;
+    // the box to cross: its low corner is k + unit * (m0, m1, m2) cells
+    const bool cells = whole && clear > 0;
+    const int sh = whole ? 1 : 0;
+    const float unit = cells ? 1.0f : (whole ? 0.25f : 0.125f);
+    const float span = cells ? (float)(2 * clear - 1) : unit;
+    const int m0 = cells ? 1 - clear : f0 >> sh, m1 = cells ? 1 - clear : f1 >> sh, m2 = cells ? 1 - clear : f2 >> sh;
+    const float l0 = (float)k0 + unit * (float)m0, l1 = (float)k1 + unit * (float)m1, l2 = (float)k2 + unit * (float)m2;
     float texit = INFINITY;
     texit = pm_box_exit(l0 * g.h, (l0 + span) * g.h, o0, r.d0, r.id0, texit);
     texit = pm_box_exit(l1 * g.h, (l1 + span) * g.h, o1, r.d1, r.id1, texit);

@@ -1,6 +1,7 @@
-"""The candidate-list walk at its edges: lists that fit, fill up between planes,
-or are shorter than one plane or one row of the stencil.  Images and counters
-equal the oracle's, bit for bit."""
+"""The candidate-list walk and the skip distance field at their edges: lists that
+fit, fill up between planes, or are shorter than one plane or one row of the
+stencil; rays that cross many clear cells at once.  Images and counters equal
+the oracle's, bit for bit."""
 import numpy as np
 import pytest
 
@@ -41,3 +42,22 @@ def test_list_walk_fill(marcher, per_cell, compensated):
     for skip in (0, 1, 4):
         got = _check(marcher, sc, skip_mode=skip, compensated=compensated)
         assert got["hits"] > 100
+
+
+@pytest.mark.parametrize("gap", [1, 2, 9, 40])
+def test_skip_over_clear_cells(marcher, gap):
+    """Three small clusters `gap` cells apart, so rays cross clear regions of
+    every radius up to and beyond the field's largest; a grid side not a
+    multiple of anything."""
+    rng = np.random.default_rng(gap)
+    h = 0.1
+    centres = np.array([[0, 0, 0], [gap + 4, 0.4, 0.3], [0.2, gap + 4, gap + 3]]) * h
+    xyz = np.concatenate([c + rng.uniform(-1.6 * h, 1.6 * h, (300, 3)) for c in centres]).astype(np.float32)
+    mid = xyz.mean(0)
+    ext = float((xyz.max(0) - xyz.min(0)).max())
+    sc = scenes.tiny_scene(xyz, h, eye=mid + np.array([0.9, 0.7, -1.1]) * ext, target=mid, width=71, height=53)
+    print(f"skip over {gap} clear cells", flush=True)
+    marcher.set_frame(60, sc.xyz, sc.h)
+    for boxes in (0, 1):
+        got = _check(marcher, sc, skip_mode=4, bound_boxes=boxes)
+        assert got["hits"] > 10
