@@ -343,6 +343,11 @@ static int build_frame(pm_ctx *c, int32_t frame, const float *d_src, uint64_t n,
     fa.sorted = (float4 *)f->fsorted.p;
     fa.cell_start = (uint32_t *)f->fcell_start.p;
     HIPCHK(c, launch_grid_build(fa, st));
+    // occupied march-grid cells (into counts, which the builds are done with)
+    uint32_t occupied = 0;
+    HIPCHK(c, launch_zero_u32((uint32_t *)f->counts.p, 1, st));
+    HIPCHK(c, launch_occupied((const uint32_t *)f->fcell_start.p, (uint32_t)fnc, (uint32_t *)f->counts.p, st));
+    HIPCHK(c, hipMemcpyAsync(&occupied, f->counts.p, sizeof(occupied), hipMemcpyDeviceToHost, st));
     HIPCHK(c, hipEventRecord(e1, st));
     HIPCHK(c, hipEventSynchronize(e1));
     float ms = 0.f;
@@ -370,6 +375,7 @@ static int build_frame(pm_ctx *c, int32_t frame, const float *d_src, uint64_t n,
     g.fox = I.forigin[0]; g.foy = I.forigin[1]; g.foz = I.forigin[2];
     g.fnx = I.fdims[0]; g.fny = I.fdims[1]; g.fnz = I.fdims[2];
     g.inv_hf = inv_hf;
+    g.sparse = n <= (uint64_t)kSparsePerCell * occupied;
 
     // skip structures: empty 27-neighbourhoods and the reference DensityGrid
     HIPCHK(c, f->empty27.ensure(nc));
@@ -1052,6 +1058,8 @@ int pm_batch_set(pm_ctx *c, const pm_settings *s, const pm_view *views, uint32_t
     B.base.s = *s;
     B.base.inv_step = 1.0f / s->step;
     B.base.counters = (unsigned long long *)c->d_counters.p;
+    B.sparse = 1;
+    for (const MarchLaunch &J : jobs) B.sparse = B.sparse && J.g.sparse;
     HIPCHK(c, c->b_hits.ensure(sizeof(uint4) * npx));
     if (s->learned) {
         set_learned(c, s, B.base);

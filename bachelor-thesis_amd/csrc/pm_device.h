@@ -42,7 +42,9 @@ struct GridDev {
     int32_t fox, foy, foz;    // fine key of fine cell (0,0,0)
     int32_t fnx, fny, fnz;
     float inv_hf;             // 2 / h
+    int sparse;               // at most kSparsePerCell particles per occupied fine cell on average
 };
+static constexpr uint32_t kSparsePerCell = 3;
 
 // ---- march-grid stencil ----
 // In fine-cell units u = inv_hf x the sample sits at offset f in [0, 1] inside
@@ -630,6 +632,148 @@ __device__ __forceinline__ Cdiff6 pm_cdiff6_lds(const GridDev &g, float qx, floa
 #pragma unroll
     for (int k = 0; k < 6; k++) out.v[k] = comp ? a.s[k] + a.c[k] : a.s[k];
     return out;
+}
+
+// ---- one list for all samples of a hit ----
+// The bisection, the FP64 step and the six central differences of a hit sample
+// points within a short segment [a, b] (one march step) and eps around it.  One
+// walk lists every particle within h of any of them, in the canonical order;
+// each sample then takes the list with its own r^2 < h^2 test, so its sum is
+// its single-sample sum, bit for bit, for about 25 candidates read instead of a
+// 25-row walk of 41 each (1 M dam break).  lst as in pm_density32_list.  False
+// (for all calling lanes, which then walk for each sample: both in one wave
+// would cost both) when some lane's box leaves the grid or spans more than two
+// cells on an axis, or its list does not fit CAP.
+template <int CAP>
+__device__ __forceinline__ bool pm_list_segment(const GridDev &g, const float a[3], const float b[3], float eps,
+                                                uint32_t *lst, int &n, uint32_t &cand)
+{
+    float lo[3], hi[3], c[3], l2 = 0.0f, big = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        // the samples' coordinates are rounded: a few ulps of room
+        big = fmaxf(big, fmaxf(fabsf(a[k]), fabsf(b[k])));
+        c[k] = 0.5f * (a[k] + b[k]);
+        const float e = b[k] - a[k];
+        l2 += e * e;
+    }
+    const float room = eps + big * 0x1p-20f;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        lo[k] = fminf(a[k], b[k]) - room;
+        hi[k] = fmaxf(a[k], b[k]) + room;
+    }
+    const float R = (g.h + 0.5f * sqrtf(l2) + room) * 1.0009765625f, R2 = R * R;
+    BoxWalk w;
+    const bool in = pm_box_begin(g, lo, hi, w) && w.nx <= 6 && w.ny <= 6 && w.nz <= 6;
+    if (__ballot(!in) != 0) return false;
+    int f = 0;                                  // entries [0, f) passed the test, [f, n) are untested
+    n = 0;
+    auto compact = [&]() {
+        _Pragma("unroll 1") for (int i = f; __ballot(i < n) != 0; i += 4) {
+            uint32_t l[4];
+            float d2[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                l[u] = lst[(i + u) * 64];
+                const float4 *const p = g.fsorted + (i + u < n ? l[u] : 0u);
+                const float rx = p->x - c[0], ry = p->y - c[1], rz = p->z - c[2];
+                d2[u] = (rx * rx + ry * ry) + rz * rz;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                lst[f * 64] = l[u];             // f <= i + u: a slot already read
+                f += (i + u < n && d2[u] < R2) ? 1 : 0;
+            }
+        }
+        n = f;
+    };
+    uint32_t pb[6], pe[6], qb[6], qe[6];
+    auto plane = [&](int jz, uint32_t (&b_)[6], uint32_t (&e_)[6]) {
+#pragma unroll
+        for (int k = 0; k < 6; k++) {
+            pm_box_row(g, w, k, jz, b_[k], e_[k]);
+            if (k >= w.ny) e_[k] = b_[k];
+        }
+    };
+    plane(0, pb, pe);
+    _Pragma("unroll 1") for (int jz = 0; __ballot(jz < w.nz) != 0; jz++) {
+        plane(jz + 1, qb, qe);                  // next plane's bounds in flight (none past the box)
+        int mp = 0;
+#pragma unroll
+        for (int k = 0; k < 6; k++) mp += (int)(pe[k] - pb[k]);
+        cand += (uint32_t)mp;
+        if (__ballot(mp != 0) != 0) {
+            bool fits = true;                   // wave-uniform
+            if (__ballot(n + mp > CAP) != 0) {
+                compact();
+                fits = __ballot(n + mp > CAP) == 0;
+            }
+#pragma unroll
+            for (int k = 0; k < 6; k++) {
+                const int m = (int)(pe[k] - pb[k]);
+                if (!fits) {                    // row by row
+                    if (__ballot(n + m > CAP) != 0) compact();
+                    if (__ballot(n + m > CAP) != 0) return false;
+                }
+                uint32_t *const q = lst + n * 64;
+#pragma unroll
+                for (int u = 0; u < 4; u++) q[u * 64] = pb[k] + (uint32_t)u;
+                if (__ballot(m > 4) != 0)
+                    for (int u = 4; u < m; u++) q[u * 64] = pb[k] + (uint32_t)u;
+                n += m;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 6; k++) { pb[k] = qb[k]; pe[k] = qe[k]; }
+    }
+    compact();
+    return true;
+}
+
+// pm_density64's sum over the listed candidates.
+__device__ __forceinline__ double pm_list_density64(const GridDev &g, const uint32_t *lst, int n, double qx, double qy,
+                                                    double qz)
+{
+    double acc = 0.0;
+    _Pragma("unroll 1") for (int i = 0; __ballot(i < n) != 0; i += 4) {
+        float4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const uint32_t l = lst[(i + u) * 64];
+            v[u] = g.fsorted[i + u < n ? l : 0u];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const double rx = (double)v[u].x - qx, ry = (double)v[u].y - qy, rz = (double)v[u].z - qz;
+            const double r2 = (rx * rx + ry * ry) + rz * rz;
+            if (i + u < n && r2 < g.h2_d) acc += pm_W_in_d(r2, g.hinv_d, g.sig_d);
+        }
+    }
+    return acc;
+}
+
+// The six central-difference densities over the listed candidates.
+__device__ __forceinline__ void pm_list_cdiff6(const GridDev &g, const uint32_t *lst, int n, const float x[3], float eps,
+                                               bool comp, float v6[6])
+{
+    const float xp[3] = { x[0] + eps, x[1] + eps, x[2] + eps }, xm[3] = { x[0] - eps, x[1] - eps, x[2] - eps };
+    Acc6 a;
+#pragma unroll
+    for (int k = 0; k < 6; k++) { a.s[k] = 0.0f; a.c[k] = 0.0f; }
+    _Pragma("unroll 1") for (int i = 0; __ballot(i < n) != 0; i += 2) {
+        float4 v[2];
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const uint32_t l = lst[(i + u) * 64];
+            v[u] = g.fsorted[i + u < n ? l : 0u];
+        }
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+            if (i + u < n) pm_acc6(g, v[u].x, v[u].y, v[u].z, x, xp, xm, comp, a);
+    }
+#pragma unroll
+    for (int k = 0; k < 6; k++) v6[k] = comp ? a.s[k] + a.c[k] : a.s[k];
 }
 
 // FP64 density; the stencil is chosen from the FP32-rounded point.

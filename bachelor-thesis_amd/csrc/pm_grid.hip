@@ -248,6 +248,28 @@ hipError_t launch_empty27(const uint32_t *cs, int32_t nx, int32_t ny, int32_t nz
     return hipGetLastError();
 }
 
+// Occupied cells of a grid: one atomic per workgroup.
+__global__ __launch_bounds__(kThreads) void k_occupied(const uint32_t *__restrict__ cs, uint32_t n, uint32_t *__restrict__ out)
+{
+    __shared__ uint32_t sum;
+    if (threadIdx.x == 0) sum = 0;
+    __syncthreads();
+    uint32_t cnt = 0;
+    for (uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kThreads)
+        cnt += cs[i + 1] != cs[i] ? 1u : 0u;
+    for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off, 64);
+    if ((threadIdx.x & 63) == 0) atomicAdd(&sum, cnt);
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(out, sum);
+}
+
+hipError_t launch_occupied(const uint32_t *cs, uint32_t n, uint32_t *out, hipStream_t st)
+{
+    const uint32_t b = (n + 8 * kThreads - 1) / (8 * kThreads);
+    hipLaunchKernelGGL(k_occupied, dim3(b < 512 ? b : 512), dim3(kThreads), 0, st, cs, n, out);
+    return hipGetLastError();
+}
+
 // Distance field of empty27: clear[c] is the Chebyshev distance, in cells, from
 // c to the nearest cell whose 27-neighbourhood holds a particle, at most
 // kClearMax (cells outside the grid hold none).  A ray inside a cell with

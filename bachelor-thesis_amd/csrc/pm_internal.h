@@ -89,6 +89,7 @@ struct BatchLaunch {
     const BatchChunk *chunks;
     uint32_t nchunks;
     uint32_t *chunk_ctr;
+    int sparse;                // every job's frame is (GridDev::sparse)
 };
 hipError_t launch_bound_grid(const GridDev &g, float iso, bool quarter_only, uint64_t *out, hipStream_t st);
 hipError_t launch_march_batch(const BatchLaunch &B, uint32_t blocks, hipStream_t st);
@@ -160,6 +161,8 @@ hipError_t launch_depth_sprites(const SpriteLaunch &S, const float4 *pts, uint32
 hipError_t launch_depth_smooth(const float *in, float *out, uint32_t W, uint32_t H, int N, const float *K,
                                hipStream_t st);
 hipError_t launch_empty27(const uint32_t *cs, int32_t nx, int32_t ny, int32_t nz, uint8_t *out, hipStream_t st);
+// Adds the number of non-empty cells among cs's n to *out.
+hipError_t launch_occupied(const uint32_t *cs, uint32_t n, uint32_t *out, hipStream_t st);
 // The distance field of empty27 (GridDev::clear); tmp: one byte per cell.
 hipError_t launch_clear(const uint8_t *empty27, int32_t nx, int32_t ny, int32_t nz, uint8_t *tmp, uint8_t *out,
                         hipStream_t st);

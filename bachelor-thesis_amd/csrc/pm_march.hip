@@ -233,6 +233,11 @@ __device__ __forceinline__ void group_finish(const MarchLaunch &L, RayState &r, 
 // keeps 16 waves on a CU.
 static constexpr int kListCap = 36;
 static constexpr int kListWords = (kListCap + kListPad) * 64;   // per wave
+// The finish kernel's list of a whole segment, unfiltered row by row: in the
+// 1 M dam break the filtered lists hold up to 41 candidates and a row up to
+// about 10 more.  Measured there (finish kernel): 36 slots 433 us, 48 355,
+// 52 226, 56 223, 60 231 (14 KB of LDS leave 11 waves on a CU).
+static constexpr int kFinCap = 56, kFinWords = (kFinCap + kListPad) * 64;
 
 struct DensList {
     const GridDev *g;
@@ -561,8 +566,8 @@ __device__ __forceinline__ void wave_propose_step(const MarchLaunch &L, RayState
 // walk, or the sum of gradW) and the pixel's outputs.  Every lane of a wave does the same kind of work
 // and none of the march's state is held, so this runs packed and short; the
 // march kernels keep only the phases that decide where the hit is.
-template <bool INSTR>
-__device__ __forceinline__ void finish_hit(const MarchLaunch &L, uint32_t px, uint32_t py, uint4 rec, float *buf,
+template <bool INSTR, bool LIST>
+__device__ __forceinline__ void finish_hit(const MarchLaunch &L, uint32_t px, uint32_t py, uint4 rec, uint32_t *lst,
                                            Counts &cn)
 {
     const pm_settings &s = L.s;
@@ -573,27 +578,51 @@ __device__ __forceinline__ void finish_hit(const MarchLaunch &L, uint32_t px, ui
     pm_ray_dir(L, px, py, d);
     const float o0 = L.cam[0], o1 = L.cam[1], o2 = L.cam[2];
     float xs[3], th;
+    const bool comp = s.compensated != 0;
     const bool fp64 = s.final_fp64 && s.bisect_iters > 0;
-    if (rec.x & 2u) {
+    const bool bracket = (rec.x & 2u) != 0;
+    const float e = s.normal_mode == PM_NORMAL_CDIFF ? s.normal_eps : 0.0f;
+    int n = 0;
+    bool listed = false;
+    if (LIST) {
+        const float a[3] = { o0 + lo * d[0], o1 + lo * d[1], o2 + lo * d[2] };
+        const float b[3] = { o0 + hi * d[0], o1 + hi * d[1], o2 + hi * d[2] };
+        uint32_t cand = 0;
+        listed = pm_list_segment<kFinCap>(g, a, b, fabsf(e), lst, n, cand);
+        if (listed) cn.cand += cand;
+    }
+    if (bracket) {
         const int n32 = fp64 ? s.bisect_iters - 1 : s.bisect_iters;
 #pragma unroll 1
         for (int it = 0; it < n32; it++) {
             const float tm = (lo + hi) * 0.5f;
             const float qx = o0 + tm * d[0], qy = o1 + tm * d[1], qz = o2 + tm * d[2];
-            uint32_t cand = 0;
-            const float rho = pm_density32_list<kListCap>(g, qx, qy, qz, s.compensated != 0, (uint32_t *)buf, cand);
-            count_sample<INSTR>(g, qx, qy, qz, cand, false, cn);
+            uint32_t cand = 0, nsup = 0;
+            float rho;
+            if (listed) {
+                float sum = 0.0f, c = 0.0f;
+                pm_list_density(g, lst, n, qx, qy, qz, sum, c, nsup);
+                rho = comp ? sum + c : sum;
+                cn.samples++;
+                if (INSTR) {
+                    cn.cst += pm_stencil_cand(g, qx, qy, qz);
+                    cn.c27 += pm_cand27(g, qx, qy, qz);
+                }
+            } else {
+                rho = pm_density32_list<kListCap>(g, qx, qy, qz, comp, lst, cand);
+                count_sample<INSTR>(g, qx, qy, qz, cand, false, cn);
+            }
             if (rho >= s.iso) hi = tm; else lo = tm;
         }
         if (!fp64) lo = hi = (lo + hi) * 0.5f;
     }
-    if ((rec.x & 2u) && fp64) {
+    if (bracket && fp64) {
         // the last bisection step in double (RayMarcher.cpp:316-326 in FP64)
         const double tmd = ((double)lo + (double)hi) * 0.5;
         const double x = (double)o0 + tmd * (double)d[0];
         const double y = (double)o1 + tmd * (double)d[1];
         const double z = (double)o2 + tmd * (double)d[2];
-        const double rho = pm_density64(g, x, y, z);
+        const double rho = listed ? pm_list_density64(g, lst, n, x, y, z) : pm_density64(g, x, y, z);
         cn.samples++;
         if (INSTR) {
             cn.cst += pm_stencil_cand(g, (float)x, (float)y, (float)z);
@@ -617,25 +646,33 @@ __device__ __forceinline__ void finish_hit(const MarchLaunch &L, uint32_t px, ui
         pm_sum_gradw(g, xs[0], xs[1], xs[2], sx, sy, sz, cand);
         pm_normalize(sx, sy, sz, nx, ny, nz);
     } else {
-        const bool comp = s.compensated != 0;
-        const float e = s.normal_eps;
         float gv[3];
-        const Cdiff6 o = pm_cdiff6_lds<kLdsCap>(g, xs[0], xs[1], xs[2], e, buf, comp);
-        if (o.cand != 0xffffffffu) {
+        if (listed) {
+            float v[6];
+            pm_list_cdiff6(g, lst, n, xs, e, comp, v);
             cn.samples += 6;
-            cn.cand += o.cand;
-            gv[0] = o.v[0] - o.v[1]; gv[1] = o.v[2] - o.v[3]; gv[2] = o.v[4] - o.v[5];
+            gv[0] = v[0] - v[1]; gv[1] = v[2] - v[3]; gv[2] = v[4] - v[5];
         } else {
-            // the fused walk's cells leave the grid: +x, -x, +y, -y, +z, -z one at a time
+            const Cdiff6 o = pm_cdiff6_lds<kLdsCap>(g, xs[0], xs[1], xs[2], e, (float *)lst, comp);
+            if (o.cand != 0xffffffffu) {
+                cn.samples += 6;
+                cn.cand += o.cand;
+                gv[0] = o.v[0] - o.v[1]; gv[1] = o.v[2] - o.v[3]; gv[2] = o.v[4] - o.v[5];
+            } else {
+                // the fused walk's cells leave the grid: +x, -x, +y, -y, +z, -z one at a time
+#pragma unroll 1
+                for (int k = 0; k < 6; k++) {
+                    const float ek = (k & 1) ? -e : e;
+                    const float q0 = k < 2 ? xs[0] + ek : xs[0], q1 = (k >> 1) == 1 ? xs[1] + ek : xs[1],
+                                q2 = k > 3 ? xs[2] + ek : xs[2];
+                    uint32_t cand = 0;
+                    const float rho = pm_density32_list<kListCap>(g, q0, q1, q2, comp, lst, cand);
+                    cn.samples++;
+                    cn.cand += cand;
 #pragma unroll
-            for (int k = 0; k < 6; k++) {
-                float q[3] = { xs[0], xs[1], xs[2] };
-                q[k >> 1] = (k & 1) ? xs[k >> 1] - e : xs[k >> 1] + e;
-                uint32_t cand = 0;
-                const float rho = pm_density32_list<kListCap>(g, q[0], q[1], q[2], comp, (uint32_t *)buf, cand);
-                cn.samples++;
-                cn.cand += cand;
-                if (k & 1) gv[k >> 1] -= rho; else gv[k >> 1] = rho;
+                    for (int a = 0; a < 3; a++)
+                        if ((k >> 1) == a) gv[a] = (k & 1) ? gv[a] - rho : rho;
+                }
             }
         }
         if (INSTR) {
@@ -663,14 +700,14 @@ __device__ __forceinline__ void finish_hit(const MarchLaunch &L, uint32_t px, ui
 
 // One 8x8 tile per wave, one pixel per lane: the lanes whose pixel holds a
 // hit record finish it.
-template <bool INSTR>
-__device__ __forceinline__ void finish_tile(const MarchLaunch &L, uint32_t tile, float *buf, Counts &cn)
+template <bool INSTR, bool LIST>
+__device__ __forceinline__ void finish_tile(const MarchLaunch &L, uint32_t tile, uint32_t *lst, Counts &cn)
 {
     const uint32_t lane = threadIdx.x & 63, tiles_x = (L.W + 7) / 8;
     const uint32_t px = (tile % tiles_x) * 8 + (lane & 7u), py = (tile / tiles_x) * 8 + (lane >> 3);
     if (px >= L.W || py >= L.H) return;
     const uint4 rec = L.hit_rec[py * L.W + px];
-    if (rec.x & 1u) finish_hit<INSTR>(L, px, py, rec, buf, cn);
+    if (rec.x & 1u) finish_hit<INSTR, LIST>(L, px, py, rec, lst, cn);
 }
 
 // Active tile i of a launch's list for wave `w` of the grid (one-wave
@@ -685,8 +722,9 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t w)
 }
 
 // Workgroups for T tiles (all of them may be active): a multiple of a full
-// round of runs; beyond kMaxWaves each wave takes several tiles.
-static constexpr uint32_t kMaxWaves = 16384;
+// round of runs; beyond kMaxWaves each wave takes several tiles (16,384 waves
+// left some with two tiles of the 4K pool: 4.9 against 3.6 ms in the finish).
+static constexpr uint32_t kMaxWaves = 65536;
 __host__ __device__ __forceinline__ uint32_t tile_waves_of(uint32_t T)
 {
     return (T + 8 * kXcdRun - 1) / (8 * kXcdRun) * (8 * kXcdRun);
@@ -961,44 +999,49 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
     flush_counts(B.base.counters, cn);
 }
 
-// Single launch: the active tiles; batch: the tiles of
-// the chunks, one chunk per workgroup at a time.  Four waves per SIMD
-// (registers capped at 128) hide more of the walks' latency than three would
-// at 150 registers.
-template <bool BATCH, bool INSTR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_finish(MarchLaunch L0, const MarchLaunch *__restrict__ jobs,
+// Single launch: a wave per active tile; batch: a wave per chunk of tiles.
+// LIST: a hit's samples share one candidate list.  It pays where the lists fit
+// (GridDev::sparse, at most 3 particles per occupied h/2 cell: 466 -> 223 us on
+// the 1 M dam break, 1.4 per cell); in denser frames (4 M pool, 8 per cell) most
+// lists overflow after they were built and their LDS costs waves (3.6 ms walking
+// for each sample, 5.3 to 7.0 ms with lists of 44 to 92 slots), so those walk.
+// Registers are capped for four waves per SIMD.
+template <bool BATCH, bool INSTR, bool LIST>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LIST ? 3 : 4, 8))) void k_finish(MarchLaunch L0, const MarchLaunch *__restrict__ jobs,
                                                 const BatchChunk *__restrict__ chunks, uint32_t nchunks)
 {
-    __shared__ float lds[4 * kListWords];
-    const uint32_t wave = threadIdx.x >> 6;
-    float *buf = lds + wave * kListWords + (threadIdx.x & 63);
+    __shared__ uint32_t lds[LIST ? kFinWords : kListWords];
+    uint32_t *lst = lds + threadIdx.x;
     Counts cn;
+    bool any = false;
     if (BATCH) {
         for (uint32_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
             const BatchChunk ch = chunks[c];
             const MarchLaunch *Lp = jobs + __builtin_amdgcn_readfirstlane(ch.job);
-            for (uint32_t t = wave; t < ch.ntiles; t += 4) finish_tile<INSTR>(*Lp, ch.tile0 + t, buf, cn);
+            for (uint32_t t = 0; t < ch.ntiles; t++) finish_tile<INSTR, LIST>(*Lp, ch.tile0 + t, lst, cn);
+            any = true;
         }
     } else {
         const uint32_t T = ((L0.W + 7) / 8) * ((L0.H + 7) / 8);
-        const uint32_t TA = L0.tile_buf[2 * (T + 1) + T];
-        // four consecutive tiles per workgroup, runs of kXcdRun per XCD
-        for (uint32_t b = blockIdx.x; 4 * b < tile_waves_of(TA); b += gridDim.x) {
-            const uint32_t local = b >> 3, i = ((local / (kXcdRun / 4)) * 8 + (b & 7u)) * kXcdRun +
-                                               (local % (kXcdRun / 4)) * 4 + wave;
-            if (i < TA) finish_tile<INSTR>(L0, L0.tile_buf[2 * (T + 1) + i], buf, cn);
+        const uint32_t *order = L0.tile_buf + 2 * (T + 1), TA = order[T];
+        for (uint32_t w = blockIdx.x; w < tile_waves_of(TA); w += gridDim.x) {
+            const uint32_t i = xcd_tile(w);
+            if (i >= TA) continue;
+            finish_tile<INSTR, LIST>(L0, order[i], lst, cn);
+            any = true;
         }
     }
-    flush_counts(L0.counters, cn);
+    if (any) flush_counts(L0.counters, cn);
 }
 
 static hipError_t launch_finish(const MarchLaunch &L0, hipStream_t st)
 {
     const uint32_t T = ((L0.W + 7) / 8) * ((L0.H + 7) / 8);
-    const uint32_t b = tile_waves_of(T) / 4;
-    const dim3 grid(b < 8192 ? b : 8192), blk(256);
-    if (L0.s.instrument) hipLaunchKernelGGL((k_finish<false, true>), grid, blk, 0, st, L0, nullptr, nullptr, 0u);
-    else hipLaunchKernelGGL((k_finish<false, false>), grid, blk, 0, st, L0, nullptr, nullptr, 0u);
+    const uint32_t need = tile_waves_of(T);
+    const dim3 grid(need < kMaxWaves ? need : kMaxWaves), blk(64);
+    if (L0.s.instrument) hipLaunchKernelGGL((k_finish<false, true, true>), grid, blk, 0, st, L0, nullptr, nullptr, 0u);
+    else if (L0.g.sparse) hipLaunchKernelGGL((k_finish<false, false, true>), grid, blk, 0, st, L0, nullptr, nullptr, 0u);
+    else hipLaunchKernelGGL((k_finish<false, false, false>), grid, blk, 0, st, L0, nullptr, nullptr, 0u);
     return hipGetLastError();
 }
 
@@ -1008,8 +1051,9 @@ hipError_t launch_march_batch(const BatchLaunch &B, uint32_t blocks, hipStream_t
     else hipLaunchKernelGGL((k_march_batch<false>), dim3(blocks), dim3(256), 0, st, B);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const uint32_t fb = B.nchunks < 8192 ? B.nchunks : 8192;
-    hipLaunchKernelGGL((k_finish<true, false>), dim3(fb), dim3(256), 0, st, B.base, B.jobs, B.chunks, B.nchunks);
+    const uint32_t fb = B.nchunks < kMaxWaves ? B.nchunks : kMaxWaves;
+    if (B.sparse) hipLaunchKernelGGL((k_finish<true, false, true>), dim3(fb), dim3(64), 0, st, B.base, B.jobs, B.chunks, B.nchunks);
+    else hipLaunchKernelGGL((k_finish<true, false, false>), dim3(fb), dim3(64), 0, st, B.base, B.jobs, B.chunks, B.nchunks);
     return hipGetLastError();
 }
 

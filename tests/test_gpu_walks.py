@@ -61,3 +61,19 @@ def test_skip_over_clear_cells(marcher, gap):
     for boxes in (0, 1):
         got = _check(marcher, sc, skip_mode=4, bound_boxes=boxes)
         assert got["hits"] > 10
+
+
+@pytest.mark.parametrize("eps,bisect,fp64", [(0.1 / 32, 8, 1), (0.02, 8, 1), (0.1 / 32, 0, 0), (0.1 / 32, 3, 0),
+                                             (-0.1 / 32, 2, 1), (0.0, 8, 1)])
+@pytest.mark.parametrize("step", [0.0125, 0.04, 0.3])
+def test_finish_list(marcher, eps, bisect, fp64, step):
+    """A hit's samples from one list: short steps (the list), steps and offsets
+    whose box spans more cells than the list takes (the walk for each sample),
+    no bisection, an offset of zero or below it; hits at the grid's edge."""
+    sc = scenes.lattice_cube(3, n_side=9, spacing=0.05, width=61, height=43)
+    sc.step, sc.normal_eps = step, eps
+    print(f"finish list eps {eps} bisect {bisect} fp64 {fp64} step {step}", flush=True)
+    marcher.set_frame(60, sc.xyz, sc.h)
+    for comp in (0, 1):
+        got = _check(marcher, sc, skip_mode=4, bisect_iters=bisect, final_fp64=fp64, compensated=comp)
+        assert got["hits"] > 50
