@@ -730,8 +730,23 @@ __host__ __device__ __forceinline__ uint32_t tile_waves_of(uint32_t T)
     return (T + 8 * kXcdRun - 1) / (8 * kXcdRun) * (8 * kXcdRun);
 }
 
-// Schedule 0: one wave per active 8x8 tile, one ray per lane up to the ray's
-// hit or miss.  As rays end, the others spread over the idle lanes (lane
+// Waves per tile of the march, as a power of two, for TA active tiles.  The
+// chip holds about 4,096 of its waves: with fewer tiles a launch lasts as long
+// as its longest tile (a ray along a face takes a hundred samples), so each tile
+// is split over four waves whose rays start with four lanes each; the samples
+// evaluated past a crossing cost less than the idle SIMDs.  March kernel for
+// one / two / four / eight waves per tile: 640x480 lattice cube (3,200 tiles)
+// 493 / 354 / 268 / 354 us, 96x64 213 / 156 / 130 / 152 us, 1080p dam break
+// (4,300) 331 / 297 / 318 / 448 us, 4K pool (19,000) 2,490 / 2,578 / 2,899 /
+// 5,184 us.
+static constexpr uint32_t kResidentWaves = 4096, kMaxSplit = 2;
+__device__ __forceinline__ uint32_t tile_split(uint32_t TA)
+{
+    return TA < kResidentWaves ? 2u : (TA < 2 * kResidentWaves ? 1u : 0u);
+}
+
+// Schedule 0: a wave per active 8x8 tile (or several, tile_split), one ray per
+// lane or lane group up to the ray's hit or miss.  As rays end, the others spread over the idle lanes (lane
 // groups), so the tile's last rays take several samples per step.  The tiles
 // come from the list by position: no queue.  (Persistent waves that drew tiles
 // from counters spent 0.30 of 0.64 ms at 1080p on the counters: 4,096 waves
@@ -753,16 +768,19 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     const bool comp = L.s.compensated != 0;
     Counts cn;
     bool any = false;
-    for (uint32_t w = blockIdx.x; w < tile_waves_of(TA); w += gridDim.x) {
+    const uint32_t sub = LEARNED ? 0u : tile_split(TA);
+    for (uint32_t w = blockIdx.x; w < tile_waves_of(TA << sub); w += gridDim.x) {
         const uint32_t i = xcd_tile(w);
-        if (i >= TA) continue;
+        if (i >= TA << sub) continue;
         any = true;
-        const uint32_t tile = order[i];
-        const uint32_t px = (tile % tiles_x) * 8 + (lane & 7u), py = (tile / tiles_x) * 8 + (lane >> 3);
+        const uint32_t tile = order[i >> sub], part = i & ((1u << sub) - 1u), rr = lane >> sub;
+        const uint32_t lw = sub >= 2 ? 2u : 3u, np = 3u - lw;   // a part is 2^lw pixels wide, 2^np in a row
+        const uint32_t px = (tile % tiles_x) * 8 + (part & ((1u << np) - 1u)) * (1u << lw) + (rr & ((1u << lw) - 1u));
+        const uint32_t py = (tile / tiles_x) * 8 + (part >> np) * (64u >> sub >> lw) + (rr >> lw);
         RayState r{};
         r.phase = PH_DONE;
-        if (px < L.W && py < L.H) ray_setup(L, r, px, py, cn);
-        int G = 1;
+        int G = 1 << sub;
+        if (px < L.W && py < L.H) ray_setup(L, r, px, py, cn, (lane & (uint32_t)(G - 1)) == 0);
         while (__ballot(r.phase != PH_DONE) != 0) {
             // The network is batched across the wave (the wave pays for it
             // whenever any lane needs it): it runs once half of the busy
@@ -1122,7 +1140,7 @@ static hipError_t launch_march_config(const MarchLaunch &L, hipStream_t st)
     hipError_t e = launch_tile_prepass(L, st);
     if (e != hipSuccess) return e;
     // a wave per tile that may be active; beyond kMaxWaves each takes several
-    const uint32_t need = tile_waves_of(tiles);
+    const uint32_t need = tile_waves_of(tiles << kMaxSplit);
     const dim3 grid(need < kMaxWaves ? need : kMaxWaves), blk(64);
     const bool instr = L.s.instrument != 0;
     if (L.s.learned) {

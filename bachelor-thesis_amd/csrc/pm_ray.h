@@ -216,10 +216,12 @@ __device__ __forceinline__ void pm_ray_dir(const MarchLaunch &L, uint32_t px, ui
 }
 
 // Ray of pixel (px, py) and its AABB interval.  Leaves phase = PH_MARCH, or
-// writes the miss and PH_DONE.
-__device__ __forceinline__ void ray_setup(const MarchLaunch &L, RayState &r, uint32_t px, uint32_t py, Counts &cn)
+// writes the miss and PH_DONE.  lead: this lane counts and writes (the others
+// of a lane group share the ray).
+__device__ __forceinline__ void ray_setup(const MarchLaunch &L, RayState &r, uint32_t px, uint32_t py, Counts &cn,
+                                          bool lead = true)
 {
-    cn.rays++;
+    if (lead) cn.rays++;
     r.idx = py * L.W + px;
     float d[3];
     pm_ray_dir(L, px, py, d);
@@ -230,9 +232,9 @@ __device__ __forceinline__ void ray_setup(const MarchLaunch &L, RayState &r, uin
         r.phase = PH_MARCH;
         r.k = 0;
         r.lrn = L.s.learned;
-        cn.in_aabb++;
+        if (lead) cn.in_aabb++;
     } else {
-        march_miss(L, r.idx);
+        if (lead) march_miss(L, r.idx);
         r.phase = PH_DONE;
     }
 }
