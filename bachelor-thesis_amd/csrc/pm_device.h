@@ -568,13 +568,14 @@ __device__ __forceinline__ Cdiff6 pm_cdiff6_lds(const GridDev &g, float qx, floa
     const float x[3] = { qx, qy, qz };
     const float xp[3] = { qx + eps, qy + eps, qz + eps }, xm[3] = { qx - eps, qy - eps, qz - eps };
     BoxWalk w;
-    if (!pm_box_begin(g, xm, xp, w)) {
+    // eps may be negative (the samples change places)
+    if (!(eps < 0.0f ? pm_box_begin(g, xp, xm, w) : pm_box_begin(g, xm, xp, w))) {
         out.cand = 0xffffffffu;
 #pragma unroll
         for (int k = 0; k < 6; k++) out.v[k] = 0.0f;
         return out;
     }
-    const float he = (g.h + eps) * 1.0009765625f;
+    const float he = (g.h + fabsf(eps)) * 1.0009765625f;
     const float R2 = he * he;
     Acc6 a;
 #pragma unroll
