@@ -247,24 +247,6 @@ __device__ __forceinline__ float pm_density32(const GridDev &g, float qx, float 
     return pm_density32(g, qx, qy, qz, compensated, cand, nsup);
 }
 
-// Candidates of q's own trimmed fine stencil (what pm_density32 visits), with no
-// particle read: the per-sample count of instrumented launches.
-__device__ __forceinline__ uint32_t pm_stencil_cand(const GridDev &g, float qx, float qy, float qz)
-{
-    FineWalk fw;
-    if (!pm_fine_begin(g, qx, qy, qz, fw)) return 0u;
-    uint32_t cand = 0;
-    _Pragma("unroll 1") for (int dz = -2; dz <= 2; dz++) {
-        const float tz2 = pm_fine_tz2(fw, dz);
-        _Pragma("unroll 1") for (int dy = -2; dy <= 2; dy++) {
-            uint32_t b, e;
-            pm_fine_row(g, fw, dy, dz, tz2, b, e);
-            cand += e - b;
-        }
-    }
-    return cand;
-}
-
 // Particles stored in the 27 search cells (cells of h) around q's cell, the
 // candidates of the reference's neighbour query (CompactNSearch's 27-cell
 // scan, Dataset.cpp:272-280): 0 when the 3x3x3 block leaves the grid.
@@ -319,6 +301,24 @@ __device__ __forceinline__ void pm_fine_plane(const GridDev &g, const FineWalk &
         P.b[i] = g.fcell_start[row + (uint32_t)lo];
         P.e[i] = g.fcell_start[row + (uint32_t)hi];
     }
+}
+
+// Candidates of q's own trimmed fine stencil (what pm_density32 visits), with no
+// particle read: the rows' bounds alone, all loads independent.
+__device__ __forceinline__ uint32_t pm_stencil_cand(const GridDev &g, float qx, float qy, float qz)
+{
+    FineWalk fw;
+    const bool in = pm_fine_begin(g, qx, qy, qz, fw);
+    if (!in) fw.base = 2u + 2u * fw.sy + 2u * fw.sz;
+    uint32_t cand = 0;
+#pragma unroll
+    for (int dz = -2; dz <= 2; dz++) {
+        RowPlane P;
+        pm_fine_plane(g, fw, in, dz, P);
+#pragma unroll
+        for (int k = 0; k < 5; k++) cand += P.e[k] - P.b[k];
+    }
+    return cand;
 }
 
 // Lists the five rows of a plane: n slots are taken; drain(n) takes the listed
@@ -641,13 +641,14 @@ __device__ __forceinline__ Cdiff6 pm_cdiff6_lds(const GridDev &g, float qx, floa
 // walk lists every particle within h of any of them, in the canonical order;
 // each sample then takes the list with its own r^2 < h^2 test, so its sum is
 // its single-sample sum, bit for bit, for about 25 candidates read instead of a
-// 25-row walk of 41 each (1 M dam break).  lst as in pm_density32_list.  False
+// 25-row walk of 41 each (1 M dam break).  (The statistics still count each
+// sample's own stencil: pm_stencil_cand, pm_box_cand.)  lst as in pm_density32_list.  False
 // (for all calling lanes, which then walk for each sample: both in one wave
 // would cost both) when some lane's box leaves the grid or spans more than two
 // cells on an axis, or its list does not fit CAP.
 template <int CAP>
 __device__ __forceinline__ bool pm_list_segment(const GridDev &g, const float a[3], const float b[3], float eps,
-                                                uint32_t *lst, int &n, uint32_t &cand)
+                                                uint32_t *lst, int &n)
 {
     float lo[3], hi[3], c[3], l2 = 0.0f, big = 0.0f;
 #pragma unroll
@@ -703,7 +704,6 @@ __device__ __forceinline__ bool pm_list_segment(const GridDev &g, const float a[
         int mp = 0;
 #pragma unroll
         for (int k = 0; k < 6; k++) mp += (int)(pe[k] - pb[k]);
-        cand += (uint32_t)mp;
         if (__ballot(mp != 0) != 0) {
             bool fits = true;                   // wave-uniform
             if (__ballot(n + mp > CAP) != 0) {
@@ -752,6 +752,26 @@ __device__ __forceinline__ double pm_list_density64(const GridDev &g, const uint
         }
     }
     return acc;
+}
+
+// Candidates of the six-sample walk's box (pm_cdiff6_lds), with no particle
+// read; 0xffffffff where that walk does not run.
+__device__ __forceinline__ uint32_t pm_box_cand(const GridDev &g, const float x[3], float eps)
+{
+    const float e = fabsf(eps);
+    const float lo[3] = { x[0] - e, x[1] - e, x[2] - e }, hi[3] = { x[0] + e, x[1] + e, x[2] + e };
+    BoxWalk w;
+    if (!pm_box_begin(g, lo, hi, w)) return 0xffffffffu;
+    uint32_t cand = 0;
+    _Pragma("unroll 1") for (int jz = 0; __ballot(jz < w.nz) != 0; jz++) {
+#pragma unroll
+        for (int k = 0; k < 6; k++) {
+            uint32_t b, en;
+            pm_box_row(g, w, k, k < w.ny ? jz : w.nz, b, en);
+            cand += en - b;
+        }
+    }
+    return cand;
 }
 
 // The six central-difference densities over the listed candidates.

@@ -587,9 +587,7 @@ __device__ __forceinline__ void finish_hit(const MarchLaunch &L, uint32_t px, ui
     if (LIST) {
         const float a[3] = { o0 + lo * d[0], o1 + lo * d[1], o2 + lo * d[2] };
         const float b[3] = { o0 + hi * d[0], o1 + hi * d[1], o2 + hi * d[2] };
-        uint32_t cand = 0;
-        listed = pm_list_segment<kFinCap>(g, a, b, fabsf(e), lst, n, cand);
-        if (listed) cn.cand += cand;
+        listed = pm_list_segment<kFinCap>(g, a, b, fabsf(e), lst, n);
     }
     if (bracket) {
         const int n32 = fp64 ? s.bisect_iters - 1 : s.bisect_iters;
@@ -603,15 +601,11 @@ __device__ __forceinline__ void finish_hit(const MarchLaunch &L, uint32_t px, ui
                 float sum = 0.0f, c = 0.0f;
                 pm_list_density(g, lst, n, qx, qy, qz, sum, c, nsup);
                 rho = comp ? sum + c : sum;
-                cn.samples++;
-                if (INSTR) {
-                    cn.cst += pm_stencil_cand(g, qx, qy, qz);
-                    cn.c27 += pm_cand27(g, qx, qy, qz);
-                }
+                cand = pm_stencil_cand(g, qx, qy, qz);
             } else {
                 rho = pm_density32_list<kListCap>(g, qx, qy, qz, comp, lst, cand);
-                count_sample<INSTR>(g, qx, qy, qz, cand, false, cn);
             }
+            count_sample<INSTR>(g, qx, qy, qz, cand, false, cn);
             if (rho >= s.iso) hi = tm; else lo = tm;
         }
         if (!fp64) lo = hi = (lo + hi) * 0.5f;
@@ -651,6 +645,7 @@ __device__ __forceinline__ void finish_hit(const MarchLaunch &L, uint32_t px, ui
             float v[6];
             pm_list_cdiff6(g, lst, n, xs, e, comp, v);
             cn.samples += 6;
+            cn.cand += pm_box_cand(g, xs, e);
             gv[0] = v[0] - v[1]; gv[1] = v[2] - v[3]; gv[2] = v[4] - v[5];
         } else {
             const Cdiff6 o = pm_cdiff6_lds<kLdsCap>(g, xs[0], xs[1], xs[2], e, (float *)lst, comp);
