@@ -17,215 +17,9 @@
 #include "pm_features.h"
 #include "pm_internal.h"
 #include "pm_ray.h"
+#include "pm_tiles.h"
 
 namespace pm {
-
-// The first sample k at or above iso is known and the ray's march ends: its
-// record (at the pixel) holds the bracket [t_{k-1}, t_k] of the bisection, or
-// t itself (the ray starts inside the surface, or no bisection is asked for).
-// Record: (1 | bracket << 1, lo, hi, 0); a miss leaves zeros.
-// lead: this lane writes (the others of a lane group share the ray).
-__device__ __forceinline__ void emit_hit(const MarchLaunch &L, RayState &r, bool lead = true)
-{
-    const pm_settings &s = L.s;
-    float lo = r.tn, hi = r.tn;
-    bool bracket = false;
-    if (r.k != 0) {
-        lo = r.tn + (float)(r.k - 1) * s.step;
-        hi = r.tn + (float)r.k * s.step;
-        bracket = s.bisect_iters > 0;
-        if (!bracket) lo = hi = (lo + hi) * 0.5f;
-    }
-    if (lead) L.hit_rec[r.idx] = make_uint4(bracket ? 3u : 1u, __float_as_uint(lo), __float_as_uint(hi), 0u);
-    r.phase = PH_DONE;
-}
-
-// First half of one step: the sample point of the lane's next FP32 density
-// evaluation, after the skips of the march phase; false when the lane takes
-// no sample this step (the ray ended, or it used up its HOPS skips).  Past an
-// exactly skipped stretch the learned march may ask for proposals again.
-template <int HOPS>
-__device__ __forceinline__ bool ray_prepare(const MarchLaunch &L, RayState &r, float &qx, float &qy, float &qz)
-{
-    const pm_settings &s = L.s;
-    const GridDev &g = L.g;
-    const float o0 = L.cam[0], o1 = L.cam[1], o2 = L.cam[2];
-
-    // at most HOPS skips per step: a lane crossing much skippable space
-    // then idles for a step instead of holding the whole wave in this loop
-    // (a skip costs a few dozen instructions, a step a density walk)
-    for (int hop = 0;; hop++) {
-        float t = r.tn + (float)r.k * s.step;
-        if (t > r.tf || (s.max_steps > 0 && r.k >= s.max_steps)) {
-            march_miss(L, r.idx);
-            r.phase = PH_DONE;
-            return false;
-        }
-        qx = o0 + t * r.d0; qy = o1 + t * r.d1; qz = o2 + t * r.d2;
-        int kn;
-        if (s.skip_mode == PM_SKIP_BOUND) kn = pm_skip_bound(g, o0, o1, o2, r, qx, qy, qz, L.inv_step);
-        else if (s.skip_mode == PM_SKIP_EMPTY) kn = pm_skip_empty(g, o0, o1, o2, r, qx, qy, qz, s.step);
-        else return true;
-        if (kn == r.k) return true;
-        r.k = kn;
-        r.lrn = s.learned;
-        if (hop == HOPS - 1) return false;
-    }
-}
-
-// The counts of one FP32 density evaluation at q (instrumented launches also
-// count its own stencil and its 27 search cells).
-template <bool INSTR>
-__device__ __forceinline__ void count_sample(const GridDev &g, float qx, float qy, float qz, uint32_t cand, bool march,
-                                             Counts &cn)
-{
-    cn.samples++;
-    cn.cand += cand;
-    if (march) {
-        cn.march++;
-        cn.mcand += cand;
-    }
-    if (INSTR) {
-        cn.cst += cand;
-        cn.c27 += pm_cand27(g, qx, qy, qz);
-    }
-}
-
-// Second half: the sample's density rho (and its stencil candidate count)
-// ends the march, asks for a proposal or moves to the next sample.
-template <bool INSTR>
-__device__ __forceinline__ void ray_finish(const MarchLaunch &L, RayState &r, float rho, uint32_t cand, float qx,
-                                           float qy, float qz, Counts &cn)
-{
-    count_sample<INSTR>(L.g, qx, qy, qz, cand, true, cn);
-    if (rho >= L.s.iso) {
-        emit_hit(L, r);
-    } else if (r.lrn && rho < L.mlp_gate_rho) {
-        r.rho = rho;
-        r.phase = PH_PROPOSE;
-    } else {
-        r.k++;
-    }
-}
-
-// One march sample of this ray and the transition it implies.  Dens(q, cand) is the FP32 density.  HOPS: skips per step before
-// a lane idles -- 16 in the single-view march, whose end is spent on few long
-// rays with idle lanes beside them; 8 in the batch, whose lanes stay busy.
-template <bool INSTR, int HOPS, class Dens>
-__device__ __forceinline__ void ray_step(const MarchLaunch &L, RayState &r, Dens dens, Counts &cn)
-{
-    float qx, qy, qz;
-    if (!ray_prepare<HOPS>(L, r, qx, qy, qz)) return;
-    uint32_t cand = 0;
-    float rho = dens(qx, qy, qz, cand);
-    ray_finish<INSTR>(L, r, rho, cand, qx, qy, qz, cn);
-}
-
-// ---- lane groups: the end of a persistent launch ----
-// Once no tile is left, a wave's remaining rays are spread over its idle lanes:
-// G lanes (a power of two) per ray, every lane of a group holding the same
-// RayState.  A step then evaluates the G lattice samples k .. k+G-1 at once and
-// takes the first at or above iso.  Each sample is computed as the one-lane
-// march computes it, and a sample the skip would pass has its density below
-// iso, so the first crossing, the bracket and the image are those of the
-// one-lane march.  Counters count what the one-lane march evaluates: the
-// samples the skip keeps, up to the crossing.
-
-// The ray's state to LDS and back (region: 64 floats per field).
-__device__ __forceinline__ void state_put(float *region, uint32_t slot, const RayState &r)
-{
-    float *p = region + slot;
-    p[0 * 64] = r.d0; p[1 * 64] = r.d1; p[2 * 64] = r.d2; p[3 * 64] = r.tn; p[4 * 64] = r.tf;
-    p[5 * 64] = __int_as_float(r.k); p[6 * 64] = __int_as_float(r.phase); p[7 * 64] = __uint_as_float(r.idx);
-    p[8 * 64] = r.id0; p[9 * 64] = r.id1; p[10 * 64] = r.id2;
-}
-
-__device__ __forceinline__ void state_get(const float *region, uint32_t slot, RayState &r)
-{
-    const float *p = region + slot;
-    r.d0 = p[0 * 64]; r.d1 = p[1 * 64]; r.d2 = p[2 * 64]; r.tn = p[3 * 64]; r.tf = p[4 * 64];
-    r.k = __float_as_int(p[5 * 64]); r.phase = __float_as_int(p[6 * 64]); r.idx = __float_as_uint(p[7 * 64]);
-    r.id0 = p[8 * 64]; r.id1 = p[9 * 64]; r.id2 = p[10 * 64];
-    r.lrn = 0;
-    if (r.phase == PH_PROPOSE) { r.phase = PH_MARCH; r.k++; }   // below iso, and no proposals in groups
-}
-
-// Widens the groups when the busy rays fit in fewer lanes: G becomes the
-// largest power of two with (busy rays) x G <= 64.  Called by all 64 lanes.
-__device__ __forceinline__ void regroup(RayState &r, int &G, float *region)
-{
-    const uint32_t lane = threadIdx.x & 63;
-    const unsigned long long lead = __ballot(r.phase != PH_DONE && (lane & (uint32_t)(G - 1)) == 0);
-    const int nb = __popcll(lead);
-    int Gn = 1;
-    while (Gn < 64 && nb * Gn * 2 <= 64) Gn *= 2;
-    if (Gn <= G || nb == 0) return;
-    if ((lead >> lane) & 1ull) state_put(region, (uint32_t)__popcll(lead & ((1ull << lane) - 1ull)), r);
-    wave_lds_sync();
-    if ((int)(lane / (uint32_t)Gn) < nb) state_get(region, lane / (uint32_t)Gn, r);
-    else r.phase = PH_DONE;
-    wave_lds_sync();
-    G = Gn;
-}
-
-// Lane j of its group: its sample of this step; false when it takes none.
-// nonskip: the sample is one the one-lane march would evaluate.
-__device__ __forceinline__ bool group_prepare(const MarchLaunch &L, RayState &r, int G, int j, float &qx, float &qy,
-                                              float &qz, bool &nonskip)
-{
-    const pm_settings &s = L.s;
-    const GridDev &g = L.g;
-    const float o0 = L.cam[0], o1 = L.cam[1], o2 = L.cam[2];
-    nonskip = false;
-    // the group's first sample, as ray_prepare finds it; the wave has few
-    // rays left, so a group may take 8 G skips in one step
-    const int hop_cap = 8 * G - 1;
-    for (int hop = 0;; hop++) {
-        float t = r.tn + (float)r.k * s.step;
-        if (t > r.tf || (s.max_steps > 0 && r.k >= s.max_steps)) {
-            if (j == 0) march_miss(L, r.idx);
-            r.phase = PH_DONE;
-            return false;
-        }
-        qx = o0 + t * r.d0; qy = o1 + t * r.d1; qz = o2 + t * r.d2;
-        int kn = r.k;
-        if (s.skip_mode == PM_SKIP_BOUND) kn = pm_skip_bound(g, o0, o1, o2, r, qx, qy, qz, L.inv_step);
-        else if (s.skip_mode == PM_SKIP_EMPTY) kn = pm_skip_empty(g, o0, o1, o2, r, qx, qy, qz, s.step);
-        if (kn == r.k) break;
-        r.k = kn;
-        if (hop == hop_cap) return false;
-    }
-    if (j == 0) { nonskip = true; return true; }
-    const int kj = r.k + j;
-    const float t = r.tn + (float)kj * s.step;
-    if (t > r.tf || (s.max_steps > 0 && kj >= s.max_steps)) return false;
-    qx = o0 + t * r.d0; qy = o1 + t * r.d1; qz = o2 + t * r.d2;
-    // (a skip returns a later sample than r.k exactly where q may be skipped)
-    nonskip = s.skip_mode == PM_SKIP_BOUND   ? pm_skip_bound(g, o0, o1, o2, r, qx, qy, qz, L.inv_step) == r.k
-              : s.skip_mode == PM_SKIP_EMPTY ? pm_skip_empty(g, o0, o1, o2, r, qx, qy, qz, s.step) == r.k
-                                             : true;
-    return true;
-}
-
-// The group's transition from its lanes' densities.  Called by all 64 lanes.
-template <bool INSTR>
-__device__ __forceinline__ void group_finish(const MarchLaunch &L, RayState &r, int G, int j, bool want, bool nonskip,
-                                             float rho, uint32_t cand, float qx, float qy, float qz, Counts &cn)
-{
-    const uint32_t lane = threadIdx.x & 63, gbase = lane & ~(uint32_t)(G - 1);
-    const unsigned long long gmask = G == 64 ? ~0ull : ((1ull << G) - 1ull);
-    const unsigned long long cross = (__ballot(want && rho >= L.s.iso) >> gbase) & gmask;
-    const unsigned long long wants = (__ballot(want) >> gbase) & gmask;
-    if (r.phase != PH_MARCH || !(wants & 1ull)) return;
-    const int jc = cross ? __ffsll((long long)cross) - 1 : G;
-    if (want && nonskip && j <= jc) count_sample<INSTR>(L.g, qx, qy, qz, cand, true, cn);
-    if (cross) {
-        r.k += jc;
-        emit_hit(L, r, j == 0);
-    } else {
-        r.k += G;
-    }
-}
 
 // FP32 density through the lane's candidate list (compensated or plain sum).
 // CAP: 36 candidates -- near the surface a stencil holds about 41, so most
@@ -705,41 +499,6 @@ __device__ __forceinline__ void finish_tile(const MarchLaunch &L, uint32_t tile,
     if (rec.x & 1u) finish_hit<INSTR, LIST>(L, px, py, rec, lst, cn);
 }
 
-// Active tile i of a launch's list for wave `w` of the grid (one-wave
-// workgroups, dispatched to the 8 XCDs round-robin): runs of kXcdRun
-// consecutive tiles go to the XCDs in turn, so neighbouring tiles share an L2
-// and every XCD gets its share of a dense region.
-static constexpr uint32_t kXcdRun = 32;
-__device__ __forceinline__ uint32_t xcd_tile(uint32_t w)
-{
-    const uint32_t local = w >> 3;
-    return ((local / kXcdRun) * 8 + (w & 7u)) * kXcdRun + local % kXcdRun;
-}
-
-// Workgroups for T tiles (all of them may be active): a multiple of a full
-// round of runs; beyond kMaxWaves each wave takes several tiles (16,384 waves
-// left some with two tiles of the 4K pool: 4.9 against 3.6 ms in the finish).
-static constexpr uint32_t kMaxWaves = 65536;
-__host__ __device__ __forceinline__ uint32_t tile_waves_of(uint32_t T)
-{
-    return (T + 8 * kXcdRun - 1) / (8 * kXcdRun) * (8 * kXcdRun);
-}
-
-// Waves per tile of the march, as a power of two, for TA active tiles.  The
-// chip holds about 4,096 of its waves: with fewer tiles a launch lasts as long
-// as its longest tile (a ray along a face takes a hundred samples), so each tile
-// is split over four waves whose rays start with four lanes each; the samples
-// evaluated past a crossing cost less than the idle SIMDs.  March kernel for
-// one / two / four / eight waves per tile: 640x480 lattice cube (3,200 tiles)
-// 493 / 354 / 268 / 354 us, 96x64 213 / 156 / 130 / 152 us, 1080p dam break
-// (4,300) 331 / 297 / 318 / 448 us, 4K pool (19,000) 2,490 / 2,578 / 2,899 /
-// 5,184 us.
-static constexpr uint32_t kResidentWaves = 4096, kMaxSplit = 2;
-__device__ __forceinline__ uint32_t tile_split(uint32_t TA)
-{
-    return TA < kResidentWaves ? 2u : (TA < 2 * kResidentWaves ? 1u : 0u);
-}
-
 // Schedule 0: a wave per active 8x8 tile (or several, tile_split), one ray per
 // lane or lane group up to the ray's hit or miss.  As rays end, the others spread over the idle lanes (lane
 // groups), so the tile's last rays take several samples per step.  The tiles
@@ -768,10 +527,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
         const uint32_t i = xcd_tile(w);
         if (i >= TA << sub) continue;
         any = true;
-        const uint32_t tile = order[i >> sub], part = i & ((1u << sub) - 1u), rr = lane >> sub;
-        const uint32_t lw = sub >= 2 ? 2u : 3u, np = 3u - lw;   // a part is 2^lw pixels wide, 2^np in a row
-        const uint32_t px = (tile % tiles_x) * 8 + (part & ((1u << np) - 1u)) * (1u << lw) + (rr & ((1u << lw) - 1u));
-        const uint32_t py = (tile / tiles_x) * 8 + (part >> np) * (64u >> sub >> lw) + (rr >> lw);
+        uint32_t px, py;
+        part_pixel(order[i >> sub], tiles_x, i, sub, lane >> sub, px, py);
         RayState r{};
         r.phase = PH_DONE;
         int G = 1 << sub;
@@ -791,13 +548,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
             if (G == 1) {
                 if (r.phase == PH_MARCH) ray_step<INSTR, 16>(L, r, DensList{ &L.g, lst, comp }, cn);
             } else {
-                const int j = (int)(lane & (uint32_t)(G - 1));
-                float qx = 0.f, qy = 0.f, qz = 0.f, rho = 0.f;
-                bool nonskip = false, want = false;
-                uint32_t cand = 0;
-                if (r.phase != PH_DONE) want = group_prepare(L, r, G, j, qx, qy, qz, nonskip);
-                if (want) rho = pm_density32_list<kListCap>(L.g, qx, qy, qz, comp, lst, cand);
-                group_finish<INSTR>(L, r, G, j, want, nonskip, rho, cand, qx, qy, qz, cn);
+                group_step<INSTR>(L, r, G, DensList{ &L.g, lst, comp }, cn);
             }
         }
     }
@@ -904,23 +655,51 @@ __global__ __launch_bounds__(256) void k_march_reference(MarchLaunch L)
     flush_counters(L.counters, rc.rays, rc.in, rc.hits, rc.samples, rc.cand, rc.ms);
 }
 
-// The reference march over the active tiles of the tile pre-pass only (tiles
-// with a pixel whose depth is not 1; the pre-pass wrote the others' misses),
-// one tile per wave, the active list spread over the 8 XCDs as
-// k_march_aniso_active spreads it.
-__global__ __launch_bounds__(256) void k_march_reference_active(MarchLaunch L)
+// The product's reference march: the active tiles of the tile pre-pass (those
+// with a pixel whose depth is not 1; the pre-pass wrote the others' misses), a
+// wave per tile or part of one.
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_ref_tiles(MarchLaunch L)
 {
-    const uint32_t T = ((L.W + 7) / 8) * ((L.H + 7) / 8);
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    __shared__ float region[kListWords];
+    __shared__ float4 hits[64];
+    uint32_t *lst = (uint32_t *)region + threadIdx.x;
+    const pm_settings &s = L.s;
+    const GridDev &g = L.g;
+    const uint32_t tiles_x = (L.W + 7) / 8, T = tiles_x * ((L.H + 7) / 8);
     const uint32_t *order = L.tile_buf + 2 * (T + 1);
-    const uint32_t count = order[T], chunk = (count + 7) / 8;
-    const uint32_t local = (blockIdx.x >> 3) * 4 + wave, i = (blockIdx.x & 7u) * chunk + local;
-    if (local >= chunk || i >= count) return;   // whole wave
-    const uint32_t tile = order[i], tiles_x = (L.W + 7) / 8;
-    const uint32_t px = (tile % tiles_x) * 8 + (lane & 7u), py = (tile / tiles_x) * 8 + (lane >> 3);
-    RefCounts rc;
-    ref_pixel(L, px, py, px < L.W && py < L.H, rc);
-    flush_counters(L.counters, rc.rays, rc.in, rc.hits, rc.samples, rc.cand, rc.ms);
+    const uint32_t TA = order[T], sub = tile_split(TA);
+    const DensList dens{ &g, lst, s.compensated != 0 };
+    Counts cn;
+    bool any = false;
+    auto normal = [&](const float p[3], float &nx, float &ny, float &nz) {
+        if (s.normal_mode == PM_NORMAL_GRADW) {
+            float sx, sy, sz;
+            uint32_t cand = 0;
+            pm_sum_gradw(g, p[0], p[1], p[2], sx, sy, sz, cand);
+            pm_normalize(sx, sy, sz, nx, ny, nz);
+            return;
+        }
+        float gv[3];
+#pragma unroll 1
+        for (int k = 0; k < 6; k++) {
+            const float e = (k & 1) ? -s.normal_eps : s.normal_eps;
+            uint32_t cand = 0;
+            const float rho = dens(k < 2 ? p[0] + e : p[0], (k >> 1) == 1 ? p[1] + e : p[1], k > 3 ? p[2] + e : p[2], cand);
+            cn.samples++;
+            cn.cand += cand;
+#pragma unroll
+            for (int a = 0; a < 3; a++)
+                if ((k >> 1) == a) gv[a] = (k & 1) ? gv[a] - rho : rho;
+        }
+        cdiff_normal(gv, nx, ny, nz);
+    };
+    for (uint32_t w = blockIdx.x; w < tile_waves_of(TA << sub); w += gridDim.x) {
+        const uint32_t i = xcd_tile(w);
+        if (i >= TA << sub) continue;
+        any = true;
+        ref_part(L, order[i >> sub], tiles_x, i, sub, region, hits, dens, normal, cn);
+    }
+    if (any) flush_counters(L.counters, cn.rays, cn.in_aabb, cn.hits, cn.samples, cn.cand, cn.march);
 }
 
 // Batched schedule: persistent waves take chunks of tiles (each chunk belongs to
@@ -1000,13 +779,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
                 ray_step<false, 8>(*Lp, r, DensList{ &Lp->g, lst, comp }, cn);
             }
         } else {
-            const int j = (int)(lane & (uint32_t)(G - 1));
-            float qx = 0.f, qy = 0.f, qz = 0.f, rho = 0.f;
-            bool nonskip = false, want = false;
-            uint32_t cand = 0;
-            if (r.phase != PH_DONE) want = group_prepare(*Lp, r, G, j, qx, qy, qz, nonskip);
-            if (want) rho = pm_density32_list<kListCap>(Lp->g, qx, qy, qz, comp, lst, cand);
-            group_finish<false>(*Lp, r, G, j, want, nonskip, rho, cand, qx, qy, qz, cn);
+            group_step<false>(*Lp, r, G, DensList{ &Lp->g, lst, comp }, cn);
         }
     }
     flush_counts(B.base.counters, cn);
@@ -1158,8 +931,8 @@ hipError_t launch_march(const MarchLaunch &L, hipStream_t st)
         if (L.tile_buf && L.s.schedule == 0) {
             hipError_t e = launch_tile_prepass(L, st);
             if (e != hipSuccess) return e;
-            const uint32_t per_xcd = ((tiles + 7) / 8 + 3) / 4;
-            hipLaunchKernelGGL(k_march_reference_active, dim3(8 * per_xcd), dim3(256), 0, st, L);
+            const uint32_t need = tile_waves_of(tiles << kMaxSplit);
+            hipLaunchKernelGGL(k_ref_tiles, dim3(need < kMaxWaves ? need : kMaxWaves), dim3(64), 0, st, L);
             return hipGetLastError();
         }
         hipLaunchKernelGGL(k_march_reference, dim3((tiles + 3) / 4), dim3(256), 0, st, L);

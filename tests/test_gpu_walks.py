@@ -14,14 +14,14 @@ KEYS = dict(O.Settings._fields_)
 COUNTERS = ("rays", "rays_in_aabb", "hits", "samples", "march_samples", "march_cand")
 
 
-def _check(marcher, sc, **kw):
+def _check(marcher, sc, counters=COUNTERS, **kw):
     c = sc.cameras[0]
     st = sc.settings(**kw)
     pos, nrm, t, got = marcher.march(60, st, c.inv_pv, c.eye, c.width, c.height)
     o = O.march(O.Grid(sc.xyz, sc.h), O.make_settings(**{k: v for k, v in st.items() if k in KEYS}), c.inv_pv, c.eye,
                 c.width, c.height)
     assert np.array_equal(pos, o[0]) and np.array_equal(nrm, o[1]) and np.array_equal(t, o[2])
-    for k in COUNTERS:
+    for k in counters:
         assert got[k] == o[3][k], (k, got[k], o[3][k])
     return got
 
@@ -77,3 +77,27 @@ def test_finish_list(marcher, eps, bisect, fp64, step):
     for comp in (0, 1):
         got = _check(marcher, sc, skip_mode=4, bisect_iters=bisect, final_fp64=fp64, compensated=comp)
         assert got["hits"] > 50
+
+
+@pytest.mark.parametrize("size", [(9, 7), (64, 40), (333, 207)])
+@pytest.mark.parametrize("normal_mode", [0, 1])
+def test_reference_groups(marcher, size, normal_mode):
+    """The reference march in lane groups: few, some and many active tiles, a
+    MaxSteps that no group size divides, every skip, both normals."""
+    from parity import depth_in_front
+    sc = scenes.lattice_cube(5, n_side=12, spacing=0.05, width=size[0], height=size[1])
+    c = sc.cameras[0]
+    print(f"reference groups {size} normals {normal_mode}", flush=True)
+    marcher.set_frame(60, sc.xyz, sc.h)
+    G = O.Grid(sc.xyz, sc.h)
+    depth = depth_in_front(c, G.bmin, G.bmax, 0.01).astype(np.float32)
+    extra = dict(iso=sc.iso)
+    for skip, steps in ((0, 37), (2, 101), (3, 1)):
+        st = dict(mode=1, max_steps=steps, step=0.013, normal_mode=normal_mode, normal_eps=sc.normal_eps,
+                  skip_mode=skip, compensated=skip & 1, **extra)
+        pos, nrm, t, got = marcher.march(60, st, c.inv_pv, c.eye, c.width, c.height, depth=depth)
+        o = O.march(G, O.make_settings(**st), c.inv_pv, c.eye, c.width, c.height, depth=depth)
+        assert np.array_equal(pos, o[0]) and np.array_equal(t, o[2])
+        assert np.array_equal(nrm, o[1], equal_nan=True)
+        for k in ("rays_in_aabb", "hits", "samples", "cand", "march_samples"):
+            assert got[k] == o[3][k], (k, got[k], o[3][k])
