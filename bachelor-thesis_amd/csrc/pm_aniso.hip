@@ -15,13 +15,19 @@
 //      AnisotropicKernel::W(G, det G, r) (Kernel.cpp:63-83), walked over the
 //      trimmed 5x5x5 march-grid stencil around q in the canonical order (the
 //      extended walk up to the cap when the list was capped).
-// One ray per lane, one 8x8 tile per wave, each lane to the end of its ray
-// (march, bisection, FP64 step, normal, outputs); schedule 1 of the configured
-// march runs persistent waves with ray refill and a finish pass over the hits
-// instead (below).  All float arithmetic is in the order of the CPU oracle
+// The product (schedule 0) takes the active tiles as the isotropic march does
+// (pm_tiles.h): a march kernel up to each ray's bracket or miss and a finish
+// kernel for bisection, FP64 step, normal and outputs, or the reference march of
+// a tile; its walks go through candidate lists.  1080p scaled dam break: 9.17
+// (one kernel, one ray per lane to its end, direct walks) -> 3.35 + 3.10 ms;
+// reference mode 12.6 -> 3.6 ms.  The direct walks below are the plain form it
+// is checked against: schedule 1 (persistent waves with ray refill and a finish
+// pass over the hits, or in reference mode one ray per lane) and the point
+// queries.  All float arithmetic is in the order of the CPU oracle
 // (oracle/pm_aniso.inc), -ffp-contract=off.
 #include "pm_internal.h"
 #include "pm_ray.h"
+#include "pm_tiles.h"
 
 namespace pm {
 
@@ -383,6 +389,225 @@ __device__ __forceinline__ typename P::T an_sum(const GridDev &g, const P &a, co
     return comp ? s + cc : s;
 }
 
+// ---- the product's walks: candidate lists ----
+// The same sums as an_cov and an_sum, each walk through the lane's candidate
+// list in LDS (pm_list_plane): a wave runs to its longest list, not to every
+// row's longest lane.  The 2h walk tests its listed candidates first and keeps
+// the neighbours in place, so the 50 instructions of a neighbour's weight and
+// moments run over neighbours only (about 60 % of the candidates).
+// 36 slots (10 KB of LDS) and 128 VGPRs keep 16 waves on a CU; a plane of the
+// 2h walk holds about 50 candidates, so a lane takes its list six times or so.
+// Measured (1080p scaled dam break, march + finish kernels): 20 slots 6.97 ms,
+// 28 6.91, 36 6.45, 60 (ten waves) 8.0; with 163 and 214 VGPRs 7.75.
+static constexpr int kAnCap = 36;
+static constexpr int kAnWords = (kAnCap + kListPad) * 64;
+
+// Bounds of the five rows of plane dz of the 2h walk: an_row's ranges.
+struct AnPlanes {
+    SWalk w;
+    float xm2, xm1, xp1, xp2;
+    bool in;
+};
+
+__device__ __forceinline__ void an_plane(const GridDev &g, const AnPlanes &A, int dz, RowPlane &P)
+{
+    const float tz = pm_fine_off(dz, A.w.f[2]);
+    const int32_t z = A.w.c[2] + dz;
+    const bool inz = A.in && z >= 0 && z < g.nz;
+#pragma unroll
+    for (int i = 0; i < 5; i++) {
+        const float ty = pm_fine_off(i - 2, A.w.f[1]);
+        const float r2 = ty * ty + tz * tz;
+        const int32_t y = A.w.c[1] + i - 2;
+        int32_t xl = A.w.c[0] + ((A.xm2 + r2 < kLimExt) ? -2 : ((A.xm1 + r2 < kLimExt) ? -1 : 0));
+        int32_t xh = A.w.c[0] + ((A.xp2 + r2 < kLimExt) ? 2 : ((A.xp1 + r2 < kLimExt) ? 1 : 0));
+        xl = xl < 0 ? 0 : xl;
+        xh = xh > g.nx - 1 ? g.nx - 1 : xh;
+        const bool kept = inz && r2 < kLimExt && y >= 0 && y < g.ny && xl <= xh;
+        const uint32_t row = (uint32_t)g.nx * ((uint32_t)y + (uint32_t)g.ny * (uint32_t)z);
+        P.b[i] = g.cell_start[kept ? row + (uint32_t)xl : 0u];
+        P.e[i] = g.cell_start[kept ? row + (uint32_t)xh + 1u : 0u];
+    }
+}
+
+template <class T>
+__device__ __forceinline__ T an_sqrt(T x)
+{
+    if constexpr (sizeof(T) == 4) return pm_sqrt_w(x);   // both kernels' values do not depend on the root's last bit below 2^-96
+    else return sqrt(x);
+}
+
+template <class P>
+__device__ __forceinline__ uint32_t an_cov_list(const GridDev &g, const P &a, const float qf[3], const typename P::T q[3],
+                                                uint32_t *lst, typename P::T c[6], uint32_t &cand)
+{
+    using T = typename P::T;
+    AnPlanes A;
+    A.in = an_centre(g, qf, 2, A.w);
+    float t;
+    t = pm_fine_off(-2, A.w.f[0]); A.xm2 = t * t;
+    t = pm_fine_off(-1, A.w.f[0]); A.xm1 = t * t;
+    t = pm_fine_off(1, A.w.f[0]); A.xp1 = t * t;
+    t = pm_fine_off(2, A.w.f[0]); A.xp2 = t * t;
+    uint32_t nx = 0;
+    T sx = (T)0, sy = (T)0, sz = (T)0;
+    T ws = (T)0, s0 = (T)0, s1 = (T)0, s2 = (T)0;
+    T c0 = (T)0, c1 = (T)0, c2 = (T)0, c3 = (T)0, c4 = (T)0, c5 = (T)0;
+    auto drain = [&](int n) {
+        int m = 0;                               // neighbours so far, in lst[0, m)
+        _Pragma("unroll 1") for (int i = 0; __ballot(i < n) != 0; i += 4) {
+            uint32_t l[4];
+            float4 v[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                l[u] = lst[(i + u) * 64];
+                v[u] = g.sorted[i + u < n ? l[u] : 0u];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const T rx = (T)v[u].x - q[0], ry = (T)v[u].y - q[1], rz = (T)v[u].z - q[2];
+                const T r2 = (rx * rx + ry * ry) + rz * rz;
+                lst[m * 64] = l[u];              // m <= i + u: a slot already read
+                m += (i + u < n && r2 < a.R2x) ? 1 : 0;
+            }
+        }
+        if (__ballot(nx == 0 && m > 0) != 0) {
+            const float4 f = g.sorted[m > 0 ? lst[0] : 0u];
+            if (nx == 0 && m > 0) { sx = (T)f.x; sy = (T)f.y; sz = (T)f.z; }
+        }
+        const int room = nx < kMaxNeighbors ? (int)(kMaxNeighbors - nx) : 0;
+        const int take = m < room ? m : room;
+        nx += (uint32_t)m;
+        _Pragma("unroll 1") for (int i = 0; __ballot(i < take) != 0; i += 2) {
+            float4 v[2];
+#pragma unroll
+            for (int u = 0; u < 2; u++) v[u] = g.sorted[i + u < take ? lst[(i + u) * 64] : 0u];
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                const T rx = (T)v[u].x - q[0], ry = (T)v[u].y - q[1], rz = (T)v[u].z - q[2];
+                const T d = an_sqrt((rx * rx + ry * ry) + rz * rz);
+                const T k = d * a.hxinv;
+                // past the list a slot adds exact zeros
+                const T wt = (i + u < take && !(d >= a.hx)) ? (T)1 - k * k * k : (T)0;
+                const T ux = (T)v[u].x - sx, uy = (T)v[u].y - sy, uz = (T)v[u].z - sz;
+                const T w0 = wt * ux, w1 = wt * uy, w2 = wt * uz;
+                ws += wt;
+                s0 += w0; s1 += w1; s2 += w2;
+                c0 += w0 * ux;
+                c1 += w1 * ux;
+                c2 += w1 * uy;
+                c3 += w2 * ux;
+                c4 += w2 * uy;
+                c5 += w2 * uz;
+            }
+        }
+    };
+    int n = 0;
+    RowPlane R, Q;
+    an_plane(g, A, -2, R);
+    _Pragma("unroll 1") for (int dz = -2; dz <= 2; dz++) {
+        if (dz < 2) an_plane(g, A, dz + 1, Q);
+#pragma unroll
+        for (int k = 0; k < 5; k++) cand += R.e[k] - R.b[k];
+        pm_list_rows<kAnCap>(R, lst, n, dz == 2, drain);
+        R = Q;
+    }
+    if (nx == 0) return 0;
+    const T inv = (T)1 / ws;
+    const T m0 = s0 * inv, m1 = s1 * inv, m2 = s2 * inv;
+    c[0] = c0 * inv - m0 * m0; c[1] = c1 * inv - m1 * m0; c[2] = c2 * inv - m1 * m1;
+    c[3] = c3 * inv - m2 * m0; c[4] = c4 * inv - m2 * m1; c[5] = c5 * inv - m2 * m2;
+    return nx;
+}
+
+template <class P, bool GRAD>
+__device__ __forceinline__ typename P::T an_sum_list(const GridDev &g, const P &a, const float qf[3],
+                                                     const typename P::T q[3], bool comp, uint32_t *lst, uint32_t &cand,
+                                                     float *grad = nullptr)
+{
+    using T = typename P::T;
+    T c[6], G[9], detG;
+    if (GRAD) grad[0] = grad[1] = grad[2] = 0.0f;
+    uint32_t cnd = 0;
+    const uint32_t nx = an_cov_list(g, a, qf, q, lst, c, cnd);
+    if (__ballot(nx > kMaxNeighbors) != 0) return an_sum(g, a, qf, q, comp, cand, grad);   // a capped list in the wave
+    cand += cnd;
+    if (nx == 0) return (T)0;
+    an_gmat(c, nx, a, G, detG);
+    T s = (T)0, cc = (T)0;
+    auto drain = [&](int n) {
+        _Pragma("unroll 1") for (int i = 0; __ballot(i < n) != 0; i += 4) {
+            float4 v[4];
+            T w[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) v[u] = g.fsorted[i + u < n ? lst[(i + u) * 64] : 0u];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const T rx = (T)v[u].x - q[0], ry = (T)v[u].y - q[1], rz = (T)v[u].z - q[2];
+                const T r2 = (rx * rx + ry * ry) + rz * rz;
+                const bool in = i + u < n && r2 < a.h2;
+                if constexpr (GRAD) {
+                    if (in) {
+                        float o0, o1, o2;
+                        an_gradW(G, detG, rx, ry, rz, a, o0, o1, o2);
+                        grad[0] += o0; grad[1] += o1; grad[2] += o2;
+                    }
+                } else {
+                    // an_W, both branches evaluated; zero outside the support
+                    const T g0 = (G[0] * rx + G[1] * ry) + G[2] * rz;
+                    const T g1 = (G[3] * rx + G[4] * ry) + G[5] * rz;
+                    const T g2 = (G[6] * rx + G[7] * ry) + G[8] * rz;
+                    const T q2 = (g0 * g0 + g1 * g1) + g2 * g2;
+                    const T qn = an_sqrt(q2) * a.hinv, qq = (T)1 - qn;
+                    const T f1 = (T)2 * qq * qq * qq, f0 = (T)6 * (qn * qn * qn - qn * qn) + (T)1;
+                    w[u] = (in && !(q2 >= a.h2)) ? (a.sig * detG) * (qn >= (T)0.5 ? f1 : f0) : (T)0;
+                }
+            }
+            if constexpr (!GRAD) {
+#pragma unroll
+                for (int u = 0; u < 4; u++) an_neu_add(s, cc, w[u]);
+            }
+        }
+    };
+    FineWalk fw;
+    const bool in = pm_fine_begin(g, qf[0], qf[1], qf[2], fw);
+    if (!in) fw.base = 2u + 2u * fw.sy + 2u * fw.sz;
+    int n = 0;
+    RowPlane R, Q;
+    pm_fine_plane(g, fw, in, -2, R);
+    _Pragma("unroll 1") for (int dz = -2; dz <= 2; dz++) {
+        if (dz < 2) pm_fine_plane(g, fw, in, dz + 1, Q);
+#pragma unroll
+        for (int k = 0; k < 5; k++) cand += R.e[k] - R.b[k];
+        pm_list_rows<kAnCap>(R, lst, n, dz == 2, drain);
+        R = Q;
+    }
+    return comp ? s + cc : s;                    // s alone is the plain sum
+}
+
+// normalize(sum gradW) at p (RayMarcher.cpp:402-409).
+__device__ __forceinline__ void an_normal_gradw(const MarchLaunch &L, const float p[3], uint32_t *lst, float &nx, float &ny,
+                                                float &nz)
+{
+    float gs[3];
+    uint32_t cand = 0;
+    an_sum_list<AnParF, true>(L.g, L.an.f, p, p, false, lst, cand, gs);
+    const float dd = (gs[0] * gs[0] + gs[1] * gs[1]) + gs[2] * gs[2];
+    const float inv = 1.0f / sqrtf(dd);
+    nx = gs[0] * inv; ny = gs[1] * inv; nz = gs[2] * inv;
+}
+
+struct AnDens {
+    const MarchLaunch *L;
+    uint32_t *lst;
+    bool comp;
+    __device__ float operator()(float x, float y, float z, uint32_t &cand) const
+    {
+        const float q[3] = { x, y, z };
+        return an_sum_list<AnParF, false>(L->g, L->an.f, q, q, comp, lst, cand);
+    }
+};
+
 __device__ __forceinline__ float an_density32(const MarchLaunch &L, float x, float y, float z, bool comp,
                                               uint32_t &cand)
 {
@@ -587,30 +812,156 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
     flush_counters(L.counters, cn.rays, cn.in_aabb, cn.hits, cn.samples, cn.cand, cn.march);
 }
 
-// The march over the active tiles only (the tile pre-pass has written every
-// pixel of the other tiles as a miss; in reference mode the active tiles are
-// those with a drawn sprite depth), one tile per wave: every
-// wave that starts has rays to march, and the heavy tiles are not dispatched
-// between thousands of empty ones.  Workgroups go to the 8 XCDs round-robin
-// (workgroup b to XCD b mod 8), so XCD x takes the x-th eighth of the active
-// list: all XCDs share the work and neighbouring tiles share an L2.  The grid
-// has a multiple of 8 workgroups and at least T / 32 per XCD.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_march_aniso_active(MarchLaunch L)
+// ---- the product: active tiles only (the tile pre-pass wrote the others) ----
+
+// The configured march up to each ray's bracket, a wave per active tile or part
+// of one (k_march_tiles' form: lane groups, hit records).
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_an_march_tiles(MarchLaunch L)
 {
-    const uint32_t T = ((L.W + 7) / 8) * ((L.H + 7) / 8);
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    __shared__ float region[kAnWords];
+    const uint32_t lane = threadIdx.x;
+    const uint32_t tiles_x = (L.W + 7) / 8, T = tiles_x * ((L.H + 7) / 8);
     const uint32_t *order = L.tile_buf + 2 * (T + 1);
-    const uint32_t count = order[T], chunk = (count + 7) / 8;
-    const uint32_t local = (blockIdx.x >> 3) * 4 + wave, i = (blockIdx.x & 7u) * chunk + local;
-    if (local >= chunk || i >= count) return;   // whole wave
-    const uint32_t tile = order[i], tiles_x = (L.W + 7) / 8;
-    const uint32_t px = (tile % tiles_x) * 8 + (lane & 7u), py = (tile / tiles_x) * 8 + (lane >> 3);
+    const uint32_t TA = order[T], sub = tile_split(TA);
+    const AnDens dens{ &L, (uint32_t *)region + lane, L.s.compensated != 0 };
     Counts cn;
-    if (px < L.W && py < L.H) {
-        if (L.s.mode == PM_MODE_REFERENCE) an_pixel_reference(L, px, py, cn);
-        else an_pixel_config(L, px, py, cn);
+    bool any = false;
+    for (uint32_t w = blockIdx.x; w < tile_waves_of(TA << sub); w += gridDim.x) {
+        const uint32_t i = xcd_tile(w);
+        if (i >= TA << sub) continue;
+        any = true;
+        uint32_t px, py;
+        part_pixel(order[i >> sub], tiles_x, i, sub, lane >> sub, px, py);
+        RayState r{};
+        r.phase = PH_DONE;
+        int G = 1 << sub;
+        if (px < L.W && py < L.H) ray_setup(L, r, px, py, cn, (lane & (uint32_t)(G - 1)) == 0);
+        while (__ballot(r.phase != PH_DONE) != 0) {
+            regroup(r, G, region);
+            group_step<false>(L, r, G, dens, cn);
+        }
     }
-    flush_counters(L.counters, cn.rays, cn.in_aabb, cn.hits, cn.samples, cn.cand, cn.march);
+    if (any) flush_counters(L.counters, cn.rays, cn.in_aabb, cn.hits, cn.samples, cn.cand, cn.march);
+}
+
+// The hits of the same tiles: bisection (the last step in FP64), normal,
+// outputs; 2^tile_split lanes per hit where the tiles do not fill the chip.
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_an_finish_tiles(MarchLaunch L)
+{
+    __shared__ float region[kAnWords];
+    const uint32_t lane = threadIdx.x;
+    uint32_t *lst = (uint32_t *)region + lane;
+    const pm_settings &s = L.s;
+    const GridDev &g = L.g;
+    const uint32_t tiles_x = (L.W + 7) / 8, T = tiles_x * ((L.H + 7) / 8);
+    const uint32_t *order = L.tile_buf + 2 * (T + 1);
+    const uint32_t TA = order[T], sub = finish_split(TA);
+    const int G = 1 << sub;
+    const bool lead = (lane & (uint32_t)(G - 1)) == 0;
+    const bool comp = s.compensated != 0, fp64 = s.final_fp64 && s.bisect_iters > 0;
+    const AnDens dens{ &L, lst, comp };
+    const float o[3] = { L.cam[0], L.cam[1], L.cam[2] };
+    Counts cn;
+    bool any = false;
+    for (uint32_t w = blockIdx.x; w < tile_waves_of(TA << sub); w += gridDim.x) {
+        const uint32_t i = xcd_tile(w);
+        if (i >= TA << sub) continue;
+        uint32_t px, py;
+        part_pixel(order[i >> sub], tiles_x, i, sub, lane >> sub, px, py);
+        const bool inside = px < L.W && py < L.H;
+        const uint32_t idx = inside ? py * L.W + px : 0u;
+        const uint4 rec = L.hit_rec[idx];
+        const bool hit = inside && (rec.x & 1u), bracket = hit && (rec.x & 2u);
+        if (__ballot(hit) == 0) continue;
+        any = true;
+        float lo = __uint_as_float(rec.y), hi = __uint_as_float(rec.z);
+        float d[3];
+        pm_ray_dir(L, px, py, d);
+        if (__ballot(bracket) != 0) {
+            float l = lo, h = hi;
+            group_bisect(L, d, l, h, fp64 ? s.bisect_iters - 1 : s.bisect_iters, bracket, G, dens, cn);
+            if (bracket) { lo = l; hi = h; }
+            if (bracket && !fp64) lo = hi = (lo + hi) * 0.5f;
+        }
+        float th = lo, xs[3] = { o[0] + lo * d[0], o[1] + lo * d[1], o[2] + lo * d[2] };
+        if (bracket && fp64) {
+            double dlo = lo, dhi = hi;
+            const double tm = (dlo + dhi) * 0.5;
+            if (lead) {
+                const double q[3] = { (double)o[0] + tm * (double)d[0], (double)o[1] + tm * (double)d[1],
+                                      (double)o[2] + tm * (double)d[2] };
+                const float qf[3] = { (float)q[0], (float)q[1], (float)q[2] };
+                uint32_t cand = 0;
+                const double rho = an_sum_list<AnParD, false>(g, L.an.d, qf, q, false, lst, cand);
+                cn.samples++;
+                if (rho >= (double)s.iso) dhi = tm; else dlo = tm;
+            }
+            const double tt = (dlo + dhi) * 0.5;
+            xs[0] = (float)((double)o[0] + tt * (double)d[0]);
+            xs[1] = (float)((double)o[1] + tt * (double)d[1]);
+            xs[2] = (float)((double)o[2] + tt * (double)d[2]);
+            th = (float)tt;
+        }
+        // the group's lanes take the leader's point
+#pragma unroll
+        for (int a = 0; a < 3; a++) xs[a] = __shfl(xs[a], (int)(lane & ~(uint32_t)(G - 1)), 64);
+        float nx = 0.f, ny = 0.f, nz = 0.f;
+        if (s.normal_mode == PM_NORMAL_GRADW) {
+            if (hit && lead) an_normal_gradw(L, xs, lst, nx, ny, nz);
+        } else {
+            float gv[3];
+            group_cdiff(xs, s.normal_eps, hit, G, dens, gv, cn);
+            cdiff_normal(gv, nx, ny, nz);
+        }
+        if (hit && lead) {
+            L.pos[idx] = make_float4(xs[0], xs[1], xs[2], 1.0f);
+            L.nrm[idx] = make_float4(nx, ny, nz, 1.0f);
+            if (L.t) L.t[idx] = th;
+            cn.hits++;
+        }
+    }
+    if (any) flush_counters(L.counters, cn.rays, cn.in_aabb, cn.hits, cn.samples, cn.cand, cn.march);
+}
+
+// The reference march (a drawn sprite depth makes a tile active).
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_an_ref_tiles(MarchLaunch L)
+{
+    __shared__ float region[kAnWords];
+    __shared__ float4 hits[64];
+    uint32_t *lst = (uint32_t *)region + threadIdx.x;
+    const pm_settings &s = L.s;
+    const uint32_t tiles_x = (L.W + 7) / 8, T = tiles_x * ((L.H + 7) / 8);
+    const uint32_t *order = L.tile_buf + 2 * (T + 1);
+    const uint32_t TA = order[T], sub = tile_split(TA);
+    const AnDens dens{ &L, lst, s.compensated != 0 };
+    Counts cn;
+    bool any = false;
+    auto normal = [&](const float p[3], float &nx, float &ny, float &nz) {
+        if (s.normal_mode == PM_NORMAL_GRADW) {
+            an_normal_gradw(L, p, lst, nx, ny, nz);
+            return;
+        }
+        float gv[3];
+#pragma unroll 1
+        for (int k = 0; k < 6; k++) {
+            const float e = (k & 1) ? -s.normal_eps : s.normal_eps;
+            uint32_t cand = 0;
+            const float rho = dens(k < 2 ? p[0] + e : p[0], (k >> 1) == 1 ? p[1] + e : p[1], k > 3 ? p[2] + e : p[2], cand);
+            cn.samples++;
+            cn.cand += cand;
+#pragma unroll
+            for (int a = 0; a < 3; a++)
+                if ((k >> 1) == a) gv[a] = (k & 1) ? gv[a] - rho : rho;
+        }
+        cdiff_normal(gv, nx, ny, nz);
+    };
+    for (uint32_t w = blockIdx.x; w < tile_waves_of(TA << sub); w += gridDim.x) {
+        const uint32_t i = xcd_tile(w);
+        if (i >= TA << sub) continue;
+        any = true;
+        ref_part(L, order[i >> sub], tiles_x, i, sub, region, hits, dens, normal, cn);
+    }
+    if (any) flush_counters(L.counters, cn.rays, cn.in_aabb, cn.hits, cn.samples, cn.cand, cn.march);
 }
 
 // ---- configured march: persistent waves, then a finish pass over the hits ----
@@ -861,9 +1212,16 @@ hipError_t launch_march_aniso(const MarchLaunch &L, hipStream_t st)
     if (L.s.schedule == 0 && L.tile_buf) {
         hipError_t e = launch_tile_prepass(L, st);
         if (e != hipSuccess) return e;
-        // 8 ceil(ceil(T / 8) / 4) workgroups: enough waves for every XCD's share
-        const uint32_t per_xcd = ((tiles + 7) / 8 + 3) / 4;
-        hipLaunchKernelGGL(k_march_aniso_active, dim3(8 * per_xcd), dim3(256), 0, st, L);
+        const uint32_t need = tile_waves_of(tiles << kMaxSplit);
+        const dim3 grid(need < kMaxWaves ? need : kMaxWaves), blk(64);
+        if (L.s.mode == PM_MODE_REFERENCE) {
+            hipLaunchKernelGGL(k_an_ref_tiles, grid, blk, 0, st, L);
+            return hipGetLastError();
+        }
+        hipLaunchKernelGGL(k_an_march_tiles, grid, blk, 0, st, L);
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(k_an_finish_tiles, grid, blk, 0, st, L);
         return hipGetLastError();
     }
     if (L.s.mode == PM_MODE_REFERENCE || L.s.schedule != 1 || !L.hit_rec) {

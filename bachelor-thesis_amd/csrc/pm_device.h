@@ -321,8 +321,45 @@ __device__ __forceinline__ uint32_t pm_stencil_cand(const GridDev &g, float qx, 
     return cand;
 }
 
-// Lists the five rows of a plane: n slots are taken; drain(n) takes the listed
-// candidates in order.  Called by any set of lanes; those drain together.
+// Candidates b .. b + m - 1 into the slots from n: four at once (those past the
+// row are the next row's slots, or padding), then the rest.
+__device__ __forceinline__ void pm_list_put(uint32_t *lst, int n, uint32_t b, int m)
+{
+    uint32_t *const q = lst + n * 64;
+#pragma unroll
+    for (int k = 0; k < 4; k++) q[k * 64] = b + (uint32_t)k;
+    if (__ballot(m > 4) != 0)
+        for (int k = 4; k < m; k++) q[k * 64] = b + (uint32_t)k;
+}
+
+// Lists the five rows of a plane, n slots taken so far, row by row: a list is
+// filled to its last slot before the lanes take theirs, and whatever is listed
+// at the end of the last plane is taken.  drain(n) takes the listed candidates
+// in order; it is expanded once here, which is what a long one wants (the
+// anisotropic walk's, expanded at every row, ran 1.5 to 2 times slower).
+// Called by any set of lanes; those drain together.
+template <int CAP, class Drain>
+__device__ __forceinline__ void pm_list_rows(const RowPlane &P, uint32_t *lst, int &n, bool last, Drain &&drain)
+{
+    _Pragma("unroll 1") for (int i = 0; i < 5; i++) {
+        uint32_t b = P.b[0], e = P.e[0];
+#pragma unroll
+        for (int k = 1; k < 5; k++) { b = i == k ? P.b[k] : b; e = i == k ? P.e[k] : e; }
+        while (true) {
+            const int m = (int)(e - b), take = m < CAP - n ? m : CAP - n;
+            pm_list_put(lst, n, b, take);
+            n += take;
+            b += (uint32_t)take;
+            const bool more = __ballot(b < e) != 0;
+            if (!more && !(last && i == 4)) break;
+            drain(n);
+            n = 0;
+            if (!more) break;
+        }
+    }
+}
+
+// The same where a plane usually fits: one check per plane.
 template <int CAP, class Drain>
 __device__ __forceinline__ void pm_list_plane(const RowPlane &P, uint32_t *lst, int &n, Drain &&drain)
 {
@@ -334,32 +371,14 @@ __device__ __forceinline__ void pm_list_plane(const RowPlane &P, uint32_t *lst, 
         drain(n);
         n = 0;
         if (__ballot(mp > CAP) != 0) {        // a plane longer than the list (dense clusters)
-            _Pragma("unroll 1") for (int i = 0; i < 5; i++) {
-                uint32_t b = P.b[0], e = P.e[0];
-#pragma unroll
-                for (int k = 1; k < 5; k++) { b = i == k ? P.b[k] : b; e = i == k ? P.e[k] : e; }
-                while (__ballot(b < e) != 0) {
-                    const int take = min((int)(e - b), CAP - n);
-                    for (int k = 0; k < take; k++) lst[(n + k) * 64] = b + (uint32_t)k;
-                    n += take;
-                    b += (uint32_t)take;
-                    if (__ballot(b < e) != 0) { drain(n); n = 0; }
-                }
-            }
+            pm_list_rows<CAP>(P, lst, n, false, drain);
             return;
         }
     }
 #pragma unroll
     for (int i = 0; i < 5; i++) {
-        const uint32_t b = P.b[i];
-        const int m = (int)(P.e[i] - b);
-        // four slots at once; those past the row are the next row's
-        uint32_t *const q = lst + n * 64;
-#pragma unroll
-        for (int k = 0; k < 4; k++) q[k * 64] = b + (uint32_t)k;
-        if (__ballot(m > 4) != 0)
-            for (int k = 4; k < m; k++) q[k * 64] = b + (uint32_t)k;
-        n += m;
+        pm_list_put(lst, n, P.b[i], (int)(P.e[i] - P.b[i]));
+        n += (int)(P.e[i] - P.b[i]);
     }
 }
 

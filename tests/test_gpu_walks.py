@@ -80,18 +80,20 @@ def test_finish_list(marcher, eps, bisect, fp64, step):
 
 
 @pytest.mark.parametrize("size", [(9, 7), (64, 40), (333, 207)])
+@pytest.mark.parametrize("aniso", [0, 1])
 @pytest.mark.parametrize("normal_mode", [0, 1])
-def test_reference_groups(marcher, size, normal_mode):
+def test_reference_groups(marcher, size, aniso, normal_mode):
     """The reference march in lane groups: few, some and many active tiles, a
-    MaxSteps that no group size divides, every skip, both normals."""
+    MaxSteps that no group size divides, every skip, both normals; and the
+    anisotropic configured march and its finish at the same sizes."""
     from parity import depth_in_front
     sc = scenes.lattice_cube(5, n_side=12, spacing=0.05, width=size[0], height=size[1])
     c = sc.cameras[0]
-    print(f"reference groups {size} normals {normal_mode}", flush=True)
+    print(f"reference groups {size} aniso {aniso} normals {normal_mode}", flush=True)
     marcher.set_frame(60, sc.xyz, sc.h)
     G = O.Grid(sc.xyz, sc.h)
     depth = depth_in_front(c, G.bmin, G.bmax, 0.01).astype(np.float32)
-    extra = dict(iso=sc.iso)
+    extra = dict(scenes.ANISO_SETTINGS, iso=1.0) if aniso else dict(iso=sc.iso)
     for skip, steps in ((0, 37), (2, 101), (3, 1)):
         st = dict(mode=1, max_steps=steps, step=0.013, normal_mode=normal_mode, normal_eps=sc.normal_eps,
                   skip_mode=skip, compensated=skip & 1, **extra)
@@ -101,3 +103,6 @@ def test_reference_groups(marcher, size, normal_mode):
         assert np.array_equal(nrm, o[1], equal_nan=True)
         for k in ("rays_in_aabb", "hits", "samples", "cand", "march_samples"):
             assert got[k] == o[3][k], (k, got[k], o[3][k])
+    if aniso:
+        _check(marcher, sc, counters=("rays", "hits", "samples", "cand", "march_samples"), skip_mode=4,
+               normal_mode=normal_mode, **extra)
