@@ -821,7 +821,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     __shared__ float region[kAnWords];
     const uint32_t lane = threadIdx.x;
     const uint32_t tiles_x = (L.W + 7) / 8, T = tiles_x * ((L.H + 7) / 8);
-    const uint32_t *order = L.tile_buf + 2 * (T + 1);
+    const uint32_t *order = L.tile_buf;
     const uint32_t TA = order[T], sub = tile_split(TA);
     const AnDens dens{ &L, (uint32_t *)region + lane, L.s.compensated != 0 };
     Counts cn;
@@ -854,7 +854,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     const pm_settings &s = L.s;
     const GridDev &g = L.g;
     const uint32_t tiles_x = (L.W + 7) / 8, T = tiles_x * ((L.H + 7) / 8);
-    const uint32_t *order = L.tile_buf + 2 * (T + 1);
+    const uint32_t *order = L.tile_buf;
     const uint32_t TA = order[T], sub = finish_split(TA);
     const int G = 1 << sub;
     const bool lead = (lane & (uint32_t)(G - 1)) == 0;
@@ -931,7 +931,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     uint32_t *lst = (uint32_t *)region + threadIdx.x;
     const pm_settings &s = L.s;
     const uint32_t tiles_x = (L.W + 7) / 8, T = tiles_x * ((L.H + 7) / 8);
-    const uint32_t *order = L.tile_buf + 2 * (T + 1);
+    const uint32_t *order = L.tile_buf;
     const uint32_t TA = order[T], sub = tile_split(TA);
     const AnDens dens{ &L, lst, s.compensated != 0 };
     Counts cn;

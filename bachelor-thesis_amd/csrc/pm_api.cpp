@@ -720,7 +720,7 @@ static int march_launch(pm_ctx *c, int32_t frame, const pm_settings *s, const fl
         if (na) {
             L.tile_buf = na->tiles;
         } else {
-            HIPCHK(c, c->d_tiles.ensure(sizeof(uint32_t) * (3 * (tiles + 1) + scan_tmp_size((uint32_t)(tiles + 1)))));
+            HIPCHK(c, c->d_tiles.ensure(sizeof(uint32_t) * tile_words(tiles)));
             L.tile_buf = (uint32_t *)c->d_tiles.p;
         }
     }
@@ -738,8 +738,7 @@ static int march_launch(pm_ctx *c, int32_t frame, const pm_settings *s, const fl
             L.depth = (const float *)c->d_depth.p;
         }
     }
-    if (na) HIPCHK(c, launch_zero_u64(L.counters, kCtrWords, c->stream));
-    else HIPCHK(c, hipMemsetAsync(c->d_counters.p, 0, sizeof(unsigned long long) * kCtrWords, c->stream));
+    HIPCHK(c, launch_zero_u64(L.counters, kCtrWords, c->stream));
     HIPCHK(c, hipEventRecord(c->ev_k0, c->stream));
     HIPCHK(c, launch_march(L, c->stream));
     HIPCHK(c, hipEventRecord(c->ev_k1, c->stream));

@@ -64,8 +64,8 @@ struct MarchLaunch {
     int32_t mlp_min_skip;      // below this many steps the ray continues step by step
     int32_t mlp_max_skip;      // longest jump, in steps
     float mlp_gate_rho;        // a sample asks for a proposal only below this density
-    // tiles with a ray entering the AABB, in row order: scratch of
-    // 3 (T + 1) + scan_tmp_size(T + 1) u32; null = every tile
+    // the active tiles of the tile pre-pass (tile_words(T) u32: the list, its
+    // length at T, masks); null = every tile
     uint32_t *tile_buf;
     float inv_step;            // 1 / s.step (bound skip)
     // per pixel: the hit handed from the march to k_finish (1 | fp64 << 1,
@@ -122,13 +122,11 @@ struct GridBuildArgs {
     float4 *scattered;     // n: cell-major, arbitrary order inside a cell
 };
 size_t scan_tmp_size(uint32_t len);
-// Exclusive scan of len u32 (out may not alias in); tmp of scan_tmp_size(len).
-hipError_t launch_scan_u32(const uint32_t *in, uint32_t *out, uint32_t len, uint32_t *tmp, hipStream_t st);
 hipError_t launch_grid_build(const GridBuildArgs &a, hipStream_t st);
 
-// The tile pre-pass of the configured march (L.tile_buf set): flags of the 8x8
-// tiles one of whose rays enters the padded AABB, their scan, the list of
-// active tiles (order[T] = their count) and the misses of the other tiles.
+// The tile pre-pass (L.tile_buf set): the list of the active tiles and the misses
+// of the others.
+inline size_t tile_words(uint64_t T) { return (size_t)(((T + 2) & ~1ull) + 2 * ((T + 63) / 64)); }
 hipError_t launch_tile_prepass(const MarchLaunch &L, hipStream_t st);
 hipError_t launch_march(const MarchLaunch &L, hipStream_t st);
 // The anisotropic march (configured or reference mode), one kernel.

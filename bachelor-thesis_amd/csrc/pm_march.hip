@@ -45,46 +45,83 @@ struct DensList {
 
 static constexpr int kLdsCap = 32;   // floats per lane of the six-sample walk's compaction
 
-// Tile pre-pass.  tile_buf = flag[T+1] | pos[T+1] |
-// order[T+1] | scan scratch: flag = 1 for a tile one of whose rays enters the
-// padded AABB (the ray set-up and slab test of ray_setup, bit for bit) -- in
-// reference mode, one of whose pixels has a depth other than 1 -- pos
-// its exclusive scan, order the active tiles in row order (order[T] = their
-// count).  The march takes only active tiles; k_miss_tiles writes
-// the misses of the others.
+// Tile pre-pass: the 8x8 tiles one of whose rays enters the padded AABB (the ray
+// set-up and slab test of ray_setup, bit for bit) -- in reference mode, one of
+// whose pixels has a depth other than 1.  The march takes only these active
+// tiles; the others' pixels are misses.
+__device__ __forceinline__ bool tile_ray_active(const MarchLaunch &L, uint32_t px, uint32_t py)
+{
+    if (px >= L.W || py >= L.H) return false;
+    if (L.s.mode == PM_MODE_REFERENCE) return L.depth[py * L.W + px] != 1.0f;
+    const float cx = (float)px * (2.0f / (float)L.W) - 1.0f;
+    const float cy = (float)py * (2.0f / (float)L.H) - 1.0f;
+    float wx, wy, wz, d[3], tn, tf;
+    pm_unproject(L.M, cx, cy, 1.0f, wx, wy, wz);
+    pm_normalize(wx - L.cam[0], wy - L.cam[1], wz - L.cam[2], d[0], d[1], d[2]);
+    const float o[3] = { L.cam[0], L.cam[1], L.cam[2] };
+    return pm_slab(o, d, L.g.bmin, L.g.bmax, tn, tf);
+}
+
+// Two launches list the active tiles in row order and write the misses of the
+// others: tile_buf[0, count) the tiles, tile_buf[T] = count, then (64-bit
+// aligned) one mask of active tiles per 64.  The first takes 64 tiles per
+// workgroup, four per wave; the second adds up the masks before its own, which
+// at these sizes (507 masks at 1080p) is cheaper than a scan's launches.  Bound
+// by the miss writes (36 B per ray).  (Flags, a three-launch scan, a compaction
+// and the misses were six launches: 45 us at 1080p, 17 at 96x64.  One launch
+// that appended each workgroup's tiles with an atomic saved 3 us more but lost
+// the row order: march kernel of the 640x480 lattice cube 228 -> 337 us, finish
+// kernel of the 4K pool 3.6 -> 4.0 ms.)
+__device__ __forceinline__ unsigned long long *tile_masks(const MarchLaunch &L, uint32_t T)
+{
+    return (unsigned long long *)(L.tile_buf + ((T + 2u) & ~1u));
+}
+
+__global__ __launch_bounds__(1024) void k_tile_masks(MarchLaunch L, uint32_t T)
+{
+    __shared__ uint32_t nib[16];
+    const uint32_t wave = threadIdx.x >> 6, j = threadIdx.x & 63u, tiles_x = (L.W + 7) / 8;
+    const uint32_t t0 = blockIdx.x * 64 + wave * 4;
+    uint32_t m = 0;
+    for (uint32_t k = 0; k < 4 && t0 + k < T; k++) {
+        const uint32_t t = t0 + k;
+        const uint32_t px = (t % tiles_x) * 8 + (j & 7u), py = (t / tiles_x) * 8 + (j >> 3);
+        if (__ballot(tile_ray_active(L, px, py)) != 0) m |= 1u << k;
+        else if (px < L.W && py < L.H) write_miss(L, py * L.W + px);
+    }
+    if (j == 0) nib[wave] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long mask = 0;
+        for (uint32_t w = 0; w < 16; w++) mask |= (unsigned long long)nib[w] << (4 * w);
+        tile_masks(L, T)[blockIdx.x] = mask;
+    }
+}
+
+__global__ __launch_bounds__(64) void k_tile_list(MarchLaunch L, uint32_t T)
+{
+    const unsigned long long *masks = tile_masks(L, T);
+    const uint32_t b = blockIdx.x, lane = threadIdx.x;
+    uint32_t before = 0;
+    for (uint32_t i = lane; i < b; i += 64) before += (uint32_t)__popcll(masks[i]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off, 64);
+    const unsigned long long m = masks[b];
+    if ((m >> lane) & 1ull) L.tile_buf[before + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = b * 64 + lane;
+    if (b == gridDim.x - 1 && lane == 0) L.tile_buf[T] = before + (uint32_t)__popcll(m);
+}
+
+// The flags and the misses on their own (a batch lists its tiles on the host):
+// tile_buf[t] = 1 for an active tile, tile_buf[T] = 0.
 __global__ __launch_bounds__(256) void k_tile_flags(MarchLaunch L, uint32_t T)
 {
     // one wave per tile, one lane per ray
     const uint32_t t = blockIdx.x * 4 + (threadIdx.x >> 6), j = threadIdx.x & 63u;
     if (t > T) return;   // whole wave
-    bool enters = false;
-    if (t < T) {
-        const uint32_t tiles_x = (L.W + 7) / 8;
-        const uint32_t px = (t % tiles_x) * 8 + (j & 7u), py = (t / tiles_x) * 8 + (j >> 3);
-        if (px < L.W && py < L.H && L.s.mode == PM_MODE_REFERENCE) {
-            enters = L.depth[py * L.W + px] != 1.0f;   // the reference march starts where a sprite was drawn
-        } else if (px < L.W && py < L.H) {
-            const float cx = (float)px * (2.0f / (float)L.W) - 1.0f;
-            const float cy = (float)py * (2.0f / (float)L.H) - 1.0f;
-            float wx, wy, wz, d[3], tn, tf;
-            pm_unproject(L.M, cx, cy, 1.0f, wx, wy, wz);
-            pm_normalize(wx - L.cam[0], wy - L.cam[1], wz - L.cam[2], d[0], d[1], d[2]);
-            const float o[3] = { L.cam[0], L.cam[1], L.cam[2] };
-            enters = pm_slab(o, d, L.g.bmin, L.g.bmax, tn, tf);
-        }
-    }
+    const uint32_t tiles_x = (L.W + 7) / 8;
+    const bool enters = t < T && tile_ray_active(L, (t % tiles_x) * 8 + (j & 7u), (t / tiles_x) * 8 + (j >> 3));
     const unsigned long long m = __ballot(enters);
-    if (j == 0) L.tile_buf[t] = m != 0ull ? 1u : 0u;   // flag[T] = 0 closes the scan
-}
-
-__global__ __launch_bounds__(256) void k_tile_compact(uint32_t *tile_buf, uint32_t T)
-{
-    const uint32_t t = blockIdx.x * 256 + threadIdx.x;
-    if (t > T) return;
-    const uint32_t *flag = tile_buf, *pos = tile_buf + (T + 1);
-    uint32_t *order = tile_buf + 2 * (T + 1);
-    if (t == T) order[T] = pos[T];
-    else if (flag[t]) order[pos[t]] = t;
+    if (j == 0) L.tile_buf[t] = m != 0ull ? 1u : 0u;
 }
 
 // Pixels of the inactive tiles are written as misses here.  (They are not
@@ -517,7 +554,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     const uint32_t lane = threadIdx.x;
     uint32_t *lst = (uint32_t *)region + lane;
     const uint32_t tiles_x = (L.W + 7) / 8, T = tiles_x * ((L.H + 7) / 8);
-    const uint32_t *order = L.tile_buf + 2 * (T + 1);
+    const uint32_t *order = L.tile_buf;
     const uint32_t TA = order[T];
     const bool comp = L.s.compensated != 0;
     Counts cn;
@@ -666,7 +703,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     const pm_settings &s = L.s;
     const GridDev &g = L.g;
     const uint32_t tiles_x = (L.W + 7) / 8, T = tiles_x * ((L.H + 7) / 8);
-    const uint32_t *order = L.tile_buf + 2 * (T + 1);
+    const uint32_t *order = L.tile_buf;
     const uint32_t TA = order[T], sub = tile_split(TA);
     const DensList dens{ &g, lst, s.compensated != 0 };
     Counts cn;
@@ -809,7 +846,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LIST ? 3 : 4
         }
     } else {
         const uint32_t T = ((L0.W + 7) / 8) * ((L0.H + 7) / 8);
-        const uint32_t *order = L0.tile_buf + 2 * (T + 1), TA = order[T];
+        const uint32_t *order = L0.tile_buf, TA = order[T];
         for (uint32_t w = blockIdx.x; w < tile_waves_of(TA); w += gridDim.x) {
             const uint32_t i = xcd_tile(w);
             if (i >= TA) continue;
@@ -856,7 +893,7 @@ hipError_t launch_zero_u32(uint32_t *p, uint32_t n, hipStream_t st)
 
 hipError_t launch_zero_u64(unsigned long long *p, uint32_t n, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, p, n);
+    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(128), 0, st, p, n);
     return hipGetLastError();
 }
 
@@ -889,12 +926,9 @@ hipError_t launch_miss_tiles(const MarchLaunch &L, uint32_t T, hipStream_t st)
 hipError_t launch_tile_prepass(const MarchLaunch &L, hipStream_t st)
 {
     const uint32_t tiles = ((L.W + 7) / 8) * ((L.H + 7) / 8);
-    uint32_t *flag = L.tile_buf, *pos = L.tile_buf + (tiles + 1);
-    hipLaunchKernelGGL(k_tile_flags, dim3((tiles + 1 + 3) / 4), dim3(256), 0, st, L, tiles);
-    hipError_t e = launch_scan_u32(flag, pos, tiles + 1, L.tile_buf + 3 * (tiles + 1), st);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_tile_compact, dim3((tiles + 1 + 255) / 256), dim3(256), 0, st, L.tile_buf, tiles);
-    hipLaunchKernelGGL(k_miss_tiles, dim3((tiles + 3) / 4), dim3(256), 0, st, L, tiles);
+    const uint32_t groups = (tiles + 63) / 64;
+    hipLaunchKernelGGL(k_tile_masks, dim3(groups), dim3(1024), 0, st, L, tiles);
+    hipLaunchKernelGGL(k_tile_list, dim3(groups), dim3(64), 0, st, L, tiles);
     return hipGetLastError();
 }
 

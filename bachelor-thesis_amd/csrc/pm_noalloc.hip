@@ -30,7 +30,7 @@ namespace pm {
 // ceil(W/8) ceil(H/8) <= W H / 64 + (W + H) / 8 + 1 < 36864.
 constexpr uint32_t kNoAllocMaxTiles = 36864;
 constexpr size_t kNoAllocHitBytes = sizeof(uint4) * (size_t)PM_NOALLOC_MAX_PIXELS;
-constexpr size_t kNoAllocTileWords = 3 * (kNoAllocMaxTiles + 1) + 2048;   // scan scratch <= (T + 1) / 256 + 2
+constexpr size_t kNoAllocTileWords = kNoAllocMaxTiles + 2 + 2 * (kNoAllocMaxTiles / 64 + 1);
 constexpr size_t kNoAllocTileOff = kNoAllocHitBytes;
 constexpr size_t kNoAllocCtrOff = kNoAllocTileOff + ((sizeof(uint32_t) * kNoAllocTileWords + 255) & ~(size_t)255);
 constexpr size_t kNoAllocBandOff = kNoAllocCtrOff + sizeof(unsigned long long) * kCtrWords;
@@ -64,7 +64,7 @@ bool noalloc_layout(void *base, uint32_t W, uint32_t H, NoAllocScratch &s)
 {
     const uint64_t tiles = (uint64_t)((W + 7) / 8) * ((H + 7) / 8);
     if (!base || (uint64_t)W * H > PM_NOALLOC_MAX_PIXELS || tiles > kNoAllocMaxTiles) return false;
-    if (3 * (tiles + 1) + scan_tmp_size((uint32_t)(tiles + 1)) > kNoAllocTileWords) return false;
+    if (tile_words(tiles) > kNoAllocTileWords) return false;
     uint8_t *b = (uint8_t *)base;
     s.hit_rec = (uint4 *)b;
     s.tiles = (uint32_t *)(b + kNoAllocTileOff);
