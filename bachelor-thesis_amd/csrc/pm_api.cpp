@@ -738,7 +738,7 @@ static int march_launch(pm_ctx *c, int32_t frame, const pm_settings *s, const fl
             L.depth = (const float *)c->d_depth.p;
         }
     }
-    HIPCHK(c, launch_zero_u64(L.counters, kCtrWords, c->stream));
+    if (!L.tile_buf) HIPCHK(c, launch_zero_u64(L.counters, kCtrWords, c->stream));   // else the pre-pass does
     HIPCHK(c, hipEventRecord(c->ev_k0, c->stream));
     HIPCHK(c, launch_march(L, c->stream));
     HIPCHK(c, hipEventRecord(c->ev_k1, c->stream));

@@ -82,6 +82,7 @@ __global__ __launch_bounds__(1024) void k_tile_masks(MarchLaunch L, uint32_t T)
     __shared__ uint32_t nib[16];
     const uint32_t wave = threadIdx.x >> 6, j = threadIdx.x & 63u, tiles_x = (L.W + 7) / 8;
     const uint32_t t0 = blockIdx.x * 64 + wave * 4;
+    if (blockIdx.x == 0 && threadIdx.x < (uint32_t)kCtrWords) L.counters[threadIdx.x] = 0ull;   // the march's, before it
     uint32_t m = 0;
     for (uint32_t k = 0; k < 4 && t0 + k < T; k++) {
         const uint32_t t = t0 + k;
@@ -857,11 +858,141 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LIST ? 3 : 4
     if (any) flush_counts(L0.counters, cn);
 }
 
+// The finish of a small image: four lanes per hit, so the bisection takes four
+// rounds instead of seven (ten samples), the six central differences two, and a tile's hits
+// are spread over four waves.  It does more work in all (ten samples for
+// seven, the FP64 sample by one lane of four), so it gains where a hit's own
+// serial chain bounds the launch and loses once the waves fill the chip.  The
+// image's tiles are known here, its hits are not, so each line lies where an
+// image full of hits still gains:
+// - a sparse frame (k_finish with a list otherwise): 96x64 lattice 87 -> 59 us;
+//   256x192 (768 tiles) dam 131 -> 86, full lattice 94 -> 71; 288x224 (1008) dam
+//   134 -> 85 but full lattice 96 -> 110, 360x360 (2025) 115 -> 195;
+// - a dense frame, where one hit's walks take milliseconds: 96x64 pool of
+//   400,000 1698 -> 898 us, 800x600 (7500) 2400 -> 905; 1,000,000 at 1280x720
+//   (14400) 3482 -> 1518; 1920x1080 (32400) 1837 -> 2080 at 400,000 and
+//   2996 -> 2310 at 1,000,000; 4,000,000 at 3840x2160 3513 -> 7682.
+static constexpr uint32_t kGroupTiles = 800, kGroupTilesDense = 16384;
+
+// FP32 density of one of a hit's samples from the hit's list, or by its own walk.
+struct FinishDens {
+    const GridDev *g;
+    uint32_t *lst;
+    int n;
+    bool listed, comp, count;
+    __device__ float operator()(float x, float y, float z, uint32_t &cand) const
+    {
+        uint32_t c = 0, nsup = 0;
+        float rho;
+        if (listed) {
+            float sum = 0.0f, cc = 0.0f;
+            pm_list_density(*g, lst, n, x, y, z, sum, cc, nsup);
+            rho = comp ? sum + cc : sum;
+            if (count) c = pm_stencil_cand(*g, x, y, z);
+        } else {
+            rho = pm_density32_list<kListCap>(*g, x, y, z, comp, lst, c);
+        }
+        if (count) cand += c;
+        return rho;
+    }
+};
+
+template <bool LIST>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_finish_groups(MarchLaunch L)
+{
+    __shared__ uint32_t lds[kFinWords];
+    const uint32_t lane = threadIdx.x;
+    uint32_t *lst = lds + lane;
+    const pm_settings &s = L.s;
+    const GridDev &g = L.g;
+    const uint32_t tiles_x = (L.W + 7) / 8, T = tiles_x * ((L.H + 7) / 8), sub = 2;
+    const uint32_t *order = L.tile_buf, TA = order[T];
+    constexpr int G = 4;
+    const uint32_t gbase = lane & ~(uint32_t)(G - 1);
+    const bool lead = lane == gbase, comp = s.compensated != 0, fp64 = s.final_fp64 && s.bisect_iters > 0;
+    const float e = s.normal_mode == PM_NORMAL_CDIFF ? s.normal_eps : 0.0f;
+    const float o[3] = { L.cam[0], L.cam[1], L.cam[2] };
+    Counts cn;
+    bool any = false;
+    for (uint32_t w = blockIdx.x; w < tile_waves_of(TA << sub); w += gridDim.x) {
+        const uint32_t i = xcd_tile(w);
+        if (i >= TA << sub) continue;
+        uint32_t px, py;
+        part_pixel(order[i >> sub], tiles_x, i, sub, lane >> sub, px, py);
+        const bool inside = px < L.W && py < L.H;
+        const uint32_t idx = inside ? py * L.W + px : 0u;
+        const uint4 rec = L.hit_rec[idx];
+        const bool hit = inside && (rec.x & 1u), bracket = hit && (rec.x & 2u);
+        if (__ballot(hit) == 0) continue;
+        any = true;
+        float lo = __uint_as_float(rec.y), hi = __uint_as_float(rec.z);
+        float d[3];
+        pm_ray_dir(L, px, py, d);
+        FinishDens dens{ &g, lst, 0, false, comp, true };
+        if (LIST && hit) {
+            const float a[3] = { o[0] + lo * d[0], o[1] + lo * d[1], o[2] + lo * d[2] };
+            const float b[3] = { o[0] + hi * d[0], o[1] + hi * d[1], o[2] + hi * d[2] };
+            dens.listed = pm_list_segment<kFinCap>(g, a, b, fabsf(e), lst, dens.n);
+        }
+        if (__ballot(bracket) != 0) {
+            float l = lo, h = hi;
+            group_bisect(L, d, l, h, fp64 ? s.bisect_iters - 1 : s.bisect_iters, bracket, G, dens, cn);
+            if (bracket) { lo = l; hi = h; }
+            if (bracket && !fp64) lo = hi = (lo + hi) * 0.5f;
+        }
+        float th = lo, xs[3] = { o[0] + lo * d[0], o[1] + lo * d[1], o[2] + lo * d[2] };
+        if (bracket && fp64 && lead) {
+            double dlo = lo, dhi = hi;
+            const double tm = (dlo + dhi) * 0.5;
+            const double x = (double)o[0] + tm * (double)d[0], y = (double)o[1] + tm * (double)d[1],
+                         z = (double)o[2] + tm * (double)d[2];
+            const double rho = dens.listed ? pm_list_density64(g, lst, dens.n, x, y, z) : pm_density64(g, x, y, z);
+            cn.samples++;
+            if (rho >= (double)s.iso) dhi = tm; else dlo = tm;
+            const double tt = (dlo + dhi) * 0.5;
+            xs[0] = (float)((double)o[0] + tt * (double)d[0]);
+            xs[1] = (float)((double)o[1] + tt * (double)d[1]);
+            xs[2] = (float)((double)o[2] + tt * (double)d[2]);
+            th = (float)tt;
+        }
+#pragma unroll
+        for (int a = 0; a < 3; a++) xs[a] = __shfl(xs[a], (int)gbase, 64);   // the leader's point
+        float nx = 0.f, ny = 0.f, nz = 0.f;
+        if (s.normal_mode == PM_NORMAL_GRADW) {
+            if (hit && lead) {
+                float sx, sy, sz;
+                uint32_t cand = 0;
+                pm_sum_gradw(g, xs[0], xs[1], xs[2], sx, sy, sz, cand);
+                pm_normalize(sx, sy, sz, nx, ny, nz);
+            }
+        } else {
+            // counted as the six-sample walk's box, or where that leaves the grid sample by sample
+            const uint32_t box = hit ? pm_box_cand(g, xs, e) : 0u;
+            dens.count = box == 0xffffffffu;
+            if (hit && lead && !dens.count) cn.cand += box;
+            float gv[3];
+            group_cdiff(xs, e, hit, G, dens, gv, cn);
+            cdiff_normal(gv, nx, ny, nz);
+        }
+        if (hit && lead) {
+            L.pos[idx] = make_float4(xs[0], xs[1], xs[2], 1.0f);
+            L.nrm[idx] = make_float4(nx, ny, nz, 1.0f);
+            if (L.t) L.t[idx] = th;
+            cn.hits++;
+        }
+    }
+    if (any) flush_counters(L.counters, cn.rays, cn.in_aabb, cn.hits, cn.samples, cn.cand, cn.march);
+}
+
 static hipError_t launch_finish(const MarchLaunch &L0, hipStream_t st)
 {
     const uint32_t T = ((L0.W + 7) / 8) * ((L0.H + 7) / 8);
     const uint32_t need = tile_waves_of(T);
     const dim3 grid(need < kMaxWaves ? need : kMaxWaves), blk(64);
+    if (T < (L0.g.sparse ? kGroupTiles : kGroupTilesDense) && !L0.s.instrument) {
+        hipLaunchKernelGGL(L0.g.sparse ? k_finish_groups<true> : k_finish_groups<false>, dim3(tile_waves_of(T << 2)), blk, 0, st, L0);
+        return hipGetLastError();
+    }
     if (L0.s.instrument) hipLaunchKernelGGL((k_finish<false, true, true>), grid, blk, 0, st, L0, nullptr, nullptr, 0u);
     else if (L0.g.sparse) hipLaunchKernelGGL((k_finish<false, false, true>), grid, blk, 0, st, L0, nullptr, nullptr, 0u);
     else hipLaunchKernelGGL((k_finish<false, false, false>), grid, blk, 0, st, L0, nullptr, nullptr, 0u);

@@ -106,3 +106,28 @@ def test_reference_groups(marcher, size, aniso, normal_mode):
     if aniso:
         _check(marcher, sc, counters=("rays", "hits", "samples", "cand", "march_samples"), skip_mode=4,
                normal_mode=normal_mode, **extra)
+
+
+@pytest.mark.parametrize("tiles", [(7, 9), (8, 8), (13, 5), (47, 17), (25, 32), (25, 33)])
+@pytest.mark.parametrize("per_cell", [1, 12])
+def test_tile_list_and_group_finish(marcher, tiles, per_cell):
+    """Tile counts around a mask's 64 (63, 64, 65) and around the finish rule's
+    line for sparse frames (799, 800, 825), ragged right and lower edges; 12 per
+    h/2 cell is a dense frame, whose small images all finish in lane groups.
+    Both normals, offsets that leave the list, no bisection, no FP64 step."""
+    rng = np.random.default_rng(per_cell)
+    h = 0.1
+    base = np.stack(np.meshgrid(*[np.arange(8)] * 3, indexing="ij"), -1).reshape(-1, 1, 3) * (h / 2)
+    xyz = (base + rng.uniform(0, h / 2, (base.shape[0], per_cell, 3))).reshape(-1, 3).astype(np.float32)
+    sc = scenes.tiny_scene(xyz, h, eye=(0.9, 0.8, -0.7), target=(0.2, 0.2, 0.2), width=8 * tiles[0] - 3,
+                           height=8 * tiles[1] - 5)
+    sc.iso *= per_cell
+    print(f"tile list and group finish, {tiles} tiles, {per_cell} per cell", flush=True)
+    marcher.set_frame(60, sc.xyz, sc.h)
+    for kw in (dict(normal_mode=0), dict(normal_mode=1), dict(normal_eps=0.03, final_fp64=0, bisect_iters=5),
+               dict(normal_eps=-0.004, bisect_iters=0), dict(bisect_iters=1, compensated=1)):
+        # the empty-cell skip counts every sample's whole stencil; the differences' box counts
+        # are the oracle's where the offset is the scene's own
+        keys = COUNTERS if "normal_mode" in kw and kw["normal_mode"] or "normal_eps" in kw else COUNTERS + ("cand",)
+        got = _check(marcher, sc, counters=keys, skip_mode=1, **kw)
+        assert got["hits"] > 100
