@@ -111,17 +111,16 @@ struct pm_ctx {
     // training set written by the trace logger
     DevBuf ds_feat, ds_label, ds_hit, ds_count, ds_meta;
     uint64_t ds_cap = 0;
-    // batched views: job and tile-chunk tables, all views' images, the captured launch
+    // batched views: job and tile tables, all views' images, the captured launch
     uint64_t frame_epoch = 0;           // bumped whenever a frame's device buffers may move
     uint64_t batch_epoch = ~0ull;
-    DevBuf b_jobs, b_chunks, b_img, b_ctr, b_flags, b_hits;
+    DevBuf b_jobs, b_tiles, b_img, b_flags, b_hits;
     unsigned long long b_rays0 = 0;     // rays of inactive tiles (written once as misses)
     bool prepass = false;               // the last single-view march ran the tile pre-pass
     std::vector<uint64_t> b_off;        // per view: first pixel in b_img
     std::vector<uint32_t> b_w, b_h;
     uint64_t b_npx = 0;
     BatchLaunch b_launch{};
-    uint32_t b_blocks = 0;
     hipGraph_t b_graph = nullptr;
     hipGraphExec_t b_exec = nullptr;
     bool b_ready = false;
@@ -233,7 +232,7 @@ void pm_destroy(pm_ctx *c)
     c->ds_feat.release(); c->ds_label.release(); c->ds_hit.release(); c->ds_count.release(); c->ds_meta.release();
     if (c->b_exec) hipGraphExecDestroy(c->b_exec);
     if (c->b_graph) hipGraphDestroy(c->b_graph);
-    c->b_jobs.release(); c->b_chunks.release(); c->b_img.release(); c->b_ctr.release(); c->b_flags.release();
+    c->b_jobs.release(); c->b_tiles.release(); c->b_img.release(); c->b_flags.release();
     c->b_hits.release();
     if (c->h_stage) hipHostFree(c->h_stage);
     if (c->h_counters) hipHostFree(c->h_counters);
@@ -903,13 +902,10 @@ int pm_get_stats(pm_ctx *c, pm_stats *out)
 
 // ---- batched views x frames ----
 
-static constexpr uint32_t kChunkTiles = 16;   // 8x8 tiles per queue entry (1024 rays)
-
 static int batch_enqueue_launch(pm_ctx *c)
 {
     HIPCHK(c, launch_init_counters(c->b_launch.base.counters, kCtrWords, c->b_rays0, c->stream));
-    HIPCHK(c, launch_zero_u32(c->b_launch.chunk_ctr, 1, c->stream));
-    HIPCHK(c, launch_march_batch(c->b_launch, c->b_blocks, c->stream));
+    HIPCHK(c, launch_march_batch(c->b_launch, c->stream));
     return PM_OK;
 }
 
@@ -1003,15 +999,14 @@ int pm_batch_set(pm_ctx *c, const pm_settings *s, const pm_view *views, uint32_t
         J.nrm = nrm + c->b_off[v];
         J.t = tt + c->b_off[v];
     }
-    // queue: views by decreasing ray count (longest first), each as runs of
-    // kChunkTiles consecutive tiles
+    // views by decreasing ray count (longest first)
     std::vector<uint32_t> order(n_views);
     for (uint32_t v = 0; v < n_views; v++) order[v] = v;
     std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) {
         return (uint64_t)c->b_w[a] * c->b_h[a] > (uint64_t)c->b_w[b] * c->b_h[b];
     });
     // Tiles none of whose rays enters the frame's AABB are answered once, here:
-    // their misses are written now and the queue holds only the other tiles
+    // their misses are written now and the list holds only the other tiles
     // (the images are identical; a run marches only tiles with work).
     std::vector<uint64_t> foff(n_views + 1, 0);
     for (uint32_t v = 0; v < n_views; v++)
@@ -1033,26 +1028,22 @@ int pm_batch_set(pm_ctx *c, const pm_settings *s, const pm_view *views, uint32_t
     }
     std::vector<uint32_t> flags(foff[n_views]);
     HIPCHK(c, copy_sync(c, flags.data(), c->b_flags.p, sizeof(uint32_t) * flags.size(), hipMemcpyDeviceToHost));
-    std::vector<BatchChunk> chunks;
+    std::vector<BatchTile> list;
     c->b_rays0 = 0;
     for (uint32_t v : order) {
         const uint32_t W = c->b_w[v], H = c->b_h[v], tx = (W + 7) / 8;
         const uint32_t tiles = (uint32_t)(foff[v + 1] - foff[v] - 1);
         const uint32_t *fl = flags.data() + foff[v];
-        for (uint32_t t = 0; t < tiles;) {
-            if (!fl[t]) {
-                const uint32_t x0 = (t % tx) * 8, y0 = (t / tx) * 8;
-                c->b_rays0 += (uint64_t)std::min(8u, W - x0) * std::min(8u, H - y0);
-                t++;
+        for (uint32_t t = 0; t < tiles; t++) {
+            if (fl[t]) {
+                list.push_back(BatchTile{ v, t });
                 continue;
             }
-            uint32_t t0 = t, n = 0;
-            while (t < tiles && fl[t] && n < kChunkTiles) { t++; n++; }
-            chunks.push_back(BatchChunk{ v, t0, n, 0u });
+            const uint32_t x0 = (t % tx) * 8, y0 = (t / tx) * 8;
+            c->b_rays0 += (uint64_t)std::min(8u, W - x0) * std::min(8u, H - y0);
         }
     }
-    if (chunks.empty()) chunks.push_back(BatchChunk{ order[0], 0u, 0u, 0u });   // nothing to march
-    if (chunks.size() >= (1ull << 32)) return fail(c, PM_ERR_SIZE, "pm_batch_set: too many tiles");
+    if (list.size() >= (1ull << 31)) return fail(c, PM_ERR_SIZE, "pm_batch_set: too many tiles");
 
     BatchLaunch &B = c->b_launch;
     B = BatchLaunch{};
@@ -1078,15 +1069,13 @@ int pm_batch_set(pm_ctx *c, const pm_settings *s, const pm_view *views, uint32_t
         J.mlp_gate_rho = B.base.mlp_gate_rho;
     }
     HIPCHK(c, c->b_jobs.ensure(sizeof(MarchLaunch) * jobs.size()));
-    HIPCHK(c, c->b_chunks.ensure(sizeof(BatchChunk) * chunks.size()));
-    HIPCHK(c, c->b_ctr.ensure(256));
+    HIPCHK(c, c->b_tiles.ensure(sizeof(BatchTile) * (list.size() + 1)));
     HIPCHK(c, copy_sync(c, c->b_jobs.p, jobs.data(), sizeof(MarchLaunch) * jobs.size(), hipMemcpyHostToDevice));
-    HIPCHK(c, copy_sync(c, c->b_chunks.p, chunks.data(), sizeof(BatchChunk) * chunks.size(), hipMemcpyHostToDevice));
+    if (!list.empty())
+        HIPCHK(c, copy_sync(c, c->b_tiles.p, list.data(), sizeof(BatchTile) * list.size(), hipMemcpyHostToDevice));
     B.jobs = (const MarchLaunch *)c->b_jobs.p;
-    B.chunks = (const BatchChunk *)c->b_chunks.p;
-    B.nchunks = (uint32_t)chunks.size();
-    B.chunk_ctr = (uint32_t *)c->b_ctr.p;
-    c->b_blocks = std::min<uint32_t>(1024u, (B.nchunks + 3) / 4 * 4);
+    B.tiles = (const BatchTile *)c->b_tiles.p;
+    B.ntiles = (uint32_t)list.size();
 
     if (use_graph) {
         HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));

@@ -75,24 +75,22 @@ struct MarchLaunch {
     AnisoDev an;               // s.anisotropic
 };
 
-// Batched launch: many (view, frame) jobs in one persistent kernel; every job
+// Batched launch: many (view, frame) jobs in one march and one finish; every job
 // is a complete MarchLaunch in device memory (read through a wave-uniform
 // pointer, so its fields stay in scalar registers and the scalar cache).
-// A run of consecutive 8x8 tiles of one job; waves take chunks, so the job's
-// parameters stay uniform across a wave.
-struct BatchChunk {
-    uint32_t job, tile0, ntiles, pad;
+// An active 8x8 tile of one job.
+struct BatchTile {
+    uint32_t job, tile;
 };
 struct BatchLaunch {
     MarchLaunch base;          // settings, counters and network (each job repeats them)
     const MarchLaunch *jobs;
-    const BatchChunk *chunks;
-    uint32_t nchunks;
-    uint32_t *chunk_ctr;
+    const BatchTile *tiles;    // the active tiles of all jobs
+    uint32_t ntiles;
     int sparse;                // every job's frame is (GridDev::sparse)
 };
 hipError_t launch_bound_grid(const GridDev &g, float iso, bool quarter_only, uint64_t *out, hipStream_t st);
-hipError_t launch_march_batch(const BatchLaunch &B, uint32_t blocks, hipStream_t st);
+hipError_t launch_march_batch(const BatchLaunch &B, hipStream_t st);
 hipError_t launch_zero_u32(uint32_t *p, uint32_t n, hipStream_t st);
 hipError_t launch_zero_u64(unsigned long long *p, uint32_t n, hipStream_t st);
 // counters[0..n) = 0 except counters[C_RAYS] = rays0 (rays answered without marching)

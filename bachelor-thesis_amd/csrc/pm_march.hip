@@ -547,17 +547,47 @@ __device__ __forceinline__ void finish_tile(const MarchLaunch &L, uint32_t tile,
 // candidate lists or the network's activations (never both at once).
 // INSTR adds the per-sample counts of instrumented launches.
 template <bool LEARNED, bool INSTR>
+__device__ __forceinline__ void march_part(const MarchLaunch &L, uint32_t tile, uint32_t i, uint32_t sub, float *region,
+                                           Counts &cn)
+{
+    const uint32_t lane = threadIdx.x;
+    uint32_t *lst = (uint32_t *)region + lane;
+    const bool comp = L.s.compensated != 0;
+    uint32_t px, py;
+    part_pixel(tile, (L.W + 7) / 8, i, sub, lane >> sub, px, py);
+    RayState r{};
+    r.phase = PH_DONE;
+    int G = 1 << sub;
+    if (px < L.W && py < L.H) ray_setup(L, r, px, py, cn, (lane & (uint32_t)(G - 1)) == 0);
+    while (__ballot(r.phase != PH_DONE) != 0) {
+        // The network is batched across the wave (the wave pays for it
+        // whenever any lane needs it): it runs once half of the busy
+        // lanes wait for a proposal, or when few rays are left; waiting
+        // lanes sit out.  Lane groups take no proposals: the learned march
+        // groups its last 16 rays only.
+        const int nbusy = __popcll(__ballot(r.phase != PH_DONE));
+        if (LEARNED && G == 1) {
+            const int nwant = __popcll(__ballot(r.phase == PH_PROPOSE));
+            if (nwant > 0 && (2 * nwant >= nbusy || nbusy <= 16)) wave_propose_step(L, r, cn, region);
+        }
+        if (!LEARNED || nbusy <= 16) regroup(r, G, region);
+        if (G == 1) {
+            if (r.phase == PH_MARCH) ray_step<INSTR, 16>(L, r, DensList{ &L.g, lst, comp }, cn);
+        } else {
+            group_step<INSTR>(L, r, G, DensList{ &L.g, lst, comp }, cn);
+        }
+    }
+}
+
+template <bool LEARNED, bool INSTR>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_march_tiles(MarchLaunch L)
 {
     // the lanes' candidate lists, or X[64][32] + H[32][64] bf16 + Y[64]
     static_assert(kListWords >= 2112, "network region");
     __shared__ float region[kListWords];
-    const uint32_t lane = threadIdx.x;
-    uint32_t *lst = (uint32_t *)region + lane;
-    const uint32_t tiles_x = (L.W + 7) / 8, T = tiles_x * ((L.H + 7) / 8);
+    const uint32_t T = ((L.W + 7) / 8) * ((L.H + 7) / 8);
     const uint32_t *order = L.tile_buf;
     const uint32_t TA = order[T];
-    const bool comp = L.s.compensated != 0;
     Counts cn;
     bool any = false;
     const uint32_t sub = LEARNED ? 0u : tile_split(TA);
@@ -565,30 +595,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
         const uint32_t i = xcd_tile(w);
         if (i >= TA << sub) continue;
         any = true;
-        uint32_t px, py;
-        part_pixel(order[i >> sub], tiles_x, i, sub, lane >> sub, px, py);
-        RayState r{};
-        r.phase = PH_DONE;
-        int G = 1 << sub;
-        if (px < L.W && py < L.H) ray_setup(L, r, px, py, cn, (lane & (uint32_t)(G - 1)) == 0);
-        while (__ballot(r.phase != PH_DONE) != 0) {
-            // The network is batched across the wave (the wave pays for it
-            // whenever any lane needs it): it runs once half of the busy
-            // lanes wait for a proposal, or when few rays are left; waiting
-            // lanes sit out.  Lane groups take no proposals: the learned march
-            // groups its last 16 rays only.
-            const int nbusy = __popcll(__ballot(r.phase != PH_DONE));
-            if (LEARNED && G == 1) {
-                const int nwant = __popcll(__ballot(r.phase == PH_PROPOSE));
-                if (nwant > 0 && (2 * nwant >= nbusy || nbusy <= 16)) wave_propose_step(L, r, cn, region);
-            }
-            if (!LEARNED || nbusy <= 16) regroup(r, G, region);
-            if (G == 1) {
-                if (r.phase == PH_MARCH) ray_step<INSTR, 16>(L, r, DensList{ &L.g, lst, comp }, cn);
-            } else {
-                group_step<INSTR>(L, r, G, DensList{ &L.g, lst, comp }, cn);
-            }
-        }
+        march_part<LEARNED, INSTR>(L, order[i >> sub], i, sub, region, cn);
     }
     if (any) flush_counts(L.counters, cn);
 }
@@ -740,90 +747,31 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     if (any) flush_counters(L.counters, cn.rays, cn.in_aabb, cn.hits, cn.samples, cn.cand, cn.march);
 }
 
-// Batched schedule: persistent waves take chunks of tiles (each chunk belongs to
-// one (view, frame) job) from one counter; inside a chunk lanes are refilled
-// ray by ray as in k_march_persist; a wave moves to its next chunk -- and
-// loads that job's grid and camera -- once all its lanes are idle.
+// The march of a batch: as k_march_tiles, over the active tiles of all views
+// (B.tiles, the largest view first), each tile with its own job's grid and
+// camera.  The tiles are the work items because their number bounds a small
+// batch: persistent waves that drew runs of 16 tiles from a counter left most of
+// the chip idle on eight views of 0.6 MP in all.  March and finish: those 4.68 ->
+// 0.55 ms; one view of 0.03 MP 2.0 -> 0.28; 64 views, 23 MP, 8.4 -> 5.2; 64
+// views, 45 MP of two 1,024,000-particle frames, 14.0 -> 7.4, learned 14.7 -> 8.1.
 template <bool LEARNED>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_march_batch(BatchLaunch B)
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_march_batch(BatchLaunch B)
 {
-    constexpr int kRegion = kListWords;
-    __shared__ float lds[4 * kRegion];
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    float *region = lds + wave * kRegion;
-    uint32_t *lst = (uint32_t *)region + lane;
-    const bool comp = B.base.s.compensated != 0;
-
-    const MarchLaunch *Lp = B.jobs;
+    __shared__ float region[kListWords];
     Counts cn;
-    RayState r{};
-    r.phase = PH_DONE;
-    uint32_t tile = 0, tile_i = 0, ntiles = 0, tile0 = 0;
-    int qpos = 64;
-    bool exhausted = false;
-    const unsigned long long lt_mask = (1ull << lane) - 1ull;
-    // lane groups while a chunk drains (its last rays, before the next job)
-    int G = 1;
-    const bool group_ok = B.base.s.skip_mode == PM_SKIP_BOUND || B.base.s.skip_mode == PM_SKIP_NONE;
-
-    while (true) {
-        while (!exhausted) {
-            unsigned long long needy = __ballot(r.phase == PH_DONE);
-            if (needy == 0) break;
-            if (qpos >= 64) {
-                if (tile_i < ntiles) {
-                    tile = tile0 + tile_i++;
-                    qpos = 0;
-                } else {
-                    if (__ballot(r.phase != PH_DONE) != 0) break;    // drain before changing job
-                    uint32_t cidx = 0;
-                    if (lane == 0) cidx = atomicAdd(B.chunk_ctr, 1u);
-                    cidx = __builtin_amdgcn_readfirstlane(__shfl(cidx, 0, 64));
-                    if (cidx >= B.nchunks) { exhausted = true; break; }
-                    const BatchChunk ch = B.chunks[cidx];
-                    Lp = B.jobs + __builtin_amdgcn_readfirstlane(ch.job);
-                    tile0 = ch.tile0;
-                    ntiles = ch.ntiles;
-                    tile_i = 0;
-                    G = 1;                                        // every lane its own ray again
-                    continue;
-                }
-            }
-            int rank = __popcll(needy & lt_mask);
-            int take = __popcll(needy);
-            if (r.phase == PH_DONE && qpos + rank < 64) {
-                uint32_t j = (uint32_t)(qpos + rank);
-                const uint32_t tiles_x = (Lp->W + 7) / 8;
-                uint32_t px = (tile % tiles_x) * 8 + (j & 7u), py = (tile / tiles_x) * 8 + (j >> 3);
-                if (px < Lp->W && py < Lp->H) ray_setup(*Lp, r, px, py, cn);
-            }
-            qpos = qpos + take < 64 ? qpos + take : 64;
-        }
-        if (__ballot(r.phase != PH_DONE) == 0) {
-            if (exhausted) break;
-            continue;
-        }
-        // batched proposals, as in k_march_persist (before the lane groups)
-        const bool draining = exhausted || (qpos >= 64 && tile_i >= ntiles);
-        if (LEARNED) {
-            const int nbusy = __popcll(__ballot(r.phase != PH_DONE));
-            const int nwant = __popcll(__ballot(r.phase == PH_PROPOSE));
-            if (nwant > 0 && (2 * nwant >= nbusy || draining))
-                wave_propose_step(*Lp, r, cn, region);
-        }
-        if (group_ok && draining) regroup(r, G, region);
-        if (G == 1) {
-            if (r.phase == PH_MARCH) {
-                ray_step<false, 8>(*Lp, r, DensList{ &Lp->g, lst, comp }, cn);
-            }
-        } else {
-            group_step<false>(*Lp, r, G, DensList{ &Lp->g, lst, comp }, cn);
-        }
+    bool any = false;
+    const uint32_t sub = LEARNED ? 0u : tile_split(B.ntiles);
+    for (uint32_t w = blockIdx.x; w < tile_waves_of(B.ntiles << sub); w += gridDim.x) {
+        const uint32_t i = xcd_tile(w);
+        if (i >= B.ntiles << sub) continue;
+        any = true;
+        const BatchTile bt = B.tiles[i >> sub];
+        march_part<LEARNED, false>(B.jobs[__builtin_amdgcn_readfirstlane(bt.job)], bt.tile, i, sub, region, cn);
     }
-    flush_counts(B.base.counters, cn);
+    if (any) flush_counts(B.base.counters, cn);
 }
 
-// Single launch: a wave per active tile; batch: a wave per chunk of tiles.
+// A wave per active tile, of the view or of the batch.
 // LIST: a hit's samples share one candidate list.  It pays where the lists fit
 // (GridDev::sparse, at most 3 particles per occupied h/2 cell: 466 -> 223 us on
 // the 1 M dam break, 1.4 per cell); in denser frames (4 M pool, 8 per cell) most
@@ -832,17 +780,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 8))) voi
 // Registers are capped for four waves per SIMD.
 template <bool BATCH, bool INSTR, bool LIST>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LIST ? 3 : 4, 8))) void k_finish(MarchLaunch L0, const MarchLaunch *__restrict__ jobs,
-                                                const BatchChunk *__restrict__ chunks, uint32_t nchunks)
+                                                const BatchTile *__restrict__ tiles, uint32_t ntiles)
 {
     __shared__ uint32_t lds[LIST ? kFinWords : kListWords];
     uint32_t *lst = lds + threadIdx.x;
     Counts cn;
     bool any = false;
     if (BATCH) {
-        for (uint32_t c = blockIdx.x; c < nchunks; c += gridDim.x) {
-            const BatchChunk ch = chunks[c];
-            const MarchLaunch *Lp = jobs + __builtin_amdgcn_readfirstlane(ch.job);
-            for (uint32_t t = 0; t < ch.ntiles; t++) finish_tile<INSTR, LIST>(*Lp, ch.tile0 + t, lst, cn);
+        for (uint32_t w = blockIdx.x; w < tile_waves_of(ntiles); w += gridDim.x) {
+            const uint32_t i = xcd_tile(w);
+            if (i >= ntiles) continue;
+            const BatchTile bt = tiles[i];
+            finish_tile<INSTR, LIST>(jobs[__builtin_amdgcn_readfirstlane(bt.job)], bt.tile, lst, cn);
             any = true;
         }
     } else {
@@ -999,15 +948,19 @@ static hipError_t launch_finish(const MarchLaunch &L0, hipStream_t st)
     return hipGetLastError();
 }
 
-hipError_t launch_march_batch(const BatchLaunch &B, uint32_t blocks, hipStream_t st)
+hipError_t launch_march_batch(const BatchLaunch &B, hipStream_t st)
 {
-    if (B.base.s.learned) hipLaunchKernelGGL((k_march_batch<true>), dim3(blocks), dim3(256), 0, st, B);
-    else hipLaunchKernelGGL((k_march_batch<false>), dim3(blocks), dim3(256), 0, st, B);
+    const uint32_t need = tile_waves_of(B.ntiles << (B.base.s.learned ? 0u : tile_split(B.ntiles)));
+    const dim3 grid(need < kMaxWaves ? need : kMaxWaves), blk(64);
+    if (need == 0) return hipSuccess;   // no tile to march
+    if (B.base.s.learned) hipLaunchKernelGGL((k_march_batch<true>), grid, blk, 0, st, B);
+    else hipLaunchKernelGGL((k_march_batch<false>), grid, blk, 0, st, B);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const uint32_t fb = B.nchunks < kMaxWaves ? B.nchunks : kMaxWaves;
-    if (B.sparse) hipLaunchKernelGGL((k_finish<true, false, true>), dim3(fb), dim3(64), 0, st, B.base, B.jobs, B.chunks, B.nchunks);
-    else hipLaunchKernelGGL((k_finish<true, false, false>), dim3(fb), dim3(64), 0, st, B.base, B.jobs, B.chunks, B.nchunks);
+    const uint32_t nf = tile_waves_of(B.ntiles);
+    const dim3 fgrid(nf < kMaxWaves ? nf : kMaxWaves);
+    if (B.sparse) hipLaunchKernelGGL((k_finish<true, false, true>), fgrid, blk, 0, st, B.base, B.jobs, B.tiles, B.ntiles);
+    else hipLaunchKernelGGL((k_finish<true, false, false>), fgrid, blk, 0, st, B.base, B.jobs, B.tiles, B.ntiles);
     return hipGetLastError();
 }
 

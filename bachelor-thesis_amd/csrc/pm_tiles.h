@@ -259,7 +259,7 @@ __host__ __device__ __forceinline__ uint32_t tile_waves_of(uint32_t T)
 // (4,300) 331 / 297 / 318 / 448 us, 4K pool (19,000) 2,490 / 2,578 / 2,899 /
 // 5,184 us.
 static constexpr uint32_t kResidentWaves = 4096, kMaxSplit = 2;
-__device__ __forceinline__ uint32_t tile_split(uint32_t TA)
+__host__ __device__ __forceinline__ uint32_t tile_split(uint32_t TA)
 {
     return TA < kResidentWaves ? 2u : (TA < 2 * kResidentWaves ? 1u : 0u);
 }

@@ -131,3 +131,32 @@ def test_tile_list_and_group_finish(marcher, tiles, per_cell):
         keys = COUNTERS if "normal_mode" in kw and kw["normal_mode"] or "normal_eps" in kw else COUNTERS + ("cand",)
         got = _check(marcher, sc, counters=keys, skip_mode=1, **kw)
         assert got["hits"] > 100
+
+
+@pytest.mark.parametrize("use_graph", [False, True])
+@pytest.mark.parametrize("away", ["none", "some", "all"])
+def test_batch_tile_list(marcher, use_graph, away):
+    """The batch's tile list: views of one pixel, one ragged tile and many tiles,
+    views that look away from the particles, no active tile at all; each image
+    equals the oracle's, run after run."""
+    sc = scenes.lattice_cube(4, n_side=10, spacing=0.05, width=32, height=32)
+    print(f"batch tile list graph {use_graph} away {away}", flush=True)
+    marcher.set_frame(60, sc.xyz, sc.h)
+    st = sc.settings(skip_mode=4)
+    G = O.Grid(sc.xyz, sc.h)
+    cams = []
+    for i, (w, h) in enumerate(((1, 1), (7, 5), (130, 67), (8, 8))):
+        off = away == "all" or (away == "some" and i % 2 == 0)
+        eye = np.array([0.5, 0.6, 2.2])
+        cams.append(scenes.make_camera(eye, np.array([0.5, 0.6, 9.0]) if off else np.array([0.5, 0.5, 0.5]), w, h))
+    marcher.batch_set(st, [(60, c.width, c.height, c.inv_pv, c.eye) for c in cams], use_graph=use_graph)
+    ref = [O.march(G, O.make_settings(**st), c.inv_pv, c.eye, c.width, c.height) for c in cams]
+    assert (sum(o[3]["hits"] for o in ref) > 0) == (away != "all")
+    for _ in range(3):
+        marcher.batch_run()
+        marcher.wait()
+        for v, o in enumerate(ref):
+            for got, want in zip(marcher.batch_download(v), o[:3]):
+                assert np.array_equal(got, want.reshape(got.shape)), v
+        for k in ("rays", "hits", "samples", "march_samples"):
+            assert marcher.stats()[k] == sum(o[3][k] for o in ref), k
