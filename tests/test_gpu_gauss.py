@@ -36,3 +36,13 @@ def test_depth_smooth_1080p_timing(marcher):
     ref = O.depth_smooth(depth[:40], 8)
     assert np.array_equal(out[:20], ref[:20])           # rows whose window stays inside the slab
     print(f"1080p N=8 smoothing incl. copies: {dt * 1e3:.2f} ms", flush=True)
+
+
+@pytest.mark.parametrize("W,H", [(31, 33), (65, 32), (130, 95)])
+@pytest.mark.parametrize("N", [2, 3, 5, 12, 15, 16, 17, 30])
+def test_depth_smooth_every_window(marcher, W, H, N):
+    """Windows on both sides of a 64-wide row (N = 16), images around a tile's
+    32x32 and narrower than the window."""
+    rng = np.random.default_rng(W * 100 + N)
+    depth = rng.uniform(0.2, 1.0, (H, W)).astype(np.float32)
+    assert np.array_equal(marcher.depth_smooth(depth, N), O.depth_smooth(depth, N))
