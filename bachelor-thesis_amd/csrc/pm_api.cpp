@@ -1469,11 +1469,11 @@ int pm_mlp_forward(pm_ctx *c, const float *x, uint64_t n, float *y)
 }
 
 // One forward/backward over device rows `feat`/`label` (ids from idx, or 0..n-1),
-// partial gradients reduced in wave order; optionally one Adam step.
+// partial gradients reduced in a fixed order; optionally one Adam step.
 static int mlp_pass(pm_ctx *c, const float *feat, const float *label, const uint32_t *idx, uint32_t n, float w_over,
                     bool apply, float lr, float *loss_dev_out, float *grad_dev_out)
 {
-    uint32_t nw = n / 64;
+    const uint32_t nw = std::min(n / 64, kTrainBlocks);
     HIPCHK(c, c->mlp_partial.ensure(sizeof(float) * (size_t)nw * (PM_MLP_NPARAM + 1)));
     TrainArgs ta{};
     ta.net = mlp_dev(c);
@@ -1482,6 +1482,7 @@ static int mlp_pass(pm_ctx *c, const float *feat, const float *label, const uint
     ta.idx = idx;
     ta.inv_batch = 1.0f / (float)n;
     ta.w_over = w_over;
+    ta.ngroups = n / 64;
     ta.partial = (float *)c->mlp_partial.p;
     HIPCHK(c, launch_mlp_train(ta, nw, c->stream));
     AdamArgs aa{};

@@ -191,8 +191,10 @@ struct TrainArgs {
     const float *label;
     const uint32_t *idx;      // batch sample ids (NULL: 0..B-1)
     float inv_batch, w_over;
-    float *partial;           // [nwaves][NPARAM + 1]
+    uint32_t ngroups;         // B / 64
+    float *partial;           // [nblocks][NPARAM + 1]
 };
+static constexpr uint32_t kTrainBlocks = 512;   // most workgroups of k_mlp_train: two per CU fit its LDS
 struct AdamArgs {
     const float *partial;
     uint32_t nparts;
@@ -202,7 +204,7 @@ struct AdamArgs {
     float *grad_out;          // optional summed gradient
     float *loss_out;
 };
-hipError_t launch_mlp_train(const TrainArgs &a, uint32_t nwaves, hipStream_t st);
+hipError_t launch_mlp_train(const TrainArgs &a, uint32_t nblocks, hipStream_t st);
 hipError_t launch_mlp_adam(const AdamArgs &a, hipStream_t st);
 hipError_t launch_mlp_sync(const float *p, uint16_t *W1, uint16_t *W2, uint16_t *W2T, hipStream_t st);
 hipError_t launch_mlp_forward(const MlpDev &net, const float *feat, uint32_t n, float *y, hipStream_t st);

@@ -50,6 +50,28 @@ def test_mlp_gradient_matches_oracle(marcher):
     assert np.all(grad[M.OFF_W1:M.OFF_B1].reshape(M.H, M.K1)[:, M.NIN:] == 0)
 
 
+@pytest.mark.parametrize("rows", [64, 64 * 17, 64 * 512, 64 * 513])
+def test_mlp_gradient_rows(marcher, rows):
+    """One group of 64 rows, a partial of every sum beyond 16, and as many and
+    one more group than the training kernel has workgroups: the same BF16
+    products as the oracle's, so the gradient test's 2e-2 holds; two runs agree
+    bit for bit."""
+    rng = np.random.default_rng(rows)
+    p = M.init(3)
+    x = rng.uniform(-1, 2, (rows, M.NIN)).astype(np.float32)
+    t = rng.uniform(0, 4, rows).astype(np.float32)
+    marcher.mlp_set(p)
+    loss, grad = marcher.mlp_grad(x, t, 4.0)
+    lo, go = M.loss_grad(p, x, t, 4.0)
+    assert loss == pytest.approx(lo, rel=2e-3)
+    for a, b in ((M.OFF_W1, M.OFF_B1), (M.OFF_B1, M.OFF_W2), (M.OFF_W2, M.OFF_B2), (M.OFF_B2, M.OFF_W3),
+                 (M.OFF_W3, M.OFF_B3), (M.OFF_B3, M.NPARAM)):
+        u, v = grad[a:b].astype(np.float64), go[a:b]
+        assert np.linalg.norm(u - v) < 2e-2 * max(np.linalg.norm(v), 1e-30)
+    again = marcher.mlp_grad(x, t, 4.0)
+    assert again[0] == loss and np.array_equal(again[1], grad)
+
+
 def test_mlp_training_fits_smooth_target(marcher):
     """Adam on a device dataset of traces lowers the loss; determinism of two runs."""
     sc = scenes.dam_break(5, nx=40, ny=80, nz=40, width=480, height=270)
