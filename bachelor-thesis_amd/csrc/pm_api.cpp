@@ -43,7 +43,7 @@ struct DevBuf {
 struct Frame {
     pm_frame_info info{};
     GridDev g{};
-    DevBuf sorted, cell_start, cell_of, counts, cursor, scan_tmp, xyz, bounds_partial, bounds, scattered;
+    DevBuf sorted, cell_start, counts, slots, indices, scan_tmp, xyz, bounds_partial, bounds;
     DevBuf empty27, clear, clear_tmp, dg_box, dg_cons, dg_count, coarse, bound;
     DevBuf fsorted, fcell_start;    // march grid (cells of h/2)
     bool bound_ok = false;      // bound holds the sub-box bits for bound_iso and bound_boxes
@@ -56,8 +56,8 @@ struct Frame {
     void release()
     {
         coarse.release();
-        sorted.release(); cell_start.release(); cell_of.release(); counts.release(); cursor.release();
-        scan_tmp.release(); xyz.release(); bounds_partial.release(); bounds.release(); scattered.release();
+        sorted.release(); cell_start.release(); counts.release(); slots.release(); indices.release();
+        scan_tmp.release(); xyz.release(); bounds_partial.release(); bounds.release();
         empty27.release(); clear.release(); clear_tmp.release(); dg_box.release(); dg_cons.release(); dg_count.release(); bound.release();
         fsorted.release(); fcell_start.release();
         for (hipEvent_t &e : bound_ev)
@@ -299,6 +299,9 @@ static int build_frame(pm_ctx *c, int32_t frame, const float *d_src, uint64_t n,
     const float inv_hf = 2.0f * inv_h;
     uint64_t fnc = 1;
     for (int ax = 0; ax < 3; ax++) {
+        // a key beyond an int32 would differ between host and device
+        if (!(I.pmin[ax] * inv_hf > -2147483008.0f && I.pmax[ax] * inv_hf < 2147483008.0f))
+            return fail(c, PM_ERR_SIZE, "pm_set_frame: coordinates beyond 2^30 h");
         int32_t kmin = host_key(I.pmin[ax], inv_hf), kmax = host_key(I.pmax[ax], inv_hf);
         I.forigin[ax] = kmin - 4;
         I.fdims[ax] = kmax - kmin + 9;
@@ -307,55 +310,36 @@ static int build_frame(pm_ctx *c, int32_t frame, const float *d_src, uint64_t n,
     if (fnc >= (1ull << 31)) return fail(c, PM_ERR_SIZE, "pm_set_frame: march grid of %llu cells exceeds 2^31", (unsigned long long)fnc);
     I.fncells = fnc;
 
-    // scratch of both builds sized once, before either is queued
-    const uint64_t mc = fnc > nc ? fnc : nc;
     HIPCHK(c, f->sorted.ensure(sizeof(float4) * n));
     HIPCHK(c, f->cell_start.ensure(sizeof(uint32_t) * (nc + 1)));
     HIPCHK(c, f->fsorted.ensure(sizeof(float4) * n));
     HIPCHK(c, f->fcell_start.ensure(sizeof(uint32_t) * (fnc + 1)));
-    HIPCHK(c, f->cell_of.ensure(sizeof(uint32_t) * n));
-    HIPCHK(c, f->scattered.ensure(sizeof(float4) * n));
-    HIPCHK(c, f->counts.ensure(sizeof(uint32_t) * (mc + 1)));
-    HIPCHK(c, f->cursor.ensure(sizeof(uint32_t) * mc));
-    HIPCHK(c, f->scan_tmp.ensure(sizeof(uint32_t) * scan_tmp_size((uint32_t)(mc + 1))));
+    HIPCHK(c, f->slots.ensure(sizeof(uint32_t) * n));
+    HIPCHK(c, f->indices.ensure(sizeof(uint32_t) * n));
+    HIPCHK(c, f->counts.ensure(sizeof(uint32_t) * fnc));
+    const size_t scan_words = scan_tmp_size((uint32_t)nc, (uint32_t)fnc);
+    HIPCHK(c, f->scan_tmp.ensure(sizeof(uint32_t) * (scan_words + 2)));
 
     GridBuildArgs a{};
-    a.xyz = d_src; a.n = n; a.inv_h = inv_h;
-    a.ox = I.origin[0]; a.oy = I.origin[1]; a.oz = I.origin[2];
-    a.nx = I.dims[0]; a.ny = I.dims[1]; a.nz = I.dims[2];
+    a.xyz = d_src; a.n = n;
+    a.inv_hf = inv_hf;
+    for (int ax = 0; ax < 3; ax++) {
+        a.fo[ax] = I.forigin[ax]; a.fn[ax] = I.fdims[ax];
+        a.dorg[ax] = I.origin[ax]; a.dn[ax] = I.dims[ax];
+    }
     a.ncells = (uint32_t)nc;
-    a.cell_of = (uint32_t *)f->cell_of.p;
+    a.fncells = (uint32_t)fnc;
     a.counts = (uint32_t *)f->counts.p;
-    a.cursor = (uint32_t *)f->cursor.p;
-    a.scan_tmp = (uint32_t *)f->scan_tmp.p;
+    a.slot = (uint32_t *)f->slots.p;
+    a.index = (uint32_t *)f->indices.p;
     a.sorted = (float4 *)f->sorted.p;
+    a.fsorted = (float4 *)f->fsorted.p;
     a.cell_start = (uint32_t *)f->cell_start.p;
-    a.scattered = (float4 *)f->scattered.p;
+    a.fcell_start = (uint32_t *)f->fcell_start.p;
+    a.scan_tmp = (uint32_t *)f->scan_tmp.p;
+    a.occupied = a.scan_tmp + scan_words;
     HIPCHK(c, launch_grid_build(a, st));
-
-    GridBuildArgs fa = a;   // the march grid: same build, cells of h/2
-    fa.inv_h = inv_hf;
-    fa.ox = I.forigin[0]; fa.oy = I.forigin[1]; fa.oz = I.forigin[2];
-    fa.nx = I.fdims[0]; fa.ny = I.fdims[1]; fa.nz = I.fdims[2];
-    fa.ncells = (uint32_t)fnc;
-    fa.counts = (uint32_t *)f->counts.p;
-    fa.cursor = (uint32_t *)f->cursor.p;
-    fa.scan_tmp = (uint32_t *)f->scan_tmp.p;
-    fa.sorted = (float4 *)f->fsorted.p;
-    fa.cell_start = (uint32_t *)f->fcell_start.p;
-    HIPCHK(c, launch_grid_build(fa, st));
-    // occupied march-grid cells (into counts, which the builds are done with)
-    uint32_t occupied = 0;
-    HIPCHK(c, launch_zero_u32((uint32_t *)f->counts.p, 1, st));
-    HIPCHK(c, launch_occupied((const uint32_t *)f->fcell_start.p, (uint32_t)fnc, (uint32_t *)f->counts.p, st));
-    HIPCHK(c, hipMemcpyAsync(&occupied, f->counts.p, sizeof(occupied), hipMemcpyDeviceToHost, st));
     HIPCHK(c, hipEventRecord(e1, st));
-    HIPCHK(c, hipEventSynchronize(e1));
-    float ms = 0.f;
-    hipEventElapsedTime(&ms, e0, e1);
-    I.build_ms = ms;
-    hipEventDestroy(e0);
-    hipEventDestroy(e1);
 
     GridDev &g = f->g;
     g.sorted = (const float4 *)f->sorted.p;
@@ -376,7 +360,6 @@ static int build_frame(pm_ctx *c, int32_t frame, const float *d_src, uint64_t n,
     g.fox = I.forigin[0]; g.foy = I.forigin[1]; g.foz = I.forigin[2];
     g.fnx = I.fdims[0]; g.fny = I.fdims[1]; g.fnz = I.fdims[2];
     g.inv_hf = inv_hf;
-    g.sparse = n <= (uint64_t)kSparsePerCell * occupied;
 
     // skip structures: empty 27-neighbourhoods and the reference DensityGrid
     HIPCHK(c, f->empty27.ensure(nc));
@@ -402,7 +385,15 @@ static int build_frame(pm_ctx *c, int32_t frame, const float *d_src, uint64_t n,
     HIPCHK(c, f->coarse.ensure(4ull * f->cg.nx * f->cg.ny * f->cg.nz));
     f->cg.count = (const uint32_t *)f->coarse.p;
     HIPCHK(c, launch_coarse_counts(g, f->cg, (uint32_t *)f->coarse.p, st));
+    uint32_t occupied[2] = { 0, 0 };
+    HIPCHK(c, hipMemcpyAsync(occupied, a.occupied, sizeof(occupied), hipMemcpyDeviceToHost, st));
     HIPCHK(c, hipStreamSynchronize(st));
+    g.sparse = n <= (uint64_t)kSparsePerCell * occupied[1];
+    float ms = 0.f;
+    hipEventElapsedTime(&ms, e0, e1);
+    I.build_ms = ms;
+    hipEventDestroy(e0);
+    hipEventDestroy(e1);
     return PM_OK;
 }
 

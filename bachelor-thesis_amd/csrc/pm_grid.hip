@@ -3,8 +3,8 @@
 // and of Frame::ComputeAABB (Dataset.cpp:78-92).
 //
 // Pipeline (one stream, no host round trip except the extent read-back):
-//   bounds reduce -> cell id + histogram (atomics) -> exclusive scan ->
-//   scatter into cell-major float4 -> per-cell sort by input index.
+//   bounds reduce -> histogram (atomics) -> exclusive scan -> indices placed
+//   cell by cell -> per-cell sort by input index into cell-major float4.
 // The per-cell sort makes the stored order deterministic (cell, input index),
 // which is the canonical neighbour order the density sums follow.
 // All passes are HBM-bound streaming passes over n particles or C cells.
@@ -87,127 +87,224 @@ __global__ void k_fill_u32(uint32_t *__restrict__ p, uint64_t n, uint32_t v)
         p[i] = v;
 }
 
+// Both grids of a frame are built together from one histogram, the march grid's:
+// a cell of h is 2x2x2 cells of h/2 (the keys are floor-like and 2/h is exact, so
+// key(x, 1/h) = key(x, 2/h) >> 1, of negative coordinates too), so its count is
+// the sum of eight and its particles are four runs of the march grid's order.
+// The atomics bound the build (25 G/s): one per particle, which also gives the
+// particle its place, where a histogram and a cursor for each grid took four.  Only the 4-byte index is placed; the particle
+// itself is read by the ranking pass, which ranks it in both grids.  A launch's
+// workgroups take contiguous runs of particles per XCD (xcd_run): neighbours in
+// the input meet in the same cells, and their atomics and stores in one L2.
+// 1.02 M particles: both sorts 250 us in 18 launches, now 105 in 7 (count 41, place
+// 14, rank 28); the 4 M pool's, unevenly dense, 1,630 us, now 513 (rank 264).
+
+// The blockIdx-th of `blocks` work items, contiguous runs for each of the 8 XCDs
+// (workgroups are dispatched round-robin over them); >= blocks: none.
+__device__ __forceinline__ uint64_t xcd_run(uint64_t blocks)
+{
+    const uint64_t per = (blocks + 7) / 8;
+    return (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
+}
+
+// Cell of the march grid relative to its origin.
+__device__ __forceinline__ void fine_cell(const GridBuildArgs &a, float x, float y, float z, int32_t k[3])
+{
+    k[0] = pm_key(x, a.inv_hf) - a.fo[0];
+    k[1] = pm_key(y, a.inv_hf) - a.fo[1];
+    k[2] = pm_key(z, a.inv_hf) - a.fo[2];
+}
+
+__device__ __forceinline__ uint32_t fine_lin(const GridBuildArgs &a, int32_t x, int32_t y, int32_t z)
+{
+    return (uint32_t)x + (uint32_t)a.fn[0] * ((uint32_t)y + (uint32_t)a.fn[1] * (uint32_t)z);
+}
+
 __global__ __launch_bounds__(kThreads) void k_cell_count(GridBuildArgs a)
 {
-    uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
+    const uint64_t i = xcd_run((a.n + kThreads - 1) / kThreads) * kThreads + threadIdx.x;
     if (i >= a.n) return;
-    int32_t cx = pm_key(a.xyz[3 * i + 0], a.inv_h) - a.ox;
-    int32_t cy = pm_key(a.xyz[3 * i + 1], a.inv_h) - a.oy;
-    int32_t cz = pm_key(a.xyz[3 * i + 2], a.inv_h) - a.oz;
-    uint32_t c = (uint32_t)cx + (uint32_t)a.nx * ((uint32_t)cy + (uint32_t)a.ny * (uint32_t)cz);
-    a.cell_of[i] = c;
-    atomicAdd(&a.counts[c], 1u);
+    int32_t k[3];
+    fine_cell(a, a.xyz[3 * i + 0], a.xyz[3 * i + 1], a.xyz[3 * i + 2], k);
+    a.slot[i] = atomicAdd(&a.counts[fine_lin(a, k[0], k[1], k[2])], 1u);
 }
 
 // ---- exclusive scan of u32 (len up to 2^31), 1024 elements per block ----
 static constexpr int kScanPer = 4;
 static constexpr int kScanBlock = kThreads * kScanPer;
 
-size_t scan_tmp_size(uint32_t len)
+static inline uint32_t scan_blocks(uint32_t len) { return (len + kScanBlock - 1) / kScanBlock; }
+
+// Per block of the scan its sum and its number of nonzero elements.
+size_t scan_tmp_size(uint32_t ncells, uint32_t fncells)
 {
-    return (size_t)((len + kScanBlock - 1) / kScanBlock) + 1;
+    return 2 * ((size_t)scan_blocks(ncells + 1) + scan_blocks(fncells + 1));
 }
 
+// Exclusive scan of one value per thread: within waves by shuffles, then over the
+// waves' sums (sh: one u32 per wave).
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t *sh, uint32_t &total)
 {
-    // Hillis-Steele over 256 thread totals in LDS.
-    sh[threadIdx.x] = v;
-    __syncthreads();
-    for (int off = 1; off < kThreads; off <<= 1) {
-        uint32_t add = (int)threadIdx.x >= off ? sh[threadIdx.x - off] : 0u;
-        __syncthreads();
-        sh[threadIdx.x] += add;
-        __syncthreads();
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    uint32_t incl = v;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t o = __shfl_up(incl, off, 64);
+        if ((int)lane >= off) incl += o;
     }
-    total = sh[kThreads - 1];
-    uint32_t incl = sh[threadIdx.x];
+    __syncthreads();                               // sh may still be read from the last call
+    if (lane == 63) sh[wave] = incl;
     __syncthreads();
-    return incl - v;
+    uint32_t before = 0;
+    total = 0;
+    for (uint32_t w = 0; w < nw; w++) {
+        const uint32_t s = sh[w];
+        before += w < wave ? s : 0u;
+        total += s;
+    }
+    return before + incl - v;
 }
 
-__global__ __launch_bounds__(kThreads) void k_scan_blocks(const uint32_t *__restrict__ in, uint32_t *__restrict__ out,
-                                                          uint32_t len, uint32_t *__restrict__ block_sums)
+// Particles in cell c of the search grid: its eight march-grid cells.  Particles
+// lie at least two cells inside the search grid; its border cells, whose march
+// cells may lie outside the march grid, hold none.
+__device__ __forceinline__ uint32_t dense_count(const GridBuildArgs &a, uint32_t c)
 {
-    __shared__ uint32_t sh[kThreads];
-    uint32_t base = blockIdx.x * kScanBlock + threadIdx.x * kScanPer;
-    uint32_t v[kScanPer], sum = 0;
-    for (int j = 0; j < kScanPer; j++) {
-        v[j] = base + j < len ? in[base + j] : 0u;
-        sum += v[j];
+    const int32_t x = (int32_t)(c % (uint32_t)a.dn[0]), yz = (int32_t)(c / (uint32_t)a.dn[0]);
+    const int32_t y = yz % a.dn[1], z = yz / a.dn[1];
+    if (x < 2 || y < 2 || z < 2 || x > a.dn[0] - 3 || y > a.dn[1] - 3 || z > a.dn[2] - 3) return 0;
+    const int32_t fx = 2 * (x + a.dorg[0]) - a.fo[0], fy = 2 * (y + a.dorg[1]) - a.fo[1], fz = 2 * (z + a.dorg[2]) - a.fo[2];
+    uint32_t s = 0;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const uint32_t row = fine_lin(a, fx, fy + (r & 1), fz + (r >> 1));
+        s += a.counts[row] + a.counts[row + 1];
     }
+    return s;
+}
+
+// Blocks 0 .. nb0 - 1 scan the search grid's counts, the others the march grid's.
+__global__ __launch_bounds__(kThreads) void k_scan_blocks(GridBuildArgs a, uint32_t nb0)
+{
+    __shared__ uint32_t sh[kThreads / 64], occ;
+    const bool fine = blockIdx.x >= nb0;
+    const uint32_t ncells = fine ? a.fncells : a.ncells, blk = blockIdx.x - (fine ? nb0 : 0u);
+    uint32_t *out = fine ? a.fcell_start : a.cell_start;
+    const uint32_t base = blk * kScanBlock + threadIdx.x * kScanPer;
+    uint32_t v[kScanPer], sum = 0, cells = 0;
+    for (int j = 0; j < kScanPer; j++) {
+        v[j] = base + j >= ncells ? 0u : (fine ? a.counts[base + j] : dense_count(a, base + j));
+        sum += v[j];
+        cells += v[j] != 0;
+    }
+    if (threadIdx.x == 0) occ = 0;
     uint32_t total;
     uint32_t ex = block_excl_scan(sum, sh, total);
     for (int j = 0; j < kScanPer; j++) {
-        if (base + j < len) out[base + j] = ex;
+        if (base + j <= ncells) out[base + j] = ex;
         ex += v[j];
     }
-    if (threadIdx.x == 0) block_sums[blockIdx.x] = total;
-}
-
-__global__ __launch_bounds__(kThreads) void k_scan_sums(uint32_t *__restrict__ sums, uint32_t nb)
-{
-    __shared__ uint32_t sh[kThreads];
-    uint32_t carry = 0;
-    for (uint32_t base = 0; base < nb; base += kThreads) {
-        uint32_t i = base + threadIdx.x;
-        uint32_t v = i < nb ? sums[i] : 0u;
-        uint32_t total;
-        uint32_t ex = block_excl_scan(v, sh, total);
-        if (i < nb) sums[i] = ex + carry;
-        carry += total;
+    for (int off = 32; off > 0; off >>= 1) cells += __shfl_xor(cells, off, 64);
+    if ((threadIdx.x & 63) == 0) atomicAdd(&occ, cells);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        a.scan_tmp[2 * blockIdx.x] = total;
+        a.scan_tmp[2 * blockIdx.x + 1] = occ;
     }
 }
 
-__global__ __launch_bounds__(kThreads) void k_scan_add(uint32_t *__restrict__ out, uint32_t len,
-                                                       const uint32_t *__restrict__ sums)
+// One workgroup per grid: its blocks' sums in place, its occupied cells.
+__global__ __launch_bounds__(1024) void k_scan_sums(GridBuildArgs a, uint32_t nb0, uint32_t nb1)
 {
-    uint32_t base = blockIdx.x * kScanBlock + threadIdx.x * kScanPer;
-    uint32_t add = sums[blockIdx.x];
+    __shared__ uint32_t sh[16], occ;
+    const uint32_t first = blockIdx.x ? nb0 : 0u, nb = blockIdx.x ? nb1 : nb0;
+    uint32_t carry = 0, cells = 0;
+    if (threadIdx.x == 0) occ = 0;
+    for (uint32_t base = 0; base < nb; base += 1024) {
+        const uint32_t i = base + threadIdx.x;
+        uint2 *p = (uint2 *)a.scan_tmp + first + i;
+        const uint2 v = i < nb ? *p : make_uint2(0u, 0u);
+        cells += v.y;
+        uint32_t total;
+        const uint32_t ex = block_excl_scan(v.x, sh, total);
+        if (i < nb) p->x = ex + carry;
+        carry += total;
+    }
+    for (int off = 32; off > 0; off >>= 1) cells += __shfl_xor(cells, off, 64);
+    if ((threadIdx.x & 63) == 0) atomicAdd(&occ, cells);
+    __syncthreads();
+    if (threadIdx.x == 0) a.occupied[blockIdx.x] = occ;
+}
+
+__global__ __launch_bounds__(kThreads) void k_scan_add(GridBuildArgs a, uint32_t nb0)
+{
+    const bool fine = blockIdx.x >= nb0;
+    const uint32_t ncells = fine ? a.fncells : a.ncells, blk = blockIdx.x - (fine ? nb0 : 0u);
+    uint32_t *out = fine ? a.fcell_start : a.cell_start;
+    const uint32_t base = blk * kScanBlock + threadIdx.x * kScanPer;
+    const uint32_t add = a.scan_tmp[2 * blockIdx.x];
     for (int j = 0; j < kScanPer; j++)
-        if (base + j < len) out[base + j] += add;
+        if (base + j <= ncells) out[base + j] += add;
 }
 
-__global__ __launch_bounds__(kThreads) void k_scatter(GridBuildArgs a)
+// The particles' indices in the march grid's order, arbitrary inside a cell.
+__global__ __launch_bounds__(kThreads) void k_place(GridBuildArgs a)
 {
-    uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
+    const uint64_t i = xcd_run((a.n + kThreads - 1) / kThreads) * kThreads + threadIdx.x;
     if (i >= a.n) return;
-    uint32_t c = a.cell_of[i];
-    uint32_t slot = a.cell_start[c] + atomicAdd(&a.cursor[c], 1u);
-    a.scattered[slot] = make_float4(a.xyz[3 * i + 0], a.xyz[3 * i + 1], a.xyz[3 * i + 2], __uint_as_float((uint32_t)i));
+    int32_t k[3];
+    fine_cell(a, a.xyz[3 * i + 0], a.xyz[3 * i + 1], a.xyz[3 * i + 2], k);
+    a.index[a.fcell_start[fine_lin(a, k[0], k[1], k[2])] + a.slot[i]] = (uint32_t)i;
 }
 
-// Order inside each cell by input index: the particle at scattered slot s goes
-// to cell_start[c] + (number of particles of its cell with a smaller index).
-// One thread per particle, read-only over its own cell: no dependent swaps and
-// no atomics, so dense cells cost O(k) per particle in parallel rather than an
+// Order inside each cell by input index: a particle goes to its cell's start +
+// (number of particles of the cell with a smaller index), in both grids.  One
+// thread per particle, read-only over its own cells: no dependent swaps and no
+// atomics, so dense cells cost O(k) per particle in parallel rather than an
 // O(k^2) serial insertion sort.
 __global__ __launch_bounds__(kThreads) void k_cell_rank(GridBuildArgs a)
 {
-    uint64_t s = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
+    const uint64_t s = xcd_run((a.n + kThreads - 1) / kThreads) * kThreads + threadIdx.x;
     if (s >= a.n) return;
-    const float4 v = a.scattered[s];
-    const uint32_t key = __float_as_uint(v.w);
-    const uint32_t c = a.cell_of[key];
-    const uint32_t b = a.cell_start[c], e = a.cell_start[c + 1];
-    uint32_t rank = 0;
-    for (uint32_t j = b; j < e; j++) rank += __float_as_uint(a.scattered[j].w) < key ? 1u : 0u;
-    a.sorted[b + rank] = v;
+    const uint32_t key = a.index[s];
+    const float x = a.xyz[3 * (uint64_t)key], y = a.xyz[3 * (uint64_t)key + 1], z = a.xyz[3 * (uint64_t)key + 2];
+    int32_t k[3];
+    fine_cell(a, x, y, z, k);
+    // search-grid cell, and its first march-grid cell
+    const int32_t d[3] = { (k[0] + a.fo[0]) >> 1, (k[1] + a.fo[1]) >> 1, (k[2] + a.fo[2]) >> 1 };
+    const int32_t f[3] = { 2 * d[0] - a.fo[0], 2 * d[1] - a.fo[1], 2 * d[2] - a.fo[2] };
+    const uint32_t own = fine_lin(a, k[0], k[1], k[2]);
+    uint32_t rank = 0, frank = 0, own_b = 0;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const uint32_t row = fine_lin(a, f[0], f[1] + (r & 1), f[2] + (r >> 1));
+        const uint32_t b = a.fcell_start[row], m = a.fcell_start[row + 1], e = a.fcell_start[row + 2];
+        uint32_t lo = 0, hi = 0;
+        for (uint32_t j = b; j < m; j++) lo += a.index[j] < key ? 1u : 0u;
+        for (uint32_t j = m; j < e; j++) hi += a.index[j] < key ? 1u : 0u;
+        rank += lo + hi;
+        if (row == own) { frank = lo; own_b = b; }
+        if (row + 1 == own) { frank = hi; own_b = m; }
+    }
+    const uint32_t c = (uint32_t)(d[0] - a.dorg[0]) +
+                       (uint32_t)a.dn[0] * ((uint32_t)(d[1] - a.dorg[1]) + (uint32_t)a.dn[1] * (uint32_t)(d[2] - a.dorg[2]));
+    const float4 v = make_float4(x, y, z, __uint_as_float(key));
+    a.fsorted[own_b + frank] = v;
+    a.sorted[a.cell_start[c] + rank] = v;
 }
 
 hipError_t launch_grid_build(const GridBuildArgs &a, hipStream_t st)
 {
-    uint32_t len = a.ncells + 1;
-    uint32_t fill_blocks = (uint32_t)((len + kThreads - 1) / kThreads);
-    if (fill_blocks > 65535) fill_blocks = 65535;
-    hipLaunchKernelGGL(k_fill_u32, dim3(fill_blocks), dim3(kThreads), 0, st, a.counts, (uint64_t)len, 0u);
-    hipLaunchKernelGGL(k_fill_u32, dim3(fill_blocks), dim3(kThreads), 0, st, a.cursor, (uint64_t)a.ncells, 0u);
-    uint32_t pblocks = (uint32_t)((a.n + kThreads - 1) / kThreads);
+    const uint32_t fill = (a.fncells + kThreads - 1) / kThreads;
+    hipLaunchKernelGGL(k_fill_u32, dim3(fill < 65535 ? fill : 65535), dim3(kThreads), 0, st, a.counts,
+                       (uint64_t)a.fncells, 0u);
+    const uint32_t pblocks = 8 * (uint32_t)(((a.n + kThreads - 1) / kThreads + 7) / 8);
     hipLaunchKernelGGL(k_cell_count, dim3(pblocks), dim3(kThreads), 0, st, a);
-    uint32_t nb = (len + kScanBlock - 1) / kScanBlock;
-    hipLaunchKernelGGL(k_scan_blocks, dim3(nb), dim3(kThreads), 0, st, a.counts, a.cell_start, len, a.scan_tmp);
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(kThreads), 0, st, a.scan_tmp, nb);
-    hipLaunchKernelGGL(k_scan_add, dim3(nb), dim3(kThreads), 0, st, a.cell_start, len, a.scan_tmp);
-    hipLaunchKernelGGL(k_scatter, dim3(pblocks), dim3(kThreads), 0, st, a);
+    const uint32_t nb0 = scan_blocks(a.ncells + 1), nb1 = scan_blocks(a.fncells + 1);
+    hipLaunchKernelGGL(k_scan_blocks, dim3(nb0 + nb1), dim3(kThreads), 0, st, a, nb0);
+    hipLaunchKernelGGL(k_scan_sums, dim3(2), dim3(1024), 0, st, a, nb0, nb1);
+    hipLaunchKernelGGL(k_scan_add, dim3(nb0 + nb1), dim3(kThreads), 0, st, a, nb0);
+    hipLaunchKernelGGL(k_place, dim3(pblocks), dim3(kThreads), 0, st, a);
     hipLaunchKernelGGL(k_cell_rank, dim3(pblocks), dim3(kThreads), 0, st, a);
     return hipGetLastError();
 }
@@ -236,28 +333,6 @@ hipError_t launch_empty27(const uint32_t *cs, int32_t nx, int32_t ny, int32_t nz
 {
     uint32_t n = (uint32_t)nx * ny * nz;
     hipLaunchKernelGGL(k_empty27, dim3((n + kThreads - 1) / kThreads), dim3(kThreads), 0, st, cs, nx, ny, nz, out);
-    return hipGetLastError();
-}
-
-// Occupied cells of a grid: one atomic per workgroup.
-__global__ __launch_bounds__(kThreads) void k_occupied(const uint32_t *__restrict__ cs, uint32_t n, uint32_t *__restrict__ out)
-{
-    __shared__ uint32_t sum;
-    if (threadIdx.x == 0) sum = 0;
-    __syncthreads();
-    uint32_t cnt = 0;
-    for (uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kThreads)
-        cnt += cs[i + 1] != cs[i] ? 1u : 0u;
-    for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off, 64);
-    if ((threadIdx.x & 63) == 0) atomicAdd(&sum, cnt);
-    __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(out, sum);
-}
-
-hipError_t launch_occupied(const uint32_t *cs, uint32_t n, uint32_t *out, hipStream_t st)
-{
-    const uint32_t b = (n + 8 * kThreads - 1) / (8 * kThreads);
-    hipLaunchKernelGGL(k_occupied, dim3(b < 512 ? b : 512), dim3(kThreads), 0, st, cs, n, out);
     return hipGetLastError();
 }
 

@@ -105,21 +105,23 @@ hipError_t launch_bounds_reduce(const float *xyz, uint64_t n, float *partial, ui
                                 float *out, hipStream_t st);
 uint32_t bounds_partials(uint64_t n);
 
+// The search grid (cells of h) and the march grid (cells of h/2) of a frame.
 struct GridBuildArgs {
     const float *xyz;      // device AoS float3
     uint64_t n;
-    float inv_h;
-    int32_t ox, oy, oz, nx, ny, nz;
-    uint32_t ncells;
-    uint32_t *cell_of;     // n
-    uint32_t *counts;      // ncells + 1 (scan in place into cell_start)
-    uint32_t *cursor;      // ncells
-    uint32_t *scan_tmp;    // scan_tmp_size(ncells + 1)
-    float4 *sorted;        // n
-    uint32_t *cell_start;  // ncells + 1
-    float4 *scattered;     // n: cell-major, arbitrary order inside a cell
+    float inv_hf;          // 2 / h
+    int32_t fo[3], fn[3];  // march grid: origin, cells per axis
+    int32_t dorg[3], dn[3];   // search grid
+    uint32_t ncells, fncells;
+    uint32_t *counts;      // fncells, zeroed by the build
+    uint32_t *slot;        // n: place inside the march-grid cell, arbitrary order
+    uint32_t *index;       // n: input indices, march cell by march cell
+    float4 *sorted, *fsorted;             // n
+    uint32_t *cell_start, *fcell_start;   // ncells + 1, fncells + 1
+    uint32_t *scan_tmp;    // scan_tmp_size of both grids
+    uint32_t *occupied;    // [2]: search and march cells that hold a particle
 };
-size_t scan_tmp_size(uint32_t len);
+size_t scan_tmp_size(uint32_t ncells, uint32_t fncells);
 hipError_t launch_grid_build(const GridBuildArgs &a, hipStream_t st);
 
 // The tile pre-pass (L.tile_buf set): the list of the active tiles and the misses
@@ -157,8 +159,6 @@ hipError_t launch_depth_sprites(const SpriteLaunch &S, const float4 *pts, uint32
 hipError_t launch_depth_smooth(const float *in, float *out, uint32_t W, uint32_t H, int N, const float *K,
                                hipStream_t st);
 hipError_t launch_empty27(const uint32_t *cs, int32_t nx, int32_t ny, int32_t nz, uint8_t *out, hipStream_t st);
-// Adds the number of non-empty cells among cs's n to *out.
-hipError_t launch_occupied(const uint32_t *cs, uint32_t n, uint32_t *out, hipStream_t st);
 // The distance field of empty27 (GridDev::clear); tmp: one byte per cell.
 hipError_t launch_clear(const uint8_t *empty27, int32_t nx, int32_t ny, int32_t nz, uint8_t *tmp, uint8_t *out,
                         hipStream_t st);

@@ -51,6 +51,26 @@ def test_grid_negative_coordinates(marcher):
     _grid_equal(marcher, 2, xyz, 0.1)
 
 
+@pytest.mark.parametrize("n", [1, 255, 257, 20000])
+def test_grid_cell_borders(marcher, n):
+    """Coordinates on and one ulp beside the borders of the cells of h/2, of both
+    signs, duplicates among them: the search grid built from the march grid's
+    cells is the one of its own keys."""
+    rng = np.random.default_rng(n)
+    h = np.float32(0.1)
+    xyz = (rng.integers(-9, 10, (n, 3)) * (h / 2)).astype(np.float32)
+    up, down = rng.random((n, 3)) < 0.2, rng.random((n, 3)) < 0.2
+    xyz[up] = np.nextafter(xyz[up], np.float32(9))
+    xyz[down] = np.nextafter(xyz[down], np.float32(-9))
+    marcher.set_frame(3, xyz, float(h))
+    _grid_equal(marcher, 3, xyz, float(h))
+
+
+def test_grid_refuses_keys_beyond_int32(marcher):
+    with pytest.raises(Exception, match="2\\^30 h"):
+        marcher.set_frame(3, np.full((4, 3), 2.0e9, np.float32), 1.0)
+
+
 def test_neighbor_counts(marcher):
     sc = scenes.lattice_cube(1)
     marcher.set_frame(0, sc.xyz, sc.h)
