@@ -139,24 +139,20 @@ __device__ __forceinline__ int32_t pm_key(float x, float inv_h)
     return x >= 0.0f ? (int32_t)v : (int32_t)v - 1;
 }
 
-// sqrtf(x) for the kernel weight, x >= 0: the hardware square root (within one
-// ulp) corrected to the correctly rounded result by the signs of the residuals
-// x - s' s of its neighbours s' = s -+ 1 ulp -- the expansion the compiler emits
-// for sqrtf at x >= 2^-96, without its scaling of smaller inputs and its
-// special-value fix-up.  Below 2^-96 the residuals may round: the result is
-// then still within an ulp of the hardware's (at 0 the lower neighbour is a NaN
-// and every test fails), there q = sqrt(x) / h < 2^-14 for any h > 2^-34, and
-// W(q) = sigma (6 (q^3 - q^2) + 1) rounds to sigma exactly whatever the last
-// bit of the root.
+// sqrtf(x) for the kernel weight, x >= 0: x rsq(x), one ulp or two off, and one
+// Newton step whose residual is exact.  Equal to sqrtf for every float from 2^-96
+// to 2^64 (all of them compared on gfx950), six instructions instead of nine
+// (the hardware root and the residuals of both neighbours).  The march's kernels
+// issue VALU instructions 75 to 97 % of the time, half of them for weights.
+// Below 2^-96 the residual may round, and below 2^-126 and at 0 the factor is
+// capped (the result lies in [0, 2^-62]): there q = sqrt(x) / h < 2^-14 for any
+// h > 2^-34, and W(q) = sigma (6 (q^3 - q^2) + 1) rounds to sigma exactly whatever
+// the last bits of the root.
 __device__ __forceinline__ float pm_sqrt_w(float x)
 {
-    const float s = __builtin_amdgcn_sqrtf(x);
-    const float sm = __uint_as_float(__float_as_uint(s) - 1u);
-    const float sp = __uint_as_float(__float_as_uint(s) + 1u);
-    const float rm = __builtin_fmaf(-sm, s, x);
-    const float rp = __builtin_fmaf(-sp, s, x);
-    const float t = rm <= 0.0f ? sm : s;
-    return rp > 0.0f ? sp : t;
+    const float y = fminf(__builtin_amdgcn_rsqf(x), 0x1p63f);
+    const float s = x * y;
+    return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * y, s);
 }
 
 // Kernel.cpp:16-32 on a squared distance known to be < h^2.
@@ -180,14 +176,12 @@ __device__ __forceinline__ double pm_W_in_d(double r2, double hinv, double sig)
     return sig * (6.0 * (q * q * q - q * q) + 1.0);
 }
 
-// Neumaier-compensated accumulation (exact same branches as the oracle).
+// Neumaier-compensated accumulation of weights (the oracle's branches on |s| and
+// |w|: neither is negative, so the larger and the smaller do).
 __device__ __forceinline__ void pm_neu_add(float &s, float &c, float w)
 {
-    float t = s + w;
-    bool big = fabsf(s) >= fabsf(w);
-    float a = big ? s : w;
-    float b = big ? w : s;
-    c += (a - t) + b;
+    const float t = s + w;
+    c += (fmaxf(s, w) - t) + fminf(s, w);
     s = t;
 }
 
@@ -416,6 +410,7 @@ __device__ __forceinline__ void pm_list_density(const GridDev &g, const uint32_t
         for (int u = 0; u < 4; u++) {
             const float rx = vx[u] - qx, ry = vy[u] - qy, rz = vz[u] - qz;
             r2[u] = (rx * rx + ry * ry) + rz * rz;
+            asm volatile("" : "+v"(r2[u]));   // here, so that the next loads take v's registers (else 12 copies per round)
         }
         const int i0 = i;
         i += 4;
@@ -567,11 +562,10 @@ __device__ __forceinline__ void pm_acc6(const GridDev &g, float px, float py, fl
     r2[5] = sxy + rzm * rzm;
 #pragma unroll
     for (int k = 0; k < 6; k++) {
-        if (r2[k] < g.h2) {
-            const float w = pm_W_in(r2[k], g.inv_h, g.sig);
-            if (comp) pm_neu_add(a.s[k], a.c[k], w);
-            else a.s[k] += w;
-        }
+        // outside the support: an exact zero
+        const float w = r2[k] < g.h2 ? pm_W_sel(r2[k], g.inv_h, g.sig) : 0.0f;
+        if (comp) pm_neu_add(a.s[k], a.c[k], w);
+        else a.s[k] += w;
     }
 }
 
