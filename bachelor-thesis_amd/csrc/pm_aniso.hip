@@ -419,8 +419,9 @@ __device__ __forceinline__ void an_plane(const GridDev &g, const AnPlanes &A, in
         const float ty = pm_fine_off(i - 2, A.w.f[1]);
         const float r2 = ty * ty + tz * tz;
         const int32_t y = A.w.c[1] + i - 2;
-        int32_t xl = A.w.c[0] + ((A.xm2 + r2 < kLimExt) ? -2 : ((A.xm1 + r2 < kLimExt) ? -1 : 0));
-        int32_t xh = A.w.c[0] + ((A.xp2 + r2 < kLimExt) ? 2 : ((A.xp1 + r2 < kLimExt) ? 1 : 0));
+        // adds with carry: a farther cell is kept only with the nearer one
+        int32_t xl = A.w.c[0] - (A.xm1 + r2 < kLimExt ? 1 : 0) - (A.xm2 + r2 < kLimExt ? 1 : 0);
+        int32_t xh = A.w.c[0] + (A.xp1 + r2 < kLimExt ? 1 : 0) + (A.xp2 + r2 < kLimExt ? 1 : 0);
         xl = xl < 0 ? 0 : xl;
         xh = xh > g.nx - 1 ? g.nx - 1 : xh;
         const bool kept = inz && r2 < kLimExt && y >= 0 && y < g.ny && xl <= xh;

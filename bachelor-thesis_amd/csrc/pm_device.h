@@ -286,14 +286,14 @@ __device__ __forceinline__ void pm_fine_plane(const GridDev &g, const FineWalk &
     for (int i = 0; i < 5; i++) {
         const float ty = pm_fine_off(i - 2, w.fy);
         const float r2 = ty * ty + tz2;
-        const bool kept = r2 < PM_FINE_LIM;
-        int lo = (w.xm2 + r2 < PM_FINE_LIM) ? -2 : ((w.xm1 + r2 < PM_FINE_LIM) ? -1 : 0);
-        int hi = (w.xp2 + r2 < PM_FINE_LIM) ? 3 : ((w.xp1 + r2 < PM_FINE_LIM) ? 2 : 1);
-        lo = kept ? lo : 0;
-        hi = kept ? hi : 0;
+        // One compare and one add with carry each: a farther cell is kept only
+        // with the nearer one, and none where r2 alone reaches the limit.
         const uint32_t row = row0 + (uint32_t)((i - 2) * (int)w.sy);
-        P.b[i] = g.fcell_start[row + (uint32_t)lo];
-        P.e[i] = g.fcell_start[row + (uint32_t)hi];
+        const uint32_t lo = row - (w.xm1 + r2 < PM_FINE_LIM ? 1u : 0u) - (w.xm2 + r2 < PM_FINE_LIM ? 1u : 0u);
+        const uint32_t hi = row + (r2 < PM_FINE_LIM ? 1u : 0u) + (w.xp1 + r2 < PM_FINE_LIM ? 1u : 0u) +
+                            (w.xp2 + r2 < PM_FINE_LIM ? 1u : 0u);
+        P.b[i] = g.fcell_start[lo];
+        P.e[i] = g.fcell_start[hi];
     }
 }
 
