@@ -18,6 +18,7 @@
 #include <string>
 #include <vector>
 
+#include "pm_copy.h"
 #include "pm_internal.h"
 #include "pmarch.h"
 
@@ -99,6 +100,7 @@ struct pm_ctx {
     // pinned staging for asynchronous hand-off
     void *h_stage = nullptr;
     size_t h_stage_cap = 0;
+    CopyPool copies;                   // shares large copies out of it
     unsigned long long *h_counters = nullptr;
     float *user_pos = nullptr, *user_nrm = nullptr, *user_t = nullptr;
     bool pending = false;
@@ -181,6 +183,19 @@ static hipError_t zero_sync(pm_ctx *c, void *dst, size_t bytes)
     hipError_t e = hipMemsetAsync(dst, 0, bytes, c->stream);
     if (e != hipSuccess) return e;
     return hipStreamSynchronize(c->stream);
+}
+
+// Room for `need` bytes of pinned staging (no march may be in flight).
+static hipError_t ensure_stage(pm_ctx *c, size_t need)
+{
+    if (need <= c->h_stage_cap) return hipSuccess;
+    if (c->h_stage) hipHostFree(c->h_stage);
+    c->h_stage = nullptr;
+    c->h_stage_cap = 0;
+    const hipError_t e = hipHostMalloc(&c->h_stage, need, hipHostMallocDefault);
+    if (e == hipSuccess) c->h_stage_cap = need;
+    else (void)hipGetLastError();      // reported here, not by the next launch
+    return e;
 }
 
 // Every point of a BGEO file, read as the data arrives (pm_bgeo.cpp).
@@ -740,13 +755,7 @@ static int march_launch(pm_ctx *c, int32_t frame, const pm_settings *s, const fl
     c->user_t = t_out;
     if (positions_out || normals_out || t_out) {
         size_t need = (positions_out ? 16 * npx : 0) + (normals_out ? 16 * npx : 0) + (t_out ? 4 * npx : 0);
-        if (need > c->h_stage_cap) {
-            if (c->h_stage) hipHostFree(c->h_stage);
-            c->h_stage = nullptr;
-            c->h_stage_cap = 0;
-            HIPCHK(c, hipHostMalloc(&c->h_stage, need, hipHostMallocDefault));
-            c->h_stage_cap = need;
-        }
+        HIPCHK(c, ensure_stage(c, need));
         char *p = (char *)c->h_stage;
         if (positions_out) { HIPCHK(c, hipMemcpyAsync(p, c->d_pos.p, 16 * npx, hipMemcpyDeviceToHost, c->stream)); p += 16 * npx; }
         if (normals_out) { HIPCHK(c, hipMemcpyAsync(p, c->d_nrm.p, 16 * npx, hipMemcpyDeviceToHost, c->stream)); p += 16 * npx; }
@@ -804,9 +813,15 @@ static int complete(pm_ctx *c)
 {
     uint64_t npx = c->npx;
     const char *p = (const char *)c->h_stage;
-    if (c->user_pos) { memcpy(c->user_pos, p, 16 * npx); p += 16 * npx; }
-    if (c->user_nrm) { memcpy(c->user_nrm, p, 16 * npx); p += 16 * npx; }
-    if (c->user_t) { memcpy(c->user_t, p, 4 * npx); }
+    float *const user[3] = { c->user_pos, c->user_nrm, c->user_t };
+    CopyPool::Range r[3];
+    int nr = 0;
+    for (int k = 0; k < 3; k++) {
+        if (!user[k]) continue;
+        r[nr] = { user[k], p, (k < 2 ? 16 : 4) * npx };
+        p += r[nr++].bytes;
+    }
+    c->copies.copy(r, nr);
     c->user_pos = c->user_nrm = c->user_t = nullptr;
     pm_stats &S = c->stats;
     memset(&S, 0, sizeof(S));
@@ -1121,9 +1136,28 @@ int pm_batch_download(pm_ctx *c, uint32_t view, float *positions, float *normals
     const float4 *pos = (const float4 *)c->b_img.p;
     const float4 *nrm = pos + c->b_npx;
     const float *tt = (const float *)(nrm + c->b_npx);
-    if (positions) HIPCHK(c, copy_sync(c, positions, pos + o, 16 * n, hipMemcpyDeviceToHost));
-    if (normals) HIPCHK(c, copy_sync(c, normals, nrm + o, 16 * n, hipMemcpyDeviceToHost));
-    if (t) HIPCHK(c, copy_sync(c, t, tt + o, 4 * n, hipMemcpyDeviceToHost));
+    float *const dst[3] = { positions, normals, t };
+    const void *const src[3] = { pos + o, nrm + o, tt + o };
+    const size_t bytes[3] = { 16 * n, 16 * n, 4 * n };
+    size_t need = 0;
+    for (int k = 0; k < 3; k++) need += dst[k] ? bytes[k] : 0;
+    // one wait and a shared copy; small views and those beyond 64 MB of staging copy image by image
+    if (need >= kCopyShared && need <= (64u << 20) && ensure_stage(c, need) == hipSuccess) {
+        CopyPool::Range r[3];
+        int nr = 0;
+        char *p = (char *)c->h_stage;
+        for (int k = 0; k < 3; k++) {
+            if (!dst[k]) continue;
+            HIPCHK(c, hipMemcpyAsync(p, src[k], bytes[k], hipMemcpyDeviceToHost, c->stream));
+            r[nr++] = { dst[k], p, bytes[k] };
+            p += bytes[k];
+        }
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        c->copies.copy(r, nr);
+        return PM_OK;
+    }
+    for (int k = 0; k < 3; k++)
+        if (dst[k]) HIPCHK(c, copy_sync(c, dst[k], src[k], bytes[k], hipMemcpyDeviceToHost));
     return PM_OK;
 }
 
