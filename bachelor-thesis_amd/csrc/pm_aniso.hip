@@ -845,8 +845,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     if (any) flush_counters(L.counters, cn.rays, cn.in_aabb, cn.hits, cn.samples, cn.cand, cn.march);
 }
 
-// The hits of the same tiles: bisection (the last step in FP64), normal,
-// outputs; 2^tile_split lanes per hit where the tiles do not fill the chip.
+// The hits of the same tiles: bisection (the last step in FP64), point, and the
+// normal where it is a sum of gradients (central differences: k_an_normals);
+// 2^finish_split lanes per hit where the tiles do not fill the chip.
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_an_finish_tiles(MarchLaunch L)
 {
     __shared__ float region[kAnWords];
@@ -903,22 +904,75 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
             xs[2] = (float)((double)o[2] + tt * (double)d[2]);
             th = (float)tt;
         }
-        // the group's lanes take the leader's point
-#pragma unroll
-        for (int a = 0; a < 3; a++) xs[a] = __shfl(xs[a], (int)(lane & ~(uint32_t)(G - 1)), 64);
-        float nx = 0.f, ny = 0.f, nz = 0.f;
-        if (s.normal_mode == PM_NORMAL_GRADW) {
-            if (hit && lead) an_normal_gradw(L, xs, lst, nx, ny, nz);
-        } else {
-            float gv[3];
-            group_cdiff(xs, s.normal_eps, hit, G, dens, gv, cn);
-            cdiff_normal(gv, nx, ny, nz);
-        }
         if (hit && lead) {
             L.pos[idx] = make_float4(xs[0], xs[1], xs[2], 1.0f);
-            L.nrm[idx] = make_float4(nx, ny, nz, 1.0f);
             if (L.t) L.t[idx] = th;
+            if (s.normal_mode == PM_NORMAL_GRADW) {
+                float nx, ny, nz;
+                an_normal_gradw(L, xs, lst, nx, ny, nz);
+                L.nrm[idx] = make_float4(nx, ny, nz, 1.0f);
+            }
             cn.hits++;
+        }
+    }
+    if (any) flush_counters(L.counters, cn.rays, cn.in_aabb, cn.hits, cn.samples, cn.cand, cn.march);
+}
+
+// Central-difference normals of the hits whose points k_an_finish_tiles wrote:
+// six lanes per hit, ten hits per wave, seven waves per active tile (the hits in
+// the order of the tile's pixels; a wave without any ends at once).  The six
+// samples of a hit lie eps apart, so its lanes list nearly the same candidates,
+// and a launch has seven times the waves of the tiles, whose longest ones bound
+// the launch otherwise (3,700 tiles with hits on 4,096 wave slots at 1080p).
+// With the samples one after another in the finish 3,010 us, apart 1,762 + 958.
+static constexpr uint32_t kNormHits = 10, kNormParts = 7;
+
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_an_normals(MarchLaunch L)
+{
+    __shared__ uint32_t region[kAnWords];
+    __shared__ uint32_t pixel[64];
+    const uint32_t lane = threadIdx.x;
+    uint32_t *lst = region + lane;
+    const pm_settings &s = L.s;
+    const uint32_t tiles_x = (L.W + 7) / 8, T = tiles_x * ((L.H + 7) / 8);
+    const uint32_t *order = L.tile_buf;
+    const uint32_t TA = order[T];
+    const AnDens dens{ &L, lst, s.compensated != 0 };
+    const uint32_t j = lane / 6, k = lane % 6;                 // hit of the part; +x, -x, +y, -y, +z, -z
+    Counts cn;
+    bool any = false;
+    for (uint32_t w = blockIdx.x; w < tile_waves_of(TA * kNormParts); w += gridDim.x) {
+        const uint32_t i = xcd_tile(w);
+        if (i >= TA * kNormParts) continue;
+        const uint32_t tile = order[i / kNormParts], first = i % kNormParts * kNormHits;
+        const uint32_t px = (tile % tiles_x) * 8 + (lane & 7u), py = (tile / tiles_x) * 8 + (lane >> 3);
+        const bool inside = px < L.W && py < L.H;
+        const uint32_t mine = inside ? py * L.W + px : 0u;
+        const bool hit = inside && (L.hit_rec[mine].x & 1u);
+        const unsigned long long hits = __ballot(hit);
+        const uint32_t n = (uint32_t)__popcll(hits);
+        if (first >= n) continue;
+        any = true;
+        wave_lds_sync();                                       // the last round's reads are done
+        if (hit) pixel[__popcll(hits & ((1ull << lane) - 1ull))] = mine;
+        wave_lds_sync();
+        const bool want = j < kNormHits && first + j < n;
+        const uint32_t idx = want ? pixel[first + j] : 0u;
+        float rho = 0.0f;
+        if (want) {
+            const float4 p = L.pos[idx];
+            const float e = k & 1u ? -s.normal_eps : s.normal_eps;
+            uint32_t cand = 0;
+            rho = dens(k < 2 ? p.x + e : p.x, (k >> 1) == 1 ? p.y + e : p.y, k >= 4 ? p.z + e : p.z, cand);
+            cn.samples++;
+            cn.cand += cand;
+        }
+        const float d = rho - __shfl_down(rho, 1, 64);         // lanes k = 0, 2, 4: along x, y, z
+        const float gv[3] = { d, __shfl_down(d, 2, 64), __shfl_down(d, 4, 64) };
+        if (want && k == 0) {
+            float nx, ny, nz;
+            cdiff_normal(gv, nx, ny, nz);
+            L.nrm[idx] = make_float4(nx, ny, nz, 1.0f);
         }
     }
     if (any) flush_counters(L.counters, cn.rays, cn.in_aabb, cn.hits, cn.samples, cn.cand, cn.march);
@@ -1223,6 +1277,10 @@ hipError_t launch_march_aniso(const MarchLaunch &L, hipStream_t st)
         e = hipGetLastError();
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(k_an_finish_tiles, grid, blk, 0, st, L);
+        e = hipGetLastError();
+        if (e != hipSuccess || L.s.normal_mode == PM_NORMAL_GRADW) return e;
+        const uint32_t parts = tile_waves_of(tiles * kNormParts);
+        hipLaunchKernelGGL(k_an_normals, dim3(parts < kMaxWaves ? parts : kMaxWaves), blk, 0, st, L);
         return hipGetLastError();
     }
     if (L.s.mode == PM_MODE_REFERENCE || L.s.schedule != 1 || !L.hit_rec) {

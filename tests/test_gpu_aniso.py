@@ -115,6 +115,21 @@ def test_march_aniso_schedules_agree(marcher):
         assert out[0][3][k] == out[1][3][k], k
 
 
+@pytest.mark.parametrize("W,H", [(1, 1), (9, 7), (65, 33), (130, 71), (1, 50)])
+@pytest.mark.parametrize("eps", [None, -1.0])
+def test_march_aniso_normals_ragged(marcher, W, H, eps):
+    """Tiles cut by the image's border, with any number of hits against the ten of
+    a wave of the normals; offsets of both signs."""
+    sc = scenes.lattice_cube(2, width=W, height=H)
+    cam = sc.cameras[0]
+    print(f"aniso normals {W}x{H} eps={eps}", flush=True)
+    marcher.set_frame(0, sc.xyz, sc.h)
+    st = scenes.aniso_settings(sc, skip_mode=1)
+    if eps is not None:
+        st["normal_eps"] = eps * st["normal_eps"]
+    _march_pair(marcher, 0, sc, st, cam, 1)
+
+
 def test_march_aniso_dam_bitexact(marcher):
     """The dam-break column scaled to h = 0.1, 480x270, whole image."""
     sc = scenes.dam_break_aniso(0, width=480, height=270)
