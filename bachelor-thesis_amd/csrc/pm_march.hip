@@ -11,7 +11,7 @@
 // march ends where its rays' work would diverge.  (One kernel that bisected a
 // ray's hit while other lanes of the wave still marched took 23 density
 // evaluations per wave at the median, 1.11 ms at 1080p on the 1 M dam break;
-// split, 0.33 + 0.46 ms.)  Schedule 1 (k_march_simple) marches one ray per lane
+// split, 0.33 + 0.46 ms, now 0.28 + 0.25.)  Schedule 1 (k_march_simple) marches one ray per lane
 // to its end with a direct walk for every sample: the plain form the product
 // is checked against.
 #include "pm_features.h"
@@ -777,6 +777,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
 // the 1 M dam break, 1.4 per cell); in denser frames (4 M pool, 8 per cell) most
 // lists overflow after they were built and their LDS costs waves (3.6 ms walking
 // for each sample, 5.3 to 7.0 ms with lists of 44 to 92 slots), so those walk.
+// (Since then the weights take fewer instructions and the statistics count every
+// sample's own stencil: 254 us and 3.1 ms.)
 // Registers are capped for four waves per SIMD.
 template <bool BATCH, bool INSTR, bool LIST>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LIST ? 3 : 4, 8))) void k_finish(MarchLaunch L0, const MarchLaunch *__restrict__ jobs,
