@@ -706,10 +706,7 @@ __device__ __forceinline__ bool pm_list_segment(const GridDev &g, const float a[
     uint32_t pb[6], pe[6], qb[6], qe[6];
     auto plane = [&](int jz, uint32_t (&b_)[6], uint32_t (&e_)[6]) {
 #pragma unroll
-        for (int k = 0; k < 6; k++) {
-            pm_box_row(g, w, k, jz, b_[k], e_[k]);
-            if (k >= w.ny) e_[k] = b_[k];
-        }
+        for (int k = 0; k < 6; k++) pm_box_row(g, w, k, k < w.ny ? jz : w.nz, b_[k], e_[k]);   // row ny may lie past the grid
     };
     plane(0, pb, pe);
     _Pragma("unroll 1") for (int jz = 0; __ballot(jz < w.nz) != 0; jz++) {

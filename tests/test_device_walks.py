@@ -1,0 +1,142 @@
+"""The march-grid walks of csrc/pm_device.h compiled for the CPU, one lane as a
+wave of its own and every buffer checked (AddressSanitizer), so reads beyond the
+cell table show without a GPU."""
+import pathlib
+import subprocess
+
+import pytest
+
+ROOT = pathlib.Path(__file__).resolve().parents[1]
+
+# What pm_device.h needs of the HIP headers, for a wave of one lane.
+STUB = r"""
+#pragma once
+#include <cmath>
+#include <cstdint>
+#include <cstdlib>
+#define __device__
+#define __forceinline__ inline
+#define __ballot(p) ((p) ? 1ull : 0ull)
+#define __builtin_amdgcn_rsqf(x) (1.0f / std::sqrt(x))
+using std::fabs; using std::sqrt;
+struct float4 { float x, y, z, w; };
+"""
+
+# A frame's march grid as the build lays it out (cells of h/2, four cells of
+# margin, cell-major, by input index inside a cell).
+COMMON = r"""
+#include "pm_device.h"
+#include <cstdio>
+#include <cstring>
+#include <random>
+#include <vector>
+
+struct Frame {
+    std::vector<float4> sorted;
+    std::vector<uint32_t> start;
+    GridDev g{};
+    float pmin[3], pmax[3];
+    Frame(const std::vector<float4> &p, float h)
+    {
+        g.h = h; g.inv_h = 1.0f / h; g.h2 = h * h; g.inv_hf = 2.0f * g.inv_h;
+        g.sig = 8.0f / (PM_PI_F * h * h * h);
+        g.h_d = h; g.h2_d = g.h_d * g.h_d; g.hinv_d = 1.0 / g.h_d; g.sig_d = 8.0 / (PM_PI_D * g.h_d * g.h_d * g.h_d);
+        for (int a = 0; a < 3; a++) { pmin[a] = 3e38f; pmax[a] = -3e38f; }
+        for (const float4 &v : p) {
+            const float x[3] = { v.x, v.y, v.z };
+            for (int a = 0; a < 3; a++) { pmin[a] = fminf(pmin[a], x[a]); pmax[a] = fmaxf(pmax[a], x[a]); }
+        }
+        int32_t fo[3], fn[3];
+        for (int a = 0; a < 3; a++) {
+            fo[a] = pm_key(pmin[a], g.inv_hf) - 4;
+            fn[a] = pm_key(pmax[a], g.inv_hf) + 5 - fo[a];
+        }
+        g.fox = fo[0]; g.foy = fo[1]; g.foz = fo[2];
+        g.fnx = fn[0]; g.fny = fn[1]; g.fnz = fn[2];
+        const size_t nc = (size_t)fn[0] * fn[1] * fn[2];
+        std::vector<std::vector<float4>> cell(nc);
+        for (const float4 &v : p)
+            cell[(size_t)(pm_key(v.x, g.inv_hf) - fo[0]) +
+                 fn[0] * ((size_t)(pm_key(v.y, g.inv_hf) - fo[1]) + fn[1] * (size_t)(pm_key(v.z, g.inv_hf) - fo[2]))]
+                .push_back(v);
+        start.resize(nc + 1);
+        for (size_t c = 0; c < nc; c++) {
+            start[c] = (uint32_t)sorted.size();
+            sorted.insert(sorted.end(), cell[c].begin(), cell[c].end());
+        }
+        start[nc] = (uint32_t)sorted.size();
+        start.shrink_to_fit();
+        sorted.shrink_to_fit();
+        g.fcell_start = start.data();
+        g.fsorted = sorted.data();
+    }
+};
+
+static constexpr int kCap = 56;
+static uint32_t lst[(kCap + kListPad) * 64];
+
+// A jittered lattice of n[0] x n[1] x n[2] particles from `lo`.
+static std::vector<float4> lattice(const int n[3], float spacing, const float lo[3], unsigned seed)
+{
+    std::mt19937 rng(seed);
+    std::uniform_real_distribution<float> u(-0.1f * spacing, 0.1f * spacing);
+    std::vector<float4> p;
+    for (int z = 0; z < n[2]; z++)
+        for (int y = 0; y < n[1]; y++)
+            for (int x = 0; x < n[0]; x++)
+                p.push_back({ lo[0] + x * spacing + u(rng), lo[1] + y * spacing + u(rng), lo[2] + z * spacing + u(rng), 0.0f });
+    return p;
+}
+"""
+
+
+def run(tmp_path, main):
+    # -O0: every load of the source is made, also one whose value is dropped
+    (tmp_path / "hip").mkdir()
+    (tmp_path / "hip" / "hip_runtime.h").write_text(STUB)
+    src, exe = tmp_path / "walk.cpp", tmp_path / "walk"
+    src.write_text(COMMON + main)
+    subprocess.run(["g++", "-std=c++17", "-O0", "-g", "-ffp-contract=off", "-w", "-fsanitize=address",
+                    "-I" + str(tmp_path), "-I" + str(ROOT / "bachelor-thesis_amd" / "csrc"), str(src), "-o", str(exe)],
+                   check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=300)
+    assert out.returncode == 0, (out.stdout + out.stderr)[-3000:]
+    return out.stdout
+
+
+SEGMENT_EDGE = r"""
+int main()
+{
+    const int n[3] = { 9, 7, 8 };
+    const float lo[3] = { -0.13f, 0.21f, 0.4f }, h = 0.1f, eps = h / 32, step = h / 8;
+    Frame f(lattice(n, 0.05f, lo, 1), h);
+    std::mt19937 rng(2);
+    std::uniform_real_distribution<float> u(-1.0f, 1.0f);
+    long listed = 0, last = 0;
+    for (int corner = 0; corner < 8; corner++)
+        for (int i = 0; i < 20000; i++) {
+            float a[3], b[3], len = 0.0f, d[3];
+            for (int k = 0; k < 3; k++) { d[k] = u(rng); len += d[k] * d[k]; }
+            for (int k = 0; k < 3; k++) {
+                a[k] = ((corner >> k) & 1 ? f.pmax[k] : f.pmin[k]) + 1.1f * h * u(rng);
+                b[k] = a[k] + step * d[k] / sqrtf(len);
+            }
+            int m = 0;
+            if (!pm_list_segment<kCap>(f.g, a, b, eps, lst, m)) continue;
+            listed++;
+            BoxWalk w;
+            const float l[3] = { fminf(a[0], b[0]) - eps, fminf(a[1], b[1]) - eps, fminf(a[2], b[2]) - eps };
+            const float r[3] = { fmaxf(a[0], b[0]) + eps, fmaxf(a[1], b[1]) + eps, fmaxf(a[2], b[2]) + eps };
+            pm_box_begin(f.g, l, r, w);
+            last += (int)w.kh[1] + 2 - f.g.foy == f.g.fny - 1 && (int)w.kh[2] + 2 - f.g.foz == f.g.fnz - 1;
+        }
+    std::printf("%ld %ld\n", listed, last);
+}
+"""
+
+
+def test_segment_list_at_the_grid_edge(tmp_path):
+    """Segments around every corner of the particles' box, up to the last cells
+    a 5-cell stencil fits in: no row bound is read beyond the cell table."""
+    listed, last = map(int, run(tmp_path, SEGMENT_EDGE).split())
+    assert listed > 10000 and last > 100

@@ -160,3 +160,27 @@ def test_batch_tile_list(marcher, use_graph, away):
                 assert np.array_equal(got, want.reshape(got.shape)), v
         for k in ("rays", "hits", "samples", "march_samples"):
             assert marcher.stats()[k] == sum(o[3][k] for o in ref), k
+
+
+@pytest.mark.parametrize("size", [(61, 43), (333, 207)])
+@pytest.mark.parametrize("iso", [0.0, 1e-6, 0.004])
+def test_finish_list_low_iso(marcher, size, iso):
+    """Hits beside and on the edges of the padded particle box, whose segments'
+    cells reach the grid's last rows: iso 0 (every ray that enters hits on the
+    box) and a small part of the rest density, with few and many tiles, and as a
+    batch."""
+    sc = scenes.lattice_cube(3, n_side=9, spacing=0.05, width=size[0], height=size[1])
+    sc.iso *= iso
+    c = sc.cameras[0]
+    print(f"finish list low iso {iso} {size}", flush=True)
+    marcher.set_frame(60, sc.xyz, sc.h)
+    for normal_mode in (0, 1) if iso else (0,):       # (a box hit has no particle to take gradients from)
+        got = _check(marcher, sc, skip_mode=0, normal_mode=normal_mode)
+        assert got["hits"] > 100
+    st = sc.settings(skip_mode=0)
+    pos, nrm, t, _ = marcher.march(60, st, c.inv_pv, c.eye, c.width, c.height)
+    marcher.batch_set(st, [(60, c.width, c.height, c.inv_pv, c.eye)])
+    marcher.batch_run()
+    marcher.wait()
+    for got, want in zip(marcher.batch_download(0), (pos, nrm, t)):
+        assert np.array_equal(got, want)
