@@ -482,8 +482,9 @@ struct BoxWalk {
     float xm2, xm1, xp1, xp2; // squared x-distances of the four trimmable end cells
 };
 
-// false when the cells leave the march grid (the caller then takes the six
-// samples one at a time).
+// false when the cells leave the march grid, or the box has no keys (an end that
+// is not a number, or beyond any grid): the caller then takes the samples one
+// at a time.
 __device__ __forceinline__ bool pm_box_begin(const GridDev &g, const float lo[3], const float hi[3], BoxWalk &w)
 {
     const int32_t fo[3] = { g.fox, g.foy, g.foz }, fn[3] = { g.fnx, g.fny, g.fnz };
@@ -498,7 +499,7 @@ __device__ __forceinline__ bool pm_box_begin(const GridDev &g, const float lo[3]
         w.kl[a] = (float)kl;
         w.kh[a] = (float)kh;
         c0[a] = kl - 2 - fo[a];
-        ok = ok && c0[a] >= 0 && kh + 2 - fo[a] <= fn[a] - 1;
+        ok = ok && fabsf(w.ulo[a]) < 0x1p30f && fabsf(w.uhi[a]) < 0x1p30f && c0[a] >= 0 && kh + 2 - fo[a] <= fn[a] - 1;
         if (a == 0) w.nx = kh - kl + 5;
         if (a == 1) w.ny = kh - kl + 5;
         if (a == 2) w.nz = kh - kl + 5;

@@ -140,3 +140,34 @@ def test_segment_list_at_the_grid_edge(tmp_path):
     a 5-cell stencil fits in: no row bound is read beyond the cell table."""
     listed, last = map(int, run(tmp_path, SEGMENT_EDGE).split())
     assert listed > 10000 and last > 100
+
+
+BOX_ENDS = r"""
+int main()
+{
+    const int n[3] = { 9, 7, 8 };
+    const float lo[3] = { -0.2f, -0.17f, -0.23f }, h = 0.1f;
+    Frame f(lattice(n, 0.05f, lo, 1), h);
+    const float ends[] = { NAN, INFINITY, -INFINITY, 3e38f, -3e38f, 1e9f };
+    int bad = 0;
+    for (float e : ends)
+        for (int axis = 0; axis < 3; axis++)
+            for (int side = 0; side < 3; side++) {
+                float l[3] = { 0.0f, 0.0f, 0.0f }, r[3] = { 0.01f, 0.01f, 0.01f };
+                if (side != 1) l[axis] = e;
+                if (side != 0) r[axis] = e;
+                BoxWalk w;
+                bad += pm_box_begin(f.g, l, r, w);
+            }
+    const float a[3] = { 0.0f, 0.0f, 0.0f }, b[3] = { 0.01f, 0.0f, 0.0f };
+    int m = 0;
+    bad += pm_list_segment<kCap>(f.g, a, b, NAN, lst, m);
+    std::printf("%d %d\n", bad, (int)pm_list_segment<kCap>(f.g, a, b, h / 32, lst, m));
+}
+"""
+
+
+def test_box_without_keys(tmp_path):
+    """A box end that is not a number, infinite or beyond any grid has no cells:
+    no fused walk, no list (a NaN offset would otherwise list nothing)."""
+    assert run(tmp_path, BOX_ENDS).split() == ["0", "1"]

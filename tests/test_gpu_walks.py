@@ -184,3 +184,20 @@ def test_finish_list_low_iso(marcher, size, iso):
     marcher.wait()
     for got, want in zip(marcher.batch_download(0), (pos, nrm, t)):
         assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("size", [(61, 43), (333, 207)])
+@pytest.mark.parametrize("eps", [float("nan"), 1e5])
+def test_finish_offset_without_box(marcher, size, eps):
+    """An offset that is not a number, or far beyond the grid, leaves the hits'
+    points as they are: zero normals, as the one-ray-per-lane schedule's."""
+    sc = scenes.lattice_cube(3, n_side=9, spacing=0.05, centre=(0, 0, 0), width=size[0], height=size[1])
+    c = sc.cameras[0]
+    print(f"finish offset {eps} {size}", flush=True)
+    marcher.set_frame(60, sc.xyz, sc.h)
+    st = sc.settings(skip_mode=1, normal_eps=eps)
+    got = marcher.march(60, st, c.inv_pv, c.eye, *size)
+    plain = marcher.march(60, dict(st, schedule=1), c.inv_pv, c.eye, *size)
+    assert got[3]["hits"] > 100 and got[3]["samples"] == plain[3]["samples"]
+    for a, b in zip(got[:3], plain[:3]):
+        assert np.array_equal(a, b)
