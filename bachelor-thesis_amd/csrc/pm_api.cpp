@@ -47,6 +47,7 @@ struct Frame {
     DevBuf sorted, cell_start, counts, slots, indices, scan_tmp, xyz, bounds_partial, bounds;
     DevBuf empty27, clear, clear_tmp, dg_box, dg_cons, dg_count, coarse, bound;
     DevBuf fsorted, fcell_start;    // march grid (cells of h/2)
+    bool ready = false;         // built: info, g and the buffers are one frame's
     bool bound_ok = false;      // bound holds the sub-box bits for bound_iso and bound_boxes
     hipEvent_t bound_ev[2] = { nullptr, nullptr };   // around the last bound build
     bool dg_ok = false;         // the DensityGrid flags are built
@@ -266,19 +267,73 @@ void pm_destroy(pm_ctx *c)
 
 const char *pm_last_error(const pm_ctx *c) { return c ? c->err.c_str() : "null context"; }
 
+// The events around a build's kernels, released on every way out.
+struct EventPair {
+    hipEvent_t e[2] = { nullptr, nullptr };
+    ~EventPair()
+    {
+        for (hipEvent_t x : e)
+            if (x) hipEventDestroy(x);
+    }
+};
+
+// The description of a frame with the bounds b (its grids' extents and the
+// DensityGrid's), or a refusal.  Touches no frame.
+static int frame_extent(pm_ctx *c, const float b[6], uint64_t n, float h, pm_frame_info &I, int32_t dg_dims[3])
+{
+    for (int a = 0; a < 6; a++)
+        if (!std::isfinite(b[a])) return fail(c, PM_ERR_ARG, "pm_set_frame: non-finite particle coordinate");
+    memset(&I, 0, sizeof(I));
+    I.n = n;
+    I.h = h;
+    const float inv_h = 1.0f / h, inv_hf = 2.0f * inv_h;
+    // march grid: cells of h/2 (inv 2/h, exact) and four empty cells of
+    // margin, so the 5x5x5 fine stencil of any point within h of a particle
+    // stays inside it
+    uint64_t nc = 1, fnc = 1, dgn = 1;
+    for (int a = 0; a < 3; a++) {
+        I.pmin[a] = b[a];
+        I.pmax[a] = b[3 + a];
+        // a key beyond an int32 would differ between host and device
+        if (!(I.pmin[a] * inv_hf > -2147483008.0f && I.pmax[a] * inv_hf < 2147483008.0f))
+            return fail(c, PM_ERR_SIZE, "pm_set_frame: coordinates beyond 2^30 h");
+        float pad = 1.0f * h;                           // Frame::ComputeAABB, Dataset.cpp:89-91
+        I.bmin[a] = I.pmin[a] - pad;
+        I.bmax[a] = I.pmax[a] + pad;
+        const int32_t kmin = host_key(I.pmin[a], inv_h), kmax = host_key(I.pmax[a], inv_h);
+        const int32_t fmin = host_key(I.pmin[a], inv_hf), fmax = host_key(I.pmax[a], inv_hf);
+        const int64_t d = (int64_t)kmax - kmin + 5, fd = (int64_t)fmax - fmin + 9;
+        I.origin[a] = kmin - 2;
+        I.forigin[a] = fmin - 4;
+        // (each product so far is below 2^31, each factor below 2^33)
+        nc *= (uint64_t)d;
+        fnc *= (uint64_t)fd;
+        if (nc >= (1ull << 31)) return fail(c, PM_ERR_SIZE, "pm_set_frame: grid of %llu cells or more exceeds 2^31", (unsigned long long)nc);
+        if (fnc >= (1ull << 31)) return fail(c, PM_ERR_SIZE, "pm_set_frame: march grid of %llu cells or more exceeds 2^31", (unsigned long long)fnc);
+        I.dims[a] = (int32_t)d;
+        I.fdims[a] = (int32_t)fd;
+        const float cw = 1.0f * h;                      // Dataset.cpp:96
+        dg_dims[a] = (int32_t)std::ceil((I.bmax[a] - I.bmin[a]) / cw);   // :102-104
+        dgn *= (uint64_t)dg_dims[a];
+        if (dgn >= (1ull << 31)) return fail(c, PM_ERR_SIZE, "pm_set_frame: DensityGrid too large");
+    }
+    I.ncells = nc;
+    I.fncells = fnc;
+    return PM_OK;
+}
+
+// A refusal leaves the frame as it was; a failure after that leaves it not set.
 static int build_frame(pm_ctx *c, int32_t frame, const float *d_src, uint64_t n, float h, hipStream_t st)
 {
     Frame *f;
     auto it = c->frames.find(frame);
     if (it == c->frames.end()) { f = new Frame(); c->frames[frame] = f; }
     else f = it->second;
-    c->frame_epoch++;   // a batch set before this holds the old grid's pointers
-    f->bound_ok = false;
 
-    hipEvent_t e0, e1;
-    HIPCHK(c, hipEventCreate(&e0));
-    HIPCHK(c, hipEventCreate(&e1));
-    HIPCHK(c, hipEventRecord(e0, st));
+    EventPair ev;
+    HIPCHK(c, hipEventCreate(&ev.e[0]));
+    HIPCHK(c, hipEventCreate(&ev.e[1]));
+    HIPCHK(c, hipEventRecord(ev.e[0], st));
     uint32_t np = bounds_partials(n);
     HIPCHK(c, f->bounds_partial.ensure(sizeof(float) * 6 * np));
     HIPCHK(c, f->bounds.ensure(sizeof(float) * 6));
@@ -286,44 +341,18 @@ static int build_frame(pm_ctx *c, int32_t frame, const float *d_src, uint64_t n,
     float b[6];
     HIPCHK(c, hipMemcpyAsync(b, f->bounds.p, sizeof(b), hipMemcpyDeviceToHost, st));
     HIPCHK(c, hipStreamSynchronize(st));
-    for (int a = 0; a < 6; a++)
-        if (!std::isfinite(b[a])) return fail(c, PM_ERR_ARG, "pm_set_frame: non-finite particle coordinate");
+    pm_frame_info info;
+    int32_t dg_dims[3];
+    const int rc = frame_extent(c, b, n, h, info, dg_dims);
+    if (rc) return rc;
 
+    c->frame_epoch++;   // a batch set before this holds the old grid's pointers
+    f->ready = f->bound_ok = false;
     pm_frame_info &I = f->info;
-    memset(&I, 0, sizeof(I));
-    I.n = n;
-    I.h = h;
-    float inv_h = 1.0f / h;
-    uint64_t nc = 1;
-    for (int a = 0; a < 3; a++) {
-        I.pmin[a] = b[a];
-        I.pmax[a] = b[3 + a];
-        float pad = 1.0f * h;                           // Frame::ComputeAABB, Dataset.cpp:89-91
-        I.bmin[a] = I.pmin[a] - pad;
-        I.bmax[a] = I.pmax[a] + pad;
-        int32_t kmin = host_key(I.pmin[a], inv_h), kmax = host_key(I.pmax[a], inv_h);
-        I.origin[a] = kmin - 2;
-        I.dims[a] = kmax - kmin + 5;
-        nc *= (uint64_t)I.dims[a];
-    }
-    if (nc >= (1ull << 31)) return fail(c, PM_ERR_SIZE, "pm_set_frame: grid of %llu cells exceeds 2^31", (unsigned long long)nc);
-    I.ncells = nc;
-    // march grid: cells of h/2 (inv 2/h, exact) and four empty cells of
-    // margin, so the 5x5x5 fine stencil of any point within h of a particle
-    // stays inside it
-    const float inv_hf = 2.0f * inv_h;
-    uint64_t fnc = 1;
-    for (int ax = 0; ax < 3; ax++) {
-        // a key beyond an int32 would differ between host and device
-        if (!(I.pmin[ax] * inv_hf > -2147483008.0f && I.pmax[ax] * inv_hf < 2147483008.0f))
-            return fail(c, PM_ERR_SIZE, "pm_set_frame: coordinates beyond 2^30 h");
-        int32_t kmin = host_key(I.pmin[ax], inv_hf), kmax = host_key(I.pmax[ax], inv_hf);
-        I.forigin[ax] = kmin - 4;
-        I.fdims[ax] = kmax - kmin + 9;
-        fnc *= (uint64_t)I.fdims[ax];
-    }
-    if (fnc >= (1ull << 31)) return fail(c, PM_ERR_SIZE, "pm_set_frame: march grid of %llu cells exceeds 2^31", (unsigned long long)fnc);
-    I.fncells = fnc;
+    I = info;
+    for (int a = 0; a < 3; a++) f->dg_dims[a] = dg_dims[a];
+    const float inv_h = 1.0f / h, inv_hf = 2.0f * inv_h;
+    const uint64_t nc = I.ncells, fnc = I.fncells;
 
     HIPCHK(c, f->sorted.ensure(sizeof(float4) * n));
     HIPCHK(c, f->cell_start.ensure(sizeof(uint32_t) * (nc + 1)));
@@ -354,7 +383,7 @@ static int build_frame(pm_ctx *c, int32_t frame, const float *d_src, uint64_t n,
     a.scan_tmp = (uint32_t *)f->scan_tmp.p;
     a.occupied = a.scan_tmp + scan_words;
     HIPCHK(c, launch_grid_build(a, st));
-    HIPCHK(c, hipEventRecord(e1, st));
+    HIPCHK(c, hipEventRecord(ev.e[1], st));
 
     GridDev &g = f->g;
     g.sorted = (const float4 *)f->sorted.p;
@@ -385,13 +414,6 @@ static int build_frame(pm_ctx *c, int32_t frame, const float *d_src, uint64_t n,
     HIPCHK(c, launch_clear(g.empty27, I.dims[0], I.dims[1], I.dims[2], (uint8_t *)f->clear_tmp.p,
                            (uint8_t *)f->clear.p, st));
     g.clear = (const uint8_t *)f->clear.p;
-    uint64_t dgn = 1;
-    for (int a2 = 0; a2 < 3; a2++) {
-        float cw = 1.0f * h;                            // Dataset.cpp:96
-        f->dg_dims[a2] = (int32_t)std::ceil((I.bmax[a2] - I.bmin[a2]) / cw);   // :102-104
-        dgn *= (uint64_t)f->dg_dims[a2];
-    }
-    if (dgn >= (1ull << 31)) return fail(c, PM_ERR_SIZE, "pm_set_frame: DensityGrid too large");
     g.dg_nx = f->dg_dims[0]; g.dg_ny = f->dg_dims[1]; g.dg_nz = f->dg_dims[2];
     g.dg_flag = nullptr;
     f->dg_ok = false;   // built on first use (reference march, pm_get_skip_grids)
@@ -405,10 +427,9 @@ static int build_frame(pm_ctx *c, int32_t frame, const float *d_src, uint64_t n,
     HIPCHK(c, hipStreamSynchronize(st));
     g.sparse = n <= (uint64_t)kSparsePerCell * occupied[1];
     float ms = 0.f;
-    hipEventElapsedTime(&ms, e0, e1);
+    hipEventElapsedTime(&ms, ev.e[0], ev.e[1]);
     I.build_ms = ms;
-    hipEventDestroy(e0);
-    hipEventDestroy(e1);
+    f->ready = true;
     return PM_OK;
 }
 
@@ -479,7 +500,7 @@ int pm_set_frame_device(pm_ctx *c, int32_t frame, const void *d_xyz, uint64_t n,
 static Frame *get_frame(pm_ctx *c, int32_t frame)
 {
     auto it = c->frames.find(frame);
-    return it == c->frames.end() ? nullptr : it->second;
+    return it == c->frames.end() || !it->second->ready ? nullptr : it->second;
 }
 
 int pm_frame_info_get(pm_ctx *c, int32_t frame, pm_frame_info *out)

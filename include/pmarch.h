@@ -162,7 +162,10 @@ void pm_destroy(pm_ctx *ctx);
 const char *pm_last_error(const pm_ctx *ctx);
 
 /* Frame::Frame (Dataset.cpp:9-24): copies n float3 positions (the caller keeps
- * ownership) and builds the uniform grid, AABB and skip structures on the GPU. */
+ * ownership) and builds the uniform grid, AABB and skip structures on the GPU.
+ * PM_ERR_ARG for a non-finite coordinate, PM_ERR_SIZE for coordinates beyond
+ * 2^30 h or a grid of 2^31 cells (cells of h, or of h/2); a frame refused so is
+ * left as it was. */
 int pm_set_frame(pm_ctx *ctx, int32_t frame, const float *xyz, uint64_t n, float h);
 /* Same, from positions already in device memory (frame streaming). */
 int pm_set_frame_device(pm_ctx *ctx, int32_t frame, const void *d_xyz, uint64_t n, float h);
