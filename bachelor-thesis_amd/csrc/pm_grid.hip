@@ -24,6 +24,11 @@ uint32_t bounds_partials(uint64_t n)
     return (uint32_t)b;
 }
 
+// Minimum and maximum that keep a NaN, so one anywhere shows in the bounds (and
+// the frame is refused: it has no cell).
+__device__ __forceinline__ float bounds_min(float a, float b) { return b < a || b != b ? b : a; }
+__device__ __forceinline__ float bounds_max(float a, float b) { return b > a || b != b ? b : a; }
+
 __global__ __launch_bounds__(kThreads) void k_bounds_partial(const float *__restrict__ xyz, uint64_t n,
                                                              float *__restrict__ partial)
 {
@@ -31,8 +36,8 @@ __global__ __launch_bounds__(kThreads) void k_bounds_partial(const float *__rest
     for (uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kThreads) {
         for (int a = 0; a < 3; a++) {
             float v = xyz[3 * i + a];
-            mn[a] = fminf(mn[a], v);
-            mx[a] = fmaxf(mx[a], v);
+            mn[a] = bounds_min(mn[a], v);
+            mx[a] = bounds_max(mx[a], v);
         }
     }
     __shared__ float red[6][kThreads];
@@ -41,8 +46,8 @@ __global__ __launch_bounds__(kThreads) void k_bounds_partial(const float *__rest
     for (int s = kThreads / 2; s > 0; s >>= 1) {
         if ((int)threadIdx.x < s) {
             for (int a = 0; a < 3; a++) {
-                red[a][threadIdx.x] = fminf(red[a][threadIdx.x], red[a][threadIdx.x + s]);
-                red[3 + a][threadIdx.x] = fmaxf(red[3 + a][threadIdx.x], red[3 + a][threadIdx.x + s]);
+                red[a][threadIdx.x] = bounds_min(red[a][threadIdx.x], red[a][threadIdx.x + s]);
+                red[3 + a][threadIdx.x] = bounds_max(red[3 + a][threadIdx.x], red[3 + a][threadIdx.x + s]);
             }
         }
         __syncthreads();
@@ -57,16 +62,16 @@ __global__ __launch_bounds__(kThreads) void k_bounds_final(const float *__restri
     float v[6] = { FLT_MAX, FLT_MAX, FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX };
     for (uint32_t i = threadIdx.x; i < np; i += kThreads)
         for (int a = 0; a < 3; a++) {
-            v[a] = fminf(v[a], partial[6 * i + a]);
-            v[3 + a] = fmaxf(v[3 + a], partial[6 * i + 3 + a]);
+            v[a] = bounds_min(v[a], partial[6 * i + a]);
+            v[3 + a] = bounds_max(v[3 + a], partial[6 * i + 3 + a]);
         }
     for (int a = 0; a < 6; a++) red[a][threadIdx.x] = v[a];
     __syncthreads();
     for (int s = kThreads / 2; s > 0; s >>= 1) {
         if ((int)threadIdx.x < s)
             for (int a = 0; a < 3; a++) {
-                red[a][threadIdx.x] = fminf(red[a][threadIdx.x], red[a][threadIdx.x + s]);
-                red[3 + a][threadIdx.x] = fmaxf(red[3 + a][threadIdx.x], red[3 + a][threadIdx.x + s]);
+                red[a][threadIdx.x] = bounds_min(red[a][threadIdx.x], red[a][threadIdx.x + s]);
+                red[3 + a][threadIdx.x] = bounds_max(red[3 + a][threadIdx.x], red[3 + a][threadIdx.x + s]);
             }
         __syncthreads();
     }

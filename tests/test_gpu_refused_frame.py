@@ -13,6 +13,8 @@ def _refused(kind, n):
     xyz = np.random.default_rng(1).uniform(0, 1, (n, 3)).astype(np.float32)
     if kind == "inf":
         xyz[n // 2, 1] = np.inf
+    elif kind == "nan":              # one coordinate among many
+        xyz[n // 2, 1] = np.nan
     elif kind == "far":              # every key beyond an int32
         xyz += np.float32(3.0e8)
     elif kind == "grid":             # cells of h
@@ -25,7 +27,7 @@ def _refused(kind, n):
 
 
 @pytest.mark.parametrize("stream", [False, True])
-@pytest.mark.parametrize("kind", ["inf", "far", "grid", "march grid", "product"])
+@pytest.mark.parametrize("kind", ["inf", "nan", "far", "grid", "march grid", "product"])
 def test_refused_frame(marcher, kind, stream):
     sc = scenes.lattice_cube(2, n_side=8, spacing=0.05, width=48, height=32)
     c = sc.cameras[0]
