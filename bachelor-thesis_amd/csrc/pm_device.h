@@ -781,6 +781,12 @@ __device__ __forceinline__ uint32_t pm_box_cand(const GridDev &g, const float x[
             pm_box_row(g, w, k, k < w.ny ? jz : w.nz, b, en);
             cand += en - b;
         }
+        // offsets beyond h / 4
+        _Pragma("unroll 1") for (int k = 6; __ballot(k < w.ny) != 0; k++) {
+            uint32_t b, en;
+            pm_box_row(g, w, k, k < w.ny ? jz : w.nz, b, en);
+            cand += en - b;
+        }
     }
     return cand;
 }

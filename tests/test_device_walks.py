@@ -171,3 +171,36 @@ def test_box_without_keys(tmp_path):
     """A box end that is not a number, infinite or beyond any grid has no cells:
     no fused walk, no list (a NaN offset would otherwise list nothing)."""
     assert run(tmp_path, BOX_ENDS).split() == ["0", "1"]
+
+
+BOX_CAND = r"""
+int main()
+{
+    const int n[3] = { 16, 15, 14 };
+    const float lo[3] = { -0.3f, -0.17f, 0.23f }, h = 0.1f;
+    Frame f(lattice(n, 0.05f, lo, 1), h);
+    static float buf[96 * 64];
+    std::mt19937 rng(3);
+    std::uniform_real_distribution<float> u(0.0f, 1.0f);
+    long differ = 0, most = 0, seven = 0;
+    const float offsets[] = { 0.0f, h / 32, -h / 32, 0.02f, 0.026f, 0.03f, -0.03f, 0.06f, 0.1f };
+    for (float eps : offsets)
+        for (int i = 0; i < 400; i++) {
+            float x[3];
+            for (int a = 0; a < 3; a++) x[a] = f.pmin[a] + (f.pmax[a] - f.pmin[a]) * u(rng);
+            const Cdiff6 o = pm_cdiff6_lds<96>(f.g, x[0], x[1], x[2], eps, buf, true);
+            const uint32_t c = pm_box_cand(f.g, x, eps);
+            differ += c != o.cand;
+            seven += fabsf(eps) >= 0.026f && o.cand != 0xffffffffu;
+            if (o.cand != 0xffffffffu && (long)o.cand > most) most = o.cand;
+        }
+    std::printf("%ld %ld %ld\n", differ, most, seven);
+}
+"""
+
+
+def test_box_candidates(tmp_path):
+    """The count without a walk is the six-sample walk's, also where the box
+    spans seven rows or more (offsets beyond h / 4)."""
+    differ, most, seven = map(int, run(tmp_path, BOX_CAND).split())
+    assert differ == 0 and most > 100 and seven > 500

@@ -201,3 +201,17 @@ def test_finish_offset_without_box(marcher, size, eps):
     assert got[3]["hits"] > 100 and got[3]["samples"] == plain[3]["samples"]
     for a, b in zip(got[:3], plain[:3]):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("tiles", [(25, 31), (25, 33)])
+@pytest.mark.parametrize("eps", [0.02, 0.03, 0.06])
+def test_candidates_of_wide_offsets(marcher, tiles, eps):
+    """The candidates counted for the central differences do not depend on which
+    finish the image's size selects (775 and 825 tiles), also for boxes of seven
+    rows and more."""
+    sc = scenes.lattice_cube(3, n_side=9, spacing=0.05, width=8 * tiles[0], height=8 * tiles[1])
+    sc.normal_eps = eps
+    print(f"candidates of offset {eps}, {tiles} tiles", flush=True)
+    marcher.set_frame(60, sc.xyz, sc.h)
+    got = _check(marcher, sc, counters=COUNTERS + ("cand",), skip_mode=1)
+    assert got["hits"] > 1000
