@@ -651,7 +651,7 @@ __device__ __forceinline__ Cdiff6 pm_cdiff6_lds(const GridDev &g, float qx, floa
 
 // ---- one list for all samples of a hit ----
 // The bisection, the FP64 step and the six central differences of a hit sample
-// points within a short segment [a, b] (one march step) and eps around it.  One
+// points within a short segment o + [ta, tb] d (one march step) and eps around it.  One
 // walk lists every particle within h of any of them, in the canonical order;
 // each sample then takes the list with its own r^2 < h^2 test, so its sum is
 // its single-sample sum, bit for bit, for about 25 candidates read instead of a
@@ -661,14 +661,17 @@ __device__ __forceinline__ Cdiff6 pm_cdiff6_lds(const GridDev &g, float qx, floa
 // would cost both) when some lane's box leaves the grid or spans more than two
 // cells on an axis, or its list does not fit CAP.
 template <int CAP>
-__device__ __forceinline__ bool pm_list_segment(const GridDev &g, const float a[3], const float b[3], float eps,
-                                                uint32_t *lst, int &n)
+__device__ __forceinline__ bool pm_list_segment(const GridDev &g, const float o[3], const float d[3], float ta, float tb,
+                                                float eps, uint32_t *lst, int &n)
 {
-    float lo[3], hi[3], c[3], l2 = 0.0f, big = 0.0f;
+    // the ends and the samples are rounded sums o + t d: a few ulps of the largest
+    // term of room (the FP64 sample and its point lie outside [a, b] by up to one)
+    float a[3], b[3], lo[3], hi[3], c[3], l2 = 0.0f, big = fmaxf(fabsf(ta), fabsf(tb));
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-        // the samples' coordinates are rounded: a few ulps of room
-        big = fmaxf(big, fmaxf(fabsf(a[k]), fabsf(b[k])));
+        a[k] = o[k] + ta * d[k];
+        b[k] = o[k] + tb * d[k];
+        big = fmaxf(big, fmaxf(fmaxf(fabsf(a[k]), fabsf(b[k])), fabsf(o[k])));
         c[k] = 0.5f * (a[k] + b[k]);
         const float e = b[k] - a[k];
         l2 += e * e;

@@ -417,9 +417,8 @@ __device__ __forceinline__ void finish_hit(const MarchLaunch &L, uint32_t px, ui
     int n = 0;
     bool listed = false;
     if (LIST) {
-        const float a[3] = { o0 + lo * d[0], o1 + lo * d[1], o2 + lo * d[2] };
-        const float b[3] = { o0 + hi * d[0], o1 + hi * d[1], o2 + hi * d[2] };
-        listed = pm_list_segment<kFinCap>(g, a, b, fabsf(e), lst, n);
+        const float o[3] = { o0, o1, o2 };
+        listed = pm_list_segment<kFinCap>(g, o, d, lo, hi, fabsf(e), lst, n);
     }
     if (bracket) {
         const int n32 = fp64 ? s.bisect_iters - 1 : s.bisect_iters;
@@ -880,11 +879,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
         float d[3];
         pm_ray_dir(L, px, py, d);
         FinishDens dens{ &g, lst, 0, false, comp, true };
-        if (LIST && hit) {
-            const float a[3] = { o[0] + lo * d[0], o[1] + lo * d[1], o[2] + lo * d[2] };
-            const float b[3] = { o[0] + hi * d[0], o[1] + hi * d[1], o[2] + hi * d[2] };
-            dens.listed = pm_list_segment<kFinCap>(g, a, b, fabsf(e), lst, dens.n);
-        }
+        if (LIST && hit) dens.listed = pm_list_segment<kFinCap>(g, o, d, lo, hi, fabsf(e), lst, dens.n);
         if (__ballot(bracket) != 0) {
             float l = lo, h = hi;
             group_bisect(L, d, l, h, fp64 ? s.bisect_iters - 1 : s.bisect_iters, bracket, G, dens, cn);

@@ -122,7 +122,8 @@ int main()
                 b[k] = a[k] + step * d[k] / sqrtf(len);
             }
             int m = 0;
-            if (!pm_list_segment<kCap>(f.g, a, b, eps, lst, m)) continue;
+            for (int k = 0; k < 3; k++) d[k] = b[k] - a[k];
+            if (!pm_list_segment<kCap>(f.g, a, d, 0.0f, 1.0f, eps, lst, m)) continue;
             listed++;
             BoxWalk w;
             const float l[3] = { fminf(a[0], b[0]) - eps, fminf(a[1], b[1]) - eps, fminf(a[2], b[2]) - eps };
@@ -159,17 +160,17 @@ int main()
                 BoxWalk w;
                 bad += pm_box_begin(f.g, l, r, w);
             }
-    const float a[3] = { 0.0f, 0.0f, 0.0f }, b[3] = { 0.01f, 0.0f, 0.0f };
+    const float a[3] = { 0.0f, 0.0f, 0.0f }, d[3] = { 1.0f, 0.0f, 0.0f };
     int m = 0;
-    bad += pm_list_segment<kCap>(f.g, a, b, NAN, lst, m);
-    std::printf("%d %d\n", bad, (int)pm_list_segment<kCap>(f.g, a, b, h / 32, lst, m));
+    bad += pm_list_segment<kCap>(f.g, a, d, 0.0f, 0.01f, NAN, lst, m);
+    std::printf("%d %d\n", bad, (int)pm_list_segment<kCap>(f.g, a, d, 0.0f, 0.01f, h / 32, lst, m));
 }
 """
 
 
 def test_box_without_keys(tmp_path):
-    """A box end that is not a number, infinite or beyond any grid has no cells:
-    no fused walk, no list (a NaN offset would otherwise list nothing)."""
+    """An offset that is not a number, infinite or beyond any grid has no box: no
+    fused walk, no list (a NaN offset would otherwise list nothing)."""
     assert run(tmp_path, BOX_ENDS).split() == ["0", "1"]
 
 
@@ -204,3 +205,59 @@ def test_box_candidates(tmp_path):
     spans seven rows or more (offsets beyond h / 4)."""
     differ, most, seven = map(int, run(tmp_path, BOX_CAND).split())
     assert differ == 0 and most > 100 and seven > 500
+
+
+FAR_EYE = r"""
+int main()
+{
+    const int n[3] = { 12, 12, 12 };
+    const float lo3[3] = { 0.2f, 0.2f, 0.2f }, h = 0.1f, eps = h / 32;
+    Frame f(lattice(n, 0.05f, lo3, 1), h);
+    std::mt19937 rng(5);
+    std::uniform_real_distribution<float> u(-1.0f, 1.0f);
+    long listed = 0, missing = 0, within = 0;
+    const float dist[] = { 2.0f, 2e2f, 2e3f, 2e4f, 2e5f };
+    for (float D : dist)
+        for (int i = 0; i < 4000; i++) {
+            float d[3], o[3], s = 0.0f;
+            for (int k = 0; k < 3; k++) { d[k] = u(rng); s += d[k] * d[k]; }
+            for (int k = 0; k < 3; k++) {
+                d[k] /= sqrtf(s);
+                o[k] = (0.475f + 0.3f * u(rng)) - D * d[k];
+            }
+            const float lo = D, hi = lo + h / 8;
+            int m = 0;
+            if (!pm_list_segment<kCap>(f.g, o, d, lo, hi, eps, lst, m)) continue;
+            listed++;
+            for (int j = 0; j < 10; j++) {
+                // bracket ends and midpoints; the FP64 sample; the central differences of its point
+                const float t = j == 0 ? lo : j == 1 ? hi : fminf(fmaxf(lo + (hi - lo) * (0.5f + 0.5f * u(rng)), lo), hi);
+                const double td = ((double)lo + (double)t) * 0.5;
+                double q[3], h2 = f.g.h2_d;
+                for (int k = 0; k < 3; k++) {
+                    q[k] = (double)o[k] + td * (double)d[k];
+                    if (j < 4) q[k] = o[k] + t * d[k];
+                    if (j > 5) q[k] = (float)q[k];
+                }
+                if (j > 6) q[j - 7] = (float)q[j - 7] + (j & 1 ? eps : -eps);
+                for (size_t p = 0; p < f.sorted.size(); p++) {
+                    const double rx = f.sorted[p].x - q[0], ry = f.sorted[p].y - q[1], rz = f.sorted[p].z - q[2];
+                    if (!((rx * rx + ry * ry) + rz * rz < h2 * (j == 4 || j == 5 ? 1.0 : 0.999999))) continue;
+                    within++;
+                    bool found = false;
+                    for (int k = 0; k < m; k++) found = found || lst[k * 64] == p;
+                    missing += !found;
+                }
+            }
+        }
+    std::printf("%ld %ld %ld\n", listed, within, missing);
+}
+"""
+
+
+def test_segment_list_of_a_far_eye(tmp_path):
+    """Every particle within h of any of a hit's samples is in its list, from
+    20 h to 2,000,000 h away (where the coordinates' rounding outgrows h and no
+    list is made)."""
+    listed, within, missing = map(int, run(tmp_path, FAR_EYE).split())
+    assert listed > 12000 and within > 10 ** 6 and missing == 0
