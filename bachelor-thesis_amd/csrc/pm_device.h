@@ -482,9 +482,8 @@ struct BoxWalk {
     float xm2, xm1, xp1, xp2; // squared x-distances of the four trimmable end cells
 };
 
-// false when the cells leave the march grid, or the box has no keys (an end that
-// is not a number, or beyond any grid): the caller then takes the samples one
-// at a time.
+// false when the cells leave the march grid (the caller then takes the samples
+// one at a time).  The ends are finite and within 2^30 cells (pm_box_offset).
 __device__ __forceinline__ bool pm_box_begin(const GridDev &g, const float lo[3], const float hi[3], BoxWalk &w)
 {
     const int32_t fo[3] = { g.fox, g.foy, g.foz }, fn[3] = { g.fnx, g.fny, g.fnz };
@@ -499,7 +498,7 @@ __device__ __forceinline__ bool pm_box_begin(const GridDev &g, const float lo[3]
         w.kl[a] = (float)kl;
         w.kh[a] = (float)kh;
         c0[a] = kl - 2 - fo[a];
-        ok = ok && fabsf(w.ulo[a]) < 0x1p30f && fabsf(w.uhi[a]) < 0x1p30f && c0[a] >= 0 && kh + 2 - fo[a] <= fn[a] - 1;
+        ok = ok && c0[a] >= 0 && kh + 2 - fo[a] <= fn[a] - 1;
         if (a == 0) w.nx = kh - kl + 5;
         if (a == 1) w.ny = kh - kl + 5;
         if (a == 2) w.nz = kh - kl + 5;
@@ -533,6 +532,9 @@ __device__ __forceinline__ void pm_box_row(const GridDev &g, const BoxWalk &w, i
     b = kept ? lb : 0u;
     e = kept ? le : 0u;
 }
+
+// An offset a box around a point near the grid can have: its ends have keys.
+__device__ __forceinline__ bool pm_box_offset(const GridDev &g, float eps) { return fabsf(eps) < 0x1p28f * g.h; }
 
 struct Cdiff6 {
     float v[6];      // densities at +x, -x, +y, -y, +z, -z
@@ -583,7 +585,7 @@ __device__ __forceinline__ Cdiff6 pm_cdiff6_lds(const GridDev &g, float qx, floa
     const float xp[3] = { qx + eps, qy + eps, qz + eps }, xm[3] = { qx - eps, qy - eps, qz - eps };
     BoxWalk w;
     // eps may be negative (the samples change places)
-    if (!(eps < 0.0f ? pm_box_begin(g, xp, xm, w) : pm_box_begin(g, xm, xp, w))) {
+    if (!pm_box_offset(g, eps) || !(eps < 0.0f ? pm_box_begin(g, xp, xm, w) : pm_box_begin(g, xm, xp, w))) {
         out.cand = 0xffffffffu;
 #pragma unroll
         for (int k = 0; k < 6; k++) out.v[k] = 0.0f;
@@ -684,7 +686,8 @@ __device__ __forceinline__ bool pm_list_segment(const GridDev &g, const float o[
     }
     const float R = (g.h + 0.5f * sqrtf(l2) + room) * 1.0009765625f, R2 = R * R;
     BoxWalk w;
-    const bool in = pm_box_begin(g, lo, hi, w) && w.nx <= 6 && w.ny <= 6 && w.nz <= 6;
+    // (six cells hold a box narrower than h; a NaN offset has none)
+    const bool in = room < g.h && pm_box_begin(g, lo, hi, w) && w.nx <= 6 && w.ny <= 6 && w.nz <= 6;
     if (__ballot(!in) != 0) return false;
     int f = 0;                                  // entries [0, f) passed the test, [f, n) are untested
     n = 0;
@@ -710,7 +713,8 @@ __device__ __forceinline__ bool pm_list_segment(const GridDev &g, const float o[
     uint32_t pb[6], pe[6], qb[6], qe[6];
     auto plane = [&](int jz, uint32_t (&b_)[6], uint32_t (&e_)[6]) {
 #pragma unroll
-        for (int k = 0; k < 6; k++) pm_box_row(g, w, k, k < w.ny ? jz : w.nz, b_[k], e_[k]);   // row ny may lie past the grid
+        for (int k = 0; k < 6; k++)   // ny is 5 or more; row ny may lie past the grid
+            pm_box_row(g, w, k, k < 5 || k < w.ny ? jz : w.nz, b_[k], e_[k]);
     };
     plane(0, pb, pe);
     _Pragma("unroll 1") for (int jz = 0; __ballot(jz < w.nz) != 0; jz++) {
@@ -775,13 +779,13 @@ __device__ __forceinline__ uint32_t pm_box_cand(const GridDev &g, const float x[
     const float e = fabsf(eps);
     const float lo[3] = { x[0] - e, x[1] - e, x[2] - e }, hi[3] = { x[0] + e, x[1] + e, x[2] + e };
     BoxWalk w;
-    if (!pm_box_begin(g, lo, hi, w)) return 0xffffffffu;
+    if (!pm_box_offset(g, eps) || !pm_box_begin(g, lo, hi, w)) return 0xffffffffu;
     uint32_t cand = 0;
     _Pragma("unroll 1") for (int jz = 0; __ballot(jz < w.nz) != 0; jz++) {
 #pragma unroll
         for (int k = 0; k < 6; k++) {
             uint32_t b, en;
-            pm_box_row(g, w, k, k < w.ny ? jz : w.nz, b, en);
+            pm_box_row(g, w, k, k < 5 || k < w.ny ? jz : w.nz, b, en);
             cand += en - b;
         }
         // offsets beyond h / 4

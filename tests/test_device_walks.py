@@ -149,20 +149,15 @@ int main()
     const int n[3] = { 9, 7, 8 };
     const float lo[3] = { -0.2f, -0.17f, -0.23f }, h = 0.1f;
     Frame f(lattice(n, 0.05f, lo, 1), h);
-    const float ends[] = { NAN, INFINITY, -INFINITY, 3e38f, -3e38f, 1e9f };
-    int bad = 0;
-    for (float e : ends)
-        for (int axis = 0; axis < 3; axis++)
-            for (int side = 0; side < 3; side++) {
-                float l[3] = { 0.0f, 0.0f, 0.0f }, r[3] = { 0.01f, 0.01f, 0.01f };
-                if (side != 1) l[axis] = e;
-                if (side != 0) r[axis] = e;
-                BoxWalk w;
-                bad += pm_box_begin(f.g, l, r, w);
-            }
+    const float offsets[] = { NAN, INFINITY, -INFINITY, 3e38f, -3e38f, 1e9f, -1e9f };
+    static float buf[96 * 64];
     const float a[3] = { 0.0f, 0.0f, 0.0f }, d[3] = { 1.0f, 0.0f, 0.0f };
-    int m = 0;
-    bad += pm_list_segment<kCap>(f.g, a, d, 0.0f, 0.01f, NAN, lst, m);
+    int bad = 0, m = 0;
+    for (float e : offsets) {
+        bad += pm_list_segment<kCap>(f.g, a, d, 0.0f, 0.01f, fabsf(e), lst, m);
+        bad += pm_box_cand(f.g, a, e) != 0xffffffffu;
+        bad += pm_cdiff6_lds<96>(f.g, 0.0f, 0.0f, 0.0f, e, buf, true).cand != 0xffffffffu;
+    }
     std::printf("%d %d\n", bad, (int)pm_list_segment<kCap>(f.g, a, d, 0.0f, 0.01f, h / 32, lst, m));
 }
 """
