@@ -21,7 +21,6 @@
 #include <atomic>
 #include <condition_variable>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 namespace pm {
@@ -91,8 +90,9 @@ class CopyPool {
         const int want = hw > 1 ? (int)std::min(3u, hw / 2) : 0;
         try {
             for (; workers_ < want; workers_++) th_[workers_] = std::thread(&CopyPool::run, this);
-        } catch (const std::system_error &) {
-            // as many as there are
+        } catch (...) {
+            // no thread, or no memory for one: as many as there are (nothing may
+            // be thrown through the C entry that copies)
         }
         return workers_ > 0;
     }

@@ -58,3 +58,54 @@ def test_shared_copy(tmp_path):
                     "-I" + str(ROOT / "bachelor-thesis_amd" / "csrc"), str(src), "-pthread", "-o", str(exe)], check=True)
     out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
     assert out.returncode == 0 and out.stdout.strip() == "ok", out.stdout + out.stderr
+
+
+NO_MEMORY = r"""
+#include "pm_copy.h"
+#include <cstdio>
+#include <cstdlib>
+#include <new>
+
+// The next allocations of the copying thread that fail; -1: none do.
+static thread_local int left = -1;
+void *operator new(size_t n)
+{
+    if (left == 0) throw std::bad_alloc();
+    if (left > 0) left--;
+    if (void *p = malloc(n)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void *p) noexcept { free(p); }
+void operator delete(void *p, size_t) noexcept { free(p); }
+
+int main()
+{
+    const size_t n = 3 * pm::kCopyShared + 17;
+    char *a = (char *)malloc(n), *b = (char *)malloc(n);
+    for (int allowed = 0; allowed < 4; allowed++) {
+        pm::CopyPool pool;
+        for (int rep = 0; rep < 3; rep++) {
+            memset(a, 17 * rep + allowed + 1, n);
+            memset(b, 0, n);
+            const pm::CopyPool::Range r = { b, a, n };
+            left = allowed;
+            pool.copy(&r, 1);
+            left = -1;
+            if (memcmp(a, b, n) != 0) return 1;
+        }
+    }
+    std::puts("ok");
+    return 0;
+}
+"""
+
+
+def test_copy_without_memory_for_workers(tmp_path):
+    """No memory for the first, second or third worker: the copy is made by those
+    there are, and nothing is thrown."""
+    src, exe = tmp_path / "copy.cpp", tmp_path / "copy"
+    src.write_text(NO_MEMORY)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-I" + str(ROOT / "bachelor-thesis_amd" / "csrc"), str(src),
+                    "-pthread", "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert out.returncode == 0 and out.stdout.strip() == "ok", out.stdout + out.stderr
