@@ -912,7 +912,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
                 an_normal_gradw(L, xs, lst, nx, ny, nz);
                 L.nrm[idx] = make_float4(nx, ny, nz, 1.0f);
             }
-            cn.hits++;
         }
     }
     if (any) flush_counters(L.counters, cn.rays, cn.in_aabb, cn.hits, cn.samples, cn.cand, cn.march);

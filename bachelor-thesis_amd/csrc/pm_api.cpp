@@ -362,7 +362,7 @@ static int build_frame(pm_ctx *c, int32_t frame, const float *d_src, uint64_t n,
     HIPCHK(c, f->indices.ensure(sizeof(uint32_t) * n));
     HIPCHK(c, f->counts.ensure(sizeof(uint32_t) * fnc));
     const size_t scan_words = scan_tmp_size((uint32_t)nc, (uint32_t)fnc);
-    HIPCHK(c, f->scan_tmp.ensure(sizeof(uint32_t) * (scan_words + 2)));
+    HIPCHK(c, f->scan_tmp.ensure(sizeof(uint32_t) * (scan_words + 4)));
 
     GridBuildArgs a{};
     a.xyz = d_src; a.n = n;
@@ -422,10 +422,11 @@ static int build_frame(pm_ctx *c, int32_t frame, const float *d_src, uint64_t n,
     HIPCHK(c, f->coarse.ensure(4ull * f->cg.nx * f->cg.ny * f->cg.nz));
     f->cg.count = (const uint32_t *)f->coarse.p;
     HIPCHK(c, launch_coarse_counts(g, f->cg, (uint32_t *)f->coarse.p, st));
-    uint32_t occupied[2] = { 0, 0 };
+    uint32_t occupied[4] = { 0, 0, 0, 0 };
     HIPCHK(c, hipMemcpyAsync(occupied, a.occupied, sizeof(occupied), hipMemcpyDeviceToHost, st));
     HIPCHK(c, hipStreamSynchronize(st));
-    g.sparse = n <= (uint64_t)kSparsePerCell * occupied[1];
+    g.sparse = n <= (uint64_t)kSparsePerCell * occupied[2];
+    g.group_hits = group_hits(n, occupied[2], occupied[3]);
     float ms = 0.f;
     hipEventElapsedTime(&ms, ev.e[0], ev.e[1]);
     I.build_ms = ms;

@@ -43,6 +43,7 @@ struct GridDev {
     int32_t fnx, fny, fnz;
     float inv_hf;             // 2 / h
     int sparse;               // at most kSparsePerCell particles per occupied fine cell on average
+    uint32_t group_hits;      // most hits whose finish takes four lanes each (dense frames, pm_march.hip)
 };
 static constexpr uint32_t kSparsePerCell = 3;
 

@@ -140,7 +140,9 @@ static constexpr int kScanBlock = kThreads * kScanPer;
 
 static inline uint32_t scan_blocks(uint32_t len) { return (len + kScanBlock - 1) / kScanBlock; }
 
-// Per block of the scan its sum and its number of nonzero elements.
+// Per block of the scan its sum, and its number of nonzero elements (11 bits) with
+// its largest element (21 bits, at most kScanMax).
+static constexpr uint32_t kScanMax = (1u << 21) - 1u;
 size_t scan_tmp_size(uint32_t ncells, uint32_t fncells)
 {
     return 2 * ((size_t)scan_blocks(ncells + 1) + scan_blocks(fncells + 1));
@@ -191,54 +193,72 @@ __device__ __forceinline__ uint32_t dense_count(const GridBuildArgs &a, uint32_t
 // Blocks 0 .. nb0 - 1 scan the search grid's counts, the others the march grid's.
 __global__ __launch_bounds__(kThreads) void k_scan_blocks(GridBuildArgs a, uint32_t nb0)
 {
-    __shared__ uint32_t sh[kThreads / 64], occ;
+    __shared__ uint32_t sh[kThreads / 64], occ, top;
     const bool fine = blockIdx.x >= nb0;
     const uint32_t ncells = fine ? a.fncells : a.ncells, blk = blockIdx.x - (fine ? nb0 : 0u);
     uint32_t *out = fine ? a.fcell_start : a.cell_start;
     const uint32_t base = blk * kScanBlock + threadIdx.x * kScanPer;
-    uint32_t v[kScanPer], sum = 0, cells = 0;
+    uint32_t v[kScanPer], sum = 0, cells = 0, most = 0;
     for (int j = 0; j < kScanPer; j++) {
         v[j] = base + j >= ncells ? 0u : (fine ? a.counts[base + j] : dense_count(a, base + j));
         sum += v[j];
         cells += v[j] != 0;
+        most = max(most, v[j]);
     }
-    if (threadIdx.x == 0) occ = 0;
+    if (threadIdx.x == 0) occ = top = 0;
     uint32_t total;
     uint32_t ex = block_excl_scan(sum, sh, total);
     for (int j = 0; j < kScanPer; j++) {
         if (base + j <= ncells) out[base + j] = ex;
         ex += v[j];
     }
-    for (int off = 32; off > 0; off >>= 1) cells += __shfl_xor(cells, off, 64);
-    if ((threadIdx.x & 63) == 0) atomicAdd(&occ, cells);
+    for (int off = 32; off > 0; off >>= 1) {
+        cells += __shfl_xor(cells, off, 64);
+        most = max(most, (uint32_t)__shfl_xor(most, off, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        atomicAdd(&occ, cells);
+        atomicMax(&top, min(most, kScanMax));
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
         a.scan_tmp[2 * blockIdx.x] = total;
-        a.scan_tmp[2 * blockIdx.x + 1] = occ;
+        a.scan_tmp[2 * blockIdx.x + 1] = occ | top << 11;
     }
 }
 
-// One workgroup per grid: its blocks' sums in place, its occupied cells.
+// One workgroup per grid: its blocks' sums in place, its occupied cells and the
+// largest count of one.
 __global__ __launch_bounds__(1024) void k_scan_sums(GridBuildArgs a, uint32_t nb0, uint32_t nb1)
 {
-    __shared__ uint32_t sh[16], occ;
+    __shared__ uint32_t sh[16], occ, top;
     const uint32_t first = blockIdx.x ? nb0 : 0u, nb = blockIdx.x ? nb1 : nb0;
-    uint32_t carry = 0, cells = 0;
-    if (threadIdx.x == 0) occ = 0;
+    uint32_t carry = 0, cells = 0, most = 0;
+    if (threadIdx.x == 0) occ = top = 0;
     for (uint32_t base = 0; base < nb; base += 1024) {
         const uint32_t i = base + threadIdx.x;
         uint2 *p = (uint2 *)a.scan_tmp + first + i;
         const uint2 v = i < nb ? *p : make_uint2(0u, 0u);
-        cells += v.y;
+        cells += v.y & 2047u;
+        most = max(most, v.y >> 11);
         uint32_t total;
         const uint32_t ex = block_excl_scan(v.x, sh, total);
         if (i < nb) p->x = ex + carry;
         carry += total;
     }
-    for (int off = 32; off > 0; off >>= 1) cells += __shfl_xor(cells, off, 64);
-    if ((threadIdx.x & 63) == 0) atomicAdd(&occ, cells);
+    for (int off = 32; off > 0; off >>= 1) {
+        cells += __shfl_xor(cells, off, 64);
+        most = max(most, (uint32_t)__shfl_xor(most, off, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        atomicAdd(&occ, cells);
+        atomicMax(&top, most);
+    }
     __syncthreads();
-    if (threadIdx.x == 0) a.occupied[blockIdx.x] = occ;
+    if (threadIdx.x == 0) {
+        a.occupied[2 * blockIdx.x] = occ;
+        a.occupied[2 * blockIdx.x + 1] = top;
+    }
 }
 
 __global__ __launch_bounds__(kThreads) void k_scan_add(GridBuildArgs a, uint32_t nb0)

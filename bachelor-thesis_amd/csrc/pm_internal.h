@@ -119,7 +119,7 @@ struct GridBuildArgs {
     float4 *sorted, *fsorted;             // n
     uint32_t *cell_start, *fcell_start;   // ncells + 1, fncells + 1
     uint32_t *scan_tmp;    // scan_tmp_size of both grids
-    uint32_t *occupied;    // [2]: search and march cells that hold a particle
+    uint32_t *occupied;    // [4]: search cells that hold a particle, the most in one; march cells, the most in one
 };
 size_t scan_tmp_size(uint32_t ncells, uint32_t fncells);
 hipError_t launch_grid_build(const GridBuildArgs &a, hipStream_t st);
@@ -129,6 +129,9 @@ hipError_t launch_grid_build(const GridBuildArgs &a, hipStream_t st);
 inline size_t tile_words(uint64_t T) { return (size_t)(((T + 2) & ~1ull) + 2 * ((T + 63) / 64)); }
 hipError_t launch_tile_prepass(const MarchLaunch &L, hipStream_t st);
 hipError_t launch_march(const MarchLaunch &L, hipStream_t st);
+// GridDev::group_hits of a frame of n particles in `cells` march cells, at most
+// `most` in one.
+uint32_t group_hits(uint64_t n, uint32_t cells, uint32_t most);
 // The anisotropic march (configured or reference mode), one kernel.
 hipError_t launch_march_aniso(const MarchLaunch &L, hipStream_t st);
 hipError_t launch_density_aniso(const GridDev &g, const AnParF &a, const float *q, uint32_t nq, int compensated,

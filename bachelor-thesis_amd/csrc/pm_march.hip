@@ -521,7 +521,6 @@ __device__ __forceinline__ void finish_hit(const MarchLaunch &L, uint32_t px, ui
     L.pos[idx] = make_float4(xs[0], xs[1], xs[2], 1.0f);
     L.nrm[idx] = make_float4(nx, ny, nz, 1.0f);
     if (L.t) L.t[idx] = th;
-    cn.hits++;
 }
 
 // One 8x8 tile per wave, one pixel per lane: the lanes whose pixel holds a
@@ -770,6 +769,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     if (any) flush_counts(B.base.counters, cn);
 }
 
+// The hits of the launch, counted by its march.
+__device__ __forceinline__ uint32_t marched_hits(const MarchLaunch &L)
+{
+    unsigned long long n = 0;
+#pragma unroll
+    for (int k = 0; k < kCtrSlots; k++) n += L.counters[k * kCtrStride + C_HITS];
+    return (uint32_t)n;                           // at most 2^30 pixels
+}
+
 // A wave per active tile, of the view or of the batch.
 // LIST: a hit's samples share one candidate list.  It pays where the lists fit
 // (GridDev::sparse, at most 3 particles per occupied h/2 cell: 466 -> 223 us on
@@ -778,11 +786,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
 // for each sample, 5.3 to 7.0 ms with lists of 44 to 92 slots), so those walk.
 // (Since then the weights take fewer instructions and the statistics count every
 // sample's own stencil: 254 us and 3.1 ms.)
-// Registers are capped for four waves per SIMD.
+// Registers are capped for four waves per SIMD (three with lists).
+// beyond: nothing is done for launches of at most so many hits (k_finish_groups
+// takes them).
 template <bool BATCH, bool INSTR, bool LIST>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LIST ? 3 : 4, 8))) void k_finish(MarchLaunch L0, const MarchLaunch *__restrict__ jobs,
-                                                const BatchTile *__restrict__ tiles, uint32_t ntiles)
+                                                const BatchTile *__restrict__ tiles, uint32_t ntiles, uint32_t beyond)
 {
+    if (beyond != 0 && marched_hits(L0) <= beyond) return;
     __shared__ uint32_t lds[LIST ? kFinWords : kListWords];
     uint32_t *lst = lds + threadIdx.x;
     Counts cn;
@@ -812,17 +823,32 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LIST ? 3 : 4
 // rounds instead of seven (ten samples), the six central differences two, and a tile's hits
 // are spread over four waves.  It does more work in all (ten samples for
 // seven, the FP64 sample by one lane of four), so it gains where a hit's own
-// serial chain bounds the launch and loses once the waves fill the chip.  The
-// image's tiles are known here, its hits are not, so each line lies where an
-// image full of hits still gains:
-// - a sparse frame (k_finish with a list otherwise): 96x64 lattice 87 -> 59 us;
+// serial chain bounds the launch and loses once the waves fill the chip:
+// - a sparse frame (k_finish with a list otherwise): the line lies where an image
+//   full of hits still gains.  96x64 lattice 87 -> 59 us;
 //   256x192 (768 tiles) dam 131 -> 86, full lattice 94 -> 71; 288x224 (1008) dam
 //   134 -> 85 but full lattice 96 -> 110, 360x360 (2025) 115 -> 195;
-// - a dense frame, where one hit's walks take milliseconds: 96x64 pool of
-//   400,000 1698 -> 898 us, 800x600 (7500) 2400 -> 905; 1,000,000 at 1280x720
-//   (14400) 3482 -> 1518; 1920x1080 (32400) 1837 -> 2080 at 400,000 and
-//   2996 -> 2310 at 1,000,000; 4,000,000 at 3840x2160 3513 -> 7682.
-static constexpr uint32_t kGroupTiles = 800, kGroupTilesDense = 16384;
+// - a dense frame, where one hit's walks take milliseconds: the chip's 4,096 waves
+//   hold 65,536 hits of four lanes; in an uneven frame (most: the fullest h/2 cell
+//   over the mean) groups gain beyond that, its longest hits outlasting the
+//   others.  March and finish, k_finish -> groups:
+//     3.3 per cell, most 3.3: 41,000 hits 935 -> 630 us, 55,000 970 -> 966, 62,000
+//     997 -> 1027, 86,000 1084 -> 1230, 147,000 1369 -> 1748, 829,000 4057 -> 6609;
+//     pools of 5.5 to 6.2 per cell: most 5.9, 86,000 hits 1391 -> 1230, 104,000
+//     1054 -> 1256; 9.2, 78,000 1602 -> 1237, 164,000 2019 -> 2223; 19, 164,000
+//     2384 -> 2078 and 1663 -> 2012 (nearer); 17, 164,000 3763 -> 2420, 243,000 1694
+//     -> 2453.
+//   (By the image's tiles alone, up to 16,384, groups took images full of hits too:
+//   4889 us at 1280x800, k_finish 2348.)
+//   The march has counted the hits by then, so both kernels are launched where
+//   the tiles could hold more, and one of them ends at once.
+static constexpr uint32_t kGroupTiles = 800, kGroupTilesDense = 16384, kGroupHits = 65536;
+
+uint32_t group_hits(uint64_t n, uint32_t cells, uint32_t most)
+{
+    const double over = (double)most * (double)cells / (double)n;
+    return (uint32_t)fmin(kGroupHits * (1.0 + over / 8.0), 0x1p30);
+}
 
 // FP32 density of one of a hit's samples from the hit's list, or by its own walk.
 struct FinishDens {
@@ -847,9 +873,11 @@ struct FinishDens {
     }
 };
 
+// upto: nothing is done for launches of more hits (k_finish takes them).
 template <bool LIST>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_finish_groups(MarchLaunch L)
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_finish_groups(MarchLaunch L, uint32_t upto)
 {
+    if (upto != 0 && marched_hits(L) > upto) return;
     __shared__ uint32_t lds[kFinWords];
     const uint32_t lane = threadIdx.x;
     uint32_t *lst = lds + lane;
@@ -924,7 +952,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void
             L.pos[idx] = make_float4(xs[0], xs[1], xs[2], 1.0f);
             L.nrm[idx] = make_float4(nx, ny, nz, 1.0f);
             if (L.t) L.t[idx] = th;
-            cn.hits++;
         }
     }
     if (any) flush_counters(L.counters, cn.rays, cn.in_aabb, cn.hits, cn.samples, cn.cand, cn.march);
@@ -935,13 +962,16 @@ static hipError_t launch_finish(const MarchLaunch &L0, hipStream_t st)
     const uint32_t T = ((L0.W + 7) / 8) * ((L0.H + 7) / 8);
     const uint32_t need = tile_waves_of(T);
     const dim3 grid(need < kMaxWaves ? need : kMaxWaves), blk(64);
+    uint32_t upto = 0;
     if (T < (L0.g.sparse ? kGroupTiles : kGroupTilesDense) && !L0.s.instrument) {
-        hipLaunchKernelGGL(L0.g.sparse ? k_finish_groups<true> : k_finish_groups<false>, dim3(tile_waves_of(T << 2)), blk, 0, st, L0);
-        return hipGetLastError();
+        if (!L0.g.sparse && (uint64_t)T * 64 > L0.g.group_hits) upto = L0.g.group_hits;
+        hipLaunchKernelGGL(L0.g.sparse ? k_finish_groups<true> : k_finish_groups<false>, dim3(tile_waves_of(T << 2)), blk, 0, st, L0, upto);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess || upto == 0) return e;
     }
-    if (L0.s.instrument) hipLaunchKernelGGL((k_finish<false, true, true>), grid, blk, 0, st, L0, nullptr, nullptr, 0u);
-    else if (L0.g.sparse) hipLaunchKernelGGL((k_finish<false, false, true>), grid, blk, 0, st, L0, nullptr, nullptr, 0u);
-    else hipLaunchKernelGGL((k_finish<false, false, false>), grid, blk, 0, st, L0, nullptr, nullptr, 0u);
+    if (L0.s.instrument) hipLaunchKernelGGL((k_finish<false, true, true>), grid, blk, 0, st, L0, nullptr, nullptr, 0u, 0u);
+    else if (L0.g.sparse) hipLaunchKernelGGL((k_finish<false, false, true>), grid, blk, 0, st, L0, nullptr, nullptr, 0u, 0u);
+    else hipLaunchKernelGGL((k_finish<false, false, false>), grid, blk, 0, st, L0, nullptr, nullptr, 0u, upto);
     return hipGetLastError();
 }
 
@@ -956,8 +986,8 @@ hipError_t launch_march_batch(const BatchLaunch &B, hipStream_t st)
     if (e != hipSuccess) return e;
     const uint32_t nf = tile_waves_of(B.ntiles);
     const dim3 fgrid(nf < kMaxWaves ? nf : kMaxWaves);
-    if (B.sparse) hipLaunchKernelGGL((k_finish<true, false, true>), fgrid, blk, 0, st, B.base, B.jobs, B.tiles, B.ntiles);
-    else hipLaunchKernelGGL((k_finish<true, false, false>), fgrid, blk, 0, st, B.base, B.jobs, B.tiles, B.ntiles);
+    if (B.sparse) hipLaunchKernelGGL((k_finish<true, false, true>), fgrid, blk, 0, st, B.base, B.jobs, B.tiles, B.ntiles, 0u);
+    else hipLaunchKernelGGL((k_finish<true, false, false>), fgrid, blk, 0, st, B.base, B.jobs, B.tiles, B.ntiles, 0u);
     return hipGetLastError();
 }
 

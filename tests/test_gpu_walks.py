@@ -215,3 +215,38 @@ def test_candidates_of_wide_offsets(marcher, tiles, eps):
     marcher.set_frame(60, sc.xyz, sc.h)
     got = _check(marcher, sc, counters=COUNTERS + ("cand",), skip_mode=1)
     assert got["hits"] > 1000
+
+
+@pytest.mark.parametrize("extra,dist,groups", [(0, 2.6, 1), (0, 1.4, 1), (0, 1.3, 0), (0, 0.7, 0), (60, 1.1, 1), (60, 0.7, 0)])
+@pytest.mark.parametrize("learned", [0, 1])
+def test_group_finish_by_hits(marcher, extra, dist, groups, learned):
+    """The finish of a dense frame in an image of 4,800 tiles: four lanes per hit
+    up to 65,536 (1 + most / (8 mean)) hits, most the fullest h/2 cell's particles
+    (73,728 here, and about 171,000 with `extra` in one cell), a lane per hit
+    beyond, chosen on the device; images and counters are those of the
+    one-ray-per-lane schedule."""
+    from pmarch import train
+    rng = np.random.default_rng(12)
+    h = 0.1
+    base = np.stack(np.meshgrid(*[np.arange(14)] * 3, indexing="ij"), -1).reshape(-1, 1, 3) * (h / 2)
+    xyz = (base + rng.uniform(0, h / 2, (base.shape[0], 5, 3))).reshape(-1, 3)
+    xyz = np.concatenate([xyz, h * (7 + rng.uniform(0.01, 0.49, (extra, 3)))]).astype(np.float32)
+    mid = np.full(3, 0.35)
+    d = np.array([0.7, 0.6, -0.4]) / np.linalg.norm([0.7, 0.6, -0.4])
+    sc = scenes.tiny_scene(xyz, h, eye=mid + dist * d, target=mid, width=640, height=480)
+    sc.iso *= 5
+    c = sc.cameras[0]
+    print(f"group finish by hits, {extra} in a cell, distance {dist} learned {learned}", flush=True)
+    if learned:
+        marcher.mlp_set(train.load()[0])
+    marcher.set_frame(60, sc.xyz, sc.h)
+    st = sc.settings(skip_mode=4)
+    plain = marcher.march(60, dict(st, schedule=1), c.inv_pv, c.eye, c.width, c.height)
+    for _ in range(2):
+        got = marcher.march(60, dict(st, learned=learned), c.inv_pv, c.eye, c.width, c.height)
+        for a, b in zip(got[:3], plain[:3]):
+            assert np.array_equal(a, b)
+        for k in ("rays", "rays_in_aabb", "hits") + (() if learned else ("samples", "march_samples")):
+            assert got[3][k] == plain[3][k], k
+        most = 65536 * (1 + (5 + extra) / 40)
+        assert (got[3]["hits"] < 0.97 * most if groups else got[3]["hits"] > 1.03 * most) and got[3]["hits"] > 15000
