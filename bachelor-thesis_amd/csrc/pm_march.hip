@@ -830,24 +830,24 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LIST ? 3 : 4
 //   134 -> 85 but full lattice 96 -> 110, 360x360 (2025) 115 -> 195;
 // - a dense frame, where one hit's walks take milliseconds: the chip's 4,096 waves
 //   hold 65,536 hits of four lanes; in an uneven frame (most: the fullest h/2 cell
-//   over the mean) groups gain beyond that, its longest hits outlasting the
-//   others.  March and finish, k_finish -> groups:
+//   over the mean) groups gain up to four times as many, its longest hits
+//   outlasting the others.  March and finish, k_finish -> groups:
 //     3.3 per cell, most 3.3: 41,000 hits 935 -> 630 us, 55,000 970 -> 966, 62,000
 //     997 -> 1027, 86,000 1084 -> 1230, 147,000 1369 -> 1748, 829,000 4057 -> 6609;
 //     pools of 5.5 to 6.2 per cell: most 5.9, 86,000 hits 1391 -> 1230, 104,000
 //     1054 -> 1256; 9.2, 78,000 1602 -> 1237, 164,000 2019 -> 2223; 19, 164,000
-//     2384 -> 2078 and 1663 -> 2012 (nearer); 17, 164,000 3763 -> 2420, 243,000 1694
-//     -> 2453.
+//     2384 -> 2078 and 1663 -> 2012 (nearer); 17, 164,000 3763 -> 2420, 197,000 3165
+//     -> 2500, 243,000 1694 -> 2453 (nearer).
 //   (By the image's tiles alone, up to 16,384, groups took images full of hits too:
-//   4889 us at 1280x800, k_finish 2348.)
+//   the 100,000-particle pool 4889 us at 1280x800, k_finish 2348.)
 //   The march has counted the hits by then, so both kernels are launched where
 //   the tiles could hold more, and one of them ends at once.
 static constexpr uint32_t kGroupTiles = 800, kGroupTilesDense = 16384, kGroupHits = 65536;
 
 uint32_t group_hits(uint64_t n, uint32_t cells, uint32_t most)
 {
-    const double over = (double)most * (double)cells / (double)n;
-    return (uint32_t)fmin(kGroupHits * (1.0 + over / 8.0), 0x1p30);
+    const double over = (double)most * (double)cells / (double)n / 8.0;
+    return (uint32_t)(kGroupHits * (1.0 + fmin(over * over, 3.0)));
 }
 
 // FP32 density of one of a hit's samples from the hit's list, or by its own walk.
