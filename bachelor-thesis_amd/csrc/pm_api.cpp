@@ -425,7 +425,7 @@ static int build_frame(pm_ctx *c, int32_t frame, const float *d_src, uint64_t n,
     uint32_t occupied[4] = { 0, 0, 0, 0 };
     HIPCHK(c, hipMemcpyAsync(occupied, a.occupied, sizeof(occupied), hipMemcpyDeviceToHost, st));
     HIPCHK(c, hipStreamSynchronize(st));
-    g.sparse = n <= (uint64_t)kSparsePerCell * occupied[2];
+    g.sparse = 10 * n <= (uint64_t)kSparsePerTen * occupied[2];
     g.group_hits = group_hits(n, occupied[2], occupied[3]);
     float ms = 0.f;
     hipEventElapsedTime(&ms, ev.e[0], ev.e[1]);

@@ -42,10 +42,10 @@ struct GridDev {
     int32_t fox, foy, foz;    // fine key of fine cell (0,0,0)
     int32_t fnx, fny, fnz;
     float inv_hf;             // 2 / h
-    int sparse;               // at most kSparsePerCell particles per occupied fine cell on average
+    int sparse;               // at most kSparsePerTen particles per ten occupied fine cells on average
     uint32_t group_hits;      // most hits whose finish takes four lanes each (dense frames, pm_march.hip)
 };
-static constexpr uint32_t kSparsePerCell = 3;
+static constexpr uint32_t kSparsePerTen = 21;
 
 // ---- march-grid stencil ----
 // In fine-cell units u = inv_hf x the sample sits at offset f in [0, 1] inside

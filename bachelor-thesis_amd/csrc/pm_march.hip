@@ -780,12 +780,15 @@ __device__ __forceinline__ uint32_t marched_hits(const MarchLaunch &L)
 
 // A wave per active tile, of the view or of the batch.
 // LIST: a hit's samples share one candidate list.  It pays where the lists fit
-// (GridDev::sparse, at most 3 particles per occupied h/2 cell: 466 -> 223 us on
-// the 1 M dam break, 1.4 per cell); in denser frames (4 M pool, 8 per cell) most
-// lists overflow after they were built and their LDS costs waves (3.6 ms walking
-// for each sample, 5.3 to 7.0 ms with lists of 44 to 92 slots), so those walk.
-// (Since then the weights take fewer instructions and the statistics count every
-// sample's own stencil: 254 us and 3.1 ms.)
+// (GridDev::sparse, at most 2.1 particles per occupied h/2 cell); in denser frames
+// most lists overflow after they were built, and their LDS costs waves, so those
+// walk for each sample.  March and finish at 1920x1080, walk -> list, lattices of
+// 524,288 with Gaussian jitter: 1.4 per cell 846 -> 681 us, 1.8 1138 -> 992, 2.0
+// 1242 -> 1184 (at 3840x2160 2937 -> 2644), 2.04 1298 -> 1314 (an image full of hits
+// 3730 -> 3657), 2.13 1417 -> 1450 (3896 -> 3939), 2.3 1453 -> 1638, 2.9 1740 -> 2005.
+// The finish of the 1 M dam break, 1.4 per cell: 466 -> 223 us (now 254: the
+// statistics count every sample's own stencil); of the 4 M pool, 8 per cell: 3.1 ms
+// walking, 5.3 to 7.0 with lists of 44 to 92 slots.
 // Registers are capped for four waves per SIMD (three with lists).
 // beyond: nothing is done for launches of at most so many hits (k_finish_groups
 // takes them).
