@@ -658,6 +658,15 @@ static bool device_range(int device, const void *p, size_t bytes)
     return (const char *)p + bytes <= (const char *)base + size;
 }
 
+// True for host memory HIP does not know: a copy into it is staged by HIP, where
+// pinned memory takes the DMA engines' copy itself.
+static bool pageable(const void *p)
+{
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) { (void)hipGetLastError(); return true; }
+    return a.type == hipMemoryTypeUnregistered;
+}
+
 // The march of one view.  dev != nullptr: the outputs go straight into the
 // caller's device memory dev[0..2] (t may be null) and depth_in is device
 // memory; otherwise into the context's buffers, copied to the host pointers
@@ -1162,9 +1171,14 @@ int pm_batch_download(pm_ctx *c, uint32_t view, float *positions, float *normals
     const void *const src[3] = { pos + o, nrm + o, tt + o };
     const size_t bytes[3] = { 16 * n, 16 * n, 4 * n };
     size_t need = 0;
-    for (int k = 0; k < 3; k++) need += dst[k] ? bytes[k] : 0;
-    // one wait and a shared copy; small views and those beyond 64 MB of staging copy image by image
-    if (need >= kCopyShared && need <= (64u << 20) && ensure_stage(c, need) == hipSuccess) {
+    bool staged = true;
+    for (int k = 0; k < 3; k++) {
+        need += dst[k] ? bytes[k] : 0;
+        staged = staged && (!dst[k] || pageable(dst[k]));
+    }
+    // one wait and a shared copy; small views, those beyond 64 MB of staging and
+    // images into pinned memory are copied image by image
+    if (staged && need >= kCopyShared && need <= (64u << 20) && ensure_stage(c, need) == hipSuccess) {
         CopyPool::Range r[3];
         int nr = 0;
         char *p = (char *)c->h_stage;

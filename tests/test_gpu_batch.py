@@ -120,3 +120,45 @@ def test_batch_rejects_bad_views(marcher):
         marcher.batch_set(sc.settings(), [(fids[0], 0, 64, np.eye(4), np.zeros(3))])
     with pytest.raises(pmarch.PmError):
         marcher.batch_set(sc.settings(mode=1), [(fids[0], 64, 64, np.eye(4), np.zeros(3))])
+
+
+def test_batch_download_into_pinned_memory():
+    """Views into memory the caller pinned are copied there directly: no staging,
+    so the shared copy's workers are not started; one pageable image among them
+    is copied too."""
+    import ctypes
+    import os
+
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def pin(shape):
+        p = ctypes.c_void_p()
+        assert hip.hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(4 * int(np.prod(shape))), 0) == 0
+        return np.ctypeslib.as_array(ctypes.cast(p, ctypes.POINTER(ctypes.c_float)), shape)
+
+    print("batch download into pinned memory", flush=True)
+    m = pmarch.Marcher(0)
+    sc = scenes.lattice_cube(4, n_side=10, spacing=0.05, width=640, height=480)
+    c = sc.cameras[0]
+    m.set_frame(0, sc.xyz, sc.h)
+    st = sc.settings(skip_mode=4)
+    m.batch_set(st, [(0, c.width, c.height, c.inv_pv, c.eye), (0, 16, 8, c.inv_pv, c.eye)])
+    m.batch_run()
+    m.wait()
+    shapes = [(c.height, c.width, 4), (c.height, c.width, 4), (c.height, c.width)]
+    pinned, other = [pin(s) for s in shapes], [pin(s) for s in shapes]
+    small = [pin((8, 16, 4)), pin((8, 16, 4)), pin((8, 16))]
+    assert m.L.pm_batch_download(m.ctx, 1, *(p.ctypes.data for p in small)) == 0
+    before = len(os.listdir("/proc/self/task"))
+    for _ in range(2):
+        assert m.L.pm_batch_download(m.ctx, 0, *(p.ctypes.data for p in pinned)) == 0
+    assert len(os.listdir("/proc/self/task")) == before
+    plain = m.batch_download(0)
+    other[1] = np.zeros(shapes[1], np.float32)
+    assert m.L.pm_batch_download(m.ctx, 0, *(p.ctypes.data for p in other)) == 0
+    for a, b, want in zip(pinned, other, plain):
+        assert np.array_equal(a, want) and np.array_equal(b, want)
+    assert (plain[0][..., 3] > 0).sum() > 1000
+    for p in pinned + [other[0], other[2]] + small:
+        assert hip.hipHostFree(ctypes.c_void_p(p.ctypes.data)) == 0
+    m.close()
