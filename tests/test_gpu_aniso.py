@@ -203,3 +203,35 @@ def test_aniso_degenerate_neighbourhoods(marcher, case):
             assert np.array_equal(Gg[i], Go, equal_nan=True) and np.array_equal(dg[i], np.float32(do), equal_nan=True)
     assert np.array_equal(marcher.density_aniso(6, st, q), G.density_aniso(s, q), equal_nan=True)
     _march_pair(marcher, 6, sc, st, sc.cameras[0], 1)
+
+
+@pytest.mark.parametrize("iso", [100.0, 200.0, 300.0])
+@pytest.mark.parametrize("normal_mode", [0, 1])
+def test_march_aniso_capped_lists(marcher, iso, normal_mode):
+    """Waves some of whose samples have more than 8192 extended neighbours (the
+    cut of the list walk, and the direct walk for the whole wave) and some fewer:
+    the march, the reference march and their normals equal the oracle's."""
+    from parity import depth_in_front
+    rng = np.random.default_rng(5)
+    n = 11000
+    v = rng.normal(size=(n, 3))
+    v = v / np.linalg.norm(v, axis=1)[:, None] * rng.uniform(0, 1, (n, 1)) ** (1 / 3) * 0.13
+    xyz = (0.5 + v).astype(np.float32)
+    sc = scenes.tiny_scene(xyz, 0.1, eye=(1.0, 0.8, 0.1), target=(0.5, 0.5, 0.5), width=41, height=27)
+    c = sc.cameras[0]
+    print(f"aniso march capped lists iso {iso} normals {normal_mode}", flush=True)
+    marcher.set_frame(2, sc.xyz, sc.h)
+    G = O.Grid(sc.xyz, sc.h)
+    st = scenes.aniso_settings(sc, iso=iso, normal_mode=normal_mode, skip_mode=1)
+    ref = dict(mode=1, max_steps=60, step=0.006, normal_mode=normal_mode, normal_eps=sc.normal_eps, skip_mode=2,
+               compensated=0, iso=iso, **scenes.ANISO_SETTINGS)
+    near = []
+    for s, depth in ((st, None), (ref, depth_in_front(c, G.bmin, G.bmax, 0.01).astype(np.float32))):
+        pos, nrm, t, got = marcher.march(2, s, c.inv_pv, c.eye, c.width, c.height, depth=depth)
+        o = O.march(G, O.make_settings(**s), c.inv_pv, c.eye, c.width, c.height, depth=depth)
+        assert np.array_equal(pos, o[0]) and np.array_equal(t, o[2])
+        assert np.array_equal(nrm, o[1], equal_nan=True)
+        for k in ("hits", "samples", "march_samples"):
+            assert got[k] == o[3][k], (k, got[k], o[3][k])
+        near += [int((np.linalg.norm(xyz - p[:3], axis=1) < 0.2).sum()) for p in pos[pos[..., 3] > 0]]
+    assert min(near) < 8192 < max(near)

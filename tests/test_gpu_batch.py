@@ -162,3 +162,37 @@ def test_batch_download_into_pinned_memory():
     for p in pinned + [other[0], other[2]] + small:
         assert hip.hipHostFree(ctypes.c_void_p(p.ctypes.data)) == 0
     m.close()
+
+
+@pytest.mark.parametrize("dense", [(0, 1), (1, 1), (0, 0)])
+@pytest.mark.parametrize("use_graph", [False, True])
+def test_batch_of_dense_frames(marcher, dense, use_graph):
+    """A batch over sparse and dense frames (1 and 12 particles per h/2 cell): one
+    dense frame among them and all hits walk for each sample, none and they share
+    lists; each view equals the oracle's."""
+    rng = np.random.default_rng(3)
+    h = 0.1
+    base = np.stack(np.meshgrid(*[np.arange(8)] * 3, indexing="ij"), -1).reshape(-1, 1, 3) * (h / 2)
+    print(f"batch of dense frames {dense} graph {use_graph}", flush=True)
+    views, want = [], []
+    st = None
+    for f, d in enumerate(dense):
+        per = 12 if d else 1
+        xyz = (base + rng.uniform(0, h / 2, (base.shape[0], per, 3))).reshape(-1, 3).astype(np.float32)
+        sc = scenes.tiny_scene(xyz, h, eye=(0.9, 0.8, -0.7), target=(0.2, 0.2, 0.2), width=71, height=50)
+        st = st or sc.settings(skip_mode=4)
+        marcher.set_frame(60 + f, sc.xyz, sc.h)
+        G, c = O.Grid(sc.xyz, sc.h), sc.cameras[0]
+        views.append((60 + f, c.width, c.height, c.inv_pv, c.eye))
+        want.append(O.march(G, O.make_settings(**st), c.inv_pv, c.eye, c.width, c.height))
+    marcher.batch_set(st, views, use_graph=use_graph)
+    for _ in range(3):
+        marcher.batch_run()
+        marcher.wait()
+        for v, o in enumerate(want):
+            for a, b in zip(marcher.batch_download(v), o[:3]):
+                assert np.array_equal(a, b.reshape(a.shape)), v
+        got = marcher.stats()
+        for k in ("rays", "hits", "samples", "march_samples"):
+            assert got[k] == sum(o[3][k] for o in want), k
+    assert any(o[3]["hits"] > 200 for o in want)
