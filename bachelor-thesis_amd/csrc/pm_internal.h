@@ -125,8 +125,13 @@ size_t scan_tmp_size(uint32_t ncells, uint32_t fncells);
 hipError_t launch_grid_build(const GridBuildArgs &a, hipStream_t st);
 
 // The tile pre-pass (L.tile_buf set): the list of the active tiles and the misses
-// of the others.
-inline size_t tile_words(uint64_t T) { return (size_t)(((T + 2) & ~1ull) + 2 * ((T + 63) / 64)); }
+// of the others.  Its words: the list, one 64-bit mask per 64 tiles, one sum per 64
+// masks.
+inline size_t tile_words(uint64_t T)
+{
+    const uint64_t masks = (T + 63) / 64;
+    return (size_t)(((T + 2) & ~1ull) + 2 * masks + (masks + 63) / 64);
+}
 hipError_t launch_tile_prepass(const MarchLaunch &L, hipStream_t st);
 hipError_t launch_march(const MarchLaunch &L, hipStream_t st);
 // GridDev::group_hits of a frame of n particles in `cells` march cells, at most

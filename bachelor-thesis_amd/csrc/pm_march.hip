@@ -66,7 +66,10 @@ __device__ __forceinline__ bool tile_ray_active(const MarchLaunch &L, uint32_t p
 // others: tile_buf[0, count) the tiles, tile_buf[T] = count, then (64-bit
 // aligned) one mask of active tiles per 64.  The first takes 64 tiles per
 // workgroup, four per wave; the second adds up the masks before its own, which
-// at these sizes (507 masks at 1080p) is cheaper than a scan's launches.  Bound
+// at these sizes (507 masks at 1080p) is cheaper than a scan's launches.  Beyond
+// kSumMasks masks a launch between them sums the masks 64 at a time, and the
+// second adds up those (32768x16384, nothing hit: 8.1 ms without, 4.5 with; 7680x4320,
+// 8,100 masks: 353 and 323 us).  Bound
 // by the miss writes (36 B per ray).  (Flags, a three-launch scan, a compaction
 // and the misses were six launches: 45 us at 1080p, 17 at 96x64.  One launch
 // that appended each workgroup's tiles with an atomic saved 3 us more but lost
@@ -99,12 +102,33 @@ __global__ __launch_bounds__(1024) void k_tile_masks(MarchLaunch L, uint32_t T)
     }
 }
 
-__global__ __launch_bounds__(64) void k_tile_list(MarchLaunch L, uint32_t T)
+static constexpr uint32_t kSumMasks = 4096;
+__device__ __forceinline__ uint32_t *mask_sums(const MarchLaunch &L, uint32_t T)
+{
+    return (uint32_t *)(tile_masks(L, T) + (T + 63) / 64);
+}
+
+// The active tiles of 64 masks, a wave each.
+__global__ __launch_bounds__(64) void k_mask_sums(MarchLaunch L, uint32_t T)
+{
+    const uint32_t i = blockIdx.x * 64 + threadIdx.x;
+    uint32_t n = i < (T + 63) / 64 ? (uint32_t)__popcll(tile_masks(L, T)[i]) : 0u;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+    if (threadIdx.x == 0) mask_sums(L, T)[blockIdx.x] = n;
+}
+
+// summed: k_mask_sums ran.
+__global__ __launch_bounds__(64) void k_tile_list(MarchLaunch L, uint32_t T, int summed)
 {
     const unsigned long long *masks = tile_masks(L, T);
-    const uint32_t b = blockIdx.x, lane = threadIdx.x;
+    const uint32_t b = blockIdx.x, lane = threadIdx.x, first = summed ? b & ~63u : 0u;
     uint32_t before = 0;
-    for (uint32_t i = lane; i < b; i += 64) before += (uint32_t)__popcll(masks[i]);
+    if (summed) {
+        const uint32_t *sums = mask_sums(L, T);
+        for (uint32_t i = lane; i < b / 64; i += 64) before += sums[i];
+    }
+    for (uint32_t i = first + lane; i < b; i += 64) before += (uint32_t)__popcll(masks[i]);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off, 64);
     const unsigned long long m = masks[b];
@@ -1042,7 +1066,9 @@ hipError_t launch_tile_prepass(const MarchLaunch &L, hipStream_t st)
     const uint32_t tiles = ((L.W + 7) / 8) * ((L.H + 7) / 8);
     const uint32_t groups = (tiles + 63) / 64;
     hipLaunchKernelGGL(k_tile_masks, dim3(groups), dim3(1024), 0, st, L, tiles);
-    hipLaunchKernelGGL(k_tile_list, dim3(groups), dim3(64), 0, st, L, tiles);
+    const int summed = groups > kSumMasks;
+    if (summed) hipLaunchKernelGGL(k_mask_sums, dim3((groups + 63) / 64), dim3(64), 0, st, L, tiles);
+    hipLaunchKernelGGL(k_tile_list, dim3(groups), dim3(64), 0, st, L, tiles, summed);
     return hipGetLastError();
 }
 

@@ -3,7 +3,7 @@
 // pm_march_device_noalloc runs the configured isotropic march into the
 // caller's device memory without allocating anything: the buffers the march
 // needs beyond its inputs and outputs -- the per-pixel hit records, the tile
-// pre-pass's flags, scan and list, the counters and the tile-band counters --
+// pre-pass's list and masks, the counters and the tile-band counters --
 // live in one file-scope device array, `scratch`, of kNoAllocScratchBytes.
 // Each GPU holds its own copy of the array for the life of the process.  Its
 // device address is looked up once per device (hipGetSymbolAddress, with that
@@ -12,12 +12,12 @@
 //
 // Layout of the array (offsets in bytes, all 256-aligned):
 //   hit records   PM_NOALLOC_MAX_PIXELS uint4
-//   tile buffer   3 (T + 1) + scan scratch u32, T <= kNoAllocMaxTiles
+//   tile buffer   tile_words(T) u32, T <= kNoAllocMaxTiles
 //   counters      kCtrWords u64
 //   band counters 64 u32
 // Every field is rewritten by the launch before it is read (records and tile
-// lists by the kernels that produce them, the counters and band counters by
-// fill kernels at the start of the launch), so contents left by an earlier
+// lists by the kernels that produce them, the counters by the tile pre-pass, the
+// band counters not at all in this march), so contents left by an earlier
 // call do not matter.  Calls on one GPU share the array: two marches that
 // overlap on one GPU (two contexts or two threads) race.
 #include <mutex>
@@ -30,7 +30,7 @@ namespace pm {
 // ceil(W/8) ceil(H/8) <= W H / 64 + (W + H) / 8 + 1 < 36864.
 constexpr uint32_t kNoAllocMaxTiles = 36864;
 constexpr size_t kNoAllocHitBytes = sizeof(uint4) * (size_t)PM_NOALLOC_MAX_PIXELS;
-constexpr size_t kNoAllocTileWords = kNoAllocMaxTiles + 2 + 2 * (kNoAllocMaxTiles / 64 + 1);
+constexpr size_t kNoAllocTileWords = kNoAllocMaxTiles + 2 + 2 * (kNoAllocMaxTiles / 64 + 1) + kNoAllocMaxTiles / 4096 + 1;
 constexpr size_t kNoAllocTileOff = kNoAllocHitBytes;
 constexpr size_t kNoAllocCtrOff = kNoAllocTileOff + ((sizeof(uint32_t) * kNoAllocTileWords + 255) & ~(size_t)255);
 constexpr size_t kNoAllocBandOff = kNoAllocCtrOff + sizeof(unsigned long long) * kCtrWords;

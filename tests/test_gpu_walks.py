@@ -250,3 +250,22 @@ def test_group_finish_by_hits(marcher, extra, dist, groups, learned):
             assert got[3][k] == plain[3][k], k
         most = 237000 if extra else 66560
         assert (got[3]["hits"] < 0.97 * most if groups else got[3]["hits"] > 1.03 * most) and got[3]["hits"] > 15000
+
+
+@pytest.mark.parametrize("size", [(4096, 4096), (4099, 4096), (4224, 4083)])
+def test_tile_list_of_large_images(marcher, size):
+    """4,096 masks of 64 tiles, from which on they are summed in a launch of their
+    own, a few more, and 4,216 (not a multiple of 64): images and counters are
+    those of the one-ray-per-lane schedule."""
+    sc = scenes.lattice_cube(3, n_side=7, spacing=0.05, width=size[0], height=size[1])
+    c = sc.cameras[0]
+    print(f"tile list of {size}", flush=True)
+    marcher.set_frame(60, sc.xyz, sc.h)
+    st = sc.settings(skip_mode=4, bisect_iters=2)
+    got = marcher.march(60, st, c.inv_pv, c.eye, *size)
+    plain = marcher.march(60, dict(st, schedule=1), c.inv_pv, c.eye, *size)
+    for a, b in zip(got[:3], plain[:3]):
+        assert np.array_equal(a, b)
+    for k in ("rays", "rays_in_aabb", "hits", "samples"):
+        assert got[3][k] == plain[3][k], k
+    assert got[3]["hits"] > 100000
