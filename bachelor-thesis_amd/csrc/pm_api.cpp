@@ -94,8 +94,7 @@ struct pm_ctx {
     DevBuf d_pos, d_nrm, d_t, d_depth, d_counters, d_q, d_out, d_band, d_tiles;
     DevBuf d_hits;                     // per-pixel hit records of one march
     DevBuf d_gauss;                    // the smoothing tables for N = 0..31, written once
-    DevBuf d_sbig;                     // the sprite pass's large-footprint list (count + indices) ...
-    DevBuf d_stile;                    // ... and its tiles' largest depths
+    DevBuf d_stile;                    // the sprite pass's tiles' largest depths
     uint64_t npx = 0;
     bool have_t = false;
     // pinned staging for asynchronous hand-off
@@ -239,7 +238,6 @@ void pm_destroy(pm_ctx *c)
     for (auto &kv : c->frames) { kv.second->release(); delete kv.second; }
     c->d_pos.release(); c->d_nrm.release(); c->d_t.release(); c->d_depth.release();
     c->d_counters.release(); c->d_q.release(); c->d_out.release(); c->d_band.release(); c->d_tiles.release();
-    c->d_sbig.release();
     c->d_stile.release();
     c->d_gauss.release();
     c->d_hits.release();
@@ -1426,27 +1424,23 @@ static int sprites_launch(pm_ctx *c, int32_t frame, const float view[16], const 
         if (!std::isfinite(view[k]) || !std::isfinite(proj[k]) || !std::isfinite(inv_pv[k]))
             return fail(c, PM_ERR_ARG, "pm_depth_sprites: non-finite matrix entry");
     }
-    for (int k = 0; k < 3; k++) S.cam[k] = cam[k];
+    for (int k = 0; k < 3; k++) { S.cam[k] = cam[k]; S.lo[k] = f->info.pmin[k]; S.hi[k] = f->info.pmax[k]; }
     S.radius = radius;
     S.W = W;
     S.H = H;
     HIPCHK(c, hipSetDevice(c->device));
     const uint64_t npx = (uint64_t)W * H;
-    // room to list every particle with a large footprint (a wave then shares its
-    // pixels), and the tiles' depths; a sprite pass still in flight may use the
-    // old ones, so it ends before they grow
-    const size_t big_bytes = sizeof(uint32_t) * (f->info.n + 1);
+    // room for the tiles' depths; a sprite pass still in flight may use the old
+    // ones, so it ends before they grow
     const size_t tile_bytes = sizeof(uint32_t) * (size_t)((W + 7) / 8) * ((H + 7) / 8);
-    if ((c->d_sbig.cap < big_bytes || c->d_stile.cap < tile_bytes) && c->sprites_pending)
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-    HIPCHK(c, c->d_sbig.ensure(big_bytes));
+    if (c->d_stile.cap < tile_bytes && c->sprites_pending) HIPCHK(c, hipStreamSynchronize(c->stream));
     HIPCHK(c, c->d_stile.ensure(tile_bytes));
     if (d_depth) {
         if (!device_range(c->device, d_depth, 4 * npx))
             return fail(c, PM_ERR_ARG, "pm_depth_sprites_device: the image must be device memory of GPU %d, W*H floats",
                         c->device);
         HIPCHK(c, launch_depth_sprites(S, (const float4 *)f->sorted.p, (uint32_t)f->info.n, (uint32_t *)d_depth,
-                                       (uint32_t *)c->d_sbig.p, (uint32_t *)c->d_stile.p, c->stream));
+                                       (uint32_t *)c->d_stile.p, c->stream));
         HIPCHK(c, hipEventRecord(c->ev_sprites, c->stream));
         c->sprites_pending = true;
         c->sprites_frame = frame;
@@ -1454,7 +1448,7 @@ static int sprites_launch(pm_ctx *c, int32_t frame, const float view[16], const 
     }
     HIPCHK(c, c->d_out.ensure(4 * npx));
     HIPCHK(c, launch_depth_sprites(S, (const float4 *)f->sorted.p, (uint32_t)f->info.n, (uint32_t *)c->d_out.p,
-                                   (uint32_t *)c->d_sbig.p, (uint32_t *)c->d_stile.p, c->stream));
+                                   (uint32_t *)c->d_stile.p, c->stream));
     HIPCHK(c, hipMemcpyAsync(depth, c->d_out.p, 4 * npx, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     return PM_OK;

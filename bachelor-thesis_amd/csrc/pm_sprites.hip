@@ -29,7 +29,10 @@
 // (64, 8): 330 us.
 // cos(pi/2 s) is the Taylor polynomial through s^12 (error < 7e-9 on [0, 1]).
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
+
+#include <algorithm>
 
 #include "pm_internal.h"
 
@@ -177,13 +180,25 @@ __device__ __forceinline__ void sp_fragment(const SpriteLaunch &S, const float4 
 }
 
 // Footprints larger than this many pixels (a particle close to the eye: one
-// just past the near plane covers the whole image) are not drawn by their own
-// thread but listed for k_depth_sprites_big, where a wave shares the pixels.
+// just past the near plane covers the whole image), or than 32 tiles, are drawn by
+// the whole wave.
 constexpr uint32_t kSpriteBigPixels = 1024;
 
-// Below this many particles one pass draws them all: their sprites seldom cover
-// each other, and the sample's two launches cost more than the sprites.
-constexpr uint32_t kCullParticles = 4096;
+// When the sample is drawn first (whole passes, without -> with it, launches and
+// all; an estimate of what the particles draw comes from their bounding box):
+// - for many particles: the few of a small sample last as long as they hide
+//   (8,192 footprints of 2,300 pixels 119 -> 172 us, 54,000 of 1,480 419 -> 185);
+// - where footprints lie on each other, kCullOver or more over a pixel (11 over
+//   each: 98 -> 114 us, 15: 68 -> 113, 68: 115 -> 85, 615: 1257 -> 350);
+// - for a pass of some length, kCullPixels or more in all footprints (0.18 M: 44 ->
+//   50 us, 0.56 M: 64 -> 55, 0.63 M: 107 -> 70).
+// A pass has at least kSpriteWaves waves, a particle each if need be: 8,192 of
+// 2,300 pixels 138 us with 4,096 waves, 117 with 8,192; 1,000 of 63 pixels 23 us, 174
+// sixty-four to a wave.  Up to kSampleLanes64 sample sprites of more than 32 pixels
+// are drawn by 64 lanes each (eight lanes: 54,000 of 657 223 us, now 108).
+constexpr uint32_t kCullParticles = 16384;
+constexpr double kCullOver = 30.0, kCullPixels = 5e5;
+constexpr uint32_t kSampleLanes64 = 16384, kSpriteWaves = 8192, kOwnPixels = 64;
 
 // The particle of block t (of kSampleStride consecutive ones) that is drawn
 // first; hashed, so the sample has no period of a lattice's.
@@ -196,10 +211,9 @@ __device__ __forceinline__ uint32_t sp_sample(uint32_t t)
 }
 static_assert((kSampleStride & (kSampleStride - 1)) == 0, "sp_sample takes bits of the hash");
 
-// The footprint of one sprite by kSpriteLanes lanes (j: this one), pixels in
-// row order.
-constexpr uint32_t kSpriteLanes = 8;
-__device__ __forceinline__ void sp_draw(const SpriteLaunch &S, const float4 q, const SpriteBox &B, uint32_t j, uint32_t *depth)
+// The footprint of one sprite by `lanes` lanes (j: this one), pixels in row order.
+__device__ __forceinline__ void sp_draw(const SpriteLaunch &S, const float4 q, const SpriteBox &B, uint32_t j, uint32_t lanes,
+                                        uint32_t *depth)
 {
     const int bw = B.x1 - B.x0 + 1;
     int px = B.x0 + (int)j, py = B.y0;
@@ -207,47 +221,48 @@ __device__ __forceinline__ void sp_draw(const SpriteLaunch &S, const float4 q, c
         while (px > B.x1) { px -= bw; py++; }
         if (py > B.y1) break;
         sp_fragment(S, q, B, px, py, depth);
-        px += (int)kSpriteLanes;
+        px += (int)lanes;
     }
+}
+
+__device__ __forceinline__ uint32_t sp_area(const SpriteBox &B)
+{
+    return (uint32_t)(B.x1 - B.x0 + 1) * (uint32_t)(B.y1 - B.y0 + 1);
 }
 
 __device__ __forceinline__ bool sp_is_big(const SpriteBox &B)
 {
-    const uint32_t area = (uint32_t)(B.x1 - B.x0 + 1) * (uint32_t)(B.y1 - B.y0 + 1);
     const uint32_t tiles = (uint32_t)((B.x1 >> 3) - (B.x0 >> 3) + 1) * (uint32_t)((B.y1 >> 3) - (B.y0 >> 3) + 1);
-    return area > kSpriteBigPixels || tiles > 32u;
+    return sp_area(B) > kSpriteBigPixels || tiles > 32u;
 }
 
-// A sprite with a large footprint goes to the list, which has room for every
-// particle: big[0] counts them, big[1 ..] hold their indices.  The depth is the
-// minimum over all fragments (atomicMin), so who draws a sprite does not change
-// the image.
-__device__ __forceinline__ bool sp_list_big(const SpriteBox &B, uint32_t i, uint32_t *big)
-{
-    if (!sp_is_big(B)) return false;
-    big[1 + atomicAdd(big, 1u)] = i;
-    return true;
-}
-
-// The sample: kSpriteLanes lanes per sprite, so its few sprites fill the chip.
+// The sample: `lanes` lanes (8 or 64) per sprite, so its few sprites fill the chip.
+// Sprites of more than 256 pixels a lane are left to the second pass.
 __global__ __launch_bounds__(256) void k_sprites_sample(SpriteLaunch S, const float4 *__restrict__ pts, uint32_t n,
-                                                        uint32_t *depth)
+                                                        uint32_t lanes, uint32_t *depth)
 {
-    const uint32_t t = (blockIdx.x * 256u + threadIdx.x) / kSpriteLanes, j = threadIdx.x % kSpriteLanes;
+    const uint64_t g = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+    const uint32_t t = (uint32_t)(g / lanes), j = (uint32_t)g & (lanes - 1u);
     const uint32_t i = sp_sample(t);
     if (i >= n) return;
     const float4 q = pts[i];
     SpriteBox B;
     if (!sp_box(S, q, B)) return;
-    if (sp_is_big(B)) return;                                      // left to the second pass
-    sp_draw(S, q, B, j, depth);
+    if (sp_area(B) > 256u * lanes) return;
+    sp_draw(S, q, B, j, lanes, depth);
 }
 
 // All particles, or with tmax what of them is not hidden.  A lane tests one
-// particle against its footprint's tiles; the wave then draws the open
-// (particle, tile) pairs, eight lanes per pair and a row of the tile at a time.
-// (Drawn whole by the testing lane: 740 us; whole by eight lanes each 314 us;
-// with a depth test per pixel ahead of the arithmetic 450 us, a chain of loads.)
+// particle against its footprint's tiles and draws a footprint of at most `own`
+// pixels itself (up to as many as the wave has particles: a lane each then beats
+// eight lanes for one after the other; 1 M of 1.4 pixels 112 -> 68 us); the wave then
+// draws the open (particle, tile) pairs of the others, eight lanes per pair and a
+// row of the tile at a time, and the large ones in turn, all lanes on one.  (Drawn whole by the testing lane, in the 1 M
+// dam break at 1080p: 740 us; whole by eight lanes each 314 us; with a depth test
+// per pixel ahead of the arithmetic 450 us, a chain of loads.)
+// A wave takes `per` particles: with tmax from all over the cloud (scattered), so
+// every wave gets its share of the visible ones (64 neighbours each: 427 against
+// 168 us); else neighbours, read in order.
 struct SpriteItem {
     float4 q;
     int x0, x1, y0, y1;
@@ -256,25 +271,31 @@ struct SpriteItem {
 constexpr uint32_t kSpritePairs = 256;
 
 __global__ __launch_bounds__(256) void k_depth_sprites(SpriteLaunch S, const float4 *__restrict__ pts, uint32_t n,
-                                                       uint32_t *depth, uint32_t *big,
+                                                       uint32_t nw, uint32_t per, uint32_t own, uint32_t *depth,
                                                        const uint32_t *__restrict__ tmax)
 {
     __shared__ SpriteItem item[4][64];
     __shared__ uint16_t pair[4][kSpritePairs + 64];          // lane | bit << 6
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    // a wave's particles come from all over the cloud, so every wave gets its
-    // share of the visible ones (64 neighbours each: 427 against 168 us)
-    const uint32_t nw = (n + 63u) / 64u, w = blockIdx.x * 4u + wave, i = lane * nw + w;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, tiles_x = (S.W + 7) / 8;
+    const uint32_t w = blockIdx.x * 4u + wave;
+    const uint64_t i = tmax ? (uint64_t)lane * nw + w : (uint64_t)w * per + lane;
     uint32_t open = 0;
-    if (w < nw && i < n) {
+    bool big = false;
+    if (w < nw && lane < per && i < n) {
         const float4 q = pts[i];
         SpriteBox B;
-        if (sp_box(S, q, B) && !sp_list_big(B, i, big)) {
-            open = sp_open(B, tmax ? sp_near(S, q) : -1.0f, tmax, (S.W + 7) / 8);
-            item[wave][lane] = SpriteItem{ q, B.x0, B.x1, B.y0, B.y1, B.pn };
+        if (sp_box(S, q, B)) {
+            big = sp_is_big(B);
+            if (!big) open = sp_open(B, tmax ? sp_near(S, q) : -1.0f, tmax, tiles_x);
+            if (big || sp_area(B) > own) {
+                item[wave][lane] = SpriteItem{ q, B.x0, B.x1, B.y0, B.y1, B.pn };
+            } else if (open) {
+                sp_draw(S, q, B, 0u, 1u, depth);
+                open = 0;
+            }
         }
     }
-    const uint32_t g = lane / kSpriteLanes, j = lane % kSpriteLanes;
+    const uint32_t g = lane / 8u, j = lane % 8u;
     uint32_t count = 0;
     while (true) {
         const unsigned long long m = __ballot(open != 0);
@@ -288,7 +309,7 @@ __global__ __launch_bounds__(256) void k_depth_sprites(SpriteLaunch S, const flo
             if (count <= kSpritePairs) continue;
         }
         wave_lds_sync();
-        for (uint32_t k = g; k < count; k += 64u / kSpriteLanes) {
+        for (uint32_t k = g; k < count; k += 8u) {
             const uint32_t p = pair[wave][k], bit = p >> 6;
             const SpriteItem it = item[wave][p & 63u];
             SpriteBox B;
@@ -305,34 +326,33 @@ __global__ __launch_bounds__(256) void k_depth_sprites(SpriteLaunch S, const flo
         wave_lds_sync();
         count = 0;
     }
-}
-
-// The listed sprites, one per wave at a time: the lanes take the footprint's
-// pixels in turn, an 8x8 tile at a time; tiles that cannot change are left out.
-__global__ __launch_bounds__(256) void k_depth_sprites_big(SpriteLaunch S, const float4 *__restrict__ pts,
-                                                           uint32_t *depth, const uint32_t *big,
-                                                           const uint32_t *__restrict__ tmax)
-{
-    const uint32_t lane = threadIdx.x & 63u, tiles_x = (S.W + 7) / 8;
-    const uint32_t nlist = big[0];
-    const uint32_t waves = gridDim.x * 4u;
-    for (uint32_t j = blockIdx.x * 4u + (threadIdx.x >> 6); j < nlist; j += waves) {
-        const float4 q = pts[big[1 + j]];
+    // large ones: whole rows where most tiles are open, else tile by tile
+    for (unsigned long long todo = __ballot(big); todo != 0; todo &= todo - 1ull) {
+        const SpriteItem it = item[wave][(uint32_t)__ffsll((long long)todo) - 1u];
         SpriteBox B;
-        if (!sp_box(S, q, B)) continue;
-        const float zn = tmax ? sp_near(S, q) : -1.0f;
+        sp_plane(S, B);
+        B.x0 = it.x0; B.x1 = it.x1; B.y0 = it.y0; B.y1 = it.y1;
+        B.pn = it.pn;
         const uint32_t tx0 = (uint32_t)B.x0 >> 3, ty0 = (uint32_t)B.y0 >> 3;
         const uint32_t tw = ((uint32_t)B.x1 >> 3) - tx0 + 1, T = tw * (((uint32_t)B.y1 >> 3) - ty0 + 1);
-        for (uint32_t t0 = 0; t0 < T; t0 += 64u) {
-            const uint32_t t = t0 + lane;
-            bool open = t < T;
-            if (open && tmax) open = zn < __uint_as_float(tmax[(ty0 + t / tw) * tiles_x + tx0 + t % tw]);
-            unsigned long long todo = __ballot(open);
-            while (todo) {
-                const uint32_t k = t0 + (uint32_t)__ffsll((long long)todo) - 1u;
-                todo &= todo - 1ull;
+        uint32_t nopen = T;
+        const float zn = tmax ? sp_near(S, it.q) : -1.0f;
+        auto is_open = [&](uint32_t t) { return zn < __uint_as_float(tmax[(ty0 + t / tw) * tiles_x + tx0 + t % tw]); };
+        if (tmax) {
+            nopen = 0;
+            for (uint32_t t0 = 0; t0 < T; t0 += 64u)
+                nopen += (uint32_t)__popcll(__ballot(t0 + lane < T && is_open(min(t0 + lane, T - 1))));
+        }
+        if (2 * nopen > T) {
+            sp_draw(S, it.q, B, lane, 64u, depth);
+            continue;
+        }
+        for (uint32_t t0 = 0; t0 < T && nopen != 0; t0 += 64u) {
+            unsigned long long tiles = __ballot(t0 + lane < T && is_open(min(t0 + lane, T - 1)));
+            for (; tiles != 0; tiles &= tiles - 1ull) {
+                const uint32_t k = t0 + (uint32_t)__ffsll((long long)tiles) - 1u;
                 const int px = (int)((tx0 + k % tw) * 8u + (lane & 7u)), py = (int)((ty0 + k / tw) * 8u + (lane >> 3));
-                if (px >= B.x0 && px <= B.x1 && py >= B.y0 && py <= B.y1) sp_fragment(S, q, B, px, py, depth);
+                if (px >= B.x0 && px <= B.x1 && py >= B.y0 && py <= B.y1) sp_fragment(S, it.q, B, px, py, depth);
             }
         }
     }
@@ -355,11 +375,10 @@ __global__ __launch_bounds__(256) void k_tile_max(const uint32_t *__restrict__ d
     if (lane == 0) tmax[t] = v;
 }
 
-__global__ __launch_bounds__(256) void k_clear_sprites(uint32_t *depth, uint64_t n, uint32_t *big)
+__global__ __launch_bounds__(256) void k_clear_sprites(uint32_t *depth, uint64_t n)
 {
     const uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x;
     if (i < n) depth[i] = 0x3f800000u;                             // 1.0f: the depth clear value
-    if (i == 0) big[0] = 0u;
 }
 
 // Whether sp_near bounds the fragments' depths: the rows of View orthonormal,
@@ -378,22 +397,61 @@ static bool sp_cull(const SpriteLaunch &S)
            P[10] * P[15] - P[14] * P[11] > 0.0f;
 }
 
-hipError_t launch_depth_sprites(const SpriteLaunch &S, const float4 *pts, uint32_t n, uint32_t *depth, uint32_t *big,
-                                uint32_t *tmax, hipStream_t st)
+// What the particles draw, from their bounding box: the pixels of a footprint at
+// its centre, and the footprints over a pixel of its rectangle on the screen.
+struct SpriteEstimate {
+    double area, over;
+};
+static SpriteEstimate sp_estimate(const SpriteLaunch &S, uint32_t n)
+{
+    const float *V = S.view, *P = S.proj;
+    auto clip = [&](const double x[3], double c[4]) {
+        double v[4];
+        for (int r = 0; r < 4; r++) v[r] = V[r] * x[0] + V[4 + r] * x[1] + V[8 + r] * x[2] + V[12 + r];
+        for (int r = 0; r < 4; r++) c[r] = P[r] * v[0] + P[4 + r] * v[1] + P[8 + r] * v[2] + P[12 + r];
+    };
+    const double px = (double)S.W * S.H;
+    double mid[3], c[4], lo[2] = { 1.0, 1.0 }, hi[2] = { -1.0, -1.0 };
+    bool inside = false;
+    for (int k = 0; k < 8; k++) {
+        const double x[3] = { k & 1 ? S.hi[0] : S.lo[0], k & 2 ? S.hi[1] : S.lo[1], k & 4 ? S.hi[2] : S.lo[2] };
+        clip(x, c);
+        inside = inside || !(c[3] > 0.0);
+        for (int a = 0; a < 2; a++) {
+            lo[a] = fmin(lo[a], fmax(c[a] / c[3], -1.0));
+            hi[a] = fmax(hi[a], fmin(c[a] / c[3], 1.0));
+        }
+    }
+    for (int a = 0; a < 3; a++) mid[a] = 0.5 * ((double)S.lo[a] + S.hi[a]);
+    clip(mid, c);
+    const double w = fmax(c[3], 1e-3 * fabs(S.radius)), rect = inside ? 1.0 : fmax((hi[0] - lo[0]) * (hi[1] - lo[1]) / 4.0, 0.0);
+    SpriteEstimate e;
+    e.area = fmin((double)S.radius * S.radius * fabs((double)P[0] * P[5]) * px / (w * w), px);
+    e.over = n * e.area / fmax(rect * px, 1.0);
+    return e;
+}
+
+hipError_t launch_depth_sprites(const SpriteLaunch &S, const float4 *pts, uint32_t n, uint32_t *depth, uint32_t *tmax,
+                                hipStream_t st)
 {
     const uint64_t npx = (uint64_t)S.W * S.H;
-    hipLaunchKernelGGL(k_clear_sprites, dim3((unsigned)((npx + 255) / 256)), dim3(256), 0, st, depth, npx, big);
+    hipLaunchKernelGGL(k_clear_sprites, dim3((unsigned)((npx + 255) / 256)), dim3(256), 0, st, depth, npx);
     if (!n) return hipGetLastError();
     const uint32_t T = ((S.W + 7) / 8) * ((S.H + 7) / 8);
     const uint32_t *bound = nullptr;
-    if (n >= kCullParticles && sp_cull(S)) {
+    const SpriteEstimate e = sp_estimate(S, n);
+    if (n >= kCullParticles && sp_cull(S) && e.over >= kCullOver && n * e.area >= kCullPixels) {
         const uint32_t ns = (n + kSampleStride - 1) / kSampleStride;
-        hipLaunchKernelGGL(k_sprites_sample, dim3((ns * kSpriteLanes + 255) / 256), dim3(256), 0, st, S, pts, n, depth);
+        const uint32_t lanes = ns < (1u << 24) && e.area > (ns <= kSampleLanes64 ? 32.0 : 256.0) ? 64u : 8u;
+        hipLaunchKernelGGL(k_sprites_sample, dim3((uint32_t)(((uint64_t)ns * lanes + 255) / 256)), dim3(256), 0, st, S, pts, n,
+                           lanes, depth);
         hipLaunchKernelGGL(k_tile_max, dim3((T + 3) / 4), dim3(256), 0, st, (const uint32_t *)depth, S.W, S.H, tmax, T);
         bound = tmax;
     }
-    hipLaunchKernelGGL(k_depth_sprites, dim3((n + 255) / 256), dim3(256), 0, st, S, pts, n, depth, big, bound);
-    hipLaunchKernelGGL(k_depth_sprites_big, dim3(1024), dim3(256), 0, st, S, pts, depth, (const uint32_t *)big, bound);
+    // few particles: fewer to a wave, so they fill the chip
+    const uint32_t waves = std::max((n + 63u) / 64u, std::min(n, kSpriteWaves)), per = (n + waves - 1) / waves;
+    const uint32_t nw = (n + per - 1) / per, own = bound ? 0u : std::min(per, kOwnPixels);
+    hipLaunchKernelGGL(k_depth_sprites, dim3((nw + 3) / 4), dim3(256), 0, st, S, pts, n, nw, per, own, depth, bound);
     return hipGetLastError();
 }
 
