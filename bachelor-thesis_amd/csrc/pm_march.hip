@@ -30,7 +30,7 @@ static constexpr int kListWords = (kListCap + kListPad) * 64;   // per wave
 // The finish kernel's list of a whole segment, unfiltered row by row: in the
 // 1 M dam break the filtered lists hold up to 41 candidates and a row up to
 // about 10 more.  Measured there (finish kernel): 36 slots 433 us, 48 355,
-// 52 226, 56 223, 60 231 (14 KB of LDS leave 11 waves on a CU).
+// 52 226, 56 223, 60 231 (15 KB of LDS at 56 leave ten waves on a CU).
 static constexpr int kFinCap = 56, kFinWords = (kFinCap + kListPad) * 64;
 
 struct DensList {
@@ -859,14 +859,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LIST ? 3 : 4
 //   hold 65,536 hits of four lanes; in an uneven frame (most: the fullest h/2 cell
 //   over the mean) groups gain up to four times as many, its longest hits
 //   outlasting the others.  March and finish, k_finish -> groups:
-//     3.3 per cell, most 3.3: 41,000 hits 935 -> 630 us, 55,000 970 -> 966, 62,000
-//     997 -> 1027, 86,000 1084 -> 1230, 147,000 1369 -> 1748, 829,000 4057 -> 6609;
-//     pools of 5.5 to 6.2 per cell: most 5.9, 86,000 hits 1391 -> 1230, 104,000
-//     1054 -> 1256; 9.2, 78,000 1602 -> 1237, 164,000 2019 -> 2223; 19, 164,000
-//     2384 -> 2078 and 1663 -> 2012 (nearer); 17, 164,000 3763 -> 2420, 197,000 3165
-//     -> 2500, 243,000 1694 -> 2453 (nearer).
+//     even, 3.3 per cell (most 3.3): 27,000 hits 923 -> 631 us, 64,000 966 -> 889,
+//     99,000 1047 -> 1033, 134,000 1172 -> 1258, 570,000 2519 -> 3559; 9.8 per cell
+//     (2.1): 64,000 2213 -> 2036, 81,000 2244 -> 2286, 134,000 2782 -> 3164;
+//     clustered pools of 5.5 to 6.2 per cell, few hits and (near) many: most 5.9,
+//     101,000 1371 -> 1097 and (112,000) 1060 -> 1125; 9.2, 134,000 1690 -> 1437 and
+//     (149,000) 1255 -> 1329; 17, 192,000 4103 -> 2618 and (199,000) 1645 -> 1947.
 //   (By the image's tiles alone, up to 16,384, groups took images full of hits too:
-//   the 100,000-particle pool 4889 us at 1280x800, k_finish 2348.)
+//   the 100,000-particle pool at 1280x800 4889 us, k_finish 2348.)
+//   Without lists the LDS holds 16 waves a CU (sized for lists, ten: 176,000 hits of
+//   the even frame 1748 us, now 1462).
 //   The march has counted the hits by then, so both kernels are launched where
 //   the tiles could hold more, and one of them ends at once.
 static constexpr uint32_t kGroupTiles = 800, kGroupTilesDense = 16384, kGroupHits = 65536;
@@ -905,7 +907,7 @@ template <bool LIST>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_finish_groups(MarchLaunch L, uint32_t upto)
 {
     if (upto != 0 && marched_hits(L) > upto) return;
-    __shared__ uint32_t lds[kFinWords];
+    __shared__ uint32_t lds[LIST ? kFinWords : kListWords];
     const uint32_t lane = threadIdx.x;
     uint32_t *lst = lds + lane;
     const pm_settings &s = L.s;
