@@ -142,7 +142,7 @@ __device__ __forceinline__ int32_t pm_key(float x, float inv_h)
 
 // sqrtf(x) for the kernel weight, x >= 0: x rsq(x), one ulp or two off, and one
 // Newton step whose residual is exact.  Equal to sqrtf for every float from 2^-96
-// to 2^64 (all of them compared on gfx950), six instructions instead of nine
+// to 2^64 (all of them compared by tests/test_gpu_sqrt.py), six instructions instead of nine
 // (the hardware root and the residuals of both neighbours).  The march's kernels
 // issue VALU instructions 75 to 97 % of the time, half of them for weights.
 // Below 2^-96 the residual may round, and below 2^-126 and at 0 the factor is
