@@ -91,7 +91,6 @@ struct BatchLaunch {
 };
 hipError_t launch_bound_grid(const GridDev &g, float iso, bool quarter_only, uint64_t *out, hipStream_t st);
 hipError_t launch_march_batch(const BatchLaunch &B, hipStream_t st);
-hipError_t launch_zero_u32(uint32_t *p, uint32_t n, hipStream_t st);
 hipError_t launch_zero_u64(unsigned long long *p, uint32_t n, hipStream_t st);
 // counters[0..n) = 0 except counters[C_RAYS] = rays0 (rays answered without marching)
 hipError_t launch_init_counters(unsigned long long *p, uint32_t n, unsigned long long rays0, hipStream_t st);

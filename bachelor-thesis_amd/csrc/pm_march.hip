@@ -622,11 +622,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
     if (any) flush_counts(L.counters, cn);
 }
 
-__global__ void k_zero_u32(uint32_t *p, int n)
-{
-    for (int i = (int)threadIdx.x; i < n; i += (int)blockDim.x) p[i] = 0u;
-}
-
 // PerPixel_Isotropic (RayMarcher.cpp:256-344): start on the depth-buffer
 // surface, fixed step vector, MaxSteps samples, first sample with rho >= iso,
 // normal = normalize(sum gradW) (or central differences on request).
@@ -1023,12 +1018,6 @@ hipError_t launch_march_batch(const BatchLaunch &B, hipStream_t st)
 __global__ void k_zero_u64(unsigned long long *p, uint32_t n)
 {
     for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) p[i] = 0ull;
-}
-
-hipError_t launch_zero_u32(uint32_t *p, uint32_t n, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, st, p, (int)n);
-    return hipGetLastError();
 }
 
 hipError_t launch_zero_u64(unsigned long long *p, uint32_t n, hipStream_t st)

@@ -72,35 +72,10 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// C[64 x 16*NT] = A[64 x 32*KT] * B[16*NT x 32*KT]^T, bf16 in, fp32 out.
-// A rows (stride lda) and B rows (stride ldb) hold K contiguously.
-// MFMA 16x16x32 operand layout: lane l reads row (l % 16) of its A tile and of
-// its B tile, K slots 8*(l/16) .. +8; the result element acc[mi][ni][r] is
-// C[16 mi + 4 (l/16) + r][16 ni + l % 16].  A and B use the same K slots, so
-// the sum does not depend on the order the hardware assigns to them.
-template <int NT, int KT>
-__device__ __forceinline__ void wave_gemm_abt(const uint16_t *A, int lda, const uint16_t *B, int ldb,
-                                              pm_f32x4 (&acc)[4][NT])
-{
-    const int l = threadIdx.x & 63, row = l & 15, kb = l >> 4;
-#pragma unroll
-    for (int mi = 0; mi < 4; mi++)
-#pragma unroll
-        for (int ni = 0; ni < NT; ni++) acc[mi][ni] = pm_f32x4{ 0.f, 0.f, 0.f, 0.f };
-#pragma unroll
-    for (int kk = 0; kk < KT; kk++) {
-        pm_bf16x8 a[4], b[NT];
-#pragma unroll
-        for (int mi = 0; mi < 4; mi++) a[mi] = load_bf16x8(A + (16 * mi + row) * lda + 32 * kk + 8 * kb);
-#pragma unroll
-        for (int ni = 0; ni < NT; ni++) b[ni] = load_bf16x8(B + (16 * ni + row) * ldb + 32 * kk + 8 * kb);
-#pragma unroll
-        for (int mi = 0; mi < 4; mi++)
-#pragma unroll
-            for (int ni = 0; ni < NT; ni++)
-                acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mi], b[ni], acc[mi][ni], 0, 0, 0);
-    }
-}
+// MFMA 16x16x32 operand layout (C = A B^T, K contiguous in the rows of both): lane
+// l reads row (l % 16) of its A tile and of its B tile, K slots 8*(l/16) .. +8; the
+// result element acc[r] is C[4 (l/16) + r][l % 16].  A and B use the same K slots,
+// so the sum does not depend on the order the hardware assigns to them.
 
 // Forward pass of the wave's 64 samples, streaming one 16 x 16 output tile at a
 // time so that only a few accumulators are live (the caller keeps its own ray
