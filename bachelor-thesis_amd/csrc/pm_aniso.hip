@@ -1258,11 +1258,10 @@ __global__ void k_zero_band(uint32_t *p)
 hipError_t launch_march_aniso(const MarchLaunch &L, hipStream_t st)
 {
     const uint32_t tiles = ((L.W + 7) / 8) * ((L.H + 7) / 8);
-    // one ray per lane to its end (neighbouring rays of a tile sample
-    // neighbouring points, so the wave's gathers share cache lines): over the
-    // active tiles after the tile pre-pass (schedule 0), or over all tiles (no
-    // tile buffer); or (schedule 1, configured march) persistent waves with
-    // ray refill and the hit-list finish
+    // schedule 0: march, finish and normals (or the reference march) over the
+    // active tiles of the tile pre-pass.  Else the forms it is checked against:
+    // persistent waves with ray refill and the hit-list finish (configured march,
+    // schedule 1), or one ray per lane to its end over all tiles
     if (L.s.schedule == 0 && L.tile_buf) {
         hipError_t e = launch_tile_prepass(L, st);
         if (e != hipSuccess) return e;

@@ -746,10 +746,10 @@ static int march_launch(pm_ctx *c, int32_t frame, const pm_settings *s, const fl
         L.hit_rec = (uint4 *)c->d_hits.p;
     }
     if (s->anisotropic) L.an = aniso_params(f, s);
-    // tile pre-pass (active-tile list, bulk miss writes) for the persistent
+    // tile pre-pass (active-tile list, bulk miss writes) for the product
     // schedule, the anisotropic march and the reference march
-    const bool persistent = s->schedule == 0 || (!s->anisotropic && s->learned);
-    if (persistent) {
+    const bool tiled = s->schedule == 0 || (!s->anisotropic && s->learned);
+    if (tiled) {
         uint64_t tiles = (uint64_t)((W + 7) / 8) * ((H + 7) / 8);
         if (na) {
             L.tile_buf = na->tiles;

@@ -68,9 +68,9 @@ struct MarchLaunch {
     // length at T, masks); null = every tile
     uint32_t *tile_buf;
     float inv_step;            // 1 / s.step (bound skip)
-    // per pixel: the hit handed from the march to k_finish (1 | fp64 << 1,
+    // per pixel: the hit handed from the march to the finish (1 | bracket << 1,
     // lo, hi, 0), zeros for a miss; written for every pixel of a marched tile
-    // (the anisotropic march: its list of hits)
+    // (the anisotropic march's schedule 1: its list of hits)
     uint4 *hit_rec;
     AnisoDev an;               // s.anisotropic
 };
@@ -136,7 +136,8 @@ hipError_t launch_march(const MarchLaunch &L, hipStream_t st);
 // GridDev::group_hits of a frame of n particles in `cells` march cells, at most
 // `most` in one.
 uint32_t group_hits(uint64_t n, uint32_t cells, uint32_t most);
-// The anisotropic march (configured or reference mode), one kernel.
+// The anisotropic march: march, finish and normals kernels over the active tiles,
+// or the reference march of a tile; schedule 1: its own forms.
 hipError_t launch_march_aniso(const MarchLaunch &L, hipStream_t st);
 hipError_t launch_density_aniso(const GridDev &g, const AnParF &a, const float *q, uint32_t nq, int compensated,
                                 float *rho, hipStream_t st);

@@ -9,7 +9,7 @@
 namespace pm {
 
 // PH_MARCH: the next lattice sample; PH_BISECT: FP32 bisection steps (the
-// anisotropic march and the one-ray-per-lane schedule); PH_PROPOSE: waiting for
+// anisotropic march's schedule 1); PH_PROPOSE: waiting for
 // a step proposal of the learned march (taken by the whole wave at once).
 enum Phase : int {
     PH_MARCH = 0, PH_BISECT = 1, PH_DONE = 5, PH_PROPOSE = 6

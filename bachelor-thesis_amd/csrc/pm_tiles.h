@@ -97,9 +97,8 @@ __device__ __forceinline__ void ray_finish(const MarchLaunch &L, RayState &r, fl
     }
 }
 
-// One march sample of this ray and the transition it implies.  Dens(q, cand) is the FP32 density.  HOPS: skips per step before
-// a lane idles -- 16 in the single-view march, whose end is spent on few long
-// rays with idle lanes beside them; 8 in the batch, whose lanes stay busy.
+// One march sample of this ray and the transition it implies.  Dens(q, cand) is
+// the FP32 density.  HOPS: skips per step before a lane idles.
 template <bool INSTR, int HOPS, class Dens>
 __device__ __forceinline__ void ray_step(const MarchLaunch &L, RayState &r, Dens dens, Counts &cn)
 {
@@ -110,8 +109,8 @@ __device__ __forceinline__ void ray_step(const MarchLaunch &L, RayState &r, Dens
     ray_finish<INSTR>(L, r, rho, cand, qx, qy, qz, cn);
 }
 
-// ---- lane groups: the end of a persistent launch ----
-// Once no tile is left, a wave's remaining rays are spread over its idle lanes:
+// ---- lane groups ----
+// As a tile's rays end, its remaining ones are spread over the wave's idle lanes:
 // G lanes (a power of two) per ray, every lane of a group holding the same
 // RayState.  A step then evaluates the G lattice samples k .. k+G-1 at once and
 // takes the first at or above iso.  Each sample is computed as the one-lane

@@ -25,7 +25,7 @@ same march and forms.
 
 --workload batch: 64 views (W ~ U{256..1920}, H ~ U{256..1080}, seeded orbit
 cameras) over 16 consecutive frames of the 1M dam break (1 % displacement per
-frame), all 1,024 view-frames in one persistent launch replayed from a
+frame), all 1,024 view-frames in one launch replayed from a
 hipGraph; one step = one replay of the whole batch.
 
 --workload aniso_dam_1080p: the anisotropic march (PerPixel_Anisotropic, the
@@ -659,7 +659,7 @@ def bench_smooth(args):
 
 
 def bench_batch(args):
-    """64 views x 16 frames in one persistent launch from a hipGraph."""
+    """64 views x 16 frames in one launch from a hipGraph."""
     import pmarch
     from pmarch import scenes, train
 
@@ -719,7 +719,7 @@ def bench_batch(args):
         "warmup": args.warmup, "ms_per_step": round(f["ms"], 3), "higher_is_better": True, "scaling": "weak",
         "vs_baseline": None, "dtype": "f32", "data": "synthetic",
         "config": {"workload": "batch: 64 views (256..1920 x 256..1080) x 16 frames of the 1,024,000-particle dam "
-                               "break, one persistent launch replayed from a hipGraph", "views": 64, "frames": 16,
+                               "break, one launch replayed from a hipGraph", "views": 64, "frames": 16,
                    "rays_per_step": rays, "path": use},
         "roofline": {"bound": "valu", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic_for(use, "batch"),

@@ -237,14 +237,13 @@ int pm_wait(pm_ctx *ctx);
 int pm_download(pm_ctx *ctx, float *positions, float *normals, float *t);
 int pm_get_stats(pm_ctx *ctx, pm_stats *out);
 
-/* ---- batched views x frames in one persistent launch ----
+/* ---- batched views x frames in one launch ----
  * The reference renders one view per RayMarcher::Start, farmed out pixel by
  * pixel to its ThreadPool (ThreadPool.cpp:5-55) and re-started once per
  * second (AdvancedRenderer.cpp:257-298); the batch form marches many views of
- * uneven size over many resident frames in one persistent kernel.  Waves take
- * runs of 8x8 tiles of one view from a single queue ordered largest view
- * first; every view's images equal those of pm_march_async for the same
- * frame, settings and camera. */
+ * uneven size over many resident frames in one march and one finish kernel, a
+ * wave per 8x8 tile, the largest view first; every view's images equal those of
+ * pm_march_async for the same frame, settings and camera. */
 typedef struct pm_view {
     int32_t frame;      /* a frame set by pm_set_frame */
     uint32_t width, height;
@@ -252,8 +251,8 @@ typedef struct pm_view {
     float cam[3];
 } pm_view;
 /* Fixes the batch (configured march only): allocates the device images of
- * all views, uploads the tile queue and, with use_graph != 0, captures the
- * launch (counter fills + the persistent kernel) in a hipGraph. */
+ * all views, uploads the list of tiles and, with use_graph != 0, captures the
+ * launch (counter fill, march, finish) in a hipGraph. */
 int pm_batch_set(pm_ctx *ctx, const pm_settings *s, const pm_view *views, uint32_t n_views, int use_graph);
 /* Enqueues one run of the batch (graph replay or direct launch) and returns;
  * complete it with pm_query / pm_wait, which also fill pm_get_stats. */
