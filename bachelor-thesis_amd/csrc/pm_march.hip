@@ -851,9 +851,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LIST ? 3 : 4
 //   256x192 (768 tiles) dam 131 -> 86, full lattice 94 -> 71; 288x224 (1008) dam
 //   134 -> 85 but full lattice 96 -> 110, 360x360 (2025) 115 -> 195;
 // - a dense frame, where one hit's walks take milliseconds: the chip's 4,096 waves
-//   hold 65,536 hits of four lanes; in an uneven frame (most: the fullest h/2 cell
-//   over the mean) groups gain up to four times as many, its longest hits
-//   outlasting the others.  March and finish, k_finish -> groups:
+//   hold 65,536 hits of four lanes, and a quarter more still gains; in an uneven
+//   frame (most: the fullest h/2 cell over the mean) up to four times as many do,
+//   its longest hits outlasting the others.  March and finish, k_finish -> groups:
 //     even, 3.3 per cell (most 3.3): 27,000 hits 923 -> 631 us, 64,000 966 -> 889,
 //     99,000 1047 -> 1033, 134,000 1172 -> 1258, 570,000 2519 -> 3559; 9.8 per cell
 //     (2.1): 64,000 2213 -> 2036, 81,000 2244 -> 2286, 134,000 2782 -> 3164;
@@ -866,7 +866,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(LIST ? 3 : 4
 //   the even frame 1748 us, now 1462).
 //   The march has counted the hits by then, so both kernels are launched where
 //   the tiles could hold more, and one of them ends at once.
-static constexpr uint32_t kGroupTiles = 800, kGroupTilesDense = 16384, kGroupHits = 65536;
+static constexpr uint32_t kGroupTiles = 800, kGroupTilesDense = 16384, kGroupHits = 81920;
 
 uint32_t group_hits(uint64_t n, uint32_t cells, uint32_t most)
 {

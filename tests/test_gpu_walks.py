@@ -217,12 +217,12 @@ def test_candidates_of_wide_offsets(marcher, tiles, eps):
     assert got["hits"] > 1000
 
 
-@pytest.mark.parametrize("extra,dist,groups", [(0, 2.6, 1), (0, 1.5, 1), (0, 1.3, 0), (0, 0.7, 0), (60, 1.1, 1), (60, 0.7, 0)])
+@pytest.mark.parametrize("extra,dist,groups", [(0, 2.6, 1), (0, 1.5, 1), (0, 1.1, 0), (0, 0.7, 0), (40, 1.1, 1), (40, 0.7, 0)])
 @pytest.mark.parametrize("learned", [0, 1])
 def test_group_finish_by_hits(marcher, extra, dist, groups, learned):
     """The finish of a dense frame in an image of 4,800 tiles: four lanes per hit
-    up to 65,536 (1 + (most / (8 mean))^2) hits, at most four times 65,536, most the
-    fullest h/2 cell's particles (66,560 here, and 237,000 with `extra` in one cell),
+    up to 81,920 (1 + (most / (8 mean))^2) hits, at most four times 81,920, most the
+    fullest h/2 cell's particles (83,200 here, and 185,000 with `extra` in one cell),
     a lane per hit beyond, chosen on the device; images and counters are those of the
     one-ray-per-lane schedule."""
     from pmarch import train
@@ -248,7 +248,7 @@ def test_group_finish_by_hits(marcher, extra, dist, groups, learned):
             assert np.array_equal(a, b)
         for k in ("rays", "rays_in_aabb", "hits") + (() if learned else ("samples", "march_samples")):
             assert got[3][k] == plain[3][k], k
-        most = 237000 if extra else 66560
+        most = 185000 if extra else 83200
         assert (got[3]["hits"] < 0.97 * most if groups else got[3]["hits"] > 1.03 * most) and got[3]["hits"] > 15000
 
 
