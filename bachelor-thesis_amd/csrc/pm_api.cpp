@@ -858,11 +858,13 @@ static int complete(pm_ctx *c)
     // as misses are not counted on the device, so a march with the pre-pass
     // reports all W*H rays
     unsigned long long sum[C_COUNT] = {};
-    for (int k = 0; k < kCtrSlots; k++)
-        for (int i = 0; i < C_COUNT; i++) sum[i] += c->h_counters[k * kCtrStride + i];
+    for (int k = 0; k < kCtrSlots; k++) {
+        const unsigned long long *v = c->h_counters + k * kCtrStride;
+        for (int i = 0; i < C_COUNT; i++) sum[i] += v[i];
+        S.rays_in_aabb += v[C_BOX_HITS] & 0xffffffffu;
+        S.hits += v[C_BOX_HITS] >> 32;
+    }
     S.rays = c->prepass ? c->npx : sum[C_RAYS];
-    S.rays_in_aabb = sum[C_IN_AABB];
-    S.hits = sum[C_HITS];
     S.samples = sum[C_SAMPLES];
     S.cand = sum[C_CAND];
     S.march_samples = sum[C_MARCH_SAMPLES];

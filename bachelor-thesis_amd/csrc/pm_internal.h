@@ -11,9 +11,11 @@
 namespace pm {
 
 // Per-launch counters (u64 each), accumulated by the march kernels, in the
-// order of pm_stats.
+// order of pm_stats.  C_BOX_HITS: the rays in the box and 2^32 times the hits, one
+// atomic for both (a march of 800x600, a few samples per ray: 134 us, with an atomic
+// for each 168; a slot's share of the largest batch, 2^33 rays, is 2^30).
 enum Counter {
-    C_RAYS = 0, C_IN_AABB, C_HITS, C_SAMPLES, C_CAND, C_MARCH_SAMPLES, C_MLP, C_MARCH_CAND, C_CERT, C_CERT_SKIP,
+    C_RAYS = 0, C_BOX_HITS, C_SAMPLES, C_CAND, C_MARCH_SAMPLES, C_MLP, C_MARCH_CAND, C_CERT, C_CERT_SKIP,
     C_CAND_STENCIL, C_CAND27, C_COUNT
 };
 // The counters live in kCtrSlots copies, one per XCD (a workgroup adds to

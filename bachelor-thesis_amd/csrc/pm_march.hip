@@ -791,10 +791,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
 // The hits of the launch, counted by its march.
 __device__ __forceinline__ uint32_t marched_hits(const MarchLaunch &L)
 {
-    unsigned long long n = 0;
+    uint32_t n = 0;                               // at most 2^30 pixels
 #pragma unroll
-    for (int k = 0; k < kCtrSlots; k++) n += L.counters[k * kCtrStride + C_HITS];
-    return (uint32_t)n;                           // at most 2^30 pixels
+    for (int k = 0; k < kCtrSlots; k++) n += (uint32_t)(L.counters[k * kCtrStride + C_BOX_HITS] >> 32);
+    return n;
 }
 
 // A wave per active tile, of the view or of the batch.

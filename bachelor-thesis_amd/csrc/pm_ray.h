@@ -130,8 +130,7 @@ __device__ __forceinline__ void flush_counters(unsigned long long *ctr, uint32_t
     if ((threadIdx.x & 63) == 0) {
         unsigned long long *p = ctr_slot(ctr);
         if (r) atomicAdd(&p[C_RAYS], r);
-        if (a) atomicAdd(&p[C_IN_AABB], a);
-        if (h) atomicAdd(&p[C_HITS], h);
+        if (a | h) atomicAdd(&p[C_BOX_HITS], a | h << 32);
         if (s) atomicAdd(&p[C_SAMPLES], s);
         if (c) atomicAdd(&p[C_CAND], c);
         if (m) atomicAdd(&p[C_MARCH_SAMPLES], m);
@@ -150,7 +149,7 @@ struct Counts {
 __device__ __forceinline__ void flush_counts(unsigned long long *ctr, const Counts &cn)
 {
     const unsigned long long v[C_COUNT] = {
-        wave_sum(cn.rays), wave_sum(cn.in_aabb), wave_sum(cn.hits), wave_sum(cn.samples), wave_sum(cn.cand),
+        wave_sum(cn.rays), wave_sum(cn.in_aabb) | wave_sum(cn.hits) << 32, wave_sum(cn.samples), wave_sum(cn.cand),
         wave_sum(cn.march), wave_sum(cn.mlp), wave_sum(cn.mcand), wave_sum(cn.cert), wave_sum(cn.cskip),
         wave_sum(cn.cst), wave_sum(cn.c27) };
     if ((threadIdx.x & 63) == 0) {
