@@ -842,7 +842,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) void
             group_step<false>(L, r, G, dens, cn);
         }
     }
-    if (any) flush_counters(L.counters, cn.rays, cn.in_aabb, cn.hits, cn.samples, cn.cand, cn.march);
+    if (any) flush_counters(L.counters, cn.rays, box_rays(cn), all_hits(cn), cn.samples, cn.cand, cn.march);
 }
 
 // The hits of the same tiles: bisection (the last step in FP64), point, and the

@@ -146,12 +146,20 @@ struct Counts {
     unsigned long long cand = 0, mcand = 0, cst = 0, c27 = 0;
 };
 
+// A hit of the marches over tiles, counted in the upper half of in_aabb: the
+// learned march has no register left for it (a 1283x721 view 479 -> 491 us with a
+// count of its own).  A lane takes at most 2^11 tiles (the largest batch's 2^27
+// over 65,536 waves), and of each one ray and a hit per width of its groups, seven.
+static constexpr uint32_t kTileHit = 1u << 16;
+__device__ __forceinline__ uint32_t box_rays(const Counts &cn) { return cn.in_aabb & (kTileHit - 1u); }
+__device__ __forceinline__ uint32_t all_hits(const Counts &cn) { return cn.hits + cn.in_aabb / kTileHit; }
+
 __device__ __forceinline__ void flush_counts(unsigned long long *ctr, const Counts &cn)
 {
     const unsigned long long v[C_COUNT] = {
-        wave_sum(cn.rays), wave_sum(cn.in_aabb) | wave_sum(cn.hits) << 32, wave_sum(cn.samples), wave_sum(cn.cand),
-        wave_sum(cn.march), wave_sum(cn.mlp), wave_sum(cn.mcand), wave_sum(cn.cert), wave_sum(cn.cskip),
-        wave_sum(cn.cst), wave_sum(cn.c27) };
+        wave_sum(cn.rays), wave_sum(box_rays(cn) | (unsigned long long)all_hits(cn) << 32),
+        wave_sum(cn.samples), wave_sum(cn.cand), wave_sum(cn.march), wave_sum(cn.mlp), wave_sum(cn.mcand),
+        wave_sum(cn.cert), wave_sum(cn.cskip), wave_sum(cn.cst), wave_sum(cn.c27) };
     if ((threadIdx.x & 63) == 0) {
         unsigned long long *p = ctr_slot(ctr);
 #pragma unroll

@@ -88,7 +88,7 @@ __device__ __forceinline__ void ray_finish(const MarchLaunch &L, RayState &r, fl
     count_sample<INSTR>(L.g, qx, qy, qz, cand, true, cn);
     if (rho >= L.s.iso) {
         emit_hit(L, r);
-        cn.hits++;
+        cn.in_aabb += kTileHit;
     } else if (r.lrn && rho < L.mlp_gate_rho) {
         r.rho = rho;
         r.phase = PH_PROPOSE;
@@ -211,7 +211,7 @@ __device__ __forceinline__ void group_finish(const MarchLaunch &L, RayState &r, 
     if (cross) {
         r.k += jc;
         emit_hit(L, r, j == 0);
-        if (j == 0) cn.hits++;
+        if (j == 0) cn.in_aabb += kTileHit;
     } else {
         r.k += G;
     }
