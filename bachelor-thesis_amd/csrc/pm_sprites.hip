@@ -18,8 +18,8 @@
 // early depth test.
 //
 // At 1080p the dam break's 1M sprites put ~600 fragments on each drawn pixel,
-// nearly all behind others.  One particle of every kSampleStride, spread over
-// the cloud, is drawn first; the largest depth of every 8x8 pixel tile of that
+// nearly all behind others.  Where that pays (kCullParticles), one particle of
+// every kSampleStride, spread over the cloud, is drawn first; the largest depth of every 8x8 pixel tile of that
 // image then bounds what a later sprite can still change, and a sprite whose
 // nearest possible depth is not below it in any tile of its footprint is left
 // out (sp_near).  The image is the same minimum.  1080p dam break: 952 us (one
@@ -257,9 +257,10 @@ __global__ __launch_bounds__(256) void k_sprites_sample(SpriteLaunch S, const fl
 // pixels itself (up to as many as the wave has particles: a lane each then beats
 // eight lanes for one after the other; 1 M of 1.4 pixels 112 -> 68 us); the wave then
 // draws the open (particle, tile) pairs of the others, eight lanes per pair and a
-// row of the tile at a time, and the large ones in turn, all lanes on one.  (Drawn whole by the testing lane, in the 1 M
-// dam break at 1080p: 740 us; whole by eight lanes each 314 us; with a depth test
-// per pixel ahead of the arithmetic 450 us, a chain of loads.)
+// row of the tile at a time, and the large ones in turn, all lanes on one.  (1 M
+// dam break at 1080p, 168 us: drawn whole by the testing lane 740 us; whole by eight
+// lanes each 314; with a depth test per pixel ahead of the arithmetic 450, a chain
+// of loads.)
 // A wave takes `per` particles: with tmax from all over the cloud (scattered), so
 // every wave gets its share of the visible ones (64 neighbours each: 427 against
 // 168 us); else neighbours, read in order.
