@@ -287,7 +287,7 @@ def bench_aniso(args):
                    "step": scene.step, "iso": 1.0, "path": "anisotropic"},
         "roofline": {"bound": "valu", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic_for("anisotropic", args.workload),
-                     "limiter": "VALU issue of the per-lane WPCA and density walks (lane utilisation 42 %); "
+                     "limiter": "VALU issue of the per-lane WPCA and density walks (lane utilisation 72 to 78 %); "
                                 "achieved/frac are the walks' algorithmic bytes, read mostly from L1/L2"},
         "kernel_ms": round(kms, 4),
         "alg_bytes_per_launch": B,
@@ -470,10 +470,11 @@ def bench_autoplay(args):
 
 
 def sprite_pixel_tests(xyz, cam, R: float) -> int:
-    """Pixel centres k_depth_sprites tests in one pass: per particle the pixels
+    """Pixel centres in the sprites' boxes of one pass: per particle the pixels
     of its projected quad's bounding box, clamped to the image (particles with
-    a corner behind the eye draw nothing) -- the kernel's own loop bounds,
-    evaluated in FP32 in the kernel's operation order."""
+    a corner behind the eye draw nothing) -- the kernel's own bounds, evaluated
+    in FP32 in the kernel's operation order.  k_depth_sprites leaves out those
+    behind its sample's farthest depth in their tile."""
     f = np.float32
     V = np.asarray(cam.view, f).reshape(16)
     P = np.asarray(cam.proj, f).reshape(16)
@@ -559,8 +560,8 @@ def bench_sprites(args):
                    "particles": sc.n, "width": cam.width, "height": cam.height, "path": "sprites"},
         "roofline": {"bound": "valu", "achieved": round(tflops, 3), "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(tflops / FP32_PEAK_TFLOPS, 4), "traffic": None,
-                     "flops": f"{SPRITE_FLOP_PER_TEST} per pixel test x {tests} tests per pass (drawn fragments' "
-                              "extra work not counted)"},
+                     "flops": f"{SPRITE_FLOP_PER_TEST} x {tests} pixels in the sprites' boxes per pass, tested or hidden "
+                              "behind a sampled depth (drawn fragments' extra work not counted)"},
         "pixel_tests_per_pass": tests,
         "pixels_drawn": int((img < 1.0).sum()),
         "timing": "host clock over back-to-back passes on the context stream (fill + sprites kernels)",
@@ -850,8 +851,8 @@ def main():
                      "frac_of_copy": round(B / kt / 1e9 / copy, 4),
                      "hbm_gbps": round(traffic / kt / 1e9, 2) if traffic else None,
                      "hbm_frac": round(traffic / kt / 1e9 / HBM_PEAK_GBS, 4) if traffic else None,
-                     "limiter": "VALU issue of divergent per-lane stencil walks (SIMD VALU busy ~82 %, lane "
-                                "utilisation 63 % in the march); achieved/frac are the algorithmic bytes of the HBM "
+                     "limiter": "VALU issue of divergent per-lane stencil walks (SIMD VALU busy ~87 %, lane "
+                                "utilisation 62 % in the march); achieved/frac are the algorithmic bytes of the HBM "
                                 "roofline, read mostly from L1/L2 -- the HBM traffic itself is hbm_gbps"},
         "kernel_ms": round(f["kernel_ms"], 4),
         "alg_bytes_per_launch": B,
